@@ -138,8 +138,10 @@ struct fgt_solver {
     DBuf d_dir_tgt, d_dir_lev, d_dir_off, d_dir_src, d_dir_code, d_dir_flags;
     // 3-D fast path: STEP 4 folded into STEP 5 for leaves below the cutoff level
     bool fast3d = false;
-    DBuf d_s5_tasks;   // fgt::PotTask list of the 3-D STEP 5 kernel
+    DBuf d_s5_tasks;   // fgt::PotTask list of the reduced-precision STEP 5 kernel
     int n_s5 = 0, n_s5_sib = 0;   // tasks, of which the first n_s5_sib are sibling tasks
+    DBuf d_s5_sym;     // fgt::SymTask list of the FP64 STEP 5 kernel
+    int n_s5_fam = 0, n_s5_own = 0;   // families first, then single leaves
     DBuf d_p2pwS, d_fz_lev, d_fz_slot, d_fz_kids, d_fz_ksg;          // fused STEP 1+2 parents
     DBuf d_s1_box, d_s1_lev, d_s1_slot;                              // standalone STEP 1 leaves
     DBuf d_mp_slot, d_mp_first, d_mp_count, d_mp_child, d_mp_sign, d_mp_acc;  // merges of non-leaf children
@@ -152,6 +154,7 @@ struct fgt_solver {
     // per shape class)
     struct HostLists {
         std::vector<fgt::PotTask> s5;
+        std::vector<fgt::SymTask> s5_sym;
         std::vector<int> pcs_parent, pcs_child, pcs_sign;
         std::vector<int> fz_lev, fz_slot, fz_kids, fz_ksg, s1_box, s1_lev, s1_slot;
         std::vector<int> mp_slot, mp_first, mp_count, mp_child, mp_sign, mp_acc;
@@ -517,14 +520,23 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
         // the same x split sign form one task (shared x contraction).  Those
         // tasks come first (more work per task), then one task per leaf
         // evaluating its own expansion.
+        // The FP64 kernel takes all the leaf children of a parent in one task.
         std::vector<fgt::PotTask> fam, own;
+        std::vector<fgt::SymTask> sfam, sown;
         std::unordered_map<long long, int> fam_of;
+        std::unordered_map<int, int> sfam_of;
         for (size_t i = 0; i < P.leaf_box.size(); ++i) {
             const int b = P.leaf_box[i], l = P.leaf_lev[i];
             if (l > P.nlevstart) {
                 const int par = T.parent[b];
                 int sg[3];
                 for (int a = 0; a < 3; ++a) sg[a] = T.centers[3 * b + a] - T.centers[3 * par + a] < 0 ? 1 : 0;
+                auto is = sfam_of.find(par);
+                if (is == sfam_of.end()) {
+                    is = sfam_of.emplace(par, (int)sfam.size()).first;
+                    sfam.push_back({P.slot_of_box[par], l, {-1, -1, -1, -1, -1, -1, -1, -1}});
+                }
+                sfam[is->second].box[sg[0] | sg[1] << 1 | sg[2] << 2] = b;
                 const long long key = 2LL * par + sg[0];
                 auto it = fam_of.find(key);
                 if (it == fam_of.end() || fam[it->second].box[3] >= 0) {
@@ -557,8 +569,14 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
                 for (int c = 0; c < 4; ++c) pt.box[c] = -1, pt.code[c] = 0;
                 pt.box[0] = b;
                 own.push_back(pt);
+                sown.push_back({P.leaf_slot[i], l, {b, -1, -1, -1, -1, -1, -1, -1}});
             }
         }
+        S.n_s5_fam = (int)sfam.size();
+        S.n_s5_own = (int)sown.size();
+        sfam.insert(sfam.end(), sown.begin(), sown.end());
+        S.d_s5_sym.upload(sfam);
+        S.h.s5_sym = sfam;
         S.n_s5_sib = (int)fam.size();
         fam.insert(fam.end(), own.begin(), own.end());
         S.n_s5 = (int)fam.size();
@@ -872,18 +890,16 @@ void launch_direct_comps(const fgt::Geom& g, const fgt::DevTables& t, int ntask,
     }
 }
 
-// STEP 5 (3-D task kernel) for a list of output components: the one-leaf
-// tasks of components that share their x and y table kinds run once per
-// group (g3d_pw2pgh, bfgt_pwrouts.f:906-1000, likewise forms each pair of x
-// and y partial sums once for all the z kinds), the sibling tasks once per
-// component.
-void launch_pw2pot_comps(const fgt::Geom& g, const fgt::DevTables& t, int ntask, int nsib, const fgt::PotTask* tasks,
-                         const double2* expn, const std::vector<Comp>& comps, hipStream_t st) {
+// STEP 5 (3-D task kernels) for a list of output components: those that
+// share their x and y table kinds go in one pass (g3d_pw2pgh,
+// bfgt_pwrouts.f:906-1000, likewise forms each pair of x and y partial sums
+// once for all the z kinds).
+void launch_pw2pot_comps(const fgt::Geom& g, const fgt::DevTables& t, const fgt::Step5Lists& l, const double2* expn,
+                         const std::vector<Comp>& comps, hipStream_t st) {
     std::vector<fgt::ZOut> groups;
     std::vector<fgt::Kinds> gkd;
     group_comps(comps, groups, gkd);
-    for (size_t k = 0; k < groups.size(); ++k)
-        fgt::launch_pw2pot_tasks_z(g, t, ntask, nsib, tasks, expn, gkd[k], groups[k], st);
+    for (size_t k = 0; k < groups.size(); ++k) fgt::launch_pw2pot_tasks(g, t, l, expn, gkd[k], groups[k], st);
 }
 
 std::vector<Comp> components(fgt_solver& S, double* pot_override = nullptr) {
@@ -1021,7 +1037,8 @@ void execute(fgt_solver& S, hipStream_t st, bool timed, bool fork_near = false,
             mark(7);   // STEP 5 starts here (after the wait for STEP 6)
         }
         if (S.fast3d)
-            launch_pw2pot_comps(g, t, S.n_s5, S.n_s5_sib, S.d_s5_tasks.as<fgt::PotTask>(), ex, comps, st);
+            launch_pw2pot_comps(g, t, {S.n_s5, S.n_s5_sib, S.d_s5_tasks.as<fgt::PotTask>(), nullptr, S.n_s5_fam,
+                                       S.n_s5_own, S.d_s5_sym.as<fgt::SymTask>(), nullptr}, ex, comps, st);
         else
             for (const Comp& c : comps)
                 fgt::launch_pw2pot(g, t, (int)P.leaf_box.size(), S.d_leaf_box.as<int>(), S.d_leaf_lev.as<int>(),
@@ -1192,6 +1209,8 @@ struct BClass {
     std::vector<int> pcs_phase;
     DBuf s5, s5_prob;
     int n_s5 = 0, n_s5_sib = 0;
+    DBuf s5_sym, s5_symprob;
+    int n_s5_fam = 0, n_s5_own = 0;
     DBuf dir_tgt, dir_lev, dir_off, dir_src, dir_code, dir_flags, dir_prob;
     int n_dir = 0;
     double stage_ms[6] = {0, 0, 0, 0, 0, 0};   // STEPs 1-6 of the last profiled execute
@@ -1344,6 +1363,8 @@ void build_classes(fgt_batch& B) {
         std::vector<int> mch, msg, pcsp, pcsc, pcsg;
         std::vector<fgt::PotTask> sib, own;
         std::vector<int> sibp, ownp;
+        std::vector<fgt::SymTask> sfam, sown;
+        std::vector<int> sfamp, sownp;
         int maxph2 = 0, maxph4 = 0;
         for (int q = 0; q < (int)C.members.size(); ++q) {
             fgt_solver& S = *B.solvers[C.members[q]];
@@ -1378,6 +1399,10 @@ void build_classes(fgt_batch& B) {
             sibp.insert(sibp.end(), S.n_s5_sib, q);
             own.insert(own.end(), h.s5.begin() + S.n_s5_sib, h.s5.end());
             ownp.insert(ownp.end(), h.s5.size() - S.n_s5_sib, q);
+            sfam.insert(sfam.end(), h.s5_sym.begin(), h.s5_sym.begin() + S.n_s5_fam);
+            sfamp.insert(sfamp.end(), S.n_s5_fam, q);
+            sown.insert(sown.end(), h.s5_sym.begin() + S.n_s5_fam, h.s5_sym.end());
+            sownp.insert(sownp.end(), S.n_s5_own, q);
         }
         C.pp.upload(pp);
         C.n_fz = (int)fzp.size();
@@ -1461,6 +1486,12 @@ void build_classes(fgt_batch& B) {
         C.n_s5 = (int)sib.size();
         C.s5.upload(sib);
         C.s5_prob.upload(sibp);
+        C.n_s5_fam = (int)sfam.size();
+        C.n_s5_own = (int)sown.size();
+        sfam.insert(sfam.end(), sown.begin(), sown.end());
+        sfamp.insert(sfamp.end(), sownp.begin(), sownp.end());
+        C.s5_sym.upload(sfam);
+        C.s5_symprob.upload(sfamp);
         // STEP 6: every target of every problem, longest list first
         struct DT {
             int q, k, len;
@@ -1544,9 +1575,13 @@ void class_step4(const BClass& C, hipStream_t st) {
     }
 }
 void class_step5(const BClass& C, hipStream_t st) {
-    if (C.n_s5 > 0)
-        fgt::launch_pw2pot_tasks(C.g, C.t, C.n_s5, C.n_s5_sib, C.s5.as<fgt::PotTask>(), nullptr, fgt::Kinds{0, 0, 0},
-                                 fgt::OutDesc{nullptr, C.nd, 0}, st, multi(C, C.s5_prob));
+    if (C.n_s5 <= 0) return;
+    fgt::ZOut zo{};
+    zo.nz = 1;
+    zo.od[0] = fgt::OutDesc{nullptr, C.nd, 0};
+    fgt::launch_pw2pot_tasks(C.g, C.t, {C.n_s5, C.n_s5_sib, C.s5.as<fgt::PotTask>(), C.s5_prob.as<int>(), C.n_s5_fam,
+                                        C.n_s5_own, C.s5_sym.as<fgt::SymTask>(), C.s5_symprob.as<int>()},
+                             nullptr, fgt::Kinds{0, 0, 0}, zo, st, C.pp.as<fgt::ProbPtrs>());
 }
 void class_step6(const BClass& C, hipStream_t st) {
     if (C.n_dir > 0)
@@ -1758,7 +1793,6 @@ void batch_autotune(fgt_batch& B, int reps) {
         }
         {
             std::vector<int> cand{0};
-            if (C.n >= 12 && C.t.npw <= 64) cand.push_back(1);
             if (C.prec >= 1 && C.t.npw <= 80) cand.push_back(2);
             int best = cand[0];
             float bt = 1e30f;

@@ -117,6 +117,16 @@ struct PotTask {
     int code[4];
 };
 
+// One task of the symmetric 3-D STEP 1 / STEP 5 kernels: a leaf with an
+// expansion of its own (box[0]), or a family, the leaf children of the box
+// whose expansion is in `slot`.  A family's child c has bit a (x, y, z) set
+// when it is the side whose table carries the conjugate parent-child phase
+// along axis a (-1: no leaf there); lev is the leaves' level.
+struct SymTask {
+    int slot, lev;
+    int box[8];
+};
+
 // Several problems of one shape class (3-D, same norder, density count and
 // precision; plane-wave counts may differ) in one launch.  Task i of a launch belongs
 // to problem tprob[i]; the kernel then takes that problem's tables, values,
@@ -180,8 +190,8 @@ struct DevTables {
     // matrix cores, 2 BF16 hi/lo matrix cores (prec >= 1 implies expn_f32)
     int prec;
     // x-stage variant of STEP 1 / STEP 5 (tuned per shape class; -1 = the
-    // default policy): 0 VALU, 1 FP64 matrix cores (STEP 5, norder >= 12,
-    // npw <= 64), 2 the reduced-precision matrix cores (prec >= 1)
+    // default policy): 0 FP64 (VALU), 2 the reduced-precision matrix cores
+    // (prec >= 1)
     int xs1 = -1, xs5 = -1;
     size_t lds_limit;  // device LDS bytes per block
 };
@@ -191,18 +201,21 @@ struct DevTables {
 bool launch_p2pw_3d(const Geom& g, const DevTables& t, int ntask, const int* box, const int* lev,
                     const int* slot, const double* fvals, double2* expn, hipStream_t s, size_t lds_limit,
                     const Multi& mu = Multi{});
-// tasks [0, nsib): sibling tasks (up to four leaves); [nsib, ntask): one leaf
-bool launch_pw2pot_3d(const Geom& g, const DevTables& t, int ntask, int nsib, const PotTask* tasks,
-                      const double2* expn, Kinds kd, OutDesc od, hipStream_t s, size_t lds_limit,
-                      const Multi& mu = Multi{});
-// the same for the components of zo (x and y kinds kd.x, kd.y): the
-// one-leaf tasks share their x and y stages across the z kinds
+// STEP 5 in reduced precision over PotTask lists, tasks [0, nsib) sibling
+// tasks (up to four leaves), [nsib, ntask) one leaf: for the components of zo
+// (x and y kinds kd.x, kd.y) the one-leaf tasks share their x and y stages
+// across the z kinds
 bool launch_pw2pot_3d_z(const Geom& g, const DevTables& t, int ntask, int nsib, const PotTask* tasks,
                         const double2* expn, Kinds kd, const ZOut& zo, hipStream_t s, size_t lds_limit,
                         const Multi& mu = Multi{});
+// STEP 5 in FP64 arithmetic (FP64 or FP32 expansions) through the tables'
+// symmetries: tasks [0, nfam) families, then nown single leaves
+bool launch_pw2pot_sym(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks,
+                       const double2* expn, Kinds kd, const ZOut& zo, hipStream_t s, const Multi& mu = Multi{});
 bool pw2pot_3d_supported(const Geom& g, const DevTables& t);
-// true when FGT_PW2POT_VALU=1: STEP 5 keeps its x stage on the VALU
-bool pw2pot_valu_only();
+// STEP 5 runs its x stage on the reduced-precision matrix cores (else it
+// takes launch_pw2pot_sym)
+bool pw2pot_lowp(const DevTables& t);
 // Fused STEP 1 + 2 for parents with leaf children (3-D, N in {8,12,16}):
 // plev/pslot per parent, kids/ksg 8 per parent (leaf child box or -1, merge
 // sign bits).  Writes (overwrites) the parent's mp; returns false if not covered.
@@ -272,11 +285,18 @@ void launch_split(const Geom& g, const DevTables& t, int nentry, const int* pc_p
 void launch_pw2pot(const Geom& g, const DevTables& t, int ntask, const int* box,
                    const int* lev, const int* slot, const double2* expn,
                    Kinds kd, OutDesc od, hipStream_t s);
-// 3-D STEP 5 over PotTask lists (throws when the shape is not covered)
-void launch_pw2pot_tasks(const Geom& g, const DevTables& t, int ntask, int nsib, const PotTask* tasks,
-                         const double2* expn, Kinds kd, OutDesc od, hipStream_t s, const Multi& mu = Multi{});
-void launch_pw2pot_tasks_z(const Geom& g, const DevTables& t, int ntask, int nsib, const PotTask* tasks,
-                           const double2* expn, Kinds kd, const ZOut& zo, hipStream_t s);
+// 3-D STEP 5 for the components of zo, in the form pw2pot_lowp picks (throws
+// when the shape is not covered)
+struct Step5Lists {
+    int ntask, nsib;          // PotTask list (reduced precision)
+    const PotTask* tasks;
+    const int* tprob;         // its problem indices (batches)
+    int nfam, nown;           // SymTask list
+    const SymTask* sym;
+    const int* symprob;
+};
+void launch_pw2pot_tasks(const Geom& g, const DevTables& t, const Step5Lists& l, const double2* expn, Kinds kd,
+                         const ZOut& zo, hipStream_t s, const ProbPtrs* pp = nullptr);
 // flags (nullable): per entry bit0 = last of its (y,z) table group, bit1 =
 // last of its z group; entries must then be grouped in that order.
 void launch_direct(const Geom& g, const DevTables& t, int ntask, const int* tgt,

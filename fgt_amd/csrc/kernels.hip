@@ -1139,20 +1139,17 @@ void launch_split(const Geom& g, const DevTables& t, int nentry, const int* pc_p
     }
 }
 
-void launch_pw2pot_tasks(const Geom& g, const DevTables& t, int ntask, int nsib, const PotTask* tasks,
-                         const double2* expn, Kinds kd, OutDesc od, hipStream_t s, const Multi& mu) {
-    if (ntask <= 0) return;
-    if (!launch_pw2pot_3d(g, t, ntask, nsib, tasks, expn, kd, od, s, t.lds_limit, mu))
+void launch_pw2pot_tasks(const Geom& g, const DevTables& t, const Step5Lists& l, const double2* expn, Kinds kd,
+                         const ZOut& zo, hipStream_t s, const ProbPtrs* pp) {
+    const bool lowp = pw2pot_lowp(t);
+    if ((lowp ? l.ntask : l.nfam + l.nown) <= 0) return;
+    Multi mu;
+    mu.pp = pp;
+    mu.tprob = lowp ? l.tprob : l.symprob;
+    if (lowp ? !launch_pw2pot_3d_z(g, t, l.ntask, l.nsib, l.tasks, expn, kd, zo, s, t.lds_limit, mu)
+             : !launch_pw2pot_sym(g, t, l.nfam, l.nown, l.sym, expn, kd, zo, s, mu))
         throw std::runtime_error("3-D STEP 5 kernel not available for this shape");
-    check(hipGetLastError(), "k_pw2pot3 launch");
-}
-
-void launch_pw2pot_tasks_z(const Geom& g, const DevTables& t, int ntask, int nsib, const PotTask* tasks,
-                           const double2* expn, Kinds kd, const ZOut& zo, hipStream_t s) {
-    if (ntask <= 0) return;
-    if (!launch_pw2pot_3d_z(g, t, ntask, nsib, tasks, expn, kd, zo, s, t.lds_limit))
-        throw std::runtime_error("3-D STEP 5 kernel not available for this shape");
-    check(hipGetLastError(), "k_pw2pot3 launch");
+    check(hipGetLastError(), "3-D STEP 5 launch");
 }
 
 void launch_pw2pot(const Geom& g, const DevTables& t, int ntask, const int* box, const int* lev,

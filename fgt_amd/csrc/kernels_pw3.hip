@@ -748,36 +748,24 @@ __device__ __forceinline__ void pw2pot_x_lowp(const float2* __restrict__ E, cons
 }
 
 // ---------------------------------------------------------------- STEP 5
-// Tables: tabS[kind][l][v][k][i] (frequency k, node i), v = 0 the plain
+// The reduced-precision form (FP32 expansions, x stage on the matrix cores;
+// the FP64 form is k_pw2pot_sym).  Tables: tabS[kind][l][v][k][i] (frequency k, node i), v = 0 the plain
 // PW->value table, 1 / 2 the table times the + / conjugate parent->child
 // split phase.  A task (PotTask) evaluates one expansion at up to four
 // leaves: for a leaf evaluating its parent's expansion the phase is folded
 // into the tables (STEP 4 folded into STEP 5), and the x variant depends only
 // on the x split sign, so four siblings share one x contraction.
-// Per round of SR k3 slabs (4; 8 for norder 8 with a matrix-core x stage):
+// Per round of SR k3 slabs (4; 8 for norder 8):
 //   x: ff[k2][s][kk1] = sum_k1 Ux[kk1][k1] E[k3][k1][k2]   (wave = slab,
 //      or slabs w and w + 4)
 //   y: yres[s][kk1][kk2] = sum_k2 Uy[kk2][k2] ff[k2][s][kk1], per y variant
 //   z: G_c[kk3] += Re(Uz_c[kk3][k3] yres[s][zk1][zk2]), per leaf c, with one
 //      thread per output column (zk1, zk2) holding all kk3 in registers.
-// LDS: sff [k2][s][KW] (npw*64 complex, KW = 64 / SR; FP32 after a
-// reduced-precision x stage, whose FP32 results it holds exactly, else
-// FP64), yres [s][kk1][16]
+// LDS: sff [k2][s][KW] (npw*64 complex, KW = 64 / SR; the x stage's FP32
+// results, held exactly), yres [s][kk1][16]
 // (1024 complex, entry kk2 at kk2 ^ kk1), sUr [v][s][kk3] (3*SR*N complex:
 // the round's z table rows of the three variants, zero past nh).
-// MF: x stage on the FP64 matrix cores (N >= 12, npw <= 64): per slab the
-// complex product ff[kk1][k2] = sum_k1 U[kk1][k1] E[k1][k2] runs as
-// 16x16x4 tiles (rows kk1, columns 16 k2, K = 4 k1; for N = 12 the rows
-// kk1 >= N carry zero table entries).  For N = 8 half of each tile would be
-// padding and the VALU form is faster (STEP 5 over 21 norder-8 problems:
-// 4.34 vs 5.10 ms; norder 12: 5.17 VALU vs 4.53 ms here).  The table is read per
-// lane from global memory (cached); E rows stream straight into the B
-// operand.  (For STEP 1 the matrix-core form is slower: its 50 x 50 output
-// pads to 64 x 64 tiles, where the VALU form wastes only the lane padding.)
-
-// C: most leaves per task (4 for sibling tasks, 1 for a leaf's own
-// expansion; with one leaf the freed registers carry the x stage's next
-// K-step loads while the current one runs).
+// C: most leaves per task (4 for sibling tasks, 1 for a leaf's own expansion).
 // NZ: output components sharing the x and y table kinds and differing in the
 // z kind zo.kz[q] (one-leaf tasks only: all their variants are 0, so sUr
 // holds the round's rows of NZ <= 3 z kinds in place of the three
@@ -789,17 +777,16 @@ __global__ void __launch_bounds__(256, 2) k_pw2pot3(Geom g, const double2* __res
                                                 size_t ks, Kinds kd, ZOut zo, Multi mu) {
     static_assert(NZ >= 1 && NZ <= 3 && (NZ == 1 || C == 1), "z kinds are grouped for one-leaf tasks only");
     extern __shared__ double2 sm[];
-    using SF = typename std::conditional<(XS >= 2), float2, double2>::type;
-    SF* sff = reinterpret_cast<SF*>(sm);
+    static_assert(XS >= 2, "the FP64 form is k_pw2pot_sym");
+    float2* sff = reinterpret_cast<float2*>(sm);
     double2* yres = reinterpret_cast<double2*>(sff + (size_t)npw * 64);
     double2* sUr = yres + 4 * 16 * 16;
     constexpr int NQ = N / 4;
-    constexpr int PF = (N == 12) ? 6 : 8;
-    // slabs per round: 8 for norder 8 with a matrix-core x stage (each wave
+    // slabs per round: 8 for norder 8 (each wave
     // computes two slabs, and the y stage's 64 lanes are (kk1, slab) with no
     // idle half), else 4; KW: kk1 slots per (k2, slab) row of sff, per
     // (slab, kk1) group of yres
-    constexpr int SR = (N == 8 && XS >= 2) ? 8 : 4;
+    constexpr int SR = N == 8 ? 8 : 4;
     constexpr int KW = 64 / SR;
     const int tix = xcd_task(blockIdx.x, gridDim.x);
     const PotTask* __restrict__ T = tasks + tix;
@@ -872,117 +859,7 @@ __global__ void __launch_bounds__(256, 2) k_pw2pot3(Geom g, const double2* __res
                     sUr[tid] = (r + s2 < nh) ? U[(r + s2) * N + k] : make_double2(0.0, 0.0);
                 }
             }
-            // x: wave = slab, lane = k2.  Rows of E are fetched PF at a time
-            // (all loads issued before the FMAs that use them) so enough reads
-            // are in flight to cover HBM latency; lanes past npw read a valid
-            // duplicate and discard it.
-            if constexpr (XS >= 2) {
-                pw2pot_x_lowp<N, XS, SR>(E, UX, npw, nh, r, wave, lane, sff, hx);
-            } else if constexpr (XS == 1) {
-                const int k3 = r + wave;
-                if (k3 < nh) {
-                    const ET* __restrict__ Ek = E + (size_t)k3 * npw * npw;
-                    const int li = lane & 15, lk = lane >> 4;
-                    // rows kk1 >= N (N < 16) read a valid table entry and are zeroed
-                    const int lir = li < N ? li : N - 1;
-                    dbl4 are[4], aim[4];
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) are[t] = aim[t] = dbl4{0.0, 0.0, 0.0, 0.0};
-                    const int ksteps = (npw + 3) >> 2;
-                    if constexpr (C == 1 && NZ == 1) {
-                        // the next K-step's operands are loaded (always, from a
-                        // valid clamped address) before this step's products,
-                        // into two alternating register sets (with NZ > 1 the
-                        // z sums take those registers)
-                        double2 ua, ub, ea[4], eb[4];
-#define PW2POT_XLOAD(u_, e_, st)                                                             \
-    {                                                                                        \
-        const int k1c_ = min(4 * (st) + lk, npw - 1);                                        \
-        u_ = UX[k1c_ * N + lir];                                                             \
-        _Pragma("unroll") for (int t = 0; t < 4; ++t)                                        \
-            e_[t] = ldE(Ek[(size_t)k1c_ * npw + min(16 * t + li, npw - 1)]);                 \
-    }
-#define PW2POT_XSTEP(u_, e_, st)                                                             \
-    {                                                                                        \
-        const double2 um_ = (4 * (st) + lk < npw && li < N) ? u_ : make_double2(0.0, 0.0);   \
-        _Pragma("unroll") for (int t = 0; t < 4; ++t) cmfma(um_, e_[t], are[t], aim[t]);     \
-    }
-                        PW2POT_XLOAD(ua, ea, 0);
-                        for (int st = 0; st < ksteps; st += 2) {
-                            PW2POT_XLOAD(ub, eb, min(st + 1, ksteps - 1));
-                            // keep the loads above this step's products (the
-                            // scheduler would otherwise sink them to their use)
-                            __builtin_amdgcn_sched_barrier(0);
-                            PW2POT_XSTEP(ua, ea, st);
-                            if (st + 1 >= ksteps) break;
-                            PW2POT_XLOAD(ua, ea, min(st + 2, ksteps - 1));
-                            __builtin_amdgcn_sched_barrier(0);
-                            PW2POT_XSTEP(ub, eb, st + 1);
-                        }
-#undef PW2POT_XSTEP
-#undef PW2POT_XLOAD
-                    } else {
-                        for (int st = 0; st < ksteps; ++st) {
-                            const int k1 = 4 * st + lk;
-                            const bool kv = k1 < npw;
-                            const int k1c = kv ? k1 : npw - 1;
-                            double2 u = UX[k1c * N + lir];
-                            if (!kv || li >= N) u = make_double2(0.0, 0.0);
-                            double2 e[4];
-#pragma unroll
-                            for (int t = 0; t < 4; ++t) {
-                                const int k2 = 16 * t + li;
-                                e[t] = ldE(Ek[(size_t)k1c * npw + (k2 < npw ? k2 : npw - 1)]);
-                            }
-#pragma unroll
-                            for (int t = 0; t < 4; ++t) cmfma(u, e[t], are[t], aim[t]);
-                        }
-                    }
-                    // lane holds kk1 = lk + 4v for column k2 = 16t + li
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        const int k2 = 16 * t + li;
-                        if (k2 < npw)
-#pragma unroll
-                            for (int v = 0; v < 4; ++v)
-                                sff[(k2 * 4 + wave) * 16 + ((lk + 4 * v) ^ (k2 & 15))] =
-                                    make_double2(are[t][v], aim[t][v]);
-                    }
-                }
-            } else {
-                const int k3 = r + wave;
-                if (k3 < nh) {
-                    const ET* __restrict__ Ek = E + (size_t)k3 * npw * npw;
-                    for (int c = 0; c < npw; c += 64) {
-                        const int k2 = c + lane;
-                        const bool act = k2 < npw;
-                        const int k2c = act ? k2 : npw - 1;
-                        double2 acc[N];
-#pragma unroll
-                        for (int k = 0; k < N; ++k) acc[k] = make_double2(0.0, 0.0);
-                        int k1 = 0;
-                        for (; k1 + PF <= npw; k1 += PF) {
-                            double2 e[PF];
-#pragma unroll
-                            for (int u = 0; u < PF; ++u) e[u] = ldE(Ek[(size_t)(k1 + u) * npw + k2c]);
-#pragma unroll
-                            for (int u = 0; u < PF; ++u)
-#pragma unroll
-                                for (int k = 0; k < N; ++k) acc[k] = zfma(UX[(k1 + u) * N + k], e[u], acc[k]);
-                        }
-                        for (; k1 < npw; ++k1) {
-                            const double2 e = ldE(Ek[(size_t)k1 * npw + k2c]);
-#pragma unroll
-                            for (int k = 0; k < N; ++k) acc[k] = zfma(UX[k1 * N + k], e, acc[k]);
-                        }
-                        // row (k2, slab) holds 16 entries; entry k is stored at k ^ (k2 & 15)
-                        // so the 64 lanes of a write hit different banks
-                        if (act)
-#pragma unroll
-                            for (int k = 0; k < N; ++k) sff[(k2 * 4 + wave) * 16 + (k ^ (k2 & 15))] = acc[k];
-                    }
-                }
-            }
+            pw2pot_x_lowp<N, XS, SR>(E, UX, npw, nh, r, wave, lane, sff, hx);
             __syncthreads();
             for (int j = 0; j < nvy; ++j) {
                 if (j) __syncthreads();   // the z stage of the previous y variant is done with yres
@@ -995,7 +872,7 @@ __global__ void __launch_bounds__(256, 2) k_pw2pot3(Geom g, const double2* __res
 #pragma unroll
                     for (int q = 0; q < NQ; ++q) y[q] = make_double2(0.0, 0.0);
                     for (int k2 = 0; k2 < npw; ++k2) {
-                        const SF fs = sff[(k2 * SR + s) * KW + (kk1 ^ (k2 & (KW - 1)))];
+                        const float2 fs = sff[(k2 * SR + s) * KW + (kk1 ^ (k2 & (KW - 1)))];
                         const double2 f = make_double2(fs.x, fs.y);
 #pragma unroll
                         for (int q = 0; q < NQ; ++q) y[q] = zfma(UY[k2 * N + wave * NQ + q], f, y[q]);
@@ -1092,20 +969,6 @@ bool use_lowp1(const DevTables& t) {
     return t.xs1 >= 0 ? t.xs1 == 2 : (lowp_stages(t.prec) & 1) != 0;
 }
 
-// STEP 5 x-stage variant (0 VALU, 1 FP64 matrix cores, 2 reduced precision)
-int x5_variant(int n, const DevTables& t) {
-    const bool lowp_ok = t.prec >= 1 && t.npw <= kLowpMaxPw;
-    const bool f64mf_ok = n >= 12 && t.npw <= 64;
-    if (t.xs5 >= 0) {
-        if (t.xs5 == 2 && lowp_ok) return 2;
-        if (t.xs5 == 1 && f64mf_ok) return 1;
-        return 0;
-    }
-    if (lowp_ok && (lowp_stages(t.prec) & 2)) return 2;
-    if (f64mf_ok && !pw2pot_valu_only()) return 1;
-    return 0;
-}
-
 template <int N>
 bool try_p2pw3(const Geom& g, const DevTables& t, int ntask, const int* box, const int* lev, const int* slot,
                const double* fvals, double2* expn, hipStream_t s, size_t lds_limit, const Multi& mu) {
@@ -1129,28 +992,17 @@ bool try_p2pw3(const Geom& g, const DevTables& t, int ntask, const int* box, con
     return true;
 }
 
-// xs: the x-stage variant (>= 2: reduced precision, FP32 sff)
-size_t pw2pot3_lds(int n, int npw, int xs = 0) {
+size_t pw2pot3_lds(int n, int npw) {
     // sff, yres, sUr (three variants of up to eight slabs at norder 8, four above)
-    return (xs >= 2 ? sizeof(float2) : sizeof(double2)) * (size_t)npw * 64 +
-           sizeof(double2) * (4 * 16 * 16 + (n == 8 ? 24 : 12) * (size_t)n);
+    return sizeof(float2) * (size_t)npw * 64 + sizeof(double2) * (4 * 16 * 16 + (n == 8 ? 24 : 12) * (size_t)n);
 }
 
 template <int N, int XS, int C, int NZ = 1>
 void launch_pw2pot3_c(const Geom& g, const DevTables& t, int ntask, const PotTask* tasks, const double2* expn,
                       Kinds kd, const ZOut& zo, hipStream_t s, size_t lds, const Multi& mu) {
     if (ntask <= 0) return;
-    if constexpr (XS >= 2) {
-        hipLaunchKernelGGL((k_pw2pot3<N, XS, C, float2, NZ>), dim3(ntask), dim3(256), lds, s, g, t.pw2potS, t.npw,
-                           tasks, reinterpret_cast<const float2*>(expn), t.pw2potS_ks, kd, zo, mu);
-    } else {
-        if (t.expn_f32)
-            hipLaunchKernelGGL((k_pw2pot3<N, XS, C, float2, NZ>), dim3(ntask), dim3(256), lds, s, g, t.pw2potS,
-                               t.npw, tasks, reinterpret_cast<const float2*>(expn), t.pw2potS_ks, kd, zo, mu);
-        else
-            hipLaunchKernelGGL((k_pw2pot3<N, XS, C, double2, NZ>), dim3(ntask), dim3(256), lds, s, g, t.pw2potS,
-                               t.npw, tasks, expn, t.pw2potS_ks, kd, zo, mu);
-    }
+    hipLaunchKernelGGL((k_pw2pot3<N, XS, C, float2, NZ>), dim3(ntask), dim3(256), lds, s, g, t.pw2potS, t.npw, tasks,
+                       reinterpret_cast<const float2*>(expn), t.pw2potS_ks, kd, zo, mu);
 }
 
 // components zo.kz[a..a+nz) of zo as a group of their own
@@ -1188,30 +1040,10 @@ template <int N>
 bool try_pw2pot3(const Geom& g, const DevTables& t, int ntask, int nsib, const PotTask* tasks,
                  const double2* expn, Kinds kd, const ZOut& zo, hipStream_t s, size_t lds_limit, const Multi& mu) {
     const size_t lds = pw2pot3_lds(N, t.npw);
-    if (lds > lds_limit) return false;
-    if (3 * t.pw2potS_ks > 0x7fffffffULL) return false;
-    const int xs = x5_variant(N, t);
-    if (xs == 2) {
-        // reduced-precision x stage (FP32 or BF16 hi/lo matrix cores; FP32 sff)
-        const size_t lds32 = pw2pot3_lds(N, t.npw, 2);
-        if (t.prec == 2) {
-            launch_pw2pot3_typed<N, 3>(g, t, ntask, nsib, tasks, expn, kd, zo, s, lds32, mu);
-            return true;
-        }
-        if constexpr (N == 8) {
-            launch_pw2pot3_typed<N, 4>(g, t, ntask, nsib, tasks, expn, kd, zo, s, lds32, mu);
-            return true;
-        }
-        launch_pw2pot3_typed<N, 2>(g, t, ntask, nsib, tasks, expn, kd, zo, s, lds32, mu);
-        return true;
-    }
-    if constexpr (N >= 12) {
-        if (xs == 1) {
-            launch_pw2pot3_typed<N, 1>(g, t, ntask, nsib, tasks, expn, kd, zo, s, lds, mu);
-            return true;
-        }
-    }
-    launch_pw2pot3_typed<N, 0>(g, t, ntask, nsib, tasks, expn, kd, zo, s, lds, mu);
+    if (lds > lds_limit || 3 * t.pw2potS_ks > 0x7fffffffULL) return false;
+    // BF16 hi/lo, or FP32 (its table operands hoisted at norder 8)
+    if (t.prec == 2) launch_pw2pot3_typed<N, 3>(g, t, ntask, nsib, tasks, expn, kd, zo, s, lds, mu);
+    else launch_pw2pot3_typed<N, (N == 8 ? 4 : 2)>(g, t, ntask, nsib, tasks, expn, kd, zo, s, lds, mu);
     return true;
 }
 
@@ -1271,14 +1103,9 @@ int lowp_stages(int prec) {
     return v >= 0 ? v : (prec == 2 ? 3 : 2);
 }
 
-// FGT_PW2POT_VALU=1 selects the FP64 VALU x stage of STEP 5 instead of the
-// matrix-core one (for comparison runs).
-bool pw2pot_valu_only() {
-    static const bool v = [] {
-        const char* e = std::getenv("FGT_PW2POT_VALU");
-        return e && e[0] == '1';
-    }();
-    return v;
+bool pw2pot_lowp(const DevTables& t) {
+    if (t.prec < 1 || t.npw > kLowpMaxPw) return false;
+    return t.xs5 >= 0 ? t.xs5 == 2 : (lowp_stages(t.prec) & 2) != 0;
 }
 
 bool launch_p2pw_3d(const Geom& g, const DevTables& t, int ntask, const int* box, const int* lev,
@@ -1313,7 +1140,7 @@ bool p2pw_fused_3d(const Geom& g, const DevTables& t, int ntask, const int* plev
 
 bool pw2pot_3d_supported(const Geom& g, const DevTables& t) {
     if (g.ndim != 3 || (t.n != 8 && t.n != 12 && t.n != 16)) return false;
-    const size_t lds = pw2pot3_lds(t.n, t.npw);
+    const size_t lds = sizeof(double2) * ((size_t)t.npw * 64 + 4 * 16 * 16 + (t.n == 8 ? 24 : 12) * (size_t)t.n);
     const size_t lds1 = sizeof(double2) * std::max(4 * (size_t)t.n * t.n, 4 * (size_t)t.n * t.npw);
     const size_t lds2 = sizeof(double2) * std::max(8 * (size_t)t.n * t.n, 4 * (size_t)t.n * t.npw);
     return lds <= t.lds_limit && lds1 <= t.lds_limit && lds2 <= t.lds_limit;
@@ -1329,15 +1156,6 @@ bool launch_pw2pot_3d_z(const Geom& g, const DevTables& t, int ntask, int nsib, 
         case 16: return try_pw2pot3<16>(g, t, ntask, nsib, tasks, expn, kd, zo, s, lds_limit, mu);
         default: return false;
     }
-}
-
-bool launch_pw2pot_3d(const Geom& g, const DevTables& t, int ntask, int nsib, const PotTask* tasks,
-                      const double2* expn, Kinds kd, OutDesc od, hipStream_t s, size_t lds_limit, const Multi& mu) {
-    ZOut zo{};
-    zo.nz = 1;
-    zo.kz[0] = kd.z;
-    zo.od[0] = od;
-    return launch_pw2pot_3d_z(g, t, ntask, nsib, tasks, expn, kd, zo, s, lds_limit, mu);
 }
 
 }  // namespace fgt

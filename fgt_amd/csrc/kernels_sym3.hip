@@ -1,0 +1,402 @@
+// kernels_sym3.hip -- 3-D STEP 1 (values -> PW) and STEP 5 (PW -> values) in
+// FP64 through the symmetries of the 1-D tables (gfx950).
+//
+// Replaces g3d_tens_prod_to_pw (bfgt_pwrouts.f:153-222) with the STEP 2
+// shift of leaf children folded in, and g3d_pw2pgh (bfgt_pwrouts.f:719-1065)
+// with the STEP 4 shift into leaves folded in.
+//
+// The plane-wave frequencies come in pairs (k, npw-1-k) of opposite sign and
+// the nodes in pairs (i, n-1-i) about the box centre, so a 1-D table obeys
+//   T[npw-1-k][i] = conj T[k][i],   T[k][n-1-i] = conj T[k][i]
+// (first-derivative tables: -conj).  The same holds for the two children of
+// a box along an axis: the node i of one and n-1-i of the other lie
+// symmetric about the parent's centre, and their tables, which carry the
+// parent-child phase, are conjugates.  A "pair" below is two such nodes:
+// side a is node i (of the child whose table variant is 1), side b its mirror
+// image.  A leaf evaluated by itself has ceil(n/2) pairs per axis; the
+// (up to eight) leaf children of one parent together have n.
+//
+// With E = sums and D = differences over the pair being contracted,
+//   sum = Re(T) E + i Im(T) D,   the partner's sum = Re(T) E - i Im(T) D
+// (E, D complex, the table real): four real multiply-adds serve two inputs
+// and two outputs, where the plain complex form takes sixteen.  A quarter
+// of the arithmetic leaves both steps bound by the expansion bytes they
+// write and read.
+#include "kernels.h"
+
+#include <algorithm>
+
+namespace fgt {
+
+namespace {
+
+constexpr int kThreads = 256;
+
+__device__ __forceinline__ double2 cplus(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
+__device__ __forceinline__ double2 cminus(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
+
+// Touches every 64-byte line of n table entries once, eight scalar loads at a
+// time, the lines dealt to the block's waves: the scalar cache starts a
+// kernel empty, and the stages below would take its misses one by one.
+__device__ __forceinline__ void warm_table(CTab2 t, int n, int wave) {
+    const int lines = (n + 3) >> 2;
+    for (int i = 8 * wave; i < lines; i += 8 * (kThreads / 64)) {
+        double d[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) d[j] = t[4 * (long long)min(i + j, lines - 1)].x;
+        asm volatile("" ::"s"(d[0]), "s"(d[1]), "s"(d[2]), "s"(d[3]), "s"(d[4]), "s"(d[5]), "s"(d[6]), "s"(d[7]));
+    }
+}
+
+// pairs per axis of a task: a family (the leaf children of one parent) or one leaf
+template <int N, bool FAM>
+constexpr int sym_pairs() { return FAM ? N : (N + 1) / 2; }
+
+// ---------------------------------------------------------------- STEP 5
+// x pairs per block: a task's x pairs are split over blocks so that the
+// block's output columns (2 NX x nodes, 2 NP y nodes) are at most one per
+// thread and the x stage's sums stay in registers
+template <int N, bool FAM>
+constexpr int sym5_parts() { return sym_pairs<N, FAM>() <= 6 ? 1 : (sym_pairs<N, FAM>() + 3) / 4; }
+template <int N, bool FAM>
+constexpr int sym5_nx() { return (sym_pairs<N, FAM>() + sym5_parts<N, FAM>() - 1) / sym5_parts<N, FAM>(); }
+
+// k3 slabs per round: about one (slab, k2) column of the x stage per thread,
+// at most 8, the rounds of equal length
+__host__ __device__ inline int sym5_slabs(int npw) {
+    const int nh = (npw + 1) / 2;
+    const int most = kThreads / npw < 1 ? 1 : (kThreads / npw > 8 ? 8 : kThreads / npw);
+    const int rounds = (nh + most - 1) / most;
+    return (nh + rounds - 1) / rounds;
+}
+// double2 entries of the block's LDS: sff [k2][slab][x node] and yres
+// [slab][x node][y node] share it (rows padded by one entry: odd strides)
+inline size_t sym5_lds_entries(int npw, int nodx, int nody) {
+    const size_t sr = (size_t)sym5_slabs(npw);
+    return std::max(npw * (sr * nodx + 1), sr * nodx * (nody + 1));
+}
+
+// One block: x pairs [px0, px0 + NX) of one task, all k3.  Per round of SR
+// slabs:
+//   x: thread = (slab, k2) column; E rows k1 and npw-1-k1 stream from HBM,
+//      two steps ahead of their use, into 2 NX node sums;
+//   y: lane = (slab, x node), the y pairs split over the waves;
+//   z: thread = (x node, y node), all z pairs of every z kind in registers.
+// The tables are wave-uniform (scalar loads); LDS carries the transposes.
+// Bound by the expansion reads and by the latency of each round's three
+// stages (norder 8, npw 28, 8382 leaves: 84 us for 210 MB, 2.5 TB/s; the
+// sixteen-multiply-add form over half the siblings 244 us; norder 12, npw 60,
+// 4250 leaves: 402 us, 1182 before).  x pairs over more blocks at eight pairs
+// (two of four rather than one of eight: smaller LDS tiles, four blocks per
+// CU instead of three) measured 106 -> 102 us, the scalar cache's warm-up,
+// the unrolled y and z stages and one launch for both kinds of task 102 -> 84.
+template <int N, bool FAM, int NZ, typename ET>
+__device__ __forceinline__ void pw2pot_sym_block(int npw, int nd, const double2* __restrict__ tabS,
+                                                 const SymTask* __restrict__ T, int part,
+                                                 const ET* __restrict__ expn, size_t ks, Kinds kd, const ZOut& zo,
+                                                 const ProbPtrs* __restrict__ prob, double2* __restrict__ sm) {
+    constexpr int NP = sym_pairs<N, FAM>(), NX = sym5_nx<N, FAM>();
+    constexpr int NODX = 2 * NX, NODY = 2 * NP, COLS = NODX * NODY;
+    static_assert(COLS <= kThreads, "one output column per thread");
+    constexpr int YS = NODX <= 8 ? 4 : 2;                  // waves sharing one y row batch
+    constexpr int YP = (NP + YS - 1) / YS;                 // y pairs per wave
+    constexpr int ZS = COLS <= 64 ? 4 : (COLS <= 128 ? 2 : 1);   // thread groups sharing the z pairs
+    constexpr int ZP = (NP + ZS - 1) / ZS;
+    constexpr int V = FAM ? 1 : 0;
+    constexpr int KU = 3;
+    const int nh = (npw + 1) >> 1;
+    const int SR = sym5_slabs(npw);
+    const int ST = SR * NODX + 1;
+    const bool odd = (npw & 1) != 0;
+    const long long per = (long long)npw * N;
+    const long long row3 = (3LL * __builtin_amdgcn_readfirstlane(T->lev) + V) * per;
+    const int px0 = min(part * NX, NP - NX);
+    const CTab2 UX = ctab(tabS) + ((long long)(kd.x * ks) + row3 + px0);
+    const CTab2 UY = ctab(tabS) + ((long long)(kd.y * ks) + row3);
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63;
+    const int slot = __builtin_amdgcn_readfirstlane(T->slot);
+    const double sgx = kd.x == 1 ? -1.0 : 1.0, sgy = kd.y == 1 ? -1.0 : 1.0;
+    CTab2 UZ[NZ];
+#pragma unroll
+    for (int z = 0; z < NZ; ++z) UZ[z] = ctab(tabS) + ((long long)(zo.kz[z] * ks) + row3);
+    warm_table(UX, nh * N - px0, wave);
+    if (kd.y != kd.x) warm_table(UY, nh * N, wave);
+#pragma unroll
+    for (int z = 0; z < NZ; ++z)
+        if (zo.kz[z] != kd.x && zo.kz[z] != kd.y) warm_table(UZ[z], nh * N, wave);
+    // y rows and output column of this thread
+    const int yset = YS == 4 ? wave : wave >> 1, yrow0 = YS == 4 ? 0 : 64 * (wave & 1);
+    const int zset = ZS == 1 ? 0 : (ZS == 2 ? wave >> 1 : wave);
+    const int col = ZS == 1 ? tid : (ZS == 2 ? (tid & 127) : lane);
+    const bool zact = col < COLS;
+    const int zx = zact ? col % NODX : 0, zy = zact ? col / NODX : 0;
+    for (int ind = 0; ind < nd; ++ind) {
+        double GP[NZ][ZP], GQ[NZ][ZP];
+#pragma unroll
+        for (int z = 0; z < NZ; ++z)
+#pragma unroll
+            for (int q = 0; q < ZP; ++q) GP[z][q] = GQ[z][q] = 0.0;
+        const ET* __restrict__ E = expn + (size_t)(slot * 2 * nd + nd + ind) * (size_t)(nh * npw * npw);
+        for (int r = 0; r < nh; r += SR) {
+            const int cols = SR * npw;
+            // ---- x
+            for (int cb = 64 * wave; cb < cols; cb += kThreads) {
+                const int c = min(cb + lane, cols - 1);   // past the end: a duplicate of the last column
+                const int s = c / npw, k2 = c - s * npw;
+                // row base scalar, column offset per lane
+                const unsigned co = (unsigned)(min(r + s, nh - 1) * npw * npw + k2);
+                double2 P[NX], Q[NX];
+#pragma unroll
+                for (int p = 0; p < NX; ++p) P[p] = Q[p] = make_double2(0.0, 0.0);
+                ET u[KU][2], v[KU][2];   // two sets of KU frequency pairs
+                auto load = [&](ET (&e)[KU][2], int k) {
+#pragma unroll
+                    for (int j = 0; j < KU; ++j) {
+                        const int kc = min(k + j, nh - 1);
+                        const ET* __restrict__ ea = E + (size_t)(kc * npw);
+                        const ET* __restrict__ eb = E + (size_t)((npw - 1 - kc) * npw);
+                        e[j][0] = ea[co];
+                        e[j][1] = eb[co];
+                    }
+                };
+                auto apply = [&](const ET (&e)[KU][2], int k) {
+#pragma unroll
+                    for (int j = 0; j < KU; ++j) {
+                        if (k + j >= nh) break;
+                        const double2 a = ldE(e[j][0]), b = ldE(e[j][1]);
+                        // the zero frequency of an odd count pairs with itself
+                        const double2 S = (odd && k + j == nh - 1) ? a : cplus(a, b);
+                        const double2 D = cminus(a, b);
+#pragma unroll
+                        for (int p = 0; p < NX; ++p) {
+                            const double2 t = UX[(long long)(k + j) * N + p];
+                            P[p].x += t.x * S.x;
+                            P[p].y += t.x * S.y;
+                            Q[p].x += t.y * D.x;
+                            Q[p].y += t.y * D.y;
+                        }
+                    }
+                };
+                load(u, 0);
+                for (int k = 0; k < nh; k += 2 * KU) {
+                    load(v, k + KU);
+                    __builtin_amdgcn_sched_barrier(0);
+                    apply(u, k);
+                    if (k + KU >= nh) break;
+                    load(u, k + 2 * KU);
+                    __builtin_amdgcn_sched_barrier(0);
+                    apply(v, k + KU);
+                }
+                double2* __restrict__ o = sm + k2 * ST + s * NODX;
+#pragma unroll
+                for (int p = 0; p < NX; ++p) {
+                    o[p] = make_double2(P[p].x - Q[p].y, P[p].y + Q[p].x);
+                    o[NX + p] = make_double2(sgx * (P[p].x + Q[p].y), sgx * (P[p].y - Q[p].x));
+                }
+            }
+            __syncthreads();
+            // ---- y
+            const int rows = SR * NODX;
+            const int row = yrow0 + lane;
+            {
+                const double2* __restrict__ f = sm + min(row, rows - 1);
+                double2 P[YP], Q[YP];
+#pragma unroll
+                for (int p = 0; p < YP; ++p) P[p] = Q[p] = make_double2(0.0, 0.0);
+                if (yrow0 < rows) {
+                    // several steps' table and LDS reads together
+                    constexpr int YU = YP <= 2 ? 4 : 2;
+                    for (int k0 = 0; k0 < nh; k0 += YU) {
+                        double2 a[YU], b[YU], t[YU][YP];
+#pragma unroll
+                        for (int j = 0; j < YU; ++j) {
+                            const int k = min(k0 + j, nh - 1);
+                            a[j] = f[k * ST];
+                            b[j] = f[(npw - 1 - k) * ST];
+#pragma unroll
+                            for (int p = 0; p < YP; ++p) t[j][p] = UY[(long long)k * N + min(yset * YP + p, NP - 1)];
+                        }
+#pragma unroll
+                        for (int j = 0; j < YU; ++j) {
+                            if (k0 + j >= nh) break;
+                            const double2 S = (odd && k0 + j == nh - 1) ? a[j] : cplus(a[j], b[j]);
+                            const double2 D = cminus(a[j], b[j]);
+#pragma unroll
+                            for (int p = 0; p < YP; ++p) {
+                                P[p].x += t[j][p].x * S.x;
+                                P[p].y += t[j][p].x * S.y;
+                                Q[p].x += t[j][p].y * D.x;
+                                Q[p].y += t[j][p].y * D.y;
+                            }
+                        }
+                    }
+                }
+                __syncthreads();   // sff is read; yres takes its place
+                if (row < rows) {
+                    double2* __restrict__ o = sm + row * (NODY + 1);
+#pragma unroll
+                    for (int p = 0; p < YP; ++p) {
+                        const int q = yset * YP + p;
+                        if (q < NP) {
+                            o[q] = make_double2(P[p].x - Q[p].y, P[p].y + Q[p].x);
+                            o[NP + q] = make_double2(sgy * (P[p].x + Q[p].y), sgy * (P[p].y - Q[p].x));
+                        }
+                    }
+                }
+            }
+            __syncthreads();
+            // ---- z
+            if (zact) {
+                constexpr int ZU = NZ * ZP <= 4 ? 4 : (NZ * ZP <= 8 ? 2 : 1);
+                const int ns = min(SR, nh - r);
+                for (int s0 = 0; s0 < ns; s0 += ZU) {
+                    double2 yv[ZU], t[ZU][NZ][ZP];
+#pragma unroll
+                    for (int j = 0; j < ZU; ++j) {
+                        const int s = min(s0 + j, ns - 1);
+                        yv[j] = sm[(s * NODX + zx) * (NODY + 1) + zy];
+#pragma unroll
+                        for (int z = 0; z < NZ; ++z)
+#pragma unroll
+                            for (int q = 0; q < ZP; ++q)
+                                t[j][z][q] = UZ[z][(long long)(r + s) * N + min(zset * ZP + q, NP - 1)];
+                    }
+#pragma unroll
+                    for (int j = 0; j < ZU; ++j) {
+                        if (s0 + j >= ns) break;
+                        const double w = (odd && r + s0 + j == nh - 1) ? 0.5 : 1.0;
+                        const double yr = yv[j].x * w, yi = yv[j].y * w;
+#pragma unroll
+                        for (int z = 0; z < NZ; ++z)
+#pragma unroll
+                            for (int q = 0; q < ZP; ++q) {
+                                GP[z][q] += t[j][z][q].x * yr;
+                                GQ[z][q] += t[j][z][q].y * yi;
+                            }
+                    }
+                }
+            }
+            __syncthreads();
+        }
+        if (zact) {
+            // node pair -> (child bit, node): side b is the mirrored node, of
+            // the other child (family) or of the same leaf; a leaf's middle
+            // node (odd n) is its own mirror, side a
+            const int bx = zx >= NX, by = zy >= NP;
+            const int px = px0 + zx - bx * NX, py = zy - by * NP;
+            const int ix = bx ? N - 1 - px : px, iy = by ? N - 1 - py : py;
+            const bool own = px >= part * NX && (FAM || !((bx && 2 * px + 1 == N) || (by && 2 * py + 1 == N)));
+            if (own) {
+                const int cxy = FAM ? bx | by << 1 : 0;
+                const int ba = T->box[cxy], bb = T->box[FAM ? cxy | 4 : 0];
+                int node = ix + N * iy;
+                // opaque: the output addresses are formed here, not held
+                // through the whole task
+                asm volatile("" : "+v"(node));
+#pragma unroll
+                for (int z = 0; z < NZ; ++z) {
+                    double* const op = prob ? prob->pot : zo.od[z].p;
+                    const int ns = zo.od[z].ns, co = zo.od[z].coff + ind;
+                    const double sgz = zo.kz[z] == 1 ? -2.0 : 2.0;
+#pragma unroll
+                    for (int q = 0; q < ZP; ++q) {
+                        const int pz = zset * ZP + q;
+                        if (pz >= NP) break;
+                        if (ba >= 0)
+                            op[((size_t)ba * (N * N * N) + node + N * N * pz) * ns + co] += 2.0 * (GP[z][q] - GQ[z][q]);
+                        if (bb >= 0 && (FAM || 2 * pz + 1 != N))
+                            op[((size_t)bb * (N * N * N) + node + N * N * (N - 1 - pz)) * ns + co] +=
+                                sgz * (GP[z][q] + GQ[z][q]);
+                    }
+                }
+            }
+        }
+    }
+}
+
+// The families' blocks first, then the single leaves', in one launch; each
+// kind is dealt to the XCDs in contiguous runs (blocks of one task, and tasks
+// of one region, share an L2).
+template <int N, int NZ, typename ET>
+__global__ void __launch_bounds__(kThreads, (NZ > 1 && NZ * N >= 16) ? 2 : 3)
+    k_pw2pot_sym(int nd, const double2* __restrict__ tabS, int npw, const SymTask* __restrict__ tasks, int nfam,
+                 int nown, const ET* __restrict__ expn, size_t ks, Kinds kd, ZOut zo, Multi mu) {
+    constexpr int PF = sym5_parts<N, true>(), PO = sym5_parts<N, false>();
+    extern __shared__ double2 sm[];
+    const int b = blockIdx.x, nfb = nfam * PF;
+    const bool fam = b < nfb;
+    const int lin = fam ? xcd_task(b, nfb) : xcd_task(b - nfb, nown * PO);
+    const int tix = fam ? lin / PF : nfam + lin / PO, part = fam ? lin % PF : lin % PO;
+    const ProbPtrs* prob = nullptr;
+    if (mu.pp) {
+        prob = mu.pp + mu.tprob[tix];
+        npw = prob->g.npw;
+        tabS = prob->pw2potS;
+        expn = static_cast<const ET*>(prob->expn);
+    }
+    if (fam) pw2pot_sym_block<N, true, NZ, ET>(npw, nd, tabS, tasks + tix, part, expn, ks, kd, zo, prob, sm);
+    else pw2pot_sym_block<N, false, NZ, ET>(npw, nd, tabS, tasks + tix, part, expn, ks, kd, zo, prob, sm);
+}
+
+template <int N, int NZ>
+void launch_sym5_z(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks, const double2* expn,
+                   Kinds kd, const ZOut& zo, hipStream_t s, const Multi& mu) {
+    size_t lds = 0;
+    // a batch class holds smaller plane-wave counts too
+    for (int p = mu.pp ? 1 : t.npw; p <= t.npw; ++p) {
+        if (nfam) lds = std::max(lds, sym5_lds_entries(p, 2 * sym5_nx<N, true>(), 2 * sym_pairs<N, true>()));
+        if (nown) lds = std::max(lds, sym5_lds_entries(p, 2 * sym5_nx<N, false>(), 2 * sym_pairs<N, false>()));
+    }
+    lds *= sizeof(double2);
+    const dim3 grid((unsigned)(nfam * sym5_parts<N, true>() + nown * sym5_parts<N, false>())), block(kThreads);
+    if (t.expn_f32)
+        hipLaunchKernelGGL((k_pw2pot_sym<N, NZ, float2>), grid, block, lds, s, g.nd, t.pw2potS, t.npw, tasks, nfam, nown,
+                           reinterpret_cast<const float2*>(expn), t.pw2potS_ks, kd, zo, mu);
+    else
+        hipLaunchKernelGGL((k_pw2pot_sym<N, NZ, double2>), grid, block, lds, s, g.nd, t.pw2potS, t.npw, tasks, nfam, nown,
+                           expn, t.pw2potS_ks, kd, zo, mu);
+}
+
+// components zo.kz[a .. a + nz) as a group of their own
+ZOut zpart(const ZOut& zo, int a, int nz) {
+    ZOut r{};
+    r.nz = nz;
+    for (int q = 0; q < nz; ++q) {
+        r.kz[q] = zo.kz[a + q];
+        r.od[q] = zo.od[a + q];
+    }
+    return r;
+}
+
+template <int N>
+void launch_sym5(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks, const double2* expn,
+                 Kinds kd, const ZOut& zo, hipStream_t s, const Multi& mu) {
+    if (zo.nz == 1) {
+        launch_sym5_z<N, 1>(g, t, nfam, nown, tasks, expn, kd, zo, s, mu);
+    } else if (zo.nz == 2) {
+        launch_sym5_z<N, 2>(g, t, nfam, nown, tasks, expn, kd, zo, s, mu);
+    } else if constexpr (N <= 12) {
+        launch_sym5_z<N, 3>(g, t, nfam, nown, tasks, expn, kd, zo, s, mu);
+    } else {
+        // the sums of three z kinds exceed the registers
+        launch_sym5_z<N, 2>(g, t, nfam, nown, tasks, expn, kd, zpart(zo, 0, 2), s, mu);
+        launch_sym5_z<N, 1>(g, t, nfam, nown, tasks, expn, kd, zpart(zo, 2, 1), s, mu);
+    }
+}
+
+}  // namespace
+
+bool launch_pw2pot_sym(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks,
+                       const double2* expn, Kinds kd, const ZOut& zo, hipStream_t s, const Multi& mu) {
+    if (g.ndim != 3 || zo.nz < 1 || zo.nz > 3 || nfam + nown <= 0) return false;
+    switch (t.n) {
+        case 8: launch_sym5<8>(g, t, nfam, nown, tasks, expn, kd, zo, s, mu); return true;
+        case 12: launch_sym5<12>(g, t, nfam, nown, tasks, expn, kd, zo, s, mu); return true;
+        case 16: launch_sym5<16>(g, t, nfam, nown, tasks, expn, kd, zo, s, mu); return true;
+        default: return false;
+    }
+}
+
+}  // namespace fgt
