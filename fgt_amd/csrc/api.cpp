@@ -144,6 +144,7 @@ struct fgt_solver {
     int n_s5_fam = 0, n_s5_own = 0;   // families first, then single leaves
     DBuf d_p2pwS, d_fz_lev, d_fz_slot, d_fz_kids, d_fz_ksg;          // fused STEP 1+2 parents
     DBuf d_s1_box, d_s1_lev, d_s1_slot;                              // standalone STEP 1 leaves
+    DBuf d_s1_sym;     // fgt::SymTask list of the FP64 STEP 1 kernel: n_fz families, then n_s1 leaves
     DBuf d_mp_slot, d_mp_first, d_mp_count, d_mp_child, d_mp_sign, d_mp_acc;  // merges of non-leaf children
     std::vector<int> mp_level_off;
     int n_fz = 0, n_s1 = 0;
@@ -154,7 +155,7 @@ struct fgt_solver {
     // per shape class)
     struct HostLists {
         std::vector<fgt::PotTask> s5;
-        std::vector<fgt::SymTask> s5_sym;
+        std::vector<fgt::SymTask> s1_sym, s5_sym;
         std::vector<int> pcs_parent, pcs_child, pcs_sign;
         std::vector<int> fz_lev, fz_slot, fz_kids, fz_ksg, s1_box, s1_lev, s1_slot;
         std::vector<int> mp_slot, mp_first, mp_count, mp_child, mp_sign, mp_acc;
@@ -627,6 +628,7 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
         }
         S.d_p2pwS.upload(to_d2(t1));
         std::vector<int> fzl, fzs, fzk, fzg, s1b, s1l, s1s;
+        std::vector<fgt::SymTask> s1fam, s1own;
         std::vector<int> mps, mpf, mpc, mch, msg, macc;
         S.mp_level_off.assign(nl + 2, 0);
         for (int l = 0; l <= nl; ++l) {
@@ -638,6 +640,7 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
                         s1b.push_back(b);
                         s1l.push_back(l);
                         s1s.push_back(P.slot_of_box[b]);
+                        s1own.push_back({P.slot_of_box[b], l, {b, -1, -1, -1, -1, -1, -1, -1}});
                     }
                     continue;
                 }
@@ -670,6 +673,8 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
                 if (nk > 0) {
                     fzl.push_back(l);
                     fzs.push_back(P.slot_of_box[b]);
+                    s1fam.push_back({P.slot_of_box[b], l + 1, {-1, -1, -1, -1, -1, -1, -1, -1}});
+                    for (int c = 0; c < nk; ++c) s1fam.back().box[ksg[c]] = kids[c];
                     for (int c = 0; c < 8; ++c) {
                         fzk.push_back(kids[c]);
                         fzg.push_back(ksg[c]);
@@ -680,6 +685,9 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
         S.mp_level_off[nl + 1] = (int)mps.size();
         S.n_fz = (int)fzl.size();
         S.n_s1 = (int)s1b.size();
+        s1fam.insert(s1fam.end(), s1own.begin(), s1own.end());
+        S.d_s1_sym.upload(s1fam);
+        S.h.s1_sym = s1fam;
         S.d_fz_lev.upload(fzl);
         S.h.fz_lev = fzl;
         S.d_fz_slot.upload(fzs);
@@ -974,13 +982,10 @@ void execute(fgt_solver& S, hipStream_t st, bool timed, bool fork_near = false,
             // STEP 1: leaves at the cutoff level alone; every other PW leaf is
             // folded into its parent's expansion (STEP 1 + 2 fused), all levels
             // in one launch (they read only fvals)
-            fgt::launch_p2pw(g, t, S.n_s1, S.d_s1_box.as<int>(), S.d_s1_lev.as<int>(), S.d_s1_slot.as<int>(),
-                             fv, ex, st);
-            if (!fgt::p2pw_fused_3d(g, t, S.n_fz, S.d_fz_lev.as<int>(), S.d_fz_slot.as<int>(),
-                                    S.d_fz_kids.as<int>(), S.d_fz_ksg.as<int>(), fv,
-                                    ex, st))
-                throw std::runtime_error("fused STEP 1+2 kernel not available for this shape");
-            hcheck(hipGetLastError(), "k_p2pwF3 launch");
+            fgt::launch_p2pw_tasks(g, t, {S.n_s1, S.d_s1_box.as<int>(), S.d_s1_lev.as<int>(), S.d_s1_slot.as<int>(),
+                                          nullptr, S.n_fz, S.d_fz_lev.as<int>(), S.d_fz_slot.as<int>(),
+                                          S.d_fz_kids.as<int>(), S.d_fz_ksg.as<int>(), nullptr, S.n_fz, S.n_s1,
+                                          S.d_s1_sym.as<fgt::SymTask>(), nullptr}, fv, ex, st);
             mark(1);
             // STEP 2: non-leaf children, fine to coarse
             for (int l = P.nlevels - 1; l >= P.nlevstart; --l) {
@@ -1201,6 +1206,7 @@ struct BClass {
     int n_fz = 0;
     DBuf s1_box, s1_lev, s1_slot, s1_prob;
     int n_s1 = 0;
+    DBuf s1_sym, s1_symprob;   // SymTask list: n_fz families, then n_s1 leaves
     DBuf mp_slot, mp_first, mp_count, mp_child, mp_sign, mp_acc, mp_prob, mp_klev;
     std::vector<int> mp_phase;    // phase p: entries [mp_phase[p], mp_phase[p+1])
     DBuf m2l_toff, m2l_gent, m2l_soff, m2l_code, m2l_prob;
@@ -1363,7 +1369,7 @@ void build_classes(fgt_batch& B) {
         std::vector<int> mch, msg, pcsp, pcsc, pcsg;
         std::vector<fgt::PotTask> sib, own;
         std::vector<int> sibp, ownp;
-        std::vector<fgt::SymTask> sfam, sown;
+        std::vector<fgt::SymTask> sfam, sown, s1fam, s1own;
         std::vector<int> sfamp, sownp;
         int maxph2 = 0, maxph4 = 0;
         for (int q = 0; q < (int)C.members.size(); ++q) {
@@ -1393,6 +1399,8 @@ void build_classes(fgt_batch& B) {
             s1l.insert(s1l.end(), h.s1_lev.begin(), h.s1_lev.end());
             s1s.insert(s1s.end(), h.s1_slot.begin(), h.s1_slot.end());
             s1p.insert(s1p.end(), h.s1_box.size(), q);
+            s1fam.insert(s1fam.end(), h.s1_sym.begin(), h.s1_sym.begin() + S.n_fz);
+            s1own.insert(s1own.end(), h.s1_sym.begin() + S.n_fz, h.s1_sym.end());
             maxph2 = std::max(maxph2, P.nlevels - P.nlevstart);
             maxph4 = std::max(maxph4, P.nlevels - P.nlevstart);
             sib.insert(sib.end(), h.s5.begin(), h.s5.begin() + S.n_s5_sib);
@@ -1416,6 +1424,11 @@ void build_classes(fgt_batch& B) {
         C.s1_lev.upload(s1l);
         C.s1_slot.upload(s1s);
         C.s1_prob.upload(s1p);
+        s1fam.insert(s1fam.end(), s1own.begin(), s1own.end());
+        C.s1_sym.upload(s1fam);
+        std::vector<int> symp(fzp);
+        symp.insert(symp.end(), s1p.begin(), s1p.end());
+        C.s1_symprob.upload(symp);
         // STEP 2 phases (children arrays appended once per problem)
         std::vector<int> ms, mf, mc, ma, mp, mk;
         std::vector<int> chbase(C.members.size(), 0);
@@ -1537,13 +1550,12 @@ fgt::Multi multi(const BClass& C, const DBuf& prob, int off = 0, const DBuf* kle
 
 // Stages of one class (timed: per-stage events on st, for the tuner)
 void class_step1(const BClass& C, hipStream_t st) {
-    if (C.n_fz > 0 && !fgt::p2pw_fused_3d(C.g, C.t, C.n_fz, C.fz_lev.as<int>(), C.fz_slot.as<int>(),
-                                          C.fz_kids.as<int>(), C.fz_ksg.as<int>(), nullptr, nullptr, st,
-                                          multi(C, C.fz_prob)))
-        throw std::runtime_error("fused STEP 1+2 kernel not available for a batch class");
-    if (C.n_s1 > 0)
-        fgt::launch_p2pw(C.g, C.t, C.n_s1, C.s1_box.as<int>(), C.s1_lev.as<int>(), C.s1_slot.as<int>(), nullptr,
-                         nullptr, st, multi(C, C.s1_prob));
+    if (C.n_fz + C.n_s1 > 0)
+        fgt::launch_p2pw_tasks(C.g, C.t, {C.n_s1, C.s1_box.as<int>(), C.s1_lev.as<int>(), C.s1_slot.as<int>(),
+                                          C.s1_prob.as<int>(), C.n_fz, C.fz_lev.as<int>(), C.fz_slot.as<int>(),
+                                          C.fz_kids.as<int>(), C.fz_ksg.as<int>(), C.fz_prob.as<int>(), C.n_fz, C.n_s1,
+                                          C.s1_sym.as<fgt::SymTask>(), C.s1_symprob.as<int>()},
+                               nullptr, nullptr, st, C.pp.as<fgt::ProbPtrs>());
 }
 void class_step2(const BClass& C, hipStream_t st) {
     for (size_t ph = 0; ph + 1 < C.mp_phase.size(); ++ph) {

@@ -196,8 +196,9 @@ struct DevTables {
     size_t lds_limit;  // device LDS bytes per block
 };
 
-// Register-blocked 3-D STEP 1 / STEP 5 kernels (norder 8, 12, 16); return
-// false (nothing launched) when the shape is not covered.
+// 3-D STEP 1 / STEP 5 kernels (norder 8, 12, 16); each returns false (nothing
+// launched) when the shape is not covered.
+// STEP 1 with a reduced-precision x stage, leaves of the cutoff level
 bool launch_p2pw_3d(const Geom& g, const DevTables& t, int ntask, const int* box, const int* lev,
                     const int* slot, const double* fvals, double2* expn, hipStream_t s, size_t lds_limit,
                     const Multi& mu = Multi{});
@@ -216,17 +217,40 @@ bool pw2pot_3d_supported(const Geom& g, const DevTables& t);
 // STEP 5 runs its x stage on the reduced-precision matrix cores (else it
 // takes launch_pw2pot_sym)
 bool pw2pot_lowp(const DevTables& t);
-// Fused STEP 1 + 2 for parents with leaf children (3-D, N in {8,12,16}):
+// STEP 1 runs its x stage on the reduced-precision matrix cores (else it
+// takes launch_p2pw_sym)
+bool p2pw_lowp(const DevTables& t);
+// STEP 1 in FP64 arithmetic through the tables' symmetries: tasks [0, nfam)
+// families (their parent's expansion, STEP 2 folded in), then nown leaves of
+// the cutoff level
+bool launch_p2pw_sym(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks, const double* fvals,
+                     double2* expn, hipStream_t s, const Multi& mu = Multi{});
+// Fused STEP 1 + 2 with a reduced-precision x stage, for parents with leaf
+// children (3-D, N in {8,12,16}):
 // plev/pslot per parent, kids/ksg 8 per parent (leaf child box or -1, merge
 // sign bits).  Writes (overwrites) the parent's mp; returns false if not covered.
 bool p2pw_fused_3d(const Geom& g, const DevTables& t, int ntask, const int* plev, const int* pslot,
                    const int* kids, const int* ksg, const double* fvals, double2* expn, hipStream_t s,
                    const Multi& mu = Multi{});
 
+// 3-D STEP 1 in the form p2pw_lowp picks (throws when the shape is not
+// covered): leaves of the cutoff level, and parents with leaf children
+struct Step1Lists {
+    int n_s1;                 // reduced precision: leaves, then parents
+    const int *s1_box, *s1_lev, *s1_slot, *s1_prob;
+    int n_fz;
+    const int *fz_lev, *fz_slot, *fz_kids, *fz_ksg, *fz_prob;
+    int nfam, nown;           // SymTask list
+    const SymTask* sym;
+    const int* symprob;
+};
+void launch_p2pw_tasks(const Geom& g, const DevTables& t, const Step1Lists& l, const double* fvals, double2* expn,
+                       hipStream_t s, const ProbPtrs* pp = nullptr);
+
 // Stage launchers (stream-ordered; all arguments device pointers).
 void launch_p2pw(const Geom& g, const DevTables& t, int ntask, const int* box,
                  const int* lev, const int* slot, const double* fvals,
-                 double2* expn, hipStream_t s, const Multi& mu = Multi{});
+                 double2* expn, hipStream_t s);
 // par_acc (nullable): per parent, nonzero = add to the parent's current mp
 void launch_merge(const Geom& g, const DevTables& t, int ntask, const int* par_slot,
                   const int* par_first, const int* par_count, const int* pc_child,

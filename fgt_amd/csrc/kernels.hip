@@ -992,13 +992,29 @@ unsigned blocks_for(long long tot) { return (unsigned)((tot + kBlock - 1) / kBlo
 
 }  // namespace
 
-void launch_p2pw(const Geom& g, const DevTables& t, int ntask, const int* box, const int* lev,
-                 const int* slot, const double* fvals, double2* expn, hipStream_t s, const Multi& mu) {
-    if (ntask <= 0) return;
-    if (launch_p2pw_3d(g, t, ntask, box, lev, slot, fvals, expn, s, t.lds_limit, mu)) {
-        check(hipGetLastError(), "k_p2pw3 launch");
-        return;
+void launch_p2pw_tasks(const Geom& g, const DevTables& t, const Step1Lists& l, const double* fvals, double2* expn,
+                       hipStream_t s, const ProbPtrs* pp) {
+    Multi mu;
+    mu.pp = pp;
+    bool ok = true;
+    if (!p2pw_lowp(t)) {
+        mu.tprob = l.symprob;
+        if (l.nfam + l.nown > 0) ok = launch_p2pw_sym(g, t, l.nfam, l.nown, l.sym, fvals, expn, s, mu);
+    } else {
+        mu.tprob = l.s1_prob;
+        if (l.n_s1 > 0)
+            ok = launch_p2pw_3d(g, t, l.n_s1, l.s1_box, l.s1_lev, l.s1_slot, fvals, expn, s, t.lds_limit, mu);
+        mu.tprob = l.fz_prob;
+        if (ok && l.n_fz > 0)
+            ok = p2pw_fused_3d(g, t, l.n_fz, l.fz_lev, l.fz_slot, l.fz_kids, l.fz_ksg, fvals, expn, s, mu);
     }
+    if (!ok) throw std::runtime_error("3-D STEP 1 kernel not available for this shape");
+    check(hipGetLastError(), "3-D STEP 1 launch");
+}
+
+void launch_p2pw(const Geom& g, const DevTables& t, int ntask, const int* box, const int* lev,
+                 const int* slot, const double* fvals, double2* expn, hipStream_t s) {
+    if (ntask <= 0) return;
     if (t.expn_f32) throw std::runtime_error("FP32 expansions need the 3-D register-blocked kernels");
     if (g.ndim == 2) {
         const size_t lds2 = sizeof(double2) * ((size_t)t.npw * t.n + (size_t)t.n * g.pz) + sizeof(double) * t.n * t.n;

@@ -1,17 +1,15 @@
-// kernels_pw3.hip -- register-blocked 3-D plane-wave kernels for gfx950 (FP64).
+// kernels_pw3.hip -- 3-D plane-wave kernels with a reduced-precision x stage
+// on the matrix cores (gfx950); the FP64 forms are in kernels_sym3.hip.
 //
 // STEP 1 (values -> PW, g3d_tens_prod_to_pw, bfgt_pwrouts.f:153-222) and
 // STEP 5 (PW -> values, g3d_pw2pot, bfgt_pwrouts.f:719-790) for norder
 // N in {8, 12, 16}, one 256-thread block (4 waves) per task (a leaf, a
 // parent with leaf children, or up to four sibling leaves).
 //
-// Design: on the VALU, every contraction is arranged so that the 1-D table
-// operand is wave-uniform (its address depends only on loop counters and the
-// wave index), which lets it come from the scalar cache into SGPRs; the other
-// operand lives in VGPRs, so each v_fma_f64 has one scalar and one vector
-// source and LDS only carries the transposes between stages.  STEP 5's x
-// contraction for N = 12 and 16 runs on the FP64 matrix cores instead.  The half
-// (z) axis is processed in rounds of four slabs, one per wave.
+// The y and z stages run on the FP64 VALU with a wave-uniform 1-D table
+// operand (its address depends only on loop counters and the wave index, so
+// it comes from the scalar cache into SGPRs); LDS only carries the transposes
+// between stages.  The half (z) axis is processed in rounds of slabs.
 #include "kernels.h"
 
 #include <algorithm>
@@ -293,7 +291,7 @@ __global__ void __launch_bounds__(256) k_p2pw3(Geom g, const double2* __restrict
             }
             __syncthreads();
             // x: E[k3][k1][k2] = sum_m1 T[k1][m1] ff2[s][m1][k2]; wave = slab, lane = k2
-            if constexpr (XS >= 2) {
+            {
                 const int k3 = r + wave;
                 if (k3 < nh) {
                     ET* __restrict__ Ek = E + (size_t)k3 * npw * npw;
@@ -302,28 +300,6 @@ __global__ void __launch_bounds__(256) k_p2pw3(Geom g, const double2* __restrict
                         [&](int k2, int m1) { return sff2[(wave * N + m1) * npw + k2]; },
                         [&](int m1, int k1) { return T[k1 * N + m1]; },
                         [&](int k2, int k1, float2 v) { Ek[(size_t)k1 * npw + k2] = v; });
-                }
-            } else {
-                const int k3 = r + wave;
-                if (k3 < nh) {
-                    ET* __restrict__ Ek = E + (size_t)k3 * npw * npw;
-                    for (int c = 0; c < npw; c += 64) {
-                        const int k2 = c + lane;
-                        const bool act = k2 < npw;
-                        double2 f2[N];
-#pragma unroll
-                        for (int m1 = 0; m1 < N; ++m1)
-                            f2[m1] = act ? sff2[(wave * N + m1) * npw + k2] : make_double2(0.0, 0.0);
-                        for (int k1 = 0; k1 < npw; ++k1) {
-                            double2 a0 = make_double2(0.0, 0.0), a1 = make_double2(0.0, 0.0);
-#pragma unroll
-                            for (int m1 = 0; m1 < N; m1 += 2) {
-                                a0 = zfma(T[k1 * N + m1], f2[m1], a0);
-                                a1 = zfma(T[k1 * N + m1 + 1], f2[m1 + 1], a1);
-                            }
-                            if (act) stE(Ek + (size_t)k1 * npw + k2, make_double2(a0.x + a1.x, a0.y + a1.y));
-                        }
-                    }
                 }
             }
             __syncthreads();
@@ -501,7 +477,7 @@ __global__ void __launch_bounds__(256) k_p2pwF3(Geom g, const double2* __restric
             }
             __syncthreads();
             // x: E[k3][k1][k2] = sum_sx sum_m1 Tx^{sx}[k1][m1] F[sx][s][m1][k2]
-            if constexpr (XS >= 2) {
+            {
                 // K = (sx, m1); SR = 2: the two waves of a slab take alternate
                 // column tiles, SR = 4: one wave per slab takes them all
                 const int s = SR == 4 ? wave : (wave & 1), hlf = SR == 4 ? 0 : wave >> 1;
@@ -518,34 +494,6 @@ __global__ void __launch_bounds__(256) k_p2pwF3(Geom g, const double2* __restric
                         },
                         [&](int kk, int k1) { return kk >= N ? Txm[k1 * N + kk - N] : Txp[k1 * N + kk]; },
                         [&](int k2, int k1, float2 v) { Ek[(size_t)k1 * npw + k2] = v; });
-                }
-            } else {
-                const int s = wave & 1, hlf = wave >> 1;
-                const int k3 = r + s;
-                if (k3 < nh) {
-                    ET* __restrict__ Ek = E + (size_t)k3 * npw * npw;
-                    const int k1a = hlf ? (npw + 1) / 2 : 0, k1b = hlf ? npw : (npw + 1) / 2;
-                    const CTab2 Txp = T + base0 + 1 * per;
-                    const CTab2 Txm = T + base0 + 2 * per;
-                    for (int c = 0; c < npw; c += 64) {
-                        const int k2 = c + lane;
-                        const bool act = k2 < npw;
-                        double2 fp[N], fm[N];
-#pragma unroll
-                        for (int m1 = 0; m1 < N; ++m1) {
-                            fp[m1] = act ? sF[((0 * 2 + s) * N + m1) * npw + k2] : make_double2(0.0, 0.0);
-                            fm[m1] = act ? sF[((1 * 2 + s) * N + m1) * npw + k2] : make_double2(0.0, 0.0);
-                        }
-                        for (int k1 = k1a; k1 < k1b; ++k1) {
-                            double2 a0 = make_double2(0.0, 0.0), a1 = make_double2(0.0, 0.0);
-#pragma unroll
-                            for (int m1 = 0; m1 < N; ++m1) {
-                                a0 = zfma(Txp[k1 * N + m1], fp[m1], a0);
-                                a1 = zfma(Txm[k1 * N + m1], fm[m1], a1);
-                            }
-                            if (act) stE(Ek + (size_t)k1 * npw + k2, make_double2(a0.x + a1.x, a0.y + a1.y));
-                        }
-                    }
                 }
             }
             __syncthreads();
@@ -963,32 +911,18 @@ __global__ void __launch_bounds__(256, 2) k_pw2pot3(Geom g, const double2* __res
     }
 }
 
-// STEP 1 x stage on the reduced-precision matrix cores?
-bool use_lowp1(const DevTables& t) {
-    if (t.prec < 1 || t.npw > kLowpMaxPw) return false;
-    return t.xs1 >= 0 ? t.xs1 == 2 : (lowp_stages(t.prec) & 1) != 0;
-}
-
 template <int N>
 bool try_p2pw3(const Geom& g, const DevTables& t, int ntask, const int* box, const int* lev, const int* slot,
                const double* fvals, double2* expn, hipStream_t s, size_t lds_limit, const Multi& mu) {
     const size_t lds = sizeof(double2) * std::max(4 * (size_t)N * N, 4 * (size_t)N * t.npw);
     if (lds > lds_limit) return false;
-    if (use_lowp1(t)) {
-        float2* e32 = reinterpret_cast<float2*>(expn);
-        if (t.prec == 2)
-            hipLaunchKernelGGL((k_p2pw3<N, 3, float2>), dim3(ntask), dim3(256), lds, s, g, t.p2pw, t.npw, box, lev,
-                               slot, fvals, e32, mu);
-        else
-            hipLaunchKernelGGL((k_p2pw3<N, 2, float2>), dim3(ntask), dim3(256), lds, s, g, t.p2pw, t.npw, box, lev,
-                               slot, fvals, e32, mu);
-    } else if (t.expn_f32) {
-        hipLaunchKernelGGL((k_p2pw3<N, 0, float2>), dim3(ntask), dim3(256), lds, s, g, t.p2pw, t.npw, box, lev, slot,
-                           fvals, reinterpret_cast<float2*>(expn), mu);
-    } else {
-        hipLaunchKernelGGL((k_p2pw3<N, 0, double2>), dim3(ntask), dim3(256), lds, s, g, t.p2pw, t.npw, box, lev,
-                           slot, fvals, expn, mu);
-    }
+    float2* e32 = reinterpret_cast<float2*>(expn);
+    if (t.prec == 2)
+        hipLaunchKernelGGL((k_p2pw3<N, 3, float2>), dim3(ntask), dim3(256), lds, s, g, t.p2pw, t.npw, box, lev, slot,
+                           fvals, e32, mu);
+    else
+        hipLaunchKernelGGL((k_p2pw3<N, 2, float2>), dim3(ntask), dim3(256), lds, s, g, t.p2pw, t.npw, box, lev, slot,
+                           fvals, e32, mu);
     return true;
 }
 
@@ -1047,43 +981,34 @@ bool try_pw2pot3(const Geom& g, const DevTables& t, int ntask, int nsib, const P
     return true;
 }
 
-// slabs per round of the fused STEP 1 kernel: four for norder 8 with the
-// matrix-core x stage while sF (8 n npw complex) leaves room for three blocks
+// slabs per round of the fused STEP 1 kernel: four for norder 8 while sF (8 n npw complex) leaves room for three blocks
 // per CU, else two
 int p2pwF3_slabs(int n, const DevTables& t) {
-    return (n == 8 && use_lowp1(t) && t.npw <= 48) ? 4 : 2;
+    return n == 8 && t.npw <= 48 ? 4 : 2;
 }
 
 template <int N>
 void launch_p2pwF3_typed(const Geom& g, const DevTables& t, unsigned nblk, size_t lds, const int* plev,
                          const int* pslot, const int* kids, const int* ksg, const double* fvals, double2* expn,
                          hipStream_t s, const Multi& mu) {
-    if (use_lowp1(t)) {
-        float2* e32 = reinterpret_cast<float2*>(expn);
-        if constexpr (N == 8) {
-            if (p2pwF3_slabs(N, t) == 4) {
-                if (t.prec == 2)
-                    hipLaunchKernelGGL((k_p2pwF3<N, 3, float2, 4>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS,
-                                       t.npw, plev, pslot, kids, ksg, fvals, e32, mu);
-                else
-                    hipLaunchKernelGGL((k_p2pwF3<N, 2, float2, 4>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS,
-                                       t.npw, plev, pslot, kids, ksg, fvals, e32, mu);
-                return;
-            }
+    float2* e32 = reinterpret_cast<float2*>(expn);
+    if constexpr (N == 8) {
+        if (p2pwF3_slabs(N, t) == 4) {
+            if (t.prec == 2)
+                hipLaunchKernelGGL((k_p2pwF3<N, 3, float2, 4>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS, t.npw, plev,
+                                   pslot, kids, ksg, fvals, e32, mu);
+            else
+                hipLaunchKernelGGL((k_p2pwF3<N, 2, float2, 4>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS, t.npw, plev,
+                                   pslot, kids, ksg, fvals, e32, mu);
+            return;
         }
-        if (t.prec == 2)
-            hipLaunchKernelGGL((k_p2pwF3<N, 3, float2>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS, t.npw, plev,
-                               pslot, kids, ksg, fvals, e32, mu);
-        else
-            hipLaunchKernelGGL((k_p2pwF3<N, 2, float2>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS, t.npw, plev,
-                               pslot, kids, ksg, fvals, e32, mu);
-    } else if (t.expn_f32) {
-        hipLaunchKernelGGL((k_p2pwF3<N, 0, float2>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS, t.npw, plev, pslot,
-                           kids, ksg, fvals, reinterpret_cast<float2*>(expn), mu);
-    } else {
-        hipLaunchKernelGGL((k_p2pwF3<N, 0, double2>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS, t.npw, plev,
-                           pslot, kids, ksg, fvals, expn, mu);
     }
+    if (t.prec == 2)
+        hipLaunchKernelGGL((k_p2pwF3<N, 3, float2>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS, t.npw, plev, pslot,
+                           kids, ksg, fvals, e32, mu);
+    else
+        hipLaunchKernelGGL((k_p2pwF3<N, 2, float2>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS, t.npw, plev, pslot,
+                           kids, ksg, fvals, e32, mu);
 }
 
 }  // namespace
@@ -1101,6 +1026,11 @@ int lowp_stages(int prec) {
     // slower: 50 x 50-class outputs pad to 64-row / 16-column tiles with K = 8
     // or 16); BF16 hi/lo runs both stages on the matrix cores
     return v >= 0 ? v : (prec == 2 ? 3 : 2);
+}
+
+bool p2pw_lowp(const DevTables& t) {
+    if (t.prec < 1 || t.npw > kLowpMaxPw) return false;
+    return t.xs1 >= 0 ? t.xs1 == 2 : (lowp_stages(t.prec) & 1) != 0;
 }
 
 bool pw2pot_lowp(const DevTables& t) {

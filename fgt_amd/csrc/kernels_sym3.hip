@@ -386,7 +386,236 @@ void launch_sym5(const Geom& g, const DevTables& t, int nfam, int nown, const Sy
     }
 }
 
+// ---------------------------------------------------------------- STEP 1
+// k3 slabs per round: one row (slab, x node) of the y stage per lane
+template <int N, bool FAM>
+constexpr int sym1_slabs() { return 32 / sym_pairs<N, FAM>() > 8 ? 8 : 32 / sym_pairs<N, FAM>(); }
+// double2 entries of the block's LDS: sH [slab][y node][x node] and sF
+// [slab][x node][k2] (odd row length) share it
+template <int N, bool FAM>
+size_t sym1_lds_entries(int npw) {
+    const size_t nod = 2 * sym_pairs<N, FAM>(), sr = sym1_slabs<N, FAM>();
+    return std::max(sr * nod * nod, sr * nod * (size_t)(npw | 1));
+}
+
+// One block: part kp of kparts of the k3 rounds of one task, whose expansion
+// (the leaf's, or the parent's with the STEP 2 shift folded in) it overwrites.
+// Per round of SR slabs:
+//   z: thread = (x node, y node) column, its values folded over the z pairs
+//      (kept in registers for all rounds where a thread has one column);
+//   y: lane = (slab, x node), folded over the y pairs, k2 pairs dealt to the
+//      waves;
+//   x: lane = (slab, k2) column, folded over the x pairs, k1 pairs split over
+//      the waves that share a batch of columns; both frequencies of a pair
+//      are stored as they are formed.
+// Bound by the expansion writes and each round's latency (norder 8, npw 28,
+// 8382 leaves: 68 us for 210 MB, 171 us with the plain complex products;
+// norder 12, npw 60, 4250 leaves: 314 us for 1 GB, 639 before).  The part
+// count fills the device four blocks deep at most: each part reads the
+// values again.
+template <int N, bool FAM, typename ET>
+__device__ __forceinline__ void p2pw_sym_block(int npw, int nd, const double2* __restrict__ tabS,
+                                               const SymTask* __restrict__ T, int kp, int kparts,
+                                               const double* __restrict__ fvals, ET* __restrict__ expn,
+                                               double2* __restrict__ sm) {
+    constexpr int NP = sym_pairs<N, FAM>(), NOD = 2 * NP, COLS = NOD * NOD, SR = sym1_slabs<N, FAM>();
+    constexpr int NC = (COLS + kThreads - 1) / kThreads;   // columns per thread
+    constexpr int ZG = COLS <= 64 ? 4 : (COLS <= 128 ? 2 : 1);   // thread groups sharing the slabs
+    constexpr int V = FAM ? 1 : 0;
+    static_assert(SR * NOD <= 64, "one y row per lane");
+    const int nh = (npw + 1) >> 1;
+    const int nround = (nh + SR - 1) / SR;
+    const int rb = SR * (kp * nround / kparts), re = min(nh, SR * ((kp + 1) * nround / kparts));
+    if (rb >= re) return;
+    const int PW = npw | 1;
+    const long long row3 = (3LL * __builtin_amdgcn_readfirstlane(T->lev) + V) * ((long long)npw * N);
+    const CTab2 U = ctab(tabS) + row3;   // U[k*N + pair]
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63;
+    const int slot = __builtin_amdgcn_readfirstlane(T->slot);
+    warm_table(U, nh * N, wave);
+    // one folded z column: values of side a plus / minus those of side b
+    auto fold = [&](int col, int ind, double (&fe)[NP], double (&fo)[NP]) {
+        const int zx = col % NOD, zy = col / NOD;
+        const int bx = zx >= NP, by = zy >= NP;
+        const int px = zx - bx * NP, py = zy - by * NP;
+        // the middle node of a leaf with odd n has no mirror image
+        const bool on = FAM || !((bx && 2 * px + 1 == N) || (by && 2 * py + 1 == N));
+        const int cxy = FAM ? bx | by << 1 : 0;
+        const int ba = on ? T->box[cxy] : -1, bb = on ? T->box[FAM ? cxy | 4 : 0] : -1;
+        const int node = (bx ? N - 1 - px : px) + N * (by ? N - 1 - py : py);
+        const double* __restrict__ pa = fvals + ((size_t)max(ba, 0) * (N * N * N) + node) * nd + ind;
+        const double* __restrict__ pb = fvals + ((size_t)max(bb, 0) * (N * N * N) + node) * nd + ind;
+        const int st = N * N * nd;
+        double a[NP], b[NP];
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+            a[q] = ba >= 0 ? pa[q * st] : 0.0;
+            b[q] = (bb >= 0 && (FAM || 2 * q + 1 != N)) ? pb[(N - 1 - q) * st] : 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+            fe[q] = a[q] + b[q];
+            fo[q] = a[q] - b[q];
+        }
+    };
+    const int zgrp = ZG == 1 ? 0 : (ZG == 2 ? wave >> 1 : wave);
+    const int zcol = ZG == 1 ? tid : (ZG == 2 ? (tid & 127) : lane);
+    for (int ind = 0; ind < nd; ++ind) {
+        ET* __restrict__ E = expn + (size_t)(slot * 2 * nd + ind) * (size_t)(nh * npw * npw);
+        double fe[NP], fo[NP];
+        if (NC == 1 && zcol < COLS) fold(zcol, ind, fe, fo);
+        for (int r = rb; r < re; r += SR) {
+            // ---- z
+#pragma unroll 1
+            for (int c = 0; c < NC; ++c) {
+                const int col = zcol + c * kThreads;
+                if (col < COLS) {
+                    if (NC > 1) fold(col, ind, fe, fo);
+                    for (int s = zgrp; s < SR; s += ZG) {
+                        const CTab2 u = U + (long long)min(r + s, nh - 1) * N;
+                        double hr = 0.0, hi = 0.0;
+#pragma unroll
+                        for (int q = 0; q < NP; ++q) {
+                            const double2 t = u[q];
+                            hr += t.x * fe[q];
+                            hi += t.y * fo[q];
+                        }
+                        sm[s * COLS + col] = make_double2(hr, hi);
+                    }
+                }
+            }
+            __syncthreads();
+            // ---- y
+            {
+                const int row = min(lane, SR * NOD - 1);
+                const double2* __restrict__ h = sm + (row / NOD) * COLS + row % NOD;
+                double2 S[NP], D[NP];
+#pragma unroll
+                for (int q = 0; q < NP; ++q) {
+                    const double2 a = h[q * NOD], b = h[(NP + q) * NOD];
+                    S[q] = cplus(a, b);
+                    D[q] = cminus(a, b);
+                }
+                __syncthreads();   // sH is read; sF takes its place
+                double2* __restrict__ o = sm + row * PW;
+                for (int k = wave; k < nh; k += kThreads / 64) {
+                    double2 P = make_double2(0.0, 0.0), Q = make_double2(0.0, 0.0);
+#pragma unroll
+                    for (int q = 0; q < NP; ++q) {
+                        const double2 t = U[(long long)k * N + q];
+                        P.x += t.x * S[q].x;
+                        P.y += t.x * S[q].y;
+                        Q.x += t.y * D[q].x;
+                        Q.y += t.y * D[q].y;
+                    }
+                    if (lane < SR * NOD) {
+                        o[npw - 1 - k] = make_double2(P.x + Q.y, P.y - Q.x);
+                        o[k] = make_double2(P.x - Q.y, P.y + Q.x);
+                    }
+                }
+            }
+            __syncthreads();
+            // ---- x
+            {
+                const int cols = min(SR, nh - r) * npw;
+                const int nb = (cols + 63) >> 6;
+                const int ks = nb == 1 ? 4 : (nb == 2 ? 2 : 1);   // waves per batch of columns
+                const int kq = ks == 4 ? wave : (ks == 2 ? wave >> 1 : 0);
+                const int ka = kq * nh / ks, kb = (kq + 1) * nh / ks;
+                for (int b = ks == 4 ? 0 : (ks == 2 ? wave & 1 : wave); b < nb; b += 4 / ks) {
+                    const int c = min(64 * b + lane, cols - 1);
+                    const bool act = 64 * b + lane < cols;
+                    const int s = c / npw, k2 = c - s * npw;
+                    const double2* __restrict__ f = sm + s * NOD * PW + k2;
+                    double2 S[NP], D[NP];
+#pragma unroll
+                    for (int q = 0; q < NP; ++q) {
+                        const double2 u = f[q * PW], v = f[(NP + q) * PW];
+                        S[q] = cplus(u, v);
+                        D[q] = cminus(u, v);
+                    }
+                    // row base scalar, column offset per lane
+                    const unsigned co = (unsigned)((r + s) * npw * npw + k2);
+                    for (int k = ka; k < kb; ++k) {
+                        double2 P = make_double2(0.0, 0.0), Q = make_double2(0.0, 0.0);
+#pragma unroll
+                        for (int q = 0; q < NP; ++q) {
+                            const double2 t = U[(long long)k * N + q];
+                            P.x += t.x * S[q].x;
+                            P.y += t.x * S[q].y;
+                            Q.x += t.y * D[q].x;
+                            Q.y += t.y * D[q].y;
+                        }
+                        if (act) {
+                            stE(E + (size_t)(k * npw) + co, make_double2(P.x - Q.y, P.y + Q.x));
+                            if (2 * k + 1 != npw)
+                                stE(E + (size_t)((npw - 1 - k) * npw) + co, make_double2(P.x + Q.y, P.y - Q.x));
+                        }
+                    }
+                }
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// The families' blocks first, then the single leaves' (see k_pw2pot_sym).
+template <int N, typename ET>
+__global__ void __launch_bounds__(kThreads, 2)
+    k_p2pw_sym(int nd, const double2* __restrict__ tabS, int npw, const SymTask* __restrict__ tasks, int nfam,
+               int nown, int kfam, int kown, const double* __restrict__ fvals, ET* __restrict__ expn, Multi mu) {
+    extern __shared__ double2 sm[];
+    const int b = blockIdx.x, nfb = nfam * kfam;
+    const bool fam = b < nfb;
+    const int lin = fam ? xcd_task(b, nfb) : xcd_task(b - nfb, nown * kown);
+    const int tix = fam ? lin / kfam : nfam + lin / kown, kp = fam ? lin % kfam : lin % kown;
+    if (mu.pp) {
+        const ProbPtrs* prob = mu.pp + mu.tprob[tix];
+        npw = prob->g.npw;
+        tabS = prob->p2pwS;
+        fvals = prob->fvals;
+        expn = static_cast<ET*>(prob->expn);
+    }
+    if (fam) p2pw_sym_block<N, true, ET>(npw, nd, tabS, tasks + tix, kp, kfam, fvals, expn, sm);
+    else p2pw_sym_block<N, false, ET>(npw, nd, tabS, tasks + tix, kp, kown, fvals, expn, sm);
+}
+
+template <int N>
+void launch_sym1(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks, const double* fvals,
+                 double2* expn, hipStream_t s, const Multi& mu) {
+    size_t lds = 0;
+    if (nfam) lds = std::max(lds, sym1_lds_entries<N, true>(t.npw));
+    if (nown) lds = std::max(lds, sym1_lds_entries<N, false>(t.npw));
+    lds *= sizeof(double2);
+    // parts of the rounds per task: enough blocks to fill the device
+    const auto parts = [&](int n, int sr) {
+        const int rounds = ((t.npw + 1) / 2 + sr - 1) / sr;
+        return n > 0 ? std::max(1, std::min(std::min(4, rounds), 4096 / n)) : 1;
+    };
+    const int kf = parts(nfam, sym1_slabs<N, true>()), ko = parts(nown, sym1_slabs<N, false>());
+    const dim3 grid((unsigned)(nfam * kf + nown * ko)), block(kThreads);
+    if (t.expn_f32)
+        hipLaunchKernelGGL((k_p2pw_sym<N, float2>), grid, block, lds, s, g.nd, t.p2pwS, t.npw, tasks, nfam, nown, kf,
+                           ko, fvals, reinterpret_cast<float2*>(expn), mu);
+    else
+        hipLaunchKernelGGL((k_p2pw_sym<N, double2>), grid, block, lds, s, g.nd, t.p2pwS, t.npw, tasks, nfam, nown, kf,
+                           ko, fvals, expn, mu);
+}
+
 }  // namespace
+
+bool launch_p2pw_sym(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks, const double* fvals,
+                     double2* expn, hipStream_t s, const Multi& mu) {
+    if (g.ndim != 3 || nfam + nown <= 0) return false;
+    switch (t.n) {
+        case 8: launch_sym1<8>(g, t, nfam, nown, tasks, fvals, expn, s, mu); return true;
+        case 12: launch_sym1<12>(g, t, nfam, nown, tasks, fvals, expn, s, mu); return true;
+        case 16: launch_sym1<16>(g, t, nfam, nown, tasks, fvals, expn, s, mu); return true;
+        default: return false;
+    }
+}
 
 bool launch_pw2pot_sym(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks,
                        const double2* expn, Kinds kd, const ZOut& zo, hipStream_t s, const Multi& mu) {
