@@ -117,7 +117,7 @@ struct fgt_solver {
     fgt::Geom geom{};
     fgt::DevTables tabs{};
     // tables
-    DBuf d_p2pw, d_pw2pot, d_pw2potT, d_pw2potS, d_wms, d_wm2l, d_one, d_loctab, d_locband;
+    DBuf d_p2pw, d_pw2pot, d_pw2potS, d_wms, d_wm2l, d_loctab, d_locband;
     // data
     DBuf d_fvals, d_pot, d_expn;
     int ifpgh = 1;          // 1 pot, 2 + grad, 3 + hess
@@ -129,7 +129,6 @@ struct fgt_solver {
     // lists
     DBuf d_leaf_box, d_leaf_lev, d_leaf_slot;
     DBuf d_par_slot, d_par_first, d_par_count, d_pc_parent, d_pc_child, d_pc_sign, d_pc_sign_split;
-    DBuf d_m2l_tgt, d_m2l_off, d_m2l_src, d_m2l_idx;
     DBuf d_m2l_toff, d_m2l_poff, d_m2l_soff, d_m2l_so;   // STEP 3 entry streams per group
     int n_m2l_groups = 0;
     DBuf d_mb_toff, d_mb_gent, d_mb_soff, d_mb_code;     // STEP 3 over sibling bricks
@@ -138,6 +137,7 @@ struct fgt_solver {
     DBuf d_dir_tgt, d_dir_lev, d_dir_off, d_dir_src, d_dir_code, d_dir_flags;
     // 3-D fast path: STEP 4 folded into STEP 5 for leaves below the cutoff level
     bool fast3d = false;
+    bool lowp3d = false;   // the reduced-precision kernels cover the problem as well
     DBuf d_s5_tasks;   // fgt::PotTask list of the reduced-precision STEP 5 kernel
     int n_s5 = 0, n_s5_sib = 0;   // tasks, of which the first n_s5_sib are sibling tasks
     DBuf d_s5_sym;     // fgt::SymTask list of the FP64 STEP 5 kernel
@@ -159,8 +159,6 @@ struct fgt_solver {
         std::vector<int> pcs_parent, pcs_child, pcs_sign;
         std::vector<int> fz_lev, fz_slot, fz_kids, fz_ksg, s1_box, s1_lev, s1_slot;
         std::vector<int> mp_slot, mp_first, mp_count, mp_child, mp_sign, mp_acc;
-        std::vector<long long> m2l_toff, m2l_soff;
-        std::vector<int> m2l_gent, m2l_code;
         std::vector<int> dir_tgt, dir_lev, dir_off, dir_src, dir_code, dir_flags;
     } h;
     // STEP 6 on a second stream, overlapping STEPs 1-4 (it reads only fvals;
@@ -463,32 +461,24 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
 
     S.d_loctab.upload(P.loctab);
     S.d_locband.upload(P.locband);
-    std::vector<double2> one{make_double2(1.0, 0.0)};
-    S.d_one.upload(one);
     if (P.do_pw) {
         S.d_p2pw.upload(to_d2(P.p2pw));
         S.d_pw2pot.upload(to_d2(P.pw2pot));
-        std::vector<fgt::cplx> tr(P.pw2pot.size());
-        const size_t per = (size_t)n * P.npw;
-        for (size_t l = 0; l * per < P.pw2pot.size(); ++l)
-            for (int i = 0; i < n; ++i)
-                for (int k = 0; k < P.npw; ++k) tr[l * per + (size_t)k * n + i] = P.pw2pot[l * per + (size_t)i * P.npw + k];
-        S.d_pw2potT.upload(to_d2(tr));
         S.d_wms.upload(to_d2(P.wms));
         S.d_wm2l.upload(to_d2(P.wm2l));
     }
     fgt::DevTables& t = S.tabs;
     t.p2pw = S.d_p2pw.as<double2>();
     t.pw2pot = S.d_pw2pot.as<double2>();
-    t.pw2potT = S.d_pw2potT.as<double2>();
     t.pw2pot_ks = P.pw2pot_ks;
     t.loctab_ks = P.loctab_ks;
     t.lds_limit = lds_limit;
     t.n = n;
     t.npw = P.npw;
-    S.fast3d = P.do_pw && fgt::pw2pot_3d_supported(g, t);
+    S.fast3d = P.do_pw && fgt::sym3_supported(g, t);
+    S.lowp3d = S.fast3d && fgt::pw2pot_3d_supported(g, t);
     if (S.fast3d) compact_slots(S.plan);
-    t.prec = mode_precision(prec_mode, P.eps, S.fast3d);
+    t.prec = mode_precision(prec_mode, P.eps, S.lowp3d);
     t.expn_f32 = t.prec > 0 ? 1 : 0;
     if (P.do_pw) alloc_expansions(S, t.expn_f32 ? sizeof(float2) : sizeof(double2));
     if (S.fast3d) {
@@ -581,7 +571,7 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
         S.n_s5_sib = (int)fam.size();
         fam.insert(fam.end(), own.begin(), own.end());
         S.n_s5 = (int)fam.size();
-        S.d_s5_tasks.upload(fam);
+        if (S.lowp3d) S.d_s5_tasks.upload(fam);
         S.h.s5 = fam;
         // split entries, keeping non-leaf children only
         std::vector<int> pp, pcc, psg;
@@ -688,19 +678,21 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
         s1fam.insert(s1fam.end(), s1own.begin(), s1own.end());
         S.d_s1_sym.upload(s1fam);
         S.h.s1_sym = s1fam;
-        S.d_fz_lev.upload(fzl);
+        if (S.lowp3d) {
+            S.d_fz_lev.upload(fzl);
+            S.d_fz_slot.upload(fzs);
+            S.d_fz_kids.upload(fzk);
+            S.d_fz_ksg.upload(fzg);
+            S.d_s1_box.upload(s1b);
+            S.d_s1_lev.upload(s1l);
+            S.d_s1_slot.upload(s1s);
+        }
         S.h.fz_lev = fzl;
-        S.d_fz_slot.upload(fzs);
         S.h.fz_slot = fzs;
-        S.d_fz_kids.upload(fzk);
         S.h.fz_kids = fzk;
-        S.d_fz_ksg.upload(fzg);
         S.h.fz_ksg = fzg;
-        S.d_s1_box.upload(s1b);
         S.h.s1_box = s1b;
-        S.d_s1_lev.upload(s1l);
         S.h.s1_lev = s1l;
-        S.d_s1_slot.upload(s1s);
         S.h.s1_slot = s1s;
         S.d_mp_slot.upload(mps);
         S.h.mp_slot = mps;
@@ -719,58 +711,50 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
     t.pw2potS = S.d_pw2potS.as<double2>();
     t.wms = S.d_wms.as<double2>();
     t.wm2l = S.d_wm2l.as<double2>();
-    t.one = S.d_one.as<double2>();
     t.loctab = S.d_loctab.as<double>();
     t.locband = S.d_locband.as<int>();
     t.n = n;
     t.npw = P.npw;
 
-    // work lists
-    S.d_leaf_box.upload(P.leaf_box);
-    S.d_leaf_lev.upload(P.leaf_lev);
-    S.d_leaf_slot.upload(P.leaf_slot);
-    S.d_par_slot.upload(P.par_slot);
-    S.d_par_first.upload(P.par_first);
-    S.d_par_count.upload(P.par_count);
-    S.d_pc_parent.upload(P.pc_parent);
-    S.d_pc_child.upload(P.pc_child);
-    std::vector<int> sg(P.pc_sign.size()), sgs(P.pc_sign.size());
-    for (size_t i = 0; i < sg.size(); ++i) {
-        sg[i] = map_sign(ndim, P.pc_sign[i]);
-        sgs[i] = sg[i] ^ real_mask(ndim);
+    // work lists of the general path
+    if (!S.fast3d) {
+        S.d_leaf_box.upload(P.leaf_box);
+        S.d_leaf_lev.upload(P.leaf_lev);
+        S.d_leaf_slot.upload(P.leaf_slot);
+        S.d_par_slot.upload(P.par_slot);
+        S.d_par_first.upload(P.par_first);
+        S.d_par_count.upload(P.par_count);
+        S.d_pc_parent.upload(P.pc_parent);
+        S.d_pc_child.upload(P.pc_child);
+        std::vector<int> sg(P.pc_sign.size()), sgs(P.pc_sign.size());
+        for (size_t i = 0; i < sg.size(); ++i) {
+            sg[i] = map_sign(ndim, P.pc_sign[i]);
+            sgs[i] = sg[i] ^ real_mask(ndim);
+        }
+        S.d_pc_sign.upload(sg);
+        S.d_pc_sign_split.upload(sgs);
     }
-    S.d_pc_sign.upload(sg);
-    S.d_pc_sign_split.upload(sgs);
-    S.d_m2l_tgt.upload(P.m2l_tgt);
-    S.d_m2l_off.upload(P.m2l_off);
-    S.d_m2l_src.upload(P.m2l_src);
-    std::vector<int> mi(P.m2l_idx.size());
-    for (size_t i = 0; i < mi.size(); ++i) mi[i] = map_m2l(ndim, P.m2l_idx[i]);
-    S.d_m2l_idx.upload(mi);
     if (P.do_pw) {
+        // STEP 3 over sibling bricks where the lists allow them, else over
+        // target groups
         std::vector<long long> toff, soff;
         std::vector<int> gent, code;
-        S.n_m2l_groups = m2l_streams(P, fgt::m2l_group(), toff, gent, soff, code);
-        S.d_m2l_toff.upload(toff);
-        S.h.m2l_toff = toff;
-        S.d_m2l_poff.upload(gent);
-        S.h.m2l_gent = gent;
-        S.d_m2l_soff.upload(soff);
-        S.h.m2l_soff = soff;
-        S.d_m2l_so.upload(code);
-        S.h.m2l_code = code;
         if (fgt::m2l_brick_env() != 0) {
-            std::vector<long long> bt, bs;
-            std::vector<int> bg, bc;
             bool geo = false;
-            S.n_m2l_bricks = m2l_bricks(P, bt, bg, bs, bc, &geo);
+            S.n_m2l_bricks = m2l_bricks(P, toff, gent, soff, code, &geo);
             S.m2l_sep_ok = S.n_m2l_bricks > 0 && geo;
-            if (S.n_m2l_bricks > 0) {
-                S.d_mb_toff.upload(bt);
-                S.d_mb_gent.upload(bg);
-                S.d_mb_soff.upload(bs);
-                S.d_mb_code.upload(bc);
-            }
+        }
+        if (S.n_m2l_bricks > 0) {
+            S.d_mb_toff.upload(toff);
+            S.d_mb_gent.upload(gent);
+            S.d_mb_soff.upload(soff);
+            S.d_mb_code.upload(code);
+        } else {
+            S.n_m2l_groups = m2l_streams(P, fgt::m2l_group(), toff, gent, soff, code);
+            S.d_m2l_toff.upload(toff);
+            S.d_m2l_poff.upload(gent);
+            S.d_m2l_soff.upload(soff);
+            S.d_m2l_so.upload(code);
         }
     }
 
@@ -1343,7 +1327,7 @@ void build_classes(fgt_batch& B) {
             if (B.solvers[i]->plan.npw > B.solvers[big]->plan.npw) big = i;
         C.g = B.solvers[big]->geom;
         C.t = B.solvers[big]->tabs;
-        C.t.p2pw = C.t.p2pwS = C.t.pw2pot = C.t.pw2potT = C.t.pw2potS = C.t.wms = C.t.wm2l = nullptr;
+        C.t.p2pw = C.t.p2pwS = C.t.pw2pot = C.t.pw2potS = C.t.wms = C.t.wm2l = nullptr;
         C.t.loctab = nullptr;
         C.t.pw2potS_ks = C.t.loctab_ks = 0;   // the value tables (kind 0) only
         C.m2l_ept2_ok = true;
@@ -2722,7 +2706,7 @@ int fgt_solver_set_precision(fgt_solver* s, int mode) {
             throw std::invalid_argument("BF16 hi/lo contractions need eps >= 1e-3 (this plan's eps is smaller)");
         if (mode >= 1 && !s->plan.do_pw)
             throw std::invalid_argument("mixed precision: this plan forms no plane-wave expansions (near field only)");
-        if (mode >= 1 && !s->fast3d)
+        if (mode >= 1 && !s->lowp3d)
             throw std::invalid_argument("mixed precision needs the 3-D register-blocked path (ndim 3, norder 8/12/16)");
         const int f32 = mode >= 1 ? 1 : 0;
         if (f32 != s->tabs.expn_f32) {
@@ -2814,7 +2798,7 @@ int fgt_batch_set_precision(fgt_batch* b, int mode, double eps_min, int* nmixed)
         int cnt = 0;
         for (auto& S : b->solvers) {
             const double eps = S->plan.eps;
-            const bool ok = mode >= 1 && S->plan.do_pw && S->fast3d && eps >= eps_min;
+            const bool ok = mode >= 1 && S->plan.do_pw && S->lowp3d && eps >= eps_min;
             int m = 0;
             if (ok) {
                 if (mode == 1) m = eps >= kEpsFp32 ? 1 : 0;

@@ -157,11 +157,9 @@ struct Multi {
 struct DevTables {
     // per level l: value->PW  T[l][k][m] (k < npw, m < n) complex (double2)
     const double2* p2pw;
-    // per kind and level l: PW->value  U[kind][l][i][k] (i < n, k < npw),
-    // and transposed UT[kind][l][k][i]
+    // per kind and level l: PW->value  U[kind][l][i][k] (i < n, k < npw)
     const double2* pw2pot;
-    const double2* pw2potT;
-    // pw2potT and its products with the parent->child split phase of each
+    // its transpose and that times the parent->child split phase of each
     // level: pw2potS[kind][l][v][k][i], v = 0 plain, 1 = + phase, 2 = conjugate
     const double2* pw2potS;
     // p2pw and its products with the child->parent merge phase of each level:
@@ -170,8 +168,6 @@ struct DevTables {
     // merge/split 1-D phases wms[klev-1][k], M2L 1-D phases wm2l[o][k]
     const double2* wms;
     const double2* wm2l;
-    // identity table for unit axes (one complex 1.0)
-    const double2* one;
     // near-field masked tables loc[kind][l][slot][k][j], bands [l][slot][k][2];
     // loc_slots table slots per level (13 for the solve, 193 for the
     // refinement of a new tree); a pair's table slots are packed 8 bits per
@@ -179,7 +175,7 @@ struct DevTables {
     const double* loctab;
     const int* locband;
     int loc_slots = 13;
-    // kind strides (elements): pw2pot / pw2potT, pw2potS, loctab
+    // kind strides (elements): pw2pot, pw2potS, loctab
     size_t pw2pot_ks, pw2potS_ks, loctab_ks;
     int n;     // norder
     int npw;
@@ -196,8 +192,8 @@ struct DevTables {
     size_t lds_limit;  // device LDS bytes per block
 };
 
-// 3-D STEP 1 / STEP 5 kernels (norder 8, 12, 16); each returns false (nothing
-// launched) when the shape is not covered.
+// 3-D STEP 1 / STEP 5 kernels; each returns false (nothing launched) when the
+// shape is not covered.
 // STEP 1 with a reduced-precision x stage, leaves of the cutoff level
 bool launch_p2pw_3d(const Geom& g, const DevTables& t, int ntask, const int* box, const int* lev,
                     const int* slot, const double* fvals, double2* expn, hipStream_t s, size_t lds_limit,
@@ -213,6 +209,9 @@ bool launch_pw2pot_3d_z(const Geom& g, const DevTables& t, int ntask, int nsib, 
 // symmetries: tasks [0, nfam) families, then nown single leaves
 bool launch_pw2pot_sym(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks,
                        const double2* expn, Kinds kd, const ZOut& zo, hipStream_t s, const Multi& mu = Multi{});
+// the symmetric kernels cover this shape (norder 4..16, LDS)
+bool sym3_supported(const Geom& g, const DevTables& t);
+// the reduced-precision kernels cover it too (norder 8, 12, 16, LDS)
 bool pw2pot_3d_supported(const Geom& g, const DevTables& t);
 // STEP 5 runs its x stage on the reduced-precision matrix cores (else it
 // takes launch_pw2pot_sym)
@@ -330,7 +329,7 @@ void launch_direct(const Geom& g, const DevTables& t, int ntask, const int* tgt,
 bool launch_direct_3d(const Geom& g, const DevTables& t, int ntask, const int* tgt, const int* lev,
                       const int* off, const int* src, const int* code, const int* flags,
                       const double* fvals, Kinds kd, OutDesc od, hipStream_t s, const Multi& mu = Multi{});
-// 3-D register-blocked path only (norder 8, 12, 16, with flags); false
+// 3-D register-blocked path only (norder 4..16, with flags); false
 // when not covered (nothing launched)
 bool launch_direct_3d_z(const Geom& g, const DevTables& t, int ntask, const int* tgt, const int* lev,
                         const int* off, const int* src, const int* code, const int* flags,

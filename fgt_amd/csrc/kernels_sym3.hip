@@ -21,10 +21,14 @@
 // (E, D complex, the table real): four real multiply-adds serve two inputs
 // and two outputs, where the plain complex form takes sixteen.  A quarter
 // of the arithmetic leaves both steps bound by the expansion bytes they
-// write and read.
+// write and read.  Orders 4 to 16 (lower ones, and 1-D and 2-D, take the
+// general kernels: one barrier-separated pass per half-axis frequency; at
+// order 6, npw 18, 1972 leaves with two densities these took 94 us for STEP 1
+// and 304 us for STEP 5, 19 and 29 us here).
 #include "kernels.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace fgt {
 
@@ -340,6 +344,29 @@ __global__ void __launch_bounds__(kThreads, (NZ > 1 && NZ * N >= 16) ? 2 : 3)
     else pw2pot_sym_block<N, false, NZ, ET>(npw, nd, tabS, tasks + tix, part, expn, ks, kd, zo, prob, sm);
 }
 
+// f(std::integral_constant<int, n>) for the orders covered here
+template <class F>
+bool for_order(int n, F&& f) {
+    switch (n) {
+        case 4: f(std::integral_constant<int, 4>{}); return true;
+        case 5: f(std::integral_constant<int, 5>{}); return true;
+        case 6: f(std::integral_constant<int, 6>{}); return true;
+        case 7: f(std::integral_constant<int, 7>{}); return true;
+        case 8: f(std::integral_constant<int, 8>{}); return true;
+        case 9: f(std::integral_constant<int, 9>{}); return true;
+        case 10: f(std::integral_constant<int, 10>{}); return true;
+        case 11: f(std::integral_constant<int, 11>{}); return true;
+        case 12: f(std::integral_constant<int, 12>{}); return true;
+        case 13: f(std::integral_constant<int, 13>{}); return true;
+        case 14: f(std::integral_constant<int, 14>{}); return true;
+        case 15: f(std::integral_constant<int, 15>{}); return true;
+        case 16: f(std::integral_constant<int, 16>{}); return true;
+        default: return false;
+    }
+}
+// FP32 expansions exist at the orders with reduced-precision kernels
+constexpr bool has_fp32(int n) { return n == 8 || n == 12 || n == 16; }
+
 template <int N, int NZ>
 void launch_sym5_z(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks, const double2* expn,
                    Kinds kd, const ZOut& zo, hipStream_t s, const Multi& mu) {
@@ -351,12 +378,15 @@ void launch_sym5_z(const Geom& g, const DevTables& t, int nfam, int nown, const 
     }
     lds *= sizeof(double2);
     const dim3 grid((unsigned)(nfam * sym5_parts<N, true>() + nown * sym5_parts<N, false>())), block(kThreads);
-    if (t.expn_f32)
-        hipLaunchKernelGGL((k_pw2pot_sym<N, NZ, float2>), grid, block, lds, s, g.nd, t.pw2potS, t.npw, tasks, nfam, nown,
-                           reinterpret_cast<const float2*>(expn), t.pw2potS_ks, kd, zo, mu);
-    else
-        hipLaunchKernelGGL((k_pw2pot_sym<N, NZ, double2>), grid, block, lds, s, g.nd, t.pw2potS, t.npw, tasks, nfam, nown,
-                           expn, t.pw2potS_ks, kd, zo, mu);
+    if constexpr (has_fp32(N)) {
+        if (t.expn_f32) {
+            hipLaunchKernelGGL((k_pw2pot_sym<N, NZ, float2>), grid, block, lds, s, g.nd, t.pw2potS, t.npw, tasks, nfam,
+                               nown, reinterpret_cast<const float2*>(expn), t.pw2potS_ks, kd, zo, mu);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_pw2pot_sym<N, NZ, double2>), grid, block, lds, s, g.nd, t.pw2potS, t.npw, tasks, nfam, nown,
+                       expn, t.pw2potS_ks, kd, zo, mu);
 }
 
 // components zo.kz[a .. a + nz) as a group of their own
@@ -596,12 +626,15 @@ void launch_sym1(const Geom& g, const DevTables& t, int nfam, int nown, const Sy
     };
     const int kf = parts(nfam, sym1_slabs<N, true>()), ko = parts(nown, sym1_slabs<N, false>());
     const dim3 grid((unsigned)(nfam * kf + nown * ko)), block(kThreads);
-    if (t.expn_f32)
-        hipLaunchKernelGGL((k_p2pw_sym<N, float2>), grid, block, lds, s, g.nd, t.p2pwS, t.npw, tasks, nfam, nown, kf,
-                           ko, fvals, reinterpret_cast<float2*>(expn), mu);
-    else
-        hipLaunchKernelGGL((k_p2pw_sym<N, double2>), grid, block, lds, s, g.nd, t.p2pwS, t.npw, tasks, nfam, nown, kf,
-                           ko, fvals, expn, mu);
+    if constexpr (has_fp32(N)) {
+        if (t.expn_f32) {
+            hipLaunchKernelGGL((k_p2pw_sym<N, float2>), grid, block, lds, s, g.nd, t.p2pwS, t.npw, tasks, nfam, nown,
+                               kf, ko, fvals, reinterpret_cast<float2*>(expn), mu);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_p2pw_sym<N, double2>), grid, block, lds, s, g.nd, t.p2pwS, t.npw, tasks, nfam, nown, kf, ko,
+                       fvals, expn, mu);
 }
 
 }  // namespace
@@ -609,23 +642,26 @@ void launch_sym1(const Geom& g, const DevTables& t, int nfam, int nown, const Sy
 bool launch_p2pw_sym(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks, const double* fvals,
                      double2* expn, hipStream_t s, const Multi& mu) {
     if (g.ndim != 3 || nfam + nown <= 0) return false;
-    switch (t.n) {
-        case 8: launch_sym1<8>(g, t, nfam, nown, tasks, fvals, expn, s, mu); return true;
-        case 12: launch_sym1<12>(g, t, nfam, nown, tasks, fvals, expn, s, mu); return true;
-        case 16: launch_sym1<16>(g, t, nfam, nown, tasks, fvals, expn, s, mu); return true;
-        default: return false;
-    }
+    return for_order(t.n, [&](auto n) { launch_sym1<n()>(g, t, nfam, nown, tasks, fvals, expn, s, mu); });
 }
 
 bool launch_pw2pot_sym(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks,
                        const double2* expn, Kinds kd, const ZOut& zo, hipStream_t s, const Multi& mu) {
     if (g.ndim != 3 || zo.nz < 1 || zo.nz > 3 || nfam + nown <= 0) return false;
-    switch (t.n) {
-        case 8: launch_sym5<8>(g, t, nfam, nown, tasks, expn, kd, zo, s, mu); return true;
-        case 12: launch_sym5<12>(g, t, nfam, nown, tasks, expn, kd, zo, s, mu); return true;
-        case 16: launch_sym5<16>(g, t, nfam, nown, tasks, expn, kd, zo, s, mu); return true;
-        default: return false;
-    }
+    return for_order(t.n, [&](auto n) { launch_sym5<n()>(g, t, nfam, nown, tasks, expn, kd, zo, s, mu); });
+}
+
+bool sym3_supported(const Geom& g, const DevTables& t) {
+    if (g.ndim != 3) return false;
+    size_t need = 0;
+    const bool ok = for_order(t.n, [&](auto n) {
+        constexpr int N = n();
+        for (int p = 1; p <= t.npw; ++p)
+            need = std::max({need, sym1_lds_entries<N, true>(p), sym1_lds_entries<N, false>(p),
+                             sym5_lds_entries(p, 2 * sym5_nx<N, true>(), 2 * sym_pairs<N, true>()),
+                             sym5_lds_entries(p, 2 * sym5_nx<N, false>(), 2 * sym_pairs<N, false>())});
+    });
+    return ok && need * sizeof(double2) <= t.lds_limit;
 }
 
 }  // namespace fgt
