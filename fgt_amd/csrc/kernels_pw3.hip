@@ -105,9 +105,11 @@ __device__ __forceinline__ void x1_lowp_group(int npw, int lane, int c0, int cts
             cval[gi] = (c >> 1) < npw && c0 + gi * ctstep < CT;
             k1c[gi] = cval[gi] ? (c >> 1) : 0;
         }
-        // FP32: the column tiles' table operands of every K step, read once
-        // for all row tiles (the BF16 form re-reads them per row tile)
-        constexpr int KS = (KN + 3) / 4;
+        // the column tiles' table operands of every K step, read (BF16: and
+        // split) once for all row tiles (BF16 per row tile, with the result's
+        // part picked by an index through scratch: k_p2pw3 over the 779 leaves
+        // of an order-8 problem 39 us, now 30)
+        constexpr int KS = (KN + 3) / 4, KB = (KN + 15) / 16;
         float tb1[CG][XS == 2 ? KS : 1], tb2[CG][XS == 2 ? KS : 1];
         if constexpr (XS == 2) {
 #pragma unroll
@@ -123,6 +125,24 @@ __device__ __forceinline__ void x1_lowp_group(int npw, int lane, int c0, int cts
                     tb2[gi][st] = ok ? bcol(u, part[gi], 1) : 0.f;
                 }
             }
+        }
+        bf8 bh[CG][XS == 2 ? 1 : KB], bl[CG][XS == 2 ? 1 : KB];
+        if constexpr (XS != 2) {
+#pragma unroll
+            for (int st = 0; st < KB; ++st)
+#pragma unroll
+                for (int gi = 0; gi < CG; ++gi) {
+                    float bx[8];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int kk = 16 * st + 4 * lq + j;
+                        const bool ok = kk < KN && cval[gi];
+                        const double2 u = fb(kk < KN ? kk : KN - 1, k1c[gi]);
+                        bx[2 * j] = ok ? bcol(u, part[gi], 0) : 0.f;
+                        bx[2 * j + 1] = ok ? bcol(u, part[gi], 1) : 0.f;
+                    }
+                    split_bf(bx, bh[gi][st], bl[gi][st]);
+                }
         }
         // one row tile at a time (few live accumulators, high occupancy)
         for (int mt = 0; mt < MT; ++mt) {
@@ -145,7 +165,7 @@ __device__ __forceinline__ void x1_lowp_group(int npw, int lane, int c0, int cts
                 }
             } else {
 #pragma unroll
-                for (int st = 0; st < (KN + 15) / 16; ++st) {
+                for (int st = 0; st < KB; ++st) {
                     float ax[8];
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
@@ -158,20 +178,9 @@ __device__ __forceinline__ void x1_lowp_group(int npw, int lane, int c0, int cts
                     split_bf(ax, ah, al);
 #pragma unroll
                     for (int gi = 0; gi < CG; ++gi) {
-                        float bx[8];
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const int kk = 16 * st + 4 * lq + j;
-                            const bool ok = kk < KN && cval[gi];
-                            const double2 u = fb(kk < KN ? kk : KN - 1, k1c[gi]);
-                            bx[2 * j] = ok ? bcol(u, part[gi], 0) : 0.f;
-                            bx[2 * j + 1] = ok ? bcol(u, part[gi], 1) : 0.f;
-                        }
-                        bf8 bh, bl;
-                        split_bf(bx, bh, bl);
-                        acc[gi][0] = mfma_bf(ah, bh, acc[gi][0]);
-                        acc[gi][1] = mfma_bf(ah, bl, acc[gi][1]);
-                        acc[gi][1] = mfma_bf(al, bh, acc[gi][1]);
+                        acc[gi][0] = mfma_bf(ah, bh[gi][st], acc[gi][0]);
+                        acc[gi][1] = mfma_bf(ah, bl[gi][st], acc[gi][1]);
+                        acc[gi][1] = mfma_bf(al, bh[gi][st], acc[gi][1]);
                     }
                 }
             }
@@ -187,10 +196,10 @@ __device__ __forceinline__ void x1_lowp_group(int npw, int lane, int c0, int cts
                 if (cval[gi])
 #pragma unroll
                     for (int h = 0; h < 2; ++h) {
-                        const int v = 2 * part[gi] + h;
-                        const int k2 = 16 * mt + 4 * lq + v;
-                        if (k2 < npw)
-                            fw(k2, k1c[gi], part[gi] ? make_float2(q[v], o[v]) : make_float2(o[v], q[v]));
+                        // (selects of fixed elements: an index by lane goes through scratch)
+                        const int k2 = 16 * mt + 4 * lq + 2 * part[gi] + h;
+                        const float2 v = part[gi] ? make_float2(q[2 + h], o[2 + h]) : make_float2(o[h], q[h]);
+                        if (k2 < npw) fw(k2, k1c[gi], v);
                     }
             }
         }
