@@ -196,6 +196,21 @@ int map_code(int ndim, int c, int centre = 6) {
     return centre | (centre << 8) | (a0 << 16);
 }
 
+// sort key of a target's near-field entries: sources with equal keys share
+// their z and x tables
+int zxy_code(int c) { return ((c >> 16) & 255) << 8 | (c & 255); }
+// near-field tables [..][k][j] (target node, source node) as the kernels of
+// the problem read them: the 3-D ones [j][k]
+std::vector<double> loctab_for(int ndim, int n, const std::vector<double>& t) {
+    if (!fgt::direct3_orders(ndim, n)) return t;
+    std::vector<double> o(t.size());
+    const size_t nn = (size_t)n * n;
+    for (size_t b = 0; b + nn <= t.size(); b += nn)
+        for (int k = 0; k < n; ++k)
+            for (int j = 0; j < n; ++j) o[b + (size_t)j * n + k] = t[b + (size_t)k * n + j];
+    return o;
+}
+
 std::vector<double2> to_d2(const std::vector<fgt::cplx>& v) {
     std::vector<double2> o(v.size());
     for (size_t i = 0; i < v.size(); ++i) o[i] = make_double2(v[i].real(), v[i].imag());
@@ -459,7 +474,7 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
         S.d_pot.alloc(sizeof(double) * (size_t)P.nd * P.npbox * P.nboxes);
     }
 
-    S.d_loctab.upload(P.loctab);
+    S.d_loctab.upload(loctab_for(ndim, n, P.loctab));
     S.d_locband.upload(P.locband);
     if (P.do_pw) {
         S.d_p2pw.upload(to_d2(P.p2pw));
@@ -760,8 +775,8 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
 
     // near-field targets, longest list first (one block per target: the
     // longest-processing-time order shortens the tail of the launch); entries
-    // of a target sorted by (z, y, x) table slot so the 3-D kernel can share
-    // the y and z contractions within a group
+    // of a target sorted by (z, x, y) table slot so the 3-D kernel can share
+    // the x and z contractions within a group
     const int ndt = (int)P.dir_tgt.size();
     std::vector<int> order(ndt);
     for (int i = 0; i < ndt; ++i) order[i] = i;
@@ -780,8 +795,7 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
         std::vector<int> idx(b0 - a0);
         for (int i = a0; i < b0; ++i) idx[i - a0] = i;
         std::stable_sort(idx.begin(), idx.end(), [&](int x, int y) {
-            const int cx = map_code(ndim, P.dir_code[x]), cy = map_code(ndim, P.dir_code[y]);
-            return (cx >> 8) < (cy >> 8);
+            return zxy_code(map_code(ndim, P.dir_code[x])) < zxy_code(map_code(ndim, P.dir_code[y]));
         });
         for (int i = a; i < b; ++i) {
             ds[i] = P.dir_src[idx[i - a]];
@@ -789,7 +803,7 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
         }
         for (int i = a; i < b; ++i) {
             const bool last = (i + 1 == b);
-            if (last || (dc[i] >> 8) != (dc[i + 1] >> 8)) df[i] |= 1;
+            if (last || zxy_code(dc[i]) != zxy_code(dc[i + 1])) df[i] |= 1;
             if (last || (dc[i] >> 16) != (dc[i + 1] >> 16)) df[i] |= 2;
         }
     }
@@ -843,9 +857,11 @@ std::vector<Comp> components_on(int ndim, int nd, int ifpgh, double* pot, double
     return c;
 }
 
-// Output components grouped by their x and y table kinds (gkd[k]), at most
-// three z kinds per group (groups[k]).
-void group_comps(const std::vector<Comp>& comps, std::vector<fgt::ZOut>& groups, std::vector<fgt::Kinds>& gkd) {
+// Output components grouped by their x and y table kinds, at most three z
+// kinds per group, and the groups with equally many z kinds three to a launch.
+std::vector<fgt::ZGroups> group_comps(const std::vector<Comp>& comps) {
+    std::vector<fgt::ZOut> groups;
+    std::vector<fgt::Kinds> gkd;
     for (const Comp& c : comps) {
         size_t k = 0;
         while (k < groups.size() && !(gkd[k].x == c.kd.x && gkd[k].y == c.kd.y && groups[k].nz < 3)) ++k;
@@ -858,6 +874,15 @@ void group_comps(const std::vector<Comp>& comps, std::vector<fgt::ZOut>& groups,
         z.od[z.nz] = c.od;
         ++z.nz;
     }
+    std::vector<fgt::ZGroups> out;
+    for (size_t k = 0; k < groups.size(); ++k) {
+        size_t q = 0;
+        while (q < out.size() && (out[q].zo[0].nz != groups[k].nz || out[q].n == fgt::kMaxZGroups)) ++q;
+        if (q == out.size()) out.push_back(fgt::ZGroups{});
+        out[q].kd[out[q].n] = gkd[k];
+        out[q].zo[out[q].n++] = groups[k];
+    }
+    return out;
 }
 
 // STEP 6 for a list of output components: on the 3-D register-blocked
@@ -868,17 +893,15 @@ void group_comps(const std::vector<Comp>& comps, std::vector<fgt::ZOut>& groups,
 void launch_direct_comps(const fgt::Geom& g, const fgt::DevTables& t, int ntask, const int* tgt, const int* lev,
                          const int* off, const int* src, const int* code, const int* flags, const double* fvals,
                          const std::vector<Comp>& comps, hipStream_t st) {
-    std::vector<fgt::ZOut> groups;
-    std::vector<fgt::Kinds> gkd;
-    group_comps(comps, groups, gkd);
-    for (size_t k = 0; k < groups.size(); ++k) {
-        if (fgt::launch_direct_3d_z(g, t, ntask, tgt, lev, off, src, code, flags, fvals, gkd[k], groups[k], st)) {
+    for (const fgt::ZGroups& zg : group_comps(comps)) {
+        if (fgt::launch_direct_3d(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, st)) {
             hcheck(hipGetLastError(), "k_direct3 launch");
             continue;
         }
-        for (int q = 0; q < groups[k].nz; ++q)
-            fgt::launch_direct(g, t, ntask, tgt, lev, off, src, code, flags, fvals,
-                               fgt::Kinds{gkd[k].x, gkd[k].y, groups[k].kz[q]}, groups[k].od[q], st);
+        for (int k = 0; k < zg.n; ++k)
+            for (int q = 0; q < zg.zo[k].nz; ++q)
+                fgt::launch_direct(g, t, ntask, tgt, lev, off, src, code, flags, fvals,
+                                   fgt::Kinds{zg.kd[k].x, zg.kd[k].y, zg.zo[k].kz[q]}, zg.zo[k].od[q], st);
     }
 }
 
@@ -888,10 +911,7 @@ void launch_direct_comps(const fgt::Geom& g, const fgt::DevTables& t, int ntask,
 // once for all the z kinds).
 void launch_pw2pot_comps(const fgt::Geom& g, const fgt::DevTables& t, const fgt::Step5Lists& l, const double2* expn,
                          const std::vector<Comp>& comps, hipStream_t st) {
-    std::vector<fgt::ZOut> groups;
-    std::vector<fgt::Kinds> gkd;
-    group_comps(comps, groups, gkd);
-    for (size_t k = 0; k < groups.size(); ++k) fgt::launch_pw2pot_tasks(g, t, l, expn, gkd[k], groups[k], st);
+    for (const fgt::ZGroups& zg : group_comps(comps)) fgt::launch_pw2pot_tasks(g, t, l, expn, zg, st);
 }
 
 std::vector<Comp> components(fgt_solver& S, double* pot_override = nullptr) {
@@ -954,12 +974,17 @@ void execute(fgt_solver& S, hipStream_t st, bool timed, bool fork_near = false,
             hcheck(hipEventCreateWithFlags(&S.ev_join, hipEventDisableTiming), "hipEventCreate");
         }
         hcheck(hipEventRecord(S.ev_fork, st), "hipEventRecord");   // after the zeroing
+    }
+    // enqueued behind STEP 1's kernels, so these get the device first: the
+    // near field fills what they and the short launches after them leave
+    auto fork_near_field = [&] {
+        if (!fork) return;
         hcheck(hipStreamWaitEvent(S.st_near, S.ev_fork, 0), "hipStreamWaitEvent");
         if (timed) hcheck(hipEventRecord(evn[0], S.st_near), "hipEventRecord");
         near_field(S.st_near);
         if (timed) hcheck(hipEventRecord(evn[1], S.st_near), "hipEventRecord");
         hcheck(hipEventRecord(S.ev_join, S.st_near), "hipEventRecord");
-    }
+    };
     mark(0);
     if (P.do_pw) {
         if (S.fast3d) {
@@ -970,6 +995,7 @@ void execute(fgt_solver& S, hipStream_t st, bool timed, bool fork_near = false,
                                           nullptr, S.n_fz, S.d_fz_lev.as<int>(), S.d_fz_slot.as<int>(),
                                           S.d_fz_kids.as<int>(), S.d_fz_ksg.as<int>(), nullptr, S.n_fz, S.n_s1,
                                           S.d_s1_sym.as<fgt::SymTask>(), nullptr}, fv, ex, st);
+            fork_near_field();
             mark(1);
             // STEP 2: non-leaf children, fine to coarse
             for (int l = P.nlevels - 1; l >= P.nlevstart; --l) {
@@ -983,6 +1009,7 @@ void execute(fgt_solver& S, hipStream_t st, bool timed, bool fork_near = false,
             // STEP 1: every PW leaf, all levels in one launch
             fgt::launch_p2pw(g, t, (int)P.leaf_box.size(), S.d_leaf_box.as<int>(), S.d_leaf_lev.as<int>(),
                              S.d_leaf_slot.as<int>(), fv, ex, st);
+            fork_near_field();
             mark(1);
             // STEP 2: fine to coarse
             for (int l = P.nlevels - 1; l >= P.nlevstart; --l) {
@@ -1572,12 +1599,13 @@ void class_step4(const BClass& C, hipStream_t st) {
 }
 void class_step5(const BClass& C, hipStream_t st) {
     if (C.n_s5 <= 0) return;
-    fgt::ZOut zo{};
-    zo.nz = 1;
-    zo.od[0] = fgt::OutDesc{nullptr, C.nd, 0};
+    fgt::ZGroups zg{};
+    zg.n = 1;
+    zg.zo[0].nz = 1;
+    zg.zo[0].od[0] = fgt::OutDesc{nullptr, C.nd, 0};
     fgt::launch_pw2pot_tasks(C.g, C.t, {C.n_s5, C.n_s5_sib, C.s5.as<fgt::PotTask>(), C.s5_prob.as<int>(), C.n_s5_fam,
                                         C.n_s5_own, C.s5_sym.as<fgt::SymTask>(), C.s5_symprob.as<int>()},
-                             nullptr, fgt::Kinds{0, 0, 0}, zo, st, C.pp.as<fgt::ProbPtrs>());
+                             nullptr, zg, st, C.pp.as<fgt::ProbPtrs>());
 }
 void class_step6(const BClass& C, hipStream_t st) {
     if (C.n_dir > 0)
@@ -2043,7 +2071,7 @@ struct Refiner {
             fgt::make_loctab_level(P.eps, P.ipoly, n, P.delta, P.tree.boxsize[l], &tab[per * l],
                                    &band[(size_t)2 * n * nslot * l], &loccols[(size_t)2 * nslot * l],
                                    &tab[ks + per * l], &tab[2 * ks + per * l], 3);
-        d_loctab.upload(tab);
+        d_loctab.upload(loctab_for(P.ndim, n, tab));
         d_locband.upload(band);
         tr = S.tabs;
         tr.loctab = d_loctab.as<double>();
@@ -2210,13 +2238,15 @@ struct Refiner {
             }
             if (ent.empty()) continue;
             std::stable_sort(ent.begin(), ent.end(),
-                             [](const std::pair<int, int>& x, const std::pair<int, int>& y) { return (x.first >> 8) < (y.first >> 8); });
+                             [](const std::pair<int, int>& x, const std::pair<int, int>& y) {
+                                 return zxy_code(x.first) < zxy_code(y.first);
+                             });
             for (size_t j = 0; j < ent.size(); ++j) {
                 dsrc.push_back(ent[j].second);
                 dcode.push_back(ent[j].first);
                 const bool last = j + 1 == ent.size();
                 int f = 0;
-                if (last || (ent[j].first >> 8) != (ent[j + 1].first >> 8)) f |= 1;
+                if (last || zxy_code(ent[j].first) != zxy_code(ent[j + 1].first)) f |= 1;
                 if (last || (ent[j].first >> 16) != (ent[j + 1].first >> 16)) f |= 2;
                 dfl.push_back(f);
             }

@@ -57,6 +57,36 @@ struct CTab1 {
 __device__ __forceinline__ CTab2 ctab(const double2* q) { return CTab2{(cdvec2_t*)q}; }
 __device__ __forceinline__ CTab1 ctab(const double* q) { return CTab1{(cdouble_t*)q}; }
 
+// Global memory through its own address space.  A pointer that is either a
+// kernel argument or read from a per-problem descriptor is generic to the
+// compiler, which then emits flat accesses: they count on the LDS counter as
+// well, so every wait for one of them waits for all loads in flight.
+// gload / gstore: element o of a wave-uniform base (scalar base, 32-bit lane
+// offset).
+typedef float fvec2_t __attribute__((ext_vector_type(2)));
+#define FGT_GLOBAL __attribute__((address_space(1)))
+__device__ __forceinline__ double gload(const double* p, unsigned o) {
+    return ((const FGT_GLOBAL double*)p)[o];
+}
+__device__ __forceinline__ double2 gload(const double2* p, unsigned o) {
+    const dvec2_t v = ((const FGT_GLOBAL dvec2_t*)p)[o];
+    return make_double2(v.x, v.y);
+}
+__device__ __forceinline__ float2 gload(const float2* p, unsigned o) {
+    const fvec2_t v = ((const FGT_GLOBAL fvec2_t*)p)[o];
+    return make_float2(v.x, v.y);
+}
+__device__ __forceinline__ void gadd(double* p, unsigned o, double v) {
+    FGT_GLOBAL double* q = (FGT_GLOBAL double*)p + o;
+    *q += v;
+}
+__device__ __forceinline__ void gstore(double2* p, unsigned o, double2 v) {
+    ((FGT_GLOBAL dvec2_t*)p)[o] = dvec2_t{v.x, v.y};
+}
+__device__ __forceinline__ void gstore(float2* p, unsigned o, double2 v) {
+    ((FGT_GLOBAL fvec2_t*)p)[o] = fvec2_t{(float)v.x, (float)v.y};
+}
+
 // Workgroups are dealt to the 8 XCDs round-robin; give each XCD a contiguous
 // range of tasks so that tasks sharing data (children of one parent,
 // neighbouring targets, one element range of many targets) meet in the same L2.
@@ -102,6 +132,27 @@ struct ZOut {
     OutDesc od[3];
 };
 
+// Up to three such groups with equally many z kinds run in one launch (their
+// blocks side by side: a group alone leaves the device idle on small trees).
+constexpr int kMaxZGroups = 3;
+struct ZGroups {
+    int n;
+    Kinds kd[kMaxZGroups];   // x and y kinds (z unused)
+    ZOut zo[kMaxZGroups];    // equal nz
+};
+// z kinds [a, a + nz) of every group
+inline ZGroups z_kinds(const ZGroups& zg, int a, int nz) {
+    ZGroups r = zg;
+    for (int k = 0; k < zg.n; ++k) {
+        r.zo[k].nz = nz;
+        for (int q = 0; q < nz; ++q) {
+            r.zo[k].kz[q] = zg.zo[k].kz[a + q];
+            r.zo[k].od[q] = zg.zo[k].od[a + q];
+        }
+    }
+    return r;
+}
+
 // One task of the 3-D STEP 5 kernel: the local expansion in `slot`,
 // evaluated at up to four leaves of level `lev` that share the x table
 // variant vx (0 plain table; 1 / 2 table times the + / conjugate
@@ -141,7 +192,7 @@ struct ProbPtrs {
     const double2* pw2potS;   // PW->value tables [l][v][k][i] (value kind)
     const double2* wms;       // merge/split 1-D phases [klev-1][k]
     const double2* wm2l;      // M2L 1-D phases [o][k]
-    const double* loctab;     // near-field tables [l][slot][k][j] (value kind)
+    const double* loctab;     // near-field tables [l][slot][j][k] (value kind)
     const double* fvals;      // (nd, npbox, nboxes)
     double* pot;              // (nd, npbox, nboxes), accumulated into
     void* expn;               // expansion slots (FP64 or FP32 complex)
@@ -168,7 +219,8 @@ struct DevTables {
     // merge/split 1-D phases wms[klev-1][k], M2L 1-D phases wm2l[o][k]
     const double2* wms;
     const double2* wm2l;
-    // near-field masked tables loc[kind][l][slot][k][j], bands [l][slot][k][2];
+    // near-field masked tables loc[kind][l][slot][k][j] ([j][k] where
+    // direct3_orders), bands [l][slot][k][2];
     // loc_slots table slots per level (13 for the solve, 193 for the
     // refinement of a new tree); a pair's table slots are packed 8 bits per
     // kernel axis: x | y << 8 | z << 16
@@ -208,7 +260,7 @@ bool launch_pw2pot_3d_z(const Geom& g, const DevTables& t, int ntask, int nsib, 
 // STEP 5 in FP64 arithmetic (FP64 or FP32 expansions) through the tables'
 // symmetries: tasks [0, nfam) families, then nown single leaves
 bool launch_pw2pot_sym(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks,
-                       const double2* expn, Kinds kd, const ZOut& zo, hipStream_t s, const Multi& mu = Multi{});
+                       const double2* expn, const ZGroups& zg, hipStream_t s, const Multi& mu = Multi{});
 // the symmetric kernels cover this shape (norder 4..16, LDS)
 bool sym3_supported(const Geom& g, const DevTables& t);
 // the reduced-precision kernels cover it too (norder 8, 12, 16, LDS)
@@ -308,7 +360,7 @@ void launch_split(const Geom& g, const DevTables& t, int nentry, const int* pc_p
 void launch_pw2pot(const Geom& g, const DevTables& t, int ntask, const int* box,
                    const int* lev, const int* slot, const double2* expn,
                    Kinds kd, OutDesc od, hipStream_t s);
-// 3-D STEP 5 for the components of zo, in the form pw2pot_lowp picks (throws
+// 3-D STEP 5 for the components of zg, in the form pw2pot_lowp picks (throws
 // when the shape is not covered)
 struct Step5Lists {
     int ntask, nsib;          // PotTask list (reduced precision)
@@ -318,22 +370,21 @@ struct Step5Lists {
     const SymTask* sym;
     const int* symprob;
 };
-void launch_pw2pot_tasks(const Geom& g, const DevTables& t, const Step5Lists& l, const double2* expn, Kinds kd,
-                         const ZOut& zo, hipStream_t s, const ProbPtrs* pp = nullptr);
-// flags (nullable): per entry bit0 = last of its (y,z) table group, bit1 =
+void launch_pw2pot_tasks(const Geom& g, const DevTables& t, const Step5Lists& l, const double2* expn,
+                         const ZGroups& zg, hipStream_t s, const ProbPtrs* pp = nullptr);
+// flags (nullable): per entry bit0 = last of its (x,z) table group, bit1 =
 // last of its z group; entries must then be grouped in that order.
 void launch_direct(const Geom& g, const DevTables& t, int ntask, const int* tgt,
                    const int* lev, const int* off, const int* src, const int* code,
                    const int* flags, const double* fvals, Kinds kd, OutDesc od, hipStream_t s,
                    const Multi& mu = Multi{});
+// the 3-D near-field kernels cover this order (4..16); they read the near-
+// field tables as [j][k] (source node, target node)
+inline bool direct3_orders(int ndim, int n) { return ndim == 3 && n >= 4 && n <= 16; }
+// orders covered, with flags; false when not (nothing launched)
 bool launch_direct_3d(const Geom& g, const DevTables& t, int ntask, const int* tgt, const int* lev,
                       const int* off, const int* src, const int* code, const int* flags,
-                      const double* fvals, Kinds kd, OutDesc od, hipStream_t s, const Multi& mu = Multi{});
-// 3-D register-blocked path only (norder 4..16, with flags); false
-// when not covered (nothing launched)
-bool launch_direct_3d_z(const Geom& g, const DevTables& t, int ntask, const int* tgt, const int* lev,
-                        const int* off, const int* src, const int* code, const int* flags,
-                        const double* fvals, Kinds kd, const ZOut& zo, hipStream_t s);
+                      const double* fvals, const ZGroups& zg, hipStream_t s, const Multi& mu = Multi{});
 
 // Device workspace of the no-allocation entry point: a file-scope device
 // array of kScratchBytes per GPU.  scratch_region() returns its address on

@@ -1155,16 +1155,19 @@ void launch_split(const Geom& g, const DevTables& t, int nentry, const int* pc_p
     }
 }
 
-void launch_pw2pot_tasks(const Geom& g, const DevTables& t, const Step5Lists& l, const double2* expn, Kinds kd,
-                         const ZOut& zo, hipStream_t s, const ProbPtrs* pp) {
+void launch_pw2pot_tasks(const Geom& g, const DevTables& t, const Step5Lists& l, const double2* expn,
+                         const ZGroups& zg, hipStream_t s, const ProbPtrs* pp) {
     const bool lowp = pw2pot_lowp(t);
     if ((lowp ? l.ntask : l.nfam + l.nown) <= 0) return;
     Multi mu;
     mu.pp = pp;
     mu.tprob = lowp ? l.tprob : l.symprob;
-    if (lowp ? !launch_pw2pot_3d_z(g, t, l.ntask, l.nsib, l.tasks, expn, kd, zo, s, t.lds_limit, mu)
-             : !launch_pw2pot_sym(g, t, l.nfam, l.nown, l.sym, expn, kd, zo, s, mu))
-        throw std::runtime_error("3-D STEP 5 kernel not available for this shape");
+    bool ok = true;
+    if (!lowp) ok = launch_pw2pot_sym(g, t, l.nfam, l.nown, l.sym, expn, zg, s, mu);
+    else
+        for (int q = 0; q < zg.n; ++q)
+            ok = ok && launch_pw2pot_3d_z(g, t, l.ntask, l.nsib, l.tasks, expn, zg.kd[q], zg.zo[q], s, t.lds_limit, mu);
+    if (!ok) throw std::runtime_error("3-D STEP 5 kernel not available for this shape");
     check(hipGetLastError(), "3-D STEP 5 launch");
 }
 
@@ -1189,7 +1192,13 @@ void launch_direct(const Geom& g, const DevTables& t, int ntask, const int* tgt,
                    const int* off, const int* src, const int* code, const int* flags, const double* fvals,
                    Kinds kd, OutDesc od, hipStream_t s, const Multi& mu) {
     if (ntask <= 0) return;
-    if (launch_direct_3d(g, t, ntask, tgt, lev, off, src, code, flags, fvals, kd, od, s, mu)) {
+    ZGroups zg{};
+    zg.n = 1;
+    zg.kd[0] = kd;
+    zg.zo[0].nz = 1;
+    zg.zo[0].kz[0] = kd.z;
+    zg.zo[0].od[0] = od;
+    if (launch_direct_3d(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, s, mu)) {
         check(hipGetLastError(), "k_direct3 launch");
         return;
     }

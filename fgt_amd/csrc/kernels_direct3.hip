@@ -3,19 +3,26 @@
 // Replaces the per-pair banded contraction of g3d_tens_prod_to_potloc_fast
 // (src/bfgt/bfgt_local.f:1322-1618) summed over a target's list-1 sources
 // (boxfgt.f:904-928).  Sources of one target are pre-sorted on the host by
-// their (z, y, x) table slots; since the near-field operator is the
-// separable product A_z (x) A_y (x) A_x, sources that share the y and z
-// tables are summed after their x contraction, and y-results that share the
+// their (z, x, y) table slots; since the near-field operator is the
+// separable product A_z (x) A_x (x) A_y, sources that share the x and z
+// tables are summed after their y contraction, and x-results that share the
 // z table are summed before it:
-//     pot += sum_z A_z ( sum_{y | z} A_y ( sum_{x | y,z} A_x f_s ) )
-// which needs one x contraction per source, one y contraction per (y,z)
-// group and one z contraction per z group.
-// Orders 4 to 16; one block of N^2 threads (rounded up to whole waves: 64 /
-// 192 / 256 for n = 8 / 12 / 16) per target leaf; the 1-D tables (masked to their
-// significant band, zero elsewhere) are wave-uniform and read into SGPRs;
-// the partial sums live in registers between LDS transposes.  (At order 6,
-// 2094 leaves with two densities, the general kernel's barrier-separated
-// passes per source took 503 us, this one 68 us.)
+//     pot += sum_z A_z ( sum_{x | z} A_x ( sum_{y | x,z} A_y f_s ) )
+// which needs one y contraction per source, one x contraction per (x,z)
+// group and one z contraction per z group.  y goes first because the values'
+// fastest index then stays a row index of the product: neighbouring lanes
+// load neighbouring values (with x first every lane of a load fell into a
+// cache line of its own, and the L1 bounded the kernel).
+//
+// The contractions run on the FP64 matrix cores as 4x4x4 products (four
+// independent blocks per instruction).  On this card they reach the FP64
+// peak from one dependent chain (77 of 78.6 TFLOP/s; v_fma_f64 61 with four
+// waves per SIMD) and take the table as a per-lane operand: with the table in
+// SGPRs, each loaded double served one multiply-add of a wave, and the scalar
+// cache bounded the kernel at a third of the peak.  Measured (alone, then
+// beside STEP 1): order 16, 60255 pairs 460 -> 357 us, 45 % of the FP64 peak (the
+// table and output latencies at each z group are left); order 12 Hessian,
+// 4774 pairs 620 -> 187 us; order 8 gradient, 21347 pairs 228 -> 112 us.
 #include <cstdlib>
 
 #include "kernels.h"
@@ -38,206 +45,509 @@ int direct_runs(const Multi& mu) {
     return v >= 0 ? v : (mu.pp ? 1 : 0);
 }
 
-// flags per source entry: bit0 = last of its (y,z) group, bit1 = last of its z group;
-// nls table slots per level, slot codes 8 bits per axis
-template <int N>
-constexpr int direct3_block() { return (N * N + 63) / 64 * 64; }
-
-// NZ output components that differ only in their z kind (ZOut) share the x
-// and y sums; NZ = 1 is the one-component kernel (od = zo.od[0]).
-template <int N, int NZ>
-__global__ void __launch_bounds__(direct3_block<N>(), N == 16 ? (NZ == 1 ? 3 : 2) : 2)
-    k_direct3(Geom g, const double* __restrict__ loctab_a, int nls, const int* __restrict__ tgt,
-              const int* __restrict__ lev, const int* __restrict__ off, const int* __restrict__ src,
-              const int* __restrict__ code, const int* __restrict__ flags, const double* __restrict__ fvals_a,
-              size_t ks, Kinds kd, ZOut zo, Multi mu, int runs) {
-    extern __shared__ double dsm[];   // N^3 doubles (transpose buffer)
-    constexpr int NN = N * N;
-    const int task = runs ? xcd_run_task<8>(blockIdx.x, gridDim.x) : (int)blockIdx.x;
-    const double* __restrict__ loctab = loctab_a;
-    const double* __restrict__ fvals = fvals_a;
-    if (mu.pp) {
-        const ProbPtrs& q = mu.pp[mu.tprob[task]];
-        loctab = q.loctab;
-        fvals = q.fvals;
-        zo.od[0].p = q.pot;   // batches evaluate the potential only
-    }
-    const int tb = tgt[task], l = lev[task];
-    // table kind per axis (value / first / second derivative): stride ks
-    const CTab1 tabx = ctab(loctab) + (long long)(kd.x * ks + (size_t)l * nls * NN);
-    const CTab1 taby = ctab(loctab) + (long long)(kd.y * ks + (size_t)l * nls * NN);
-    CTab1 tabz[NZ];
+// A target's source entries, staged in LDS kChunk at a time: read back at a
+// wave-uniform address they keep the vector-memory counter for the values
+// and tables alone (read from global memory between the products, every step
+// waited for all loads in flight).  z group g of the chunk goes to team
+// g % TEAMS; a chunk's last entry closes its groups.
+// flags per entry: bit0 = last of its (x,z) group, bit1 = last of its z group.
+constexpr int kChunk = 256;
+template <int TEAMS>
+struct Entries {
+    int2 e[TEAMS][kChunk];   // source box; slot codes | flags << 24
+    int n[TEAMS];
+};
+struct Entry {
+    int src, code;
+    __device__ __forceinline__ int x() const { return code & 255; }
+    __device__ __forceinline__ int y() const { return (code >> 8) & 255; }
+    __device__ __forceinline__ int z() const { return (code >> 16) & 255; }
+    __device__ __forceinline__ bool xz_end() const { return (code >> 24) & 1; }
+    __device__ __forceinline__ bool z_end() const { return (code >> 25) & 1; }
+};
+__device__ __forceinline__ Entry uniform(int2 v) {
+    return Entry{__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y)};
+}
+// entries [j0, j0 + n), n <= kChunk, by the block's first wave; the caller's
+// barrier follows
+template <int TEAMS>
+__device__ __forceinline__ void stage_entries(Entries<TEAMS>& en, const int* __restrict__ src,
+                                              const int* __restrict__ code, const int* __restrict__ flags, int j0,
+                                              int n, int lane) {
+    int cnt[TEAMS], g0 = 0;
 #pragma unroll
-    for (int q = 0; q < NZ; ++q) tabz[q] = ctab(loctab) + (long long)(zo.kz[q] * ks + (size_t)l * nls * NN);
-    const int tid = threadIdx.x;
-    const bool act = tid < NN;
-    // x stage: thread = (j2, j3); y stage: thread = (k1, j3); z stage: thread = (k1, k2)
-    const int a = tid % N, bq = tid / N;
-    const int nd = g.nd;
-    const int j0 = off[task], j1e = off[task + 1];
-    for (int ind = 0; ind < nd; ++ind) {
-        double X[N], Y[N], acc[NZ][N];
+    for (int t = 0; t < TEAMS; ++t) cnt[t] = 0;
+    for (int q = 0; q < n; q += 64) {
+        const int j = q + lane;
+        const bool on = j < n;
+        const int fl = on ? (j == n - 1 ? 3 : flags[j0 + j]) : 0;
+        const int2 v = on ? make_int2(src[j0 + j], code[j0 + j] | fl << 24) : make_int2(0, 0);
+        const unsigned long long before = (1ull << lane) - 1;
+        const unsigned long long m = __ballot(fl & 2);
+        const int team = TEAMS == 1 ? 0 : (g0 + __popcll(m & before)) % TEAMS;
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
-            X[i] = Y[i] = 0.0;
-#pragma unroll
-            for (int q = 0; q < NZ; ++q) acc[q][i] = 0.0;
+        for (int t = 0; t < TEAMS; ++t) {
+            const unsigned long long mt = __ballot(on && team == t);
+            if (on && team == t) en.e[t][cnt[t] + __popcll(mt & before)] = v;
+            cnt[t] += __popcll(mt);
         }
-        for (int j = j0; j < j1e; ++j) {
-            const int sb = src[j], c = code[j], fl = flags[j];
-            const CTab1 Ax = tabx + (long long)(c & 255) * NN;
-            // ---- x: X[k1] += sum_j1 Ax[k1][j1] f[j1, j2=a, j3=bq]
-            if (act) {
-                double f[N];
-                const double* fs = fvals + ((size_t)sb * g.npbox + (size_t)N * tid) * nd + ind;
-                if (N % 2 == 0 && nd == 1) {
-                    // one density, even order: the thread's N values are
-                    // contiguous and 16-byte aligned; read them as pairs
-                    const double2* fs2 = reinterpret_cast<const double2*>(fs);
+        g0 += __popcll(m);
+    }
 #pragma unroll
-                    for (int i = 0; i < N / 2; ++i) {
-                        const double2 v = fs2[i];
-                        f[2 * i] = v.x;
-                        f[2 * i + 1] = v.y;
-                    }
-                } else {
+    for (int t = 0; t < TEAMS; ++t)
+        if (lane == 0) en.n[t] = cnt[t];
+}
+
+// Runs a team's entries: the operands of the next entry load (always, past
+// the end the last entry's again, so every path waits with exactly one set in
+// flight) during the products of this one.  OP: an entry's operands; load(e,
+// op), step(e, op).
+template <class OP, class L, class S>
+__device__ __forceinline__ void run_entries(const int2* list, int n, L&& load, S&& step) {
+    if (n <= 0) return;
+    OP a, b;
+    Entry ea = uniform(list[0]), eb = ea;
+    load(ea, a);
+    int2 nx = list[min(1, n - 1)];   // the entry after the one being loaded
+    for (int q = 0; q < n; q += 2) {
+        eb = uniform(nx);
+        load(eb, b);
+        nx = list[min(q + 2, n - 1)];
+        __builtin_amdgcn_sched_barrier(0);
+        step(ea, a);
+        __builtin_amdgcn_sched_barrier(0);
+        if (q + 1 >= n) break;
+        ea = uniform(nx);
+        load(ea, a);
+        nx = list[min(q + 3, n - 1)];
+        __builtin_amdgcn_sched_barrier(0);
+        step(eb, b);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// ------------------------------------------------------------ orders to 12
+// v_mfma_f64_4x4x4_4b (lane = 16 k + 4 b + i, block b): operands A[i][k],
+// B[k][i], result D[k][i].
+
+// T[r][h] = P[(4 h + k) * N + 4 r + i], zero past n: one 1-D table (stored
+// [source node][target node]) as the operand of its contraction.  P is
+// wave-uniform and the lane offset 32-bit (one address register, the rest
+// immediate offsets).
+template <int N, int NB>
+__device__ __forceinline__ void load_table(const double* __restrict__ P, int i, int k, double (&T)[NB][NB]) {
 #pragma unroll
-                    for (int i = 0; i < N; ++i) f[i] = fs[(size_t)i * nd];
-                }
+    for (int r = 0; r < NB; ++r)
 #pragma unroll
-                for (int k1 = 0; k1 < N; ++k1) {
-                    double s = X[k1];
-#pragma unroll
-                    for (int i = 0; i < N; ++i) s += Ax[k1 * N + i] * f[i];
-                    X[k1] = s;
-                }
+        for (int h = 0; h < NB; ++h) {
+            const int j = 4 * h + k, row = 4 * r + i;
+            if (N % 4 == 0) {
+                T[r][h] = gload(P, j * N + row);
+            } else {
+                const double v = gload(P, min(j, N - 1) * N + min(row, N - 1));
+                T[r][h] = row < N && j < N ? v : 0.0;
             }
-            if (fl & 1) {
-                // ---- y: Y[k2] += sum_j2 Ay[k2][j2] X[k1, j2, j3]
-                const CTab1 Ay = taby + (long long)((c >> 8) & 255) * NN;
-                __syncthreads();
-                if (act) {
+        }
+}
+
+template <int N> constexpr int direct3_nb() { return (N + 3) / 4; }
+// a team's exchange buffer [z][y][x] (doubles): odd rows and planes of 4
+// mod 16 put the sixteen lanes of a write into different banks
+template <int N> constexpr int direct3_row() { return 4 * direct3_nb<N>() + 1; }
+template <int N> constexpr int direct3_plane() {
+    return (4 * direct3_nb<N>() * direct3_row<N>() + 11) / 16 * 16 + 4;
+}
+template <int N> constexpr int direct3_buf() { return 4 * direct3_nb<N>() * direct3_plane<N>(); }
+
+// One block per target: TEAMS teams of W waves, each team taking every
+// TEAMS-th z group.  Wave w of a team holds the z slabs j3 = 4 (w S + s) + b,
+// s < S = NB / W, of the source values and of the y and x sums, where the
+// result of one contraction is the operand of the next as it stands; the z
+// contraction takes the x sums through LDS, the wave its rows k2 of the same
+// blocks.  A team of one wave (orders to 8) needs no barrier for that.
+// nls table slots per level, slot codes 8 bits per axis.
+// NZ output components that differ only in their z kind (ZOut) share the x
+// and y sums.
+template <int N> constexpr int direct3_waves() { return direct3_nb<N>() <= 2 ? 1 : direct3_nb<N>(); }
+// three teams where a team is one wave: one per z offset of same-level
+// neighbours, so a target's list takes a third of the time (one team measured
+// the same on lists that fill the device)
+template <int N> constexpr int direct3_teams() { return direct3_waves<N>() == 1 ? 3 : 1; }
+
+template <int N, int NZ>
+__global__ void __launch_bounds__(64 * direct3_waves<N>() * direct3_teams<N>())
+    k_direct3(int nd, const double* __restrict__ loctab, int nls, const int* __restrict__ tgt,
+              const int* __restrict__ lev, const int* __restrict__ off, const int* __restrict__ src,
+              const int* __restrict__ code, const int* __restrict__ flags, const double* __restrict__ fvals,
+              size_t ks, ZGroups zg, int ntask, Multi mu, int runs) {
+    constexpr int NB = direct3_nb<N>(), W = direct3_waves<N>(), TEAMS = direct3_teams<N>(), S = NB / W;
+    constexpr int NN = N * N, NPB = N * N * N;
+    constexpr int ROW = direct3_row<N>(), PLANE = direct3_plane<N>();
+    static_assert(W == 1 || TEAMS == 1, "the teams of a block share its barriers");
+    __shared__ double s_buf[TEAMS][direct3_buf<N>()];   // exchange [j3][k2][k1]
+    __shared__ Entries<TEAMS> en;
+    // blocks of one group after another's
+    const int grp = blockIdx.x / ntask, bt = blockIdx.x - grp * ntask;
+    const int task = runs ? xcd_run_task<8>(bt, ntask) : bt;
+    const Kinds kd = zg.kd[grp];
+    const ZOut& zo = zg.zo[grp];
+    const ProbPtrs* prob = nullptr;
+    if (mu.pp) {
+        prob = mu.pp + mu.tprob[task];
+        loctab = prob->loctab;
+        fvals = prob->fvals;
+    }
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int team = wave / W, w = wave % W;
+    const int i = lane & 3, b = (lane >> 2) & 3, k = lane >> 4;
+    const int tb = tgt[task], l = lev[task];
+    const int j0 = off[task], j1 = off[task + 1];
+    // table kind per axis (value / first / second derivative): stride ks
+    const double* __restrict__ tabx = loctab + (kd.x * ks + (size_t)l * nls * NN);
+    const double* __restrict__ taby = loctab + (kd.y * ks + (size_t)l * nls * NN);
+    double* __restrict__ buf = s_buf[team];
+    struct Op {
+        double F[S][NB][NB], T[NB][NB];
+    };
+    for (int ind = 0; ind < nd; ++ind) {
+        double Z[NZ][S][NB][NB];
 #pragma unroll
-                    for (int k1 = 0; k1 < N; ++k1) dsm[(bq * N + a) * N + k1] = X[k1];   // [j3][j2][k1]
-                }
-                __syncthreads();
-                if (act) {
-                    double xv[N];   // X[k1=a, j2, j3=bq]
+        for (int c = 0; c < NZ; ++c)
 #pragma unroll
-                    for (int j2 = 0; j2 < N; ++j2) xv[j2] = dsm[(bq * N + j2) * N + a];
+            for (int s = 0; s < S; ++s)
 #pragma unroll
-                    for (int k2 = 0; k2 < N; ++k2) {
-                        double s = Y[k2];
+                for (int m = 0; m < NB; ++m)
 #pragma unroll
-                        for (int j2 = 0; j2 < N; ++j2) s += Ay[k2 * N + j2] * xv[j2];
-                        Y[k2] = s;
-                    }
-                }
+                    for (int r = 0; r < NB; ++r) Z[c][s][m][r] = 0.0;
+        double Y[S][NB][NB], X[S][NB][NB];
 #pragma unroll
-                for (int i = 0; i < N; ++i) X[i] = 0.0;
-                if (fl & 2) {
-                    // ---- z: acc[q][k3] += sum_j3 Az_q[k3][j3] Y[k1, k2, j3]
-                    __syncthreads();
-                    if (act) {
+        for (int s = 0; s < S; ++s)
 #pragma unroll
-                        for (int k2 = 0; k2 < N; ++k2) dsm[(bq * N + k2) * N + a] = Y[k2];   // [j3][k2][k1]
-                    }
-                    __syncthreads();
-                    if (act) {
-                        double yv[N];   // Y[k1=a, k2=bq, j3]
+            for (int m = 0; m < NB; ++m)
 #pragma unroll
-                        for (int j3 = 0; j3 < N; ++j3) yv[j3] = dsm[(j3 * N + bq) * N + a];
+                for (int r = 0; r < NB; ++r) Y[s][m][r] = X[s][m][r] = 0.0;
+        auto load = [&](Entry e, Op& op) {
+            const double* __restrict__ f = fvals + (size_t)e.src * NPB * nd + ind;
+            // lane (i = j1, k = j2), slab j3; past n: a valid value, zeroed
 #pragma unroll
-                        for (int q = 0; q < NZ; ++q) {
-                            const CTab1 Az = tabz[q] + (long long)((c >> 16) & 255) * NN;
+            for (int s = 0; s < S; ++s)
 #pragma unroll
-                            for (int k3 = 0; k3 < N; ++k3) {
-                                double s = acc[q][k3];
+                for (int m = 0; m < NB; ++m)
 #pragma unroll
-                                for (int j3 = 0; j3 < N; ++j3) s += Az[k3 * N + j3] * yv[j3];
-                                acc[q][k3] = s;
-                            }
+                    for (int h = 0; h < NB; ++h) {
+                        const int jx = 4 * m + i, jy = 4 * h + k, jz = 4 * (w * S + s) + b;
+                        if (N % 4 == 0) {
+                            op.F[s][m][h] = gload(f, (NN * jz + N * jy + jx) * nd);
+                        } else {
+                            const double v =
+                                gload(f, (NN * min(jz, N - 1) + N * min(jy, N - 1) + min(jx, N - 1)) * nd);
+                            op.F[s][m][h] = jx < N && jy < N && jz < N ? v : 0.0;
                         }
                     }
+            load_table<N, NB>(taby + e.y() * NN, i, k, op.T);
+        };
+        auto step = [&](Entry e, Op& op) {
+            // y: Y[j1][k2] += sum_j2 f[j1][j2] Ay[k2][j2]
 #pragma unroll
-                    for (int i = 0; i < N; ++i) Y[i] = 0.0;
+            for (int h = 0; h < NB; ++h)
+#pragma unroll
+                for (int r = 0; r < NB; ++r)
+#pragma unroll
+                    for (int s = 0; s < S; ++s)
+#pragma unroll
+                        for (int m = 0; m < NB; ++m)
+                            Y[s][m][r] =
+                                __builtin_amdgcn_mfma_f64_4x4x4f64(op.F[s][m][h], op.T[r][h], Y[s][m][r], 0, 0, 0);
+            if (!e.xz_end()) return;
+            // x: X[k1][k2] += sum_j1 Ax[k1][j1] Y[j1][k2]
+            double U[NB][NB];   // (prefetched too it took a third of the registers and gained nothing)
+            load_table<N, NB>(tabx + e.x() * NN, i, k, U);
+#pragma unroll
+            for (int h = 0; h < NB; ++h)
+#pragma unroll
+                for (int r = 0; r < NB; ++r)
+#pragma unroll
+                    for (int s = 0; s < S; ++s)
+#pragma unroll
+                        for (int m = 0; m < NB; ++m)
+                            X[s][m][r] =
+                                __builtin_amdgcn_mfma_f64_4x4x4f64(U[m][h], Y[s][h][r], X[s][m][r], 0, 0, 0);
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+#pragma unroll
+                for (int m = 0; m < NB; ++m)
+#pragma unroll
+                    for (int r = 0; r < NB; ++r) Y[s][m][r] = 0.0;
+            if (!e.z_end()) return;
+            // lane: k1 = 4 m + k, k2 = 4 r + i, slab j3
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+#pragma unroll
+                for (int m = 0; m < NB; ++m)
+#pragma unroll
+                    for (int r = 0; r < NB; ++r) {
+                        buf[(4 * (w * S + s) + b) * PLANE + (4 * r + i) * ROW + 4 * m + k] = X[s][m][r];
+                        X[s][m][r] = 0.0;
+                    }
+            if (W > 1) __syncthreads();
+            else __builtin_amdgcn_wave_barrier();
+            // z: Z[k3][k1] += sum_j3 Az[k3][j3] X[j3][k1], rows k2
+            double V[S][NB][NB];
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+#pragma unroll
+                for (int h = 0; h < NB; ++h)
+#pragma unroll
+                    for (int r = 0; r < NB; ++r)
+                        V[s][h][r] = buf[(4 * h + k) * PLANE + (4 * (w * S + s) + b) * ROW + 4 * r + i];
+#pragma unroll
+            for (int c = 0; c < NZ; ++c) {
+                double A[NB][NB];
+                load_table<N, NB>(loctab + (zo.kz[c] * ks + ((size_t)l * nls + e.z()) * NN), i, k, A);
+#pragma unroll
+                for (int h = 0; h < NB; ++h)
+#pragma unroll
+                    for (int r = 0; r < NB; ++r)
+#pragma unroll
+                        for (int s = 0; s < S; ++s)
+#pragma unroll
+                            for (int m = 0; m < NB; ++m)
+                                Z[c][s][m][r] =
+                                    __builtin_amdgcn_mfma_f64_4x4x4f64(A[m][h], V[s][h][r], Z[c][s][m][r], 0, 0, 0);
+            }
+            if (W > 1) __syncthreads();   // the x sums are read
+            else __builtin_amdgcn_wave_barrier();
+        };
+        for (int c0 = j0; c0 < j1; c0 += kChunk) {
+            if (ind == 0 || j1 - j0 > kChunk) {
+                __syncthreads();
+                if (wave == 0) stage_entries<TEAMS>(en, src, code, flags, c0, min(kChunk, j1 - c0), lane);
+                __syncthreads();
+            }
+            run_entries<Op>(en.e[team], __builtin_amdgcn_readfirstlane(en.n[team]), load, step);
+        }
+        // lane: k3 = 4 m + k, k1 = 4 r + i, rows k2; the teams' sums go to
+        // the first team in order
+#pragma unroll
+        for (int c = 0; c < NZ; ++c) {
+            if (TEAMS > 1) {
+                __syncthreads();
+                if (team > 0) {
+#pragma unroll
+                    for (int s = 0; s < S; ++s)
+#pragma unroll
+                        for (int m = 0; m < NB; ++m)
+#pragma unroll
+                            for (int r = 0; r < NB; ++r)
+                                buf[(4 * m + k) * PLANE + (4 * (w * S + s) + b) * ROW + 4 * r + i] = Z[c][s][m][r];
                 }
+                __syncthreads();
+            }
+            if (team == 0) {
+                // (batches evaluate the potential only)
+                double* __restrict__ o =
+                    (prob ? prob->pot : zo.od[c].p) + (size_t)tb * NPB * zo.od[c].ns + zo.od[c].coff + ind;
+                const int ns = zo.od[c].ns;
+                int node = i + N * (4 * w * S + b) + NN * k;
+                // opaque: the output addresses are formed here, not held
+                // through the whole target
+                asm volatile("" : "+v"(node));
+#pragma unroll
+                for (int s = 0; s < S; ++s)
+#pragma unroll
+                    for (int m = 0; m < NB; ++m)
+#pragma unroll
+                        for (int r = 0; r < NB; ++r) {
+                            const int k1 = 4 * r + i, k2 = 4 * (w * S + s) + b, k3 = 4 * m + k;
+                            double v = Z[c][s][m][r];
+#pragma unroll
+                            for (int t = 1; t < TEAMS; ++t) v += s_buf[t][k3 * PLANE + k2 * ROW + k1];
+                            if (N % 4 == 0 || (k1 < N && k2 < N && k3 < N))
+                                gadd(o, (node + 4 * r + 4 * N * s + 4 * NN * m) * ns, v);
+                        }
             }
         }
-        if (act) {
+        if (TEAMS > 1) __syncthreads();   // the buffers are read
+    }
+}
+
+// ------------------------------------------------------------ orders 13-16
+// v_mfma_f64_16x16x4 (lane = 16 k + i): operands A[i][k], B[k][i], result
+// element v D[k + 4 v][i].
+typedef double dbl4 __attribute__((ext_vector_type(4)));
+
+// T[s] = P[((4 s + k) * N + i) * nd], zero where !ok or past n
+template <int N>
+__device__ __forceinline__ void load_tile(const double* __restrict__ P, int i, int k, bool ok, int nd,
+                                          double (&T)[4]) {
 #pragma unroll
-            for (int q = 0; q < NZ; ++q) {
-                const OutDesc& od = zo.od[q];
-#pragma unroll
-                for (int k3 = 0; k3 < N; ++k3)
-                    od.p[((size_t)tb * g.npbox + a + N * (bq + N * k3)) * od.ns + od.coff + ind] += acc[q][k3];
-            }
+    for (int s = 0; s < 4; ++s) {
+        const int j = 4 * s + k;
+        if (N == 16) {
+            T[s] = gload(P, (j * N + i) * nd);
+        } else {
+            const double v = gload(P, (min(j, N - 1) * N + min(i, N - 1)) * nd);
+            T[s] = ok && i < N && j < N ? v : 0.0;
         }
-        __syncthreads();
+    }
+}
+
+// One block of four waves per target, wave w the z slabs j3 = 4 w .. 4 w + 3
+// (one tile each: rows j1, columns k2), then in the z contraction the rows
+// k2 = 4 w .. 4 w + 3; otherwise as k_direct3.
+template <int N, int NZ>
+__global__ void __launch_bounds__(256, 2)
+    k_direct3w(int nd, const double* __restrict__ loctab, int nls, const int* __restrict__ tgt,
+               const int* __restrict__ lev, const int* __restrict__ off, const int* __restrict__ src,
+               const int* __restrict__ code, const int* __restrict__ flags, const double* __restrict__ fvals,
+               size_t ks, ZGroups zg, int ntask, Multi mu, int runs) {
+    constexpr int NN = N * N, NPB = N * N * N;
+    constexpr int ROW = 17, PLANE = 16 * ROW;
+    __shared__ double buf[16 * PLANE];   // exchange [j3][k2][k1]
+    __shared__ Entries<1> en;
+    // blocks of one group after another's
+    const int grp = blockIdx.x / ntask, bt = blockIdx.x - grp * ntask;
+    const int task = runs ? xcd_run_task<8>(bt, ntask) : bt;
+    const Kinds kd = zg.kd[grp];
+    const ZOut& zo = zg.zo[grp];
+    const ProbPtrs* prob = nullptr;
+    if (mu.pp) {
+        prob = mu.pp + mu.tprob[task];
+        loctab = prob->loctab;
+        fvals = prob->fvals;
+    }
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = lane & 15, k = lane >> 4;
+    const int tb = tgt[task], l = lev[task];
+    const int j0 = off[task], j1 = off[task + 1];
+    const double* __restrict__ tabx = loctab + (kd.x * ks + (size_t)l * nls * NN);
+    const double* __restrict__ taby = loctab + (kd.y * ks + (size_t)l * nls * NN);
+    struct Op {
+        double F[4][4], T[4], U[4];
+    };
+    static_assert(NZ <= 2, "the sums of three z kinds exceed the registers");
+    for (int ind = 0; ind < nd; ++ind) {
+        dbl4 Y[4], X[4], Z[NZ][4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            Y[t] = X[t] = dbl4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int c = 0; c < NZ; ++c) Z[c][t] = dbl4{0.0, 0.0, 0.0, 0.0};
+        }
+        auto load = [&](Entry e, Op& op) {
+            const double* __restrict__ f = fvals + (size_t)e.src * NPB * nd + ind;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const int j3 = 4 * w + t;
+                load_tile<N>(f + (size_t)NN * min(j3, N - 1) * nd, i, k, j3 < N, nd, op.F[t]);
+            }
+            load_tile<N>(taby + e.y() * NN, i, k, true, 1, op.T);
+            load_tile<N>(tabx + e.x() * NN, i, k, true, 1, op.U);
+        };
+        auto step = [&](Entry e, const Op& op) {
+            // y: Y[j1][k2] += sum_j2 f[j1][j2] Ay[k2][j2]
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    Y[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(op.F[t][s], op.T[s], Y[t], 0, 0, 0);
+            if (!e.xz_end()) return;
+            // x: X[k1][k2] += sum_j1 Ax[k1][j1] Y[j1][k2], element s of Y: j1 = k + 4 s
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    X[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(op.U[s], Y[t][s], X[t], 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) Y[t] = dbl4{0.0, 0.0, 0.0, 0.0};
+            if (!e.z_end()) return;
+            // lane: k1 = k + 4 v, k2 = i
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) buf[(4 * w + t) * PLANE + i * ROW + k + 4 * v] = X[t][v];
+                X[t] = dbl4{0.0, 0.0, 0.0, 0.0};
+            }
+            __syncthreads();
+            double V[4][4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) V[t][s] = buf[(4 * s + k) * PLANE + (4 * w + t) * ROW + i];
+#pragma unroll
+            for (int c = 0; c < NZ; ++c) {
+                // z: Z[k3][k1] += sum_j3 Az[k3][j3] X[j3][k1], rows k2
+                double A[4];
+                load_tile<N>(loctab + (zo.kz[c] * ks + ((size_t)l * nls + e.z()) * NN), i, k, true, 1, A);
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        Z[c][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[s], V[t][s], Z[c][t], 0, 0, 0);
+            }
+            __syncthreads();   // the x sums are read
+        };
+        for (int c0 = j0; c0 < j1; c0 += kChunk) {
+            if (ind == 0 || j1 - j0 > kChunk) {
+                __syncthreads();
+                if (w == 0) stage_entries<1>(en, src, code, flags, c0, min(kChunk, j1 - c0), lane);
+                __syncthreads();
+            }
+            run_entries<Op>(en.e[0], __builtin_amdgcn_readfirstlane(en.n[0]), load, step);
+        }
+        // lane: k3 = k + 4 v, k1 = i, rows k2 = 4 w + t (batches evaluate the
+        // potential only)
+#pragma unroll
+        for (int c = 0; c < NZ; ++c) {
+            const OutDesc& od = zo.od[c];
+            double* __restrict__ o = (prob ? prob->pot : od.p) + (size_t)tb * NPB * od.ns + od.coff + ind;
+            const int ns = od.ns;
+            int node = i + N * (4 * w) + NN * k;
+            asm volatile("" : "+v"(node));
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    if (N == 16 || (i < N && 4 * w + t < N && k + 4 * v < N))
+                        gadd(o, (node + N * t + 4 * NN * v) * ns, Z[c][t][v]);
+        }
+    }
+}
+
+template <int N, int NZ>
+void launch_direct3(const Geom& g, const DevTables& t, int ntask, const int* tgt, const int* lev, const int* off,
+                    const int* src, const int* code, const int* flags, const double* fvals, const ZGroups& zg,
+                    hipStream_t s, const Multi& mu) {
+    const int runs = direct_runs(mu);
+    const dim3 grid((unsigned)(ntask * zg.n));
+    if constexpr (N > 12) {
+        hipLaunchKernelGGL((k_direct3w<N, NZ>), grid, dim3(256), 0, s, g.nd, t.loctab, t.loc_slots, tgt, lev, off, src,
+                           code, flags, fvals, t.loctab_ks, zg, ntask, mu, runs);
+    } else {
+        hipLaunchKernelGGL((k_direct3<N, NZ>), grid, dim3(64 * direct3_waves<N>() * direct3_teams<N>()), 0, s, g.nd,
+                           t.loctab, t.loc_slots, tgt, lev, off, src, code, flags, fvals, t.loctab_ks, zg, ntask, mu,
+                           runs);
     }
 }
 
 template <int N>
 bool try_direct3(const Geom& g, const DevTables& t, int ntask, const int* tgt, const int* lev, const int* off,
-                 const int* src, const int* code, const int* flags, const double* fvals, Kinds kd, const ZOut& zo,
+                 const int* src, const int* code, const int* flags, const double* fvals, const ZGroups& zg,
                  hipStream_t s, const Multi& mu) {
-    const size_t lds = sizeof(double) * (size_t)N * N * N;
-    if (lds > t.lds_limit) return false;
-    const dim3 grid(ntask), block(direct3_block<N>());
-    const int runs = direct_runs(mu);
-    switch (zo.nz) {
-        case 1:
-            hipLaunchKernelGGL((k_direct3<N, 1>), grid, block, lds, s, g, t.loctab, t.loc_slots, tgt, lev, off, src,
-                               code, flags, fvals, t.loctab_ks, kd, zo, mu, runs);
-            return true;
-        case 2:
-            hipLaunchKernelGGL((k_direct3<N, 2>), grid, block, lds, s, g, t.loctab, t.loc_slots, tgt, lev, off, src,
-                               code, flags, fvals, t.loctab_ks, kd, zo, mu, runs);
-            return true;
+    switch (zg.zo[0].nz) {
+        case 1: launch_direct3<N, 1>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, s, mu); return true;
+        case 2: launch_direct3<N, 2>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, s, mu); return true;
         case 3:
-            if constexpr (N == 16) {
-                // three z kinds exceed the registers at norder 16 (spills):
-                // two passes, the first sharing two of them
-                ZOut a = zo, b{};
-                a.nz = 2;
-                b.nz = 1;
-                b.kz[0] = zo.kz[2];
-                b.od[0] = zo.od[2];
-                hipLaunchKernelGGL((k_direct3<N, 2>), grid, block, lds, s, g, t.loctab, t.loc_slots, tgt, lev, off,
-                                   src, code, flags, fvals, t.loctab_ks, kd, a, mu, runs);
-                hipLaunchKernelGGL((k_direct3<N, 1>), grid, block, lds, s, g, t.loctab, t.loc_slots, tgt, lev, off,
-                                   src, code, flags, fvals, t.loctab_ks, kd, b, mu, runs);
+            if constexpr (N > 12) {
+                // (three z kinds' sums exceed the registers)
+                launch_direct3<N, 2>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, z_kinds(zg, 0, 2), s, mu);
+                launch_direct3<N, 1>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, z_kinds(zg, 2, 1), s, mu);
             } else {
-                hipLaunchKernelGGL((k_direct3<N, 3>), grid, block, lds, s, g, t.loctab, t.loc_slots, tgt, lev, off,
-                                   src, code, flags, fvals, t.loctab_ks, kd, zo, mu, runs);
+                launch_direct3<N, 3>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, s, mu);
             }
             return true;
-        default:
-            return false;
-    }
-}
-
-bool direct3_covered(const Geom& g, const DevTables& t, int ntask, const int* flags) {
-    return g.ndim == 3 && ntask > 0 && flags && t.n >= 4 && t.n <= 16;
-}
-
-bool direct3_dispatch(const Geom& g, const DevTables& t, int ntask, const int* tgt, const int* lev, const int* off,
-                      const int* src, const int* code, const int* flags, const double* fvals, Kinds kd,
-                      const ZOut& zo, hipStream_t s, const Multi& mu) {
-    switch (t.n) {
-        case 4: return try_direct3<4>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, kd, zo, s, mu);
-        case 5: return try_direct3<5>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, kd, zo, s, mu);
-        case 6: return try_direct3<6>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, kd, zo, s, mu);
-        case 7: return try_direct3<7>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, kd, zo, s, mu);
-        case 8: return try_direct3<8>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, kd, zo, s, mu);
-        case 9: return try_direct3<9>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, kd, zo, s, mu);
-        case 10: return try_direct3<10>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, kd, zo, s, mu);
-        case 11: return try_direct3<11>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, kd, zo, s, mu);
-        case 12: return try_direct3<12>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, kd, zo, s, mu);
-        case 13: return try_direct3<13>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, kd, zo, s, mu);
-        case 14: return try_direct3<14>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, kd, zo, s, mu);
-        case 15: return try_direct3<15>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, kd, zo, s, mu);
-        case 16: return try_direct3<16>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, kd, zo, s, mu);
         default: return false;
     }
 }
@@ -246,20 +556,25 @@ bool direct3_dispatch(const Geom& g, const DevTables& t, int ntask, const int* t
 
 bool launch_direct_3d(const Geom& g, const DevTables& t, int ntask, const int* tgt, const int* lev,
                       const int* off, const int* src, const int* code, const int* flags,
-                      const double* fvals, Kinds kd, OutDesc od, hipStream_t s, const Multi& mu) {
-    if (!direct3_covered(g, t, ntask, flags)) return false;
-    ZOut zo{};
-    zo.nz = 1;
-    zo.kz[0] = kd.z;
-    zo.od[0] = od;
-    return direct3_dispatch(g, t, ntask, tgt, lev, off, src, code, flags, fvals, kd, zo, s, mu);
-}
-
-bool launch_direct_3d_z(const Geom& g, const DevTables& t, int ntask, const int* tgt, const int* lev,
-                        const int* off, const int* src, const int* code, const int* flags,
-                        const double* fvals, Kinds kd, const ZOut& zo, hipStream_t s) {
-    if (!direct3_covered(g, t, ntask, flags) || zo.nz < 1 || zo.nz > 3) return false;
-    return direct3_dispatch(g, t, ntask, tgt, lev, off, src, code, flags, fvals, kd, zo, s, Multi{});
+                      const double* fvals, const ZGroups& zg, hipStream_t s, const Multi& mu) {
+    if (!direct3_orders(g.ndim, t.n) || ntask <= 0 || !flags || zg.n < 1 || zg.n > kMaxZGroups) return false;
+    if ((long long)ntask * zg.n > 0x7fffffffLL) return false;
+    switch (t.n) {
+        case 4: return try_direct3<4>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, s, mu);
+        case 5: return try_direct3<5>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, s, mu);
+        case 6: return try_direct3<6>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, s, mu);
+        case 7: return try_direct3<7>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, s, mu);
+        case 8: return try_direct3<8>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, s, mu);
+        case 9: return try_direct3<9>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, s, mu);
+        case 10: return try_direct3<10>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, s, mu);
+        case 11: return try_direct3<11>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, s, mu);
+        case 12: return try_direct3<12>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, s, mu);
+        case 13: return try_direct3<13>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, s, mu);
+        case 14: return try_direct3<14>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, s, mu);
+        case 15: return try_direct3<15>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, s, mu);
+        case 16: return try_direct3<16>(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, s, mu);
+        default: return false;
+    }
 }
 
 }  // namespace fgt

@@ -159,10 +159,8 @@ __device__ __forceinline__ void pw2pot_sym_block(int npw, int nd, const double2*
 #pragma unroll
                     for (int j = 0; j < KU; ++j) {
                         const int kc = min(k + j, nh - 1);
-                        const ET* __restrict__ ea = E + (size_t)(kc * npw);
-                        const ET* __restrict__ eb = E + (size_t)((npw - 1 - kc) * npw);
-                        e[j][0] = ea[co];
-                        e[j][1] = eb[co];
+                        e[j][0] = gload(E + (size_t)(kc * npw), co);
+                        e[j][1] = gload(E + (size_t)((npw - 1 - kc) * npw), co);
                     }
                 };
                 auto apply = [&](const ET (&e)[KU][2], int k) {
@@ -301,18 +299,19 @@ __device__ __forceinline__ void pw2pot_sym_block(int npw, int nd, const double2*
                 asm volatile("" : "+v"(node));
 #pragma unroll
                 for (int z = 0; z < NZ; ++z) {
-                    double* const op = prob ? prob->pot : zo.od[z].p;
-                    const int ns = zo.od[z].ns, co = zo.od[z].coff + ind;
+                    double* const op = (prob ? prob->pot : zo.od[z].p) + zo.od[z].coff + ind;
+                    const int ns = zo.od[z].ns;
                     const double sgz = zo.kz[z] == 1 ? -2.0 : 2.0;
 #pragma unroll
                     for (int q = 0; q < ZP; ++q) {
                         const int pz = zset * ZP + q;
                         if (pz >= NP) break;
                         if (ba >= 0)
-                            op[((size_t)ba * (N * N * N) + node + N * N * pz) * ns + co] += 2.0 * (GP[z][q] - GQ[z][q]);
+                            gadd(op + (size_t)ba * (N * N * N) * ns, (node + N * N * pz) * ns,
+                                 2.0 * (GP[z][q] - GQ[z][q]));
                         if (bb >= 0 && (FAM || 2 * pz + 1 != N))
-                            op[((size_t)bb * (N * N * N) + node + N * N * (N - 1 - pz)) * ns + co] +=
-                                sgz * (GP[z][q] + GQ[z][q]);
+                            gadd(op + (size_t)bb * (N * N * N) * ns, (node + N * N * (N - 1 - pz)) * ns,
+                                 sgz * (GP[z][q] + GQ[z][q]));
                     }
                 }
             }
@@ -326,12 +325,15 @@ __device__ __forceinline__ void pw2pot_sym_block(int npw, int nd, const double2*
 template <int N, int NZ, typename ET>
 __global__ void __launch_bounds__(kThreads, (NZ > 1 && NZ * N >= 16) ? 2 : 3)
     k_pw2pot_sym(int nd, const double2* __restrict__ tabS, int npw, const SymTask* __restrict__ tasks, int nfam,
-                 int nown, const ET* __restrict__ expn, size_t ks, Kinds kd, ZOut zo, Multi mu) {
+                 int nown, const ET* __restrict__ expn, size_t ks, ZGroups zg, Multi mu) {
     constexpr int PF = sym5_parts<N, true>(), PO = sym5_parts<N, false>();
     extern __shared__ double2 sm[];
-    const int b = blockIdx.x, nfb = nfam * PF;
+    const int nfb = nfam * PF, per = nfb + nown * PO;
+    const int grp = blockIdx.x / per, b = blockIdx.x - grp * per;   // blocks of one group after another's
     const bool fam = b < nfb;
     const int lin = fam ? xcd_task(b, nfb) : xcd_task(b - nfb, nown * PO);
+    const Kinds kd = zg.kd[grp];
+    const ZOut& zo = zg.zo[grp];
     const int tix = fam ? lin / PF : nfam + lin / PO, part = fam ? lin % PF : lin % PO;
     const ProbPtrs* prob = nullptr;
     if (mu.pp) {
@@ -369,7 +371,7 @@ constexpr bool has_fp32(int n) { return n == 8 || n == 12 || n == 16; }
 
 template <int N, int NZ>
 void launch_sym5_z(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks, const double2* expn,
-                   Kinds kd, const ZOut& zo, hipStream_t s, const Multi& mu) {
+                   const ZGroups& zg, hipStream_t s, const Multi& mu) {
     size_t lds = 0;
     // a batch class holds smaller plane-wave counts too
     for (int p = mu.pp ? 1 : t.npw; p <= t.npw; ++p) {
@@ -377,42 +379,33 @@ void launch_sym5_z(const Geom& g, const DevTables& t, int nfam, int nown, const 
         if (nown) lds = std::max(lds, sym5_lds_entries(p, 2 * sym5_nx<N, false>(), 2 * sym_pairs<N, false>()));
     }
     lds *= sizeof(double2);
-    const dim3 grid((unsigned)(nfam * sym5_parts<N, true>() + nown * sym5_parts<N, false>())), block(kThreads);
+    const dim3 grid((unsigned)(zg.n * (nfam * sym5_parts<N, true>() + nown * sym5_parts<N, false>())));
+    const dim3 block(kThreads);
     if constexpr (has_fp32(N)) {
         if (t.expn_f32) {
             hipLaunchKernelGGL((k_pw2pot_sym<N, NZ, float2>), grid, block, lds, s, g.nd, t.pw2potS, t.npw, tasks, nfam,
-                               nown, reinterpret_cast<const float2*>(expn), t.pw2potS_ks, kd, zo, mu);
+                               nown, reinterpret_cast<const float2*>(expn), t.pw2potS_ks, zg, mu);
             return;
         }
     }
     hipLaunchKernelGGL((k_pw2pot_sym<N, NZ, double2>), grid, block, lds, s, g.nd, t.pw2potS, t.npw, tasks, nfam, nown,
-                       expn, t.pw2potS_ks, kd, zo, mu);
-}
-
-// components zo.kz[a .. a + nz) as a group of their own
-ZOut zpart(const ZOut& zo, int a, int nz) {
-    ZOut r{};
-    r.nz = nz;
-    for (int q = 0; q < nz; ++q) {
-        r.kz[q] = zo.kz[a + q];
-        r.od[q] = zo.od[a + q];
-    }
-    return r;
+                       expn, t.pw2potS_ks, zg, mu);
 }
 
 template <int N>
 void launch_sym5(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks, const double2* expn,
-                 Kinds kd, const ZOut& zo, hipStream_t s, const Multi& mu) {
-    if (zo.nz == 1) {
-        launch_sym5_z<N, 1>(g, t, nfam, nown, tasks, expn, kd, zo, s, mu);
-    } else if (zo.nz == 2) {
-        launch_sym5_z<N, 2>(g, t, nfam, nown, tasks, expn, kd, zo, s, mu);
+                 const ZGroups& zg, hipStream_t s, const Multi& mu) {
+    const int nz = zg.zo[0].nz;
+    if (nz == 1) {
+        launch_sym5_z<N, 1>(g, t, nfam, nown, tasks, expn, zg, s, mu);
+    } else if (nz == 2) {
+        launch_sym5_z<N, 2>(g, t, nfam, nown, tasks, expn, zg, s, mu);
     } else if constexpr (N <= 12) {
-        launch_sym5_z<N, 3>(g, t, nfam, nown, tasks, expn, kd, zo, s, mu);
+        launch_sym5_z<N, 3>(g, t, nfam, nown, tasks, expn, zg, s, mu);
     } else {
         // the sums of three z kinds exceed the registers
-        launch_sym5_z<N, 2>(g, t, nfam, nown, tasks, expn, kd, zpart(zo, 0, 2), s, mu);
-        launch_sym5_z<N, 1>(g, t, nfam, nown, tasks, expn, kd, zpart(zo, 2, 1), s, mu);
+        launch_sym5_z<N, 2>(g, t, nfam, nown, tasks, expn, z_kinds(zg, 0, 2), s, mu);
+        launch_sym5_z<N, 1>(g, t, nfam, nown, tasks, expn, z_kinds(zg, 2, 1), s, mu);
     }
 }
 
@@ -481,8 +474,8 @@ __device__ __forceinline__ void p2pw_sym_block(int npw, int nd, const double2* _
         double a[NP], b[NP];
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
-            a[q] = ba >= 0 ? pa[q * st] : 0.0;
-            b[q] = (bb >= 0 && (FAM || 2 * q + 1 != N)) ? pb[(N - 1 - q) * st] : 0.0;
+            a[q] = ba >= 0 ? gload(pa, q * st) : 0.0;
+            b[q] = (bb >= 0 && (FAM || 2 * q + 1 != N)) ? gload(pb, (N - 1 - q) * st) : 0.0;
         }
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
@@ -579,9 +572,9 @@ __device__ __forceinline__ void p2pw_sym_block(int npw, int nd, const double2* _
                             Q.y += t.y * D[q].y;
                         }
                         if (act) {
-                            stE(E + (size_t)(k * npw) + co, make_double2(P.x - Q.y, P.y + Q.x));
+                            gstore(E + (size_t)(k * npw), co, make_double2(P.x - Q.y, P.y + Q.x));
                             if (2 * k + 1 != npw)
-                                stE(E + (size_t)((npw - 1 - k) * npw) + co, make_double2(P.x + Q.y, P.y - Q.x));
+                                gstore(E + (size_t)((npw - 1 - k) * npw), co, make_double2(P.x + Q.y, P.y - Q.x));
                         }
                     }
                 }
@@ -646,9 +639,10 @@ bool launch_p2pw_sym(const Geom& g, const DevTables& t, int nfam, int nown, cons
 }
 
 bool launch_pw2pot_sym(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks,
-                       const double2* expn, Kinds kd, const ZOut& zo, hipStream_t s, const Multi& mu) {
-    if (g.ndim != 3 || zo.nz < 1 || zo.nz > 3 || nfam + nown <= 0) return false;
-    return for_order(t.n, [&](auto n) { launch_sym5<n()>(g, t, nfam, nown, tasks, expn, kd, zo, s, mu); });
+                       const double2* expn, const ZGroups& zg, hipStream_t s, const Multi& mu) {
+    if (g.ndim != 3 || zg.n < 1 || zg.n > kMaxZGroups || zg.zo[0].nz < 1 || zg.zo[0].nz > 3 || nfam + nown <= 0)
+        return false;
+    return for_order(t.n, [&](auto n) { launch_sym5<n()>(g, t, nfam, nown, tasks, expn, zg, s, mu); });
 }
 
 bool sym3_supported(const Geom& g, const DevTables& t) {
