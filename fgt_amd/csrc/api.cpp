@@ -130,7 +130,7 @@ struct fgt_solver {
     DBuf d_leaf_box, d_leaf_lev, d_leaf_slot;
     DBuf d_par_slot, d_par_first, d_par_count, d_pc_parent, d_pc_child, d_pc_sign, d_pc_sign_split;
     DBuf d_m2l_toff, d_m2l_poff, d_m2l_soff, d_m2l_so;   // STEP 3 entry streams per group
-    int n_m2l_groups = 0;
+    int n_m2l_groups = 0, m2l_group = 1;
     DBuf d_mb_toff, d_mb_gent, d_mb_soff, d_mb_code;     // STEP 3 over sibling bricks
     int n_m2l_bricks = -1;                                // -1: bricks not used
     bool m2l_sep_ok = false;                              // bricks' lists geometric: separable form
@@ -150,6 +150,10 @@ struct fgt_solver {
     int n_fz = 0, n_s1 = 0;
     DBuf d_pcs_parent, d_pcs_child, d_pcs_sign;   // splits into non-leaf children only
     std::vector<int> pcs_level_off;
+    // 2-D: leaves by cutoff box, their groups, cutoff boxes of several groups
+    bool plane = false;
+    DBuf d_pl_leaf, d_pl_group, d_pl_soff, d_pl_sslot;
+    int n_pl_leaf = 0, n_pl_group = 0, n_pl_sum = 0;
     double stage_ms[8] = {0};
     // host copies of the device work lists (the batch concatenates them
     // per shape class)
@@ -199,10 +203,68 @@ int map_code(int ndim, int c, int centre = 6) {
 // sort key of a target's near-field entries: sources with equal keys share
 // their z and x tables
 int zxy_code(int c) { return ((c >> 16) & 255) << 8 | (c & 255); }
+// 2-D lists: the PW leaves by cutoff box in groups.  A group's leaves go one
+// after another, 1 to 2 us each: as few as give each CU about four blocks
+// (what the kernel's registers allow), but two at least, since a cutoff box's
+// groups are summed afterwards.  Measured with 2 / 4 / 8 leaves: 15 / 17 / 23
+// us for 595 leaves of order 8, 82 / 77 / 70 for 4363 with three densities.
+void plane_lists(fgt_solver& S) {
+    const fgt::Plan& P = S.plan;
+    std::vector<int> par(P.nslots, -1), sign(P.nslots, 0);
+    for (size_t e = 0; e < P.pc_child.size(); ++e)
+        if (P.pc_child[e] >= 0) {
+            par[P.pc_child[e]] = P.pc_parent[e];
+            sign[P.pc_child[e]] = map_sign(2, P.pc_sign[e]);
+        }
+    const size_t nleaf = P.leaf_box.size();
+    std::vector<fgt::PlaneLeaf> leaf(nleaf);
+    std::vector<int> own(nleaf);
+    for (size_t i = 0; i < nleaf; ++i) {
+        fgt::PlaneLeaf& L = leaf[i];
+        L = {P.leaf_box[i], P.leaf_lev[i], P.leaf_slot[i], P.leaf_lev[i] - P.nlevstart, 0u, 0u};
+        // the path, fine to coarse: the bit of the parent's level
+        for (int d = L.depth - 1; d >= 0; --d) {
+            if (sign[L.slot] & 1) L.sx |= 1u << d;
+            if (sign[L.slot] & 4) L.sz |= 1u << d;
+            L.slot = par[L.slot];
+            if (L.slot < 0) throw std::logic_error("plane-wave leaf without its ancestors' slots");
+        }
+    }
+    std::vector<int> ord(nleaf);
+    for (size_t i = 0; i < nleaf; ++i) ord[i] = (int)i;
+    std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return leaf[a].slot < leaf[b].slot; });
+    std::vector<fgt::PlaneLeaf> sorted(nleaf);
+    for (size_t i = 0; i < nleaf; ++i) sorted[i] = leaf[ord[i]];
+    const int G = std::max(2, (int)((nleaf * P.nd + 1023) / 1024));
+    std::vector<fgt::PlaneGroup> groups;
+    std::vector<int> soff{0}, sslot;
+    for (size_t i = 0; i < nleaf;) {
+        size_t e = i;
+        while (e < nleaf && sorted[e].slot == sorted[i].slot) ++e;
+        const bool several = e - i > (size_t)G;   // the rest in their first leaves' slots
+        for (size_t a = i; a < e; a += G) {
+            const int slot = a == i ? sorted[i].slot : P.leaf_slot[ord[a]];
+            groups.push_back({slot, (int)a, (int)std::min(e - a, (size_t)G)});
+            if (several) sslot.push_back(slot);
+        }
+        if (several) soff.push_back((int)sslot.size());
+        i = e;
+    }
+    S.n_pl_leaf = (int)nleaf;
+    S.n_pl_group = (int)groups.size();
+    S.n_pl_sum = (int)soff.size() - 1;
+    S.d_pl_leaf.upload(sorted);
+    S.d_pl_group.upload(groups);
+    if (S.n_pl_sum) {
+        S.d_pl_soff.upload(soff);
+        S.d_pl_sslot.upload(sslot);
+    }
+}
+
 // near-field tables [..][k][j] (target node, source node) as the kernels of
-// the problem read them: the 3-D ones [j][k]
+// the problem read them, most [j][k]
 std::vector<double> loctab_for(int ndim, int n, const std::vector<double>& t) {
-    if (!fgt::direct3_orders(ndim, n)) return t;
+    if (!fgt::loctab_by_source(ndim, n)) return t;
     std::vector<double> o(t.size());
     const size_t nn = (size_t)n * n;
     for (size_t b = 0; b + nn <= t.size(); b += nn)
@@ -731,8 +793,10 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
     t.n = n;
     t.npw = P.npw;
 
+    S.plane = P.do_pw && fgt::plane_supported(g, t, P.nlevels - P.nlevstart);
+    if (S.plane) plane_lists(S);
     // work lists of the general path
-    if (!S.fast3d) {
+    if (!S.fast3d && !S.plane) {
         S.d_leaf_box.upload(P.leaf_box);
         S.d_leaf_lev.upload(P.leaf_lev);
         S.d_leaf_slot.upload(P.leaf_slot);
@@ -765,7 +829,8 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
             S.d_mb_soff.upload(soff);
             S.d_mb_code.upload(code);
         } else {
-            S.n_m2l_groups = m2l_streams(P, fgt::m2l_group(), toff, gent, soff, code);
+            S.m2l_group = fgt::m2l_group((long long)P.m2l_tgt.size() * (((long long)P.nd * P.nexp + 255) / 256));
+            S.n_m2l_groups = m2l_streams(P, S.m2l_group, toff, gent, soff, code);
             S.d_m2l_toff.upload(toff);
             S.d_m2l_poff.upload(gent);
             S.d_m2l_soff.upload(soff);
@@ -885,7 +950,19 @@ std::vector<fgt::ZGroups> group_comps(const std::vector<Comp>& comps) {
     return out;
 }
 
-// STEP 6 for a list of output components: on the 3-D register-blocked
+// 2-D components for one launch
+fgt::PlaneComps plane_comps(const std::vector<Comp>& comps) {
+    static_assert(fgt::kPlaneComps == 6, "potential, two gradient and three Hessian entries");
+    fgt::PlaneComps pc{};
+    for (const Comp& c : comps) {
+        pc.kx[pc.n] = c.kd.x;
+        pc.kz[pc.n] = c.kd.z;
+        pc.od[pc.n++] = c.od;
+    }
+    return pc;
+}
+
+// STEP 6 for a list of output components: in one launch in 2-D; on the 3-D register-blocked
 // path the components that share their x and y table kinds go in one pass
 // (their x and y sums are formed once; gnd_tens_prod_to_pghloc,
 // bfgt_local.f:756-920, shares the partial sums the same way), elsewhere
@@ -893,6 +970,11 @@ std::vector<fgt::ZGroups> group_comps(const std::vector<Comp>& comps) {
 void launch_direct_comps(const fgt::Geom& g, const fgt::DevTables& t, int ntask, const int* tgt, const int* lev,
                          const int* off, const int* src, const int* code, const int* flags, const double* fvals,
                          const std::vector<Comp>& comps, hipStream_t st) {
+    if (g.ndim == 2) {
+        if (!fgt::launch_direct_plane(g, t, ntask, tgt, lev, off, src, code, fvals, plane_comps(comps), st))
+            throw std::runtime_error("2-D STEP 6 launch failed");
+        return;
+    }
     for (const fgt::ZGroups& zg : group_comps(comps)) {
         if (fgt::launch_direct_3d(g, t, ntask, tgt, lev, off, src, code, flags, fvals, zg, st)) {
             hcheck(hipGetLastError(), "k_direct3 launch");
@@ -966,7 +1048,9 @@ void execute(fgt_solver& S, hipStream_t st, bool timed, bool fork_near = false,
                             S.d_dir_off.as<int>(), S.d_dir_src.as<int>(), S.d_dir_code.as<int>(),
                             S.d_dir_flags.as<int>(), fv, comps, sn);
     };
-    const bool fork = fork_near && P.do_pw && !P.dir_tgt.empty();
+    // (not in 2-D: the second stream's events cost more than its near field,
+    // 63 us against 32 for 595 leaves)
+    const bool fork = fork_near && !S.plane && P.do_pw && !P.dir_tgt.empty();
     if (fork) {
         if (!S.st_near) {
             hcheck(hipStreamCreateWithFlags(&S.st_near, hipStreamNonBlocking), "hipStreamCreate near");
@@ -1005,6 +1089,15 @@ void execute(fgt_solver& S, hipStream_t st, bool timed, bool fork_near = false,
                                   S.d_mp_acc.as<int>() + a, P.nlevels - l, ex, st);
             }
             mark(2);
+        } else if (S.plane) {
+            // STEPs 1 and 2 of every leaf and level
+            if (!fgt::launch_p2pw_plane(g, t, P.nlevels - P.nlevstart, S.n_pl_group, S.d_pl_group.as<fgt::PlaneGroup>(),
+                                        S.d_pl_leaf.as<fgt::PlaneLeaf>(), S.n_pl_sum, S.d_pl_soff.as<int>(),
+                                        S.d_pl_sslot.as<int>(), fv, ex, st))
+                throw std::runtime_error("2-D STEP 1 launch failed");
+            fork_near_field();
+            mark(1);
+            mark(2);
         } else {
             // STEP 1: every PW leaf, all levels in one launch
             fgt::launch_p2pw(g, t, (int)P.leaf_box.size(), S.d_leaf_box.as<int>(), S.d_leaf_lev.as<int>(),
@@ -1028,14 +1121,15 @@ void execute(fgt_solver& S, hipStream_t st, bool timed, bool fork_near = false,
             fgt::launch_m2l_brick(g, t, S.n_m2l_bricks, 2LL * P.nd * P.nexp * P.nslots, S.d_mb_toff.as<long long>(),
                                   S.d_mb_gent.as<int>(), S.d_mb_soff.as<long long>(), S.d_mb_code.as<int>(), ex, st);
         else
-            fgt::launch_m2l27(g, t, S.n_m2l_groups, fgt::m2l_group(), 2LL * P.nd * P.nexp * P.nslots,
+            fgt::launch_m2l27(g, t, S.n_m2l_groups, S.m2l_group, 2LL * P.nd * P.nexp * P.nslots,
                               S.d_m2l_toff.as<long long>(), S.d_m2l_poff.as<int>(), S.d_m2l_soff.as<long long>(),
                               S.d_m2l_so.as<int>(), ex, st, fgt::Multi{},
                               m2l_ept_default((((long long)P.nd * P.nexp) & 1) == 0));
         mark(3);
         // STEP 4: coarse to fine (fast 3-D path: only into non-leaf children;
         // leaves read their parent's expansion in STEP 5 through phased tables)
-        for (int l = P.nlevstart; l <= P.nlevels - 1; ++l) {
+        // (2-D: STEP 5 takes the cutoff boxes' expansions)
+        for (int l = P.nlevstart; !S.plane && l <= P.nlevels - 1; ++l) {
             if (S.fast3d) {
                 const int a = S.pcs_level_off[l], b = S.pcs_level_off[l + 1];
                 fgt::launch_split(g, t, b - a, S.d_pcs_parent.as<int>() + a, S.d_pcs_child.as<int>() + a,
@@ -1055,7 +1149,11 @@ void execute(fgt_solver& S, hipStream_t st, bool timed, bool fork_near = false,
         if (S.fast3d)
             launch_pw2pot_comps(g, t, {S.n_s5, S.n_s5_sib, S.d_s5_tasks.as<fgt::PotTask>(), nullptr, S.n_s5_fam,
                                        S.n_s5_own, S.d_s5_sym.as<fgt::SymTask>(), nullptr}, ex, comps, st);
-        else
+        else if (S.plane) {
+            if (!fgt::launch_pw2pot_plane(g, t, P.nlevels - P.nlevstart, S.n_pl_leaf, S.d_pl_leaf.as<fgt::PlaneLeaf>(),
+                                          ex, plane_comps(comps), st))
+                throw std::runtime_error("2-D STEP 5 launch failed");
+        } else
             for (const Comp& c : comps)
                 fgt::launch_pw2pot(g, t, (int)P.leaf_box.size(), S.d_leaf_box.as<int>(), S.d_leaf_lev.as<int>(),
                                    S.d_leaf_slot.as<int>(), ex, c.kd, c.od, st);
@@ -2117,8 +2215,13 @@ struct Refiner {
             }
         std::unordered_map<int, int> tmp;     // solve slot of a grandparent -> workspace slot
         int ns = 0;
+        // (2-D: only the cutoff boxes have theirs, so the boxes from there down)
         for (int p : parents)
-            if (p < nb0 && T.level[p] > P.nlevstart && !tmp.count(T.parent[p])) tmp[T.parent[p]] = ns++;
+            for (int q = p; q < nb0 && T.level[q] > P.nlevstart;) {
+                q = T.parent[q];
+                if (!tmp.count(q)) tmp[q] = ns++;
+                if (!S.plane) break;
+            }
         for (int p : parents) aslot[p] = ns++;
         std::vector<int> bslot(nk, -1);
         for (int i = 0; i < nk; ++i)
@@ -2128,13 +2231,21 @@ struct Refiner {
         double2* W = ws.as<double2>();
         const double2* X = S.d_expn.as<double2>();
         const size_t sb = sizeof(double2) * slot_el;
+        // entries per split level code: (source slot, target slot, sign)
+        std::map<int, std::array<std::vector<int>, 3>> splits;
         for (const auto& kv : tmp) {
+            if (S.plane && T.level[kv.first] > P.nlevstart) {
+                const int q = T.parent[kv.first];
+                auto& e = splits[P.nlevels - T.level[q]];
+                e[0].push_back(tmp.at(q));
+                e[1].push_back(kv.second);
+                e[2].push_back(split_sign(T.centers, ndim, kv.first, q));
+                continue;
+            }
             const int sl = P.slot_of_box[kv.first];
             if (sl < 0) throw std::logic_error("refinement: parent without a plane-wave slot");
             hcheck(hipMemcpyAsync(W + slot_el * kv.second, X + slot_el * sl, sb, hipMemcpyDeviceToDevice, st), "copy loc");
         }
-        // entries per split level code: (source slot, target slot, sign)
-        std::map<int, std::array<std::vector<int>, 3>> splits;
         for (int p : parents) {
             const int a = aslot[p];
             if (p < nb0) {
@@ -2160,12 +2271,12 @@ struct Refiner {
         }
         DBuf d_a, d_b, d_c;
         auto run_splits = [&]() {
-            for (auto& kv : splits) {
-                const int ne = (int)kv.second[0].size();
-                d_a.upload(kv.second[0]);
-                d_b.upload(kv.second[1]);
-                d_c.upload(kv.second[2]);
-                fgt::launch_split(g, S.tabs, ne, d_a.as<int>(), d_b.as<int>(), d_c.as<int>(), kv.first, W, st);
+            for (auto kv = splits.rbegin(); kv != splits.rend(); ++kv) {   // coarse to fine
+                const int ne = (int)kv->second[0].size();
+                d_a.upload(kv->second[0]);
+                d_b.upload(kv->second[1]);
+                d_c.upload(kv->second[2]);
+                fgt::launch_split(g, S.tabs, ne, d_a.as<int>(), d_b.as<int>(), d_c.as<int>(), kv->first, W, st);
                 hcheck(hipStreamSynchronize(st), "refinement split");
             }
             splits.clear();
@@ -2204,7 +2315,15 @@ struct Refiner {
             db.upload(pw_box);
             dl.upload(pw_lev);
             dsl.upload(pw_slot);
-            for (const Comp& c : comps)
+            DBuf dpl;   // (used until the synchronisation below)
+            if (S.plane) {
+                std::vector<fgt::PlaneLeaf> pl;
+                for (size_t i = 0; i < pw_box.size(); ++i) pl.push_back({pw_box[i], pw_lev[i], pw_slot[i], 0, 0u, 0u});
+                dpl.upload(pl);
+                if (!fgt::launch_pw2pot_plane(g, S.tabs, P.nlevels - P.nlevstart, (int)pl.size(),
+                                              dpl.as<fgt::PlaneLeaf>(), W, plane_comps(comps), st))
+                    throw std::runtime_error("2-D STEP 5 launch failed");
+            } else for (const Comp& c : comps)
                 fgt::launch_pw2pot(g, S.tabs, (int)pw_box.size(), db.as<int>(), dl.as<int>(), dsl.as<int>(), W, c.kd,
                                    c.od, st);
         }

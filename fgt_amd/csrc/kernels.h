@@ -178,6 +178,25 @@ struct SymTask {
     int box[8];
 };
 
+// 2-D: a leaf with an expansion (at `depth` levels below its cutoff box, whose
+// expansion is in `slot`; bit i of sx / sz set when the merge phase of the
+// path's level i, coarse to fine, is conjugated along that axis), and a group
+// of consecutive leaves of one cutoff box, summed into expansion `slot`.
+struct PlaneLeaf {
+    int box, lev, slot, depth;
+    unsigned sx, sz;
+};
+struct PlaneGroup {
+    int slot, first, count;
+};
+// 2-D output components: x and z table kinds, outputs
+constexpr int kPlaneComps = 6;
+struct PlaneComps {
+    int n;
+    int kx[kPlaneComps], kz[kPlaneComps];
+    OutDesc od[kPlaneComps];
+};
+
 // Several problems of one shape class (3-D, same norder, density count and
 // precision; plane-wave counts may differ) in one launch.  Task i of a launch belongs
 // to problem tprob[i]; the kernel then takes that problem's tables, values,
@@ -220,7 +239,7 @@ struct DevTables {
     const double2* wms;
     const double2* wm2l;
     // near-field masked tables loc[kind][l][slot][k][j] ([j][k] where
-    // direct3_orders), bands [l][slot][k][2];
+    // loctab_by_source), bands [l][slot][k][2];
     // loc_slots table slots per level (13 for the solve, 193 for the
     // refinement of a new tree); a pair's table slots are packed 8 bits per
     // kernel axis: x | y << 8 | z << 16
@@ -316,9 +335,11 @@ void launch_merge(const Geom& g, const DevTables& t, int ntask, const int* par_s
 // target's final entry.
 constexpr int kM2lGroup = 4;   // best at 4-5 with six blocks per CU (8 was best at four)
 constexpr int kM2lGroupMax = 12;
-// targets per STEP 3 block: kM2lGroup, or FGT_M2L_GROUP (1..kM2lGroupMax,
-// tuning runs)
-int m2l_group();
+// targets per STEP 3 block of a problem with `blocks` targets x element
+// ranges: kM2lGroup, or one where even that leaves each CU fewer than sixteen
+// blocks (178 targets of 800 elements: 13 us in groups of four, now 9), or
+// FGT_M2L_GROUP (1..kM2lGroupMax, tuning runs)
+int m2l_group(long long blocks);
 constexpr int kM2lBatch = 4;
 // longest entry stream of a group: kM2lGroupMax targets x (own + 26 list
 // entries), padded
@@ -381,10 +402,26 @@ void launch_direct(const Geom& g, const DevTables& t, int ntask, const int* tgt,
 // the 3-D near-field kernels cover this order (4..16); they read the near-
 // field tables as [j][k] (source node, target node)
 inline bool direct3_orders(int ndim, int n) { return ndim == 3 && n >= 4 && n <= 16; }
+// the near-field tables of a problem are [j][k] (the 2-D kernel reads them so
+// for every order)
+inline bool loctab_by_source(int ndim, int n) { return ndim == 2 || direct3_orders(ndim, n); }
 // orders covered, with flags; false when not (nothing launched)
 bool launch_direct_3d(const Geom& g, const DevTables& t, int ntask, const int* tgt, const int* lev,
                       const int* off, const int* src, const int* code, const int* flags,
                       const double* fvals, const ZGroups& zg, hipStream_t s, const Multi& mu = Multi{});
+
+// 2-D STEP 1 + 2, STEP 4 + 5 and STEP 6 (kernels_plane.hip); nlev: levels
+// below the cutoff.  The launchers return false on a launch error.
+bool plane_supported(const Geom& g, const DevTables& t, int nlev);
+// leaves grouped by cutoff box; sum_slots[sum_off[i] ..]: the group slots of
+// the i-th cutoff box with more than one group, its own first
+bool launch_p2pw_plane(const Geom& g, const DevTables& t, int nlev, int ngroup, const PlaneGroup* groups,
+                       const PlaneLeaf* leaves, int nsum, const int* sum_off, const int* sum_slots,
+                       const double* fvals, double2* expn, hipStream_t s);
+bool launch_pw2pot_plane(const Geom& g, const DevTables& t, int nlev, int nleaf, const PlaneLeaf* leaves,
+                         const double2* expn, const PlaneComps& pc, hipStream_t s);
+bool launch_direct_plane(const Geom& g, const DevTables& t, int ntask, const int* tgt, const int* lev, const int* off,
+                         const int* src, const int* code, const double* fvals, const PlaneComps& pc, hipStream_t s);
 
 // Device workspace of the no-allocation entry point: a file-scope device
 // array of kScratchBytes per GPU.  scratch_region() returns its address on
