@@ -124,8 +124,9 @@ struct fgt_solver {
     DBuf d_grad, d_hess;    // grad(nd,ndim,npbox,nboxes), hess(nd,nhess,npbox,nboxes)
     // extra targets (STEP 11): set up on first use
     bool t_ready = false;
-    DBuf d_t_u, d_t_leaves, d_t_centers, d_t_bsz, d_t_coefs;
+    DBuf d_t_u, d_t_child, d_t_centers, d_t_bsz, d_t_work;
     int t_nleaf = 0;
+    bool t_whole = true;    // no parent lacks a child
     // lists
     DBuf d_leaf_box, d_leaf_lev, d_leaf_slot;
     DBuf d_par_slot, d_par_first, d_par_count, d_pc_parent, d_pc_child, d_pc_sign, d_pc_sign_split;
@@ -1190,6 +1191,9 @@ void execute(fgt_solver& S, hipStream_t st, bool timed, bool fork_near = false,
 // at the targets.  Targets are assigned to leaves on the host by the
 // reference's root-to-leaf descent (child bit a set when t_a - c_a >= 0,
 // find_childbox_ind, src/common/pts_tree_nd.f:713-740) and grouped by leaf.
+// per-solver target workspaces up to this size are kept between calls
+constexpr size_t kTargetWorkKept = size_t(32) << 20;
+
 void eval_targets(fgt_solver& S, int nt, const double* targs, int ifpghtarg, double* pote, double* grade,
                   double* hesse, hipStream_t st) {
     const fgt::Plan& P = S.plan;
@@ -1201,67 +1205,77 @@ void eval_targets(fgt_solver& S, int nt, const double* targs, int ifpghtarg, dou
         std::vector<double> x(n), w(n), u((size_t)n * n);
         fgt::poly_exps(P.ipoly, n, x.data(), w.data(), u.data());
         S.d_t_u.upload(u);
-        std::vector<int> leaves;
+        std::vector<int> child((size_t)mc * P.nboxes, -1);
         std::vector<double> bsz(P.nboxes);
+        S.t_nleaf = 0;
+        S.t_whole = true;
         for (int b = 0; b < P.nboxes; ++b) {
-            if (T.nchild[b] == 0) leaves.push_back(b);
             bsz[b] = T.boxsize[T.level[b]];
+            if (T.nchild[b] == 0) {
+                ++S.t_nleaf;
+                continue;
+            }
+            for (int k = 0; k < mc; ++k) {
+                const int c = T.child[(size_t)mc * b + k];
+                child[(size_t)mc * b + k] = c >= 0 ? c : -2;
+                if (c < 0) S.t_whole = false;
+            }
         }
-        S.t_nleaf = (int)leaves.size();
-        S.d_t_leaves.upload(leaves);
+        S.d_t_child.upload(child);
         S.d_t_centers.upload(T.centers);
         S.d_t_bsz.upload(bsz);
         S.t_ready = true;
     }
-    std::vector<int> leaf(nt), perm(nt);
-    for (int it = 0; it < nt; ++it) {
-        int b = 0;
-        while (T.nchild[b] > 0) {
-            int k = 0;
-            for (int a = 0; a < ndim; ++a)
-                if (targs[(size_t)ndim * it + a] - T.centers[(size_t)ndim * b + a] >= 0) k |= 1 << a;
-            const int c = T.child[(size_t)mc * b + k];
-            if (c < 0) throw std::invalid_argument("tree has a box with a missing child");
-            b = c;
-        }
-        leaf[it] = b;
-        perm[it] = it;
-    }
-    std::stable_sort(perm.begin(), perm.end(), [&](int a, int b) { return leaf[a] < leaf[b]; });
-    std::vector<double> ts((size_t)nt * ndim);
-    std::vector<int> tbox, tfirst, tcount;
-    for (int i = 0; i < nt; ++i) {
-        for (int a = 0; a < ndim; ++a) ts[(size_t)ndim * i + a] = targs[(size_t)ndim * perm[i] + a];
-        if (i == 0 || leaf[perm[i]] != leaf[perm[i - 1]] || tcount.back() == 256) {
-            tbox.push_back(leaf[perm[i]]);
-            tfirst.push_back(i);
-            tcount.push_back(0);
-        }
-        ++tcount.back();
-    }
-    DBuf d_ts, d_perm, d_tbox, d_tfirst, d_tcount, d_out;
-    d_ts.upload(ts);
-    d_perm.upload(perm);
-    d_tbox.upload(tbox);
-    d_tfirst.upload(tfirst);
-    d_tcount.upload(tcount);
     const int nhess = ndim * (ndim + 1) / 2;
     struct Out { const DBuf* vals; int ncomp; double* host; };
     const Out outs[3] = {{&S.d_pot, 1, pote}, {&S.d_grad, ndim, grade}, {&S.d_hess, nhess, hesse}};
+    int ncdmax = 0;
+    for (int L = 0; L < ifpghtarg; ++L) ncdmax = std::max(ncdmax, nd * outs[L].ncomp);
+    // one workspace; each part starts on 16 bytes
+    const int maxtask = fgt::target_tasks_max(nt, S.t_nleaf);
+    size_t bytes = 0;
+    auto part = [&](size_t b) {
+        const size_t at = bytes;
+        bytes += (b + 15) & ~size_t(15);
+        return at;
+    };
+    const size_t a_count = part(sizeof(int) * ((size_t)P.nboxes + 2)), a_first = part(sizeof(int) * (size_t)P.nboxes),
+                 a_place = part(sizeof(int2) * (size_t)nt), a_perm = part(sizeof(int) * (size_t)nt),
+                 a_task = part(sizeof(int4) * (size_t)maxtask), a_ts = part(sizeof(double) * (size_t)nt * ndim),
+                 a_out = part(sizeof(double) * (size_t)nt * ncdmax);
+    if (S.d_t_work.bytes < bytes) S.d_t_work.alloc(bytes);
+    char* W = S.d_t_work.as<char>();
+    int* count = reinterpret_cast<int*>(W + a_count);   // then the task count and the missing-child flag
+    int *ntask = count + P.nboxes, *missing = ntask + 1;
+    int* perm = reinterpret_cast<int*>(W + a_perm);
+    int4* tasks = reinterpret_cast<int4*>(W + a_task);
+    double* ts = reinterpret_cast<double*>(W + a_ts);
+    double* out = reinterpret_cast<double*>(W + a_out);
+    hcheck(hipMemcpy(ts, targs, sizeof(double) * (size_t)nt * ndim, hipMemcpyHostToDevice), "upload targets");
+    fgt::launch_zero(count, a_first - a_count, st);
+    if (!fgt::launch_target_groups(nt, ndim, P.nlevels, P.nboxes, ts, S.d_t_centers.as<double>(),
+                                   S.d_t_child.as<int>(), count, reinterpret_cast<int*>(W + a_first),
+                                   reinterpret_cast<int2*>(W + a_place), perm, tasks, ntask, missing, st))
+        throw std::runtime_error("target grouping launch failed");
+    if (!S.t_whole) {
+        int lost = 0;
+        hcheck(hipStreamSynchronize(st), "hipStreamSynchronize");
+        hcheck(hipMemcpy(&lost, missing, sizeof lost, hipMemcpyDeviceToHost), "download target flag");
+        if (lost) throw std::invalid_argument("tree has a box with a missing child");
+    }
     for (int L = 0; L < ifpghtarg; ++L) {
         const int ncd = nd * outs[L].ncomp;
-        const size_t need = sizeof(double) * (size_t)ncd * P.npbox * P.nboxes;
-        if (S.d_t_coefs.bytes < need) S.d_t_coefs.alloc(need);
-        d_out.alloc(sizeof(double) * (size_t)ncd * nt);
-        fgt::launch_vals2coefs(ndim, n, ncd, S.d_t_u.as<double>(), S.t_nleaf, S.d_t_leaves.as<int>(),
-                               outs[L].vals->as<double>(), S.d_t_coefs.as<double>(), st);
-        hcheck(hipGetLastError(), "k_vals2coefs launch");
-        fgt::launch_evalt(ndim, n, P.ipoly, ncd, (int)tbox.size(), d_tbox.as<int>(), d_tfirst.as<int>(),
-                          d_tcount.as<int>(), S.d_t_centers.as<double>(), S.d_t_bsz.as<double>(), d_ts.as<double>(),
-                          d_perm.as<int>(), S.d_t_coefs.as<double>(), d_out.as<double>(), st);
-        hcheck(hipGetLastError(), "k_evalt launch");
+        if (!fgt::launch_targets(ndim, n, P.ipoly, ncd, maxtask, S.d_t_u.as<double>(), tasks, ntask,
+                                 S.d_t_centers.as<double>(), S.d_t_bsz.as<double>(), ts, perm,
+                                 outs[L].vals->as<double>(), out, st))
+            throw std::runtime_error("target evaluation launch failed");
         hcheck(hipStreamSynchronize(st), "hipStreamSynchronize");
-        hcheck(hipMemcpy(outs[L].host, d_out.p, d_out.bytes, hipMemcpyDeviceToHost), "download target values");
+        hcheck(hipMemcpy(outs[L].host, out, sizeof(double) * (size_t)ncd * nt, hipMemcpyDeviceToHost),
+               "download target values");
+    }
+    if (S.d_t_work.bytes > kTargetWorkKept) {
+        S.d_t_work.release();
+        S.d_t_work.bytes = 0;
     }
 }
 

@@ -431,14 +431,19 @@ constexpr size_t kScratchBytes = size_t(128) << 20;
 void* scratch_region(size_t* bytes);
 void launch_zero(void* p, size_t bytes, hipStream_t s);
 
-// Extra targets (STEP 11): values (ncd, npbox, nboxes) on the listed leaves
-// -> coefficients coefs[b][q][i] (u = values->coefficients, u(k,j) at
-// u[k + j*n]); then per task (leaf tbox, sorted targets tfirst..+tcount,
-// tcount <= 256) the expansion at each target, out[perm[t]*ncd + q].
-void launch_vals2coefs(int ndim, int n, int ncd, const double* u, int nleaf, const int* leaves, const double* vals,
-                       double* coefs, hipStream_t s);
-void launch_evalt(int ndim, int n, int ipoly, int ncd, int ntask, const int* tbox, const int* tfirst,
-                  const int* tcount, const double* centers, const double* bsize_of_box, const double* targs_sorted,
-                  const int* perm, const double* coefs, double* out, hipStream_t s);
+// Extra targets (STEP 11).  launch_target_groups groups them by leaf: child
+// [box][2^ndim] (-1 leaf, -2 missing child), count zeroed by the caller;
+// perm the targets by leaf, tasks {box, first, count, -} of at most 256 and
+// their number *ntask (<= target_tasks_max); *missing set when a target's path
+// ends at a missing child.  launch_targets evaluates values (ncd, npbox,
+// nboxes) at the targets, out[t*ncd + q] (u = values->coefficients, u(k,j) at
+// u[k + j*n]).
+int target_tasks_max(int nt, int nleaf);
+bool launch_target_groups(int nt, int ndim, int nlevels, int nboxes, const double* targs, const double* centers,
+                          const int* child, int* count, int* first, int2* place, int* perm, int4* tasks, int* ntask,
+                          int* missing, hipStream_t s);
+bool launch_targets(int ndim, int n, int ipoly, int ncd, int maxtask, const double* u, const int4* tasks,
+                    const int* ntask, const double* centers, const double* bsize_of_box, const double* targs,
+                    const int* perm, const double* vals, double* out, hipStream_t s);
 
 }  // namespace fgt
