@@ -340,7 +340,7 @@ constexpr int kM2lGroupMax = 12;
 // blocks (178 targets of 800 elements: 13 us in groups of four, now 9), or
 // FGT_M2L_GROUP (1..kM2lGroupMax, tuning runs)
 int m2l_group(long long blocks);
-constexpr int kM2lBatch = 4;
+constexpr int kM2lBatch = 2;
 // longest entry stream of a group: kM2lGroupMax targets x (own + 26 list
 // entries), padded
 constexpr int kM2lMaxEntries = kM2lGroupMax * 27 + kM2lBatch;

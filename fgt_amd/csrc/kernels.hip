@@ -145,16 +145,28 @@ __global__ void __launch_bounds__(kBlock) k_merge(Geom g, DevTables t, const int
     if (e >= tot) return;
     const int r = (int)(e % g.nexp);
     const int k2 = r % g.py, k1 = (r / g.py) % g.px, k3 = r / (g.py * g.px);
-    const int first = par_first[task], cnt = par_count[task];
+    const int first = par_first[task], cnt = par_count[task];   // 1..8
+    ET* __restrict__ dst = expn + (size_t)par_slot[task] * 2 * tot;
+    // every child's element is loaded (past the last, its own again) before
+    // the first is used
+    ET v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = gload(expn + (size_t)pc_child[first + min(i, cnt - 1)] * 2 * tot, (unsigned)e);
     // par_acc[task] != 0: the parent already holds its leaf children's part
-    double2 acc = (par_acc && par_acc[task]) ? ldE(expn[(size_t)par_slot[task] * 2 * tot + e])
-                                             : make_double2(0.0, 0.0);
-    for (int i = 0; i < cnt; ++i) {
-        const int cs = pc_child[first + i];
-        const double2 v = ldE(expn[(size_t)cs * 2 * tot + e]);
-        acc = cfma(v, ms_phase(w1, pc_sign[first + i], k1, k2, k3, g), acc);
+    double2 acc = make_double2(0.0, 0.0);
+    if (par_acc && par_acc[task]) acc = ldE(gload(dst, (unsigned)e));
+    // ms_phase per child from the two x-y products (a conjugate is exact)
+    const double2 wx = g.px > 1 ? w1[k1] : make_double2(1.0, 0.0);
+    const double2 wy = g.py > 1 ? w1[k2] : make_double2(1.0, 0.0);
+    const double2 wz = w1[k3], pa = cmul(wx, wy), pb = cmul(conjd(wx), wy);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        if (i >= cnt) break;
+        const int sg = pc_sign[first + i];
+        const double2 xy = (sg & 1) ? ((sg & 2) ? conjd(pa) : pb) : ((sg & 2) ? conjd(pb) : pa);
+        acc = cfma(ldE(v[i]), cmul(xy, (sg & 4) ? conjd(wz) : wz), acc);
     }
-    stE(expn + (size_t)par_slot[task] * 2 * tot + e, acc);
+    gstore(dst, (unsigned)e, acc);
 }
 
 // ---------------------------------------------------------------- STEP 3
@@ -328,8 +340,16 @@ __global__ void __launch_bounds__(kBlock) k_m2l27(Geom g, DevTables t, int ngrou
 // selection as k_m2l27 (w_z from three more LDS rows).  Every target's own expansion is the entry at its
 // own position (o = 13, unit phase).  toff: 8 loc offsets per brick (-1 =
 // no target there); entries padded with zero-slot entries of mask 0.
+// A thread holds the element pair (k1, k2) and (npw-1-k1, npw-1-k2) of one k3,
+// whose x-y phases are conjugate and whose z phases are the same: the LDS reads
+// of the phases, two per applied pair of expansions, serve both.  Besides
+// those the source loads from the caches bound it: short blocks (the blocks of
+// one element range then share fewer source bytes than an XCD's L2 holds), and
+// entries padded to two, not four.  Whole solves: periodic order 16 with 1245
+// targets 1864 -> 1743 us, order-8 gradient with 752 targets 452 -> 418.
+constexpr int kBrickBlock = 128;
 template <typename ET>
-__global__ void __launch_bounds__(kBlock) k_m2l_brick(Geom g, DevTables t, int nbrick, long long zero_off,
+__global__ void __launch_bounds__(kBrickBlock) k_m2l_brick(Geom g, DevTables t, int nbrick, long long zero_off,
                                                       const long long* __restrict__ toff,
                                                       const int* __restrict__ gent,
                                                       const long long* __restrict__ soff,
@@ -347,20 +367,24 @@ __global__ void __launch_bounds__(kBlock) k_m2l_brick(Geom g, DevTables t, int n
         zero_off = q.zero_off;
     }
     const long long tot = (long long)g.nd * g.nexp;
-    if ((long long)chunk * blockDim.x >= tot) return;   // past this problem's elements
-    const int npw = t.npw;
-    long long e = (long long)chunk * blockDim.x + threadIdx.x;
-    const bool ok = e < tot;
-    if (!ok) e = tot - 1;   // valid duplicate, never stored
-    const int r = (int)(e % g.nexp);
-    const int k2 = r % g.py, k1 = (r / g.py) % g.px, k3 = r / (g.py * g.px);
+    // a thread's two elements: (k1, k2) and (npw-1-k1, npw-1-k2) of one k3
+    // plane, entries p and npw^2-1-p of it (the middle one of an odd npw twice)
+    const int npw = t.npw, plane = npw * npw, half = (plane + 1) / 2;
+    const int npair = g.nd * g.pz * half;
+    const int pair = chunk * kBrickBlock + (int)threadIdx.x;
+    if (chunk * kBrickBlock >= npair) return;   // past this problem's elements
+    const bool ok = pair < npair;
+    const int pc = ok ? pair : npair - 1;   // valid duplicate, never stored
+    const int kp = pc / half, p0 = pc - kp * half;
+    const int k2 = p0 % npw, k1 = p0 / npw, k3 = kp % g.pz;
+    const long long e = (long long)kp * plane + p0, e2 = (long long)kp * plane + plane - 1 - p0;
     // rows 0-4: the w_x w_y products (row 4 = 1); row 5: c = w_z(2).  w_z
     // for oz = 0, 1, 2 is conj(c), 1, c (the table's rows are exactly that),
     // read at a uniform row (5 with a sign flip, 4, 5) instead of selected
     // from registers per pair (STEP 3 at a norder-16 periodic problem 0.745
     // -> 0.696 ms); six rows rather than eight leave room for six blocks per
     // CU in LDS instead of four
-    __shared__ double2 s_fxy[6][kBlock];
+    __shared__ double2 s_fxy[6][kBrickBlock];
     const int tid = threadIdx.x;
     {
         const double2 a = t.wm2l[2 * npw + k1];
@@ -373,6 +397,7 @@ __global__ void __launch_bounds__(kBlock) k_m2l_brick(Geom g, DevTables t, int n
         s_fxy[5][tid] = t.wm2l[2 * npw + k3];
     }
     const ET* __restrict__ eb = expn + e;
+    const ET* __restrict__ eb2 = expn + e2;
     __shared__ long long s_soff[kM2lBrickMax + 2 * kM2lBatch];
     __shared__ int s_code[kM2lBrickMax];
     const int g0 = gent[brk], n = gent[brk + 1] - g0;   // a positive multiple of kM2lBatch
@@ -381,12 +406,16 @@ __global__ void __launch_bounds__(kBlock) k_m2l_brick(Geom g, DevTables t, int n
         if (i < n) s_code[i] = scode[g0 + i];
     }
     __syncthreads();
-    double2 acc[8];
+    double2 acc[8], acc2[8];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) acc[q] = make_double2(0.0, 0.0);
-    double2 va[kM2lBatch], vb[kM2lBatch], vc[kM2lBatch];
+    for (int q = 0; q < 8; ++q) acc[q] = acc2[q] = make_double2(0.0, 0.0);
+    ET va[2 * kM2lBatch], vb[2 * kM2lBatch];
 #define M2L_LOAD(v, j)                                                                   \
-    _Pragma("unroll") for (int u = 0; u < kM2lBatch; ++u) v[u] = ldE(eb[s_soff[(j) + u]]);
+    _Pragma("unroll") for (int u = 0; u < kM2lBatch; ++u) {                                \
+        const long long so = s_soff[(j) + u];                                                \
+        v[2 * u] = eb[so];                                                                   \
+        v[2 * u + 1] = eb2[so];                                                              \
+    }
 #define M2L_APPLY(v, j)                                                                  \
     _Pragma("unroll") for (int u = 0; u < kM2lBatch; ++u) {                              \
         const int code = __builtin_amdgcn_readfirstlane(s_code[(j) + u]);                \
@@ -402,22 +431,19 @@ __global__ void __launch_bounds__(kBlock) k_m2l_brick(Geom g, DevTables t, int n
                 double2 fxy = s_fxy[(kM2lRow >> (3 * oxy)) & 7][tid];                    \
                 fxy.y = __longlong_as_double(__double_as_longlong(fxy.y) ^               \
                                              ((long long)((kM2lConj >> oxy) & 1) << 63)); \
-                acc[q] = cfma(cmul(v[u], fxy), zf, acc[q]);                              \
+                acc[q] = cfma(cmul(ldE(v[2 * u]), fxy), zf, acc[q]);                     \
+                acc2[q] = cfma(cmul(ldE(v[2 * u + 1]), conjd(fxy)), zf, acc2[q]);        \
             }                                                                            \
         }                                                                                \
     }
     constexpr int B = kM2lBatch;
     M2L_LOAD(va, 0);
-    M2L_LOAD(vb, B);
-    for (int j = 0; j < n; j += 3 * B) {
-        M2L_LOAD(vc, j + 2 * B);
+    for (int j = 0; j < n; j += 2 * B) {
+        M2L_LOAD(vb, j + B);
         M2L_APPLY(va, j);
         if (j + B >= n) break;
-        M2L_LOAD(va, j + 3 * B);
+        M2L_LOAD(va, j + 2 * B);
         M2L_APPLY(vb, j + B);
-        if (j + 2 * B >= n) break;
-        M2L_LOAD(vb, j + 4 * B);
-        M2L_APPLY(vc, j + 2 * B);
     }
 #undef M2L_APPLY
 #undef M2L_LOAD
@@ -426,7 +452,10 @@ __global__ void __launch_bounds__(kBlock) k_m2l_brick(Geom g, DevTables t, int n
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
             const long long o = to[q];
-            if (o >= 0) stE(expn + o + tot + e, acc[q]);
+            if (o >= 0) {
+                stE(expn + o + tot + e, acc[q]);
+                stE(expn + o + tot + e2, acc2[q]);
+            }
         }
     }
 }
@@ -655,7 +684,7 @@ __global__ void __launch_bounds__(kBlock) k_split(Geom g, DevTables t, int nentr
     for (int k = 0; k < kSplitEPT; ++k) {
         const long long e = e0 + (long long)k * blockDim.x;
         const long long ec = e < tot ? e : tot - 1;   // valid duplicate, never stored
-        v[k] = ldE(src[ec]);
+        v[k] = ldE(gload(src, (unsigned)ec));
         const int r = (int)(ec % g.nexp);
         const int k2 = r % g.py, k1 = (r / g.py) % g.px, k3 = r / (g.py * g.px);
         // ms_phase per child from the two x-y products (a conjugate is exact)
@@ -673,7 +702,7 @@ __global__ void __launch_bounds__(kBlock) k_split(Geom g, DevTables t, int nentr
             const long long e = e0 + (long long)k * blockDim.x;
             const double2 xy = (sg & 1) ? ((sg & 2) ? conjd(pa[k]) : pb[k]) : ((sg & 2) ? conjd(pb[k]) : pa[k]);
             const double2 ph = cmul(xy, (sg & 4) ? conjd(wz[k]) : wz[k]);
-            if (e < tot) stE(dst + e, cmul(v[k], ph));
+            if (e < tot) gstore(dst, (unsigned)e, cmul(v[k], ph));
         }
     }
 }
@@ -892,13 +921,15 @@ void launch_m2l_brick(const Geom& g, const DevTables& t, int nbrick, long long z
                       const Multi& mu) {
     if (nbrick <= 0) return;
     if (g.ndim != 3) throw std::runtime_error("k_m2l_brick: 3-D only");
-    const long long nblk = (long long)blocks_for((long long)g.nd * g.nexp) * nbrick;
-    if (nblk > 0x7fffffffLL) throw std::runtime_error("k_m2l_brick: grid too large");
+    // (element pairs)
+    const long long pairs = (long long)g.nd * g.pz * ((g.px * g.py + 1) / 2);
+    const long long nblk = ((pairs + kBrickBlock - 1) / kBrickBlock) * nbrick;
+    if (pairs > 0x7fffff00LL || nblk > 0x7fffffffLL) throw std::runtime_error("k_m2l_brick: grid too large");
     if (t.expn_f32)
-        hipLaunchKernelGGL(k_m2l_brick<float2>, dim3((unsigned)nblk), dim3(kBlock), 0, s, g, t, nbrick, zero_off,
+        hipLaunchKernelGGL(k_m2l_brick<float2>, dim3((unsigned)nblk), dim3(kBrickBlock), 0, s, g, t, nbrick, zero_off,
                            toff, gent, soff, scode, reinterpret_cast<float2*>(expn), mu);
     else
-        hipLaunchKernelGGL(k_m2l_brick<double2>, dim3((unsigned)nblk), dim3(kBlock), 0, s, g, t, nbrick, zero_off,
+        hipLaunchKernelGGL(k_m2l_brick<double2>, dim3((unsigned)nblk), dim3(kBrickBlock), 0, s, g, t, nbrick, zero_off,
                            toff, gent, soff, scode, expn, mu);
     check(hipGetLastError(), "k_m2l_brick launch");
 }
