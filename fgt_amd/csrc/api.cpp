@@ -139,9 +139,7 @@ struct fgt_solver {
     // 3-D fast path: STEP 4 folded into STEP 5 for leaves below the cutoff level
     bool fast3d = false;
     bool lowp3d = false;   // the reduced-precision kernels cover the problem as well
-    DBuf d_s5_tasks;   // fgt::PotTask list of the reduced-precision STEP 5 kernel
-    int n_s5 = 0, n_s5_sib = 0;   // tasks, of which the first n_s5_sib are sibling tasks
-    DBuf d_s5_sym;     // fgt::SymTask list of the FP64 STEP 5 kernel
+    DBuf d_s5_sym;     // fgt::SymTask list of STEP 5
     int n_s5_fam = 0, n_s5_own = 0;   // families first, then single leaves
     DBuf d_p2pwS, d_fz_lev, d_fz_slot, d_fz_kids, d_fz_ksg;          // fused STEP 1+2 parents
     DBuf d_s1_box, d_s1_lev, d_s1_slot;                              // standalone STEP 1 leaves
@@ -159,7 +157,6 @@ struct fgt_solver {
     // host copies of the device work lists (the batch concatenates them
     // per shape class)
     struct HostLists {
-        std::vector<fgt::PotTask> s5;
         std::vector<fgt::SymTask> s1_sym, s5_sym;
         std::vector<int> pcs_parent, pcs_child, pcs_sign;
         std::vector<int> fz_lev, fz_slot, fz_kids, fz_ksg, s1_box, s1_lev, s1_slot;
@@ -584,15 +581,11 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
         S.d_pw2potS.upload(to_d2(ts));
         t.pw2potS_ks = sks;
         const fgt::TreeView& T = P.tree;
-        // STEP 5 tasks: leaves below the first PW level evaluate their
-        // parent's expansion through the split-phased tables; siblings with
-        // the same x split sign form one task (shared x contraction).  Those
-        // tasks come first (more work per task), then one task per leaf
-        // evaluating its own expansion.
-        // The FP64 kernel takes all the leaf children of a parent in one task.
-        std::vector<fgt::PotTask> fam, own;
+        // STEP 5 tasks: the leaf children of a box, at levels below the first
+        // PW level, evaluate its expansion through the split-phased tables, a
+        // family in one task.  Those come first (more work per task), then one
+        // task per leaf evaluating its own expansion.
         std::vector<fgt::SymTask> sfam, sown;
-        std::unordered_map<long long, int> fam_of;
         std::unordered_map<int, int> sfam_of;
         for (size_t i = 0; i < P.leaf_box.size(); ++i) {
             const int b = P.leaf_box[i], l = P.leaf_lev[i];
@@ -606,38 +599,7 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
                     sfam.push_back({P.slot_of_box[par], l, {-1, -1, -1, -1, -1, -1, -1, -1}});
                 }
                 sfam[is->second].box[sg[0] | sg[1] << 1 | sg[2] << 2] = b;
-                const long long key = 2LL * par + sg[0];
-                auto it = fam_of.find(key);
-                if (it == fam_of.end() || fam[it->second].box[3] >= 0) {
-                    fgt::PotTask pt{};
-                    pt.slot = P.slot_of_box[par];
-                    pt.lev = l;
-                    pt.vx = 1 + sg[0];
-                    pt.nvy = 0;
-                    for (int c = 0; c < 4; ++c) pt.box[c] = -1, pt.code[c] = 0;
-                    fam_of[key] = (int)fam.size();
-                    fam.push_back(pt);
-                    it = fam_of.find(key);
-                }
-                fgt::PotTask& pt = fam[it->second];
-                const int vy = 1 + sg[1];
-                int j = 0;
-                while (j < pt.nvy && pt.vy[j] != vy) ++j;
-                if (j == pt.nvy) pt.vy[pt.nvy++] = vy;
-                int c = 0;
-                while (pt.box[c] >= 0) ++c;
-                pt.box[c] = b;
-                pt.code[c] = j | ((1 + sg[2]) << 1);
             } else {
-                fgt::PotTask pt{};
-                pt.slot = P.leaf_slot[i];
-                pt.lev = l;
-                pt.vx = 0;
-                pt.nvy = 1;
-                pt.vy[0] = pt.vy[1] = 0;
-                for (int c = 0; c < 4; ++c) pt.box[c] = -1, pt.code[c] = 0;
-                pt.box[0] = b;
-                own.push_back(pt);
                 sown.push_back({P.leaf_slot[i], l, {b, -1, -1, -1, -1, -1, -1, -1}});
             }
         }
@@ -646,11 +608,6 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
         sfam.insert(sfam.end(), sown.begin(), sown.end());
         S.d_s5_sym.upload(sfam);
         S.h.s5_sym = sfam;
-        S.n_s5_sib = (int)fam.size();
-        fam.insert(fam.end(), own.begin(), own.end());
-        S.n_s5 = (int)fam.size();
-        if (S.lowp3d) S.d_s5_tasks.upload(fam);
-        S.h.s5 = fam;
         // split entries, keeping non-leaf children only
         std::vector<int> pp, pcc, psg;
         S.pcs_level_off.assign(nl + 2, 0);
@@ -1148,8 +1105,7 @@ void execute(fgt_solver& S, hipStream_t st, bool timed, bool fork_near = false,
             mark(7);   // STEP 5 starts here (after the wait for STEP 6)
         }
         if (S.fast3d)
-            launch_pw2pot_comps(g, t, {S.n_s5, S.n_s5_sib, S.d_s5_tasks.as<fgt::PotTask>(), nullptr, S.n_s5_fam,
-                                       S.n_s5_own, S.d_s5_sym.as<fgt::SymTask>(), nullptr}, ex, comps, st);
+            launch_pw2pot_comps(g, t, {S.n_s5_fam, S.n_s5_own, S.d_s5_sym.as<fgt::SymTask>(), nullptr}, ex, comps, st);
         else if (S.plane) {
             if (!fgt::launch_pw2pot_plane(g, t, P.nlevels - P.nlevstart, S.n_pl_leaf, S.d_pl_leaf.as<fgt::PlaneLeaf>(),
                                           ex, plane_comps(comps), st))
@@ -1336,10 +1292,9 @@ struct BClass {
     int n_m2l = 0;
     DBuf pcs_parent, pcs_child, pcs_sign, pcs_prob, pcs_klev;
     std::vector<int> pcs_phase;
-    DBuf s5, s5_prob;
-    int n_s5 = 0, n_s5_sib = 0;
     DBuf s5_sym, s5_symprob;
     int n_s5_fam = 0, n_s5_own = 0;
+    int n_s5 = 0;   // x contractions: the sides of the families, and the own leaves
     DBuf dir_tgt, dir_lev, dir_off, dir_src, dir_code, dir_flags, dir_prob;
     int n_dir = 0;
     double stage_ms[6] = {0, 0, 0, 0, 0, 0};   // STEPs 1-6 of the last profiled execute
@@ -1490,8 +1445,6 @@ void build_classes(fgt_batch& B) {
         std::vector<fgt::ProbPtrs> pp;
         std::vector<int> fzl, fzs, fzk, fzg, fzp, s1b, s1l, s1s, s1p;
         std::vector<int> mch, msg, pcsp, pcsc, pcsg;
-        std::vector<fgt::PotTask> sib, own;
-        std::vector<int> sibp, ownp;
         std::vector<fgt::SymTask> sfam, sown, s1fam, s1own;
         std::vector<int> sfamp, sownp;
         int maxph2 = 0, maxph4 = 0;
@@ -1526,10 +1479,6 @@ void build_classes(fgt_batch& B) {
             s1own.insert(s1own.end(), h.s1_sym.begin() + S.n_fz, h.s1_sym.end());
             maxph2 = std::max(maxph2, P.nlevels - P.nlevstart);
             maxph4 = std::max(maxph4, P.nlevels - P.nlevstart);
-            sib.insert(sib.end(), h.s5.begin(), h.s5.begin() + S.n_s5_sib);
-            sibp.insert(sibp.end(), S.n_s5_sib, q);
-            own.insert(own.end(), h.s5.begin() + S.n_s5_sib, h.s5.end());
-            ownp.insert(ownp.end(), h.s5.size() - S.n_s5_sib, q);
             sfam.insert(sfam.end(), h.s5_sym.begin(), h.s5_sym.begin() + S.n_s5_fam);
             sfamp.insert(sfamp.end(), S.n_s5_fam, q);
             sown.insert(sown.end(), h.s5_sym.begin() + S.n_s5_fam, h.s5_sym.end());
@@ -1615,13 +1564,11 @@ void build_classes(fgt_batch& B) {
         C.pcs_klev.upload(pk4);
         // STEP 3
         class_m2l(B, C);
-        // STEP 5: every sibling task first, then the one-leaf tasks
-        C.n_s5_sib = (int)sib.size();
-        sib.insert(sib.end(), own.begin(), own.end());
-        sibp.insert(sibp.end(), ownp.begin(), ownp.end());
-        C.n_s5 = (int)sib.size();
-        C.s5.upload(sib);
-        C.s5_prob.upload(sibp);
+        // STEP 5: every family first, then the one-leaf tasks
+        C.n_s5 = (int)sown.size();
+        for (const fgt::SymTask& f : sfam)
+            for (int a = 0; a < 2; ++a)
+                C.n_s5 += f.box[a] >= 0 || f.box[a | 2] >= 0 || f.box[a | 4] >= 0 || f.box[a | 6] >= 0;
         C.n_s5_fam = (int)sfam.size();
         C.n_s5_own = (int)sown.size();
         sfam.insert(sfam.end(), sown.begin(), sown.end());
@@ -1715,8 +1662,7 @@ void class_step5(const BClass& C, hipStream_t st) {
     zg.n = 1;
     zg.zo[0].nz = 1;
     zg.zo[0].od[0] = fgt::OutDesc{nullptr, C.nd, 0};
-    fgt::launch_pw2pot_tasks(C.g, C.t, {C.n_s5, C.n_s5_sib, C.s5.as<fgt::PotTask>(), C.s5_prob.as<int>(), C.n_s5_fam,
-                                        C.n_s5_own, C.s5_sym.as<fgt::SymTask>(), C.s5_symprob.as<int>()},
+    fgt::launch_pw2pot_tasks(C.g, C.t, {C.n_s5_fam, C.n_s5_own, C.s5_sym.as<fgt::SymTask>(), C.s5_symprob.as<int>()},
                              nullptr, zg, st, C.pp.as<fgt::ProbPtrs>());
 }
 void class_step6(const BClass& C, hipStream_t st) {

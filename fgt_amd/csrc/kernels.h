@@ -153,22 +153,7 @@ inline ZGroups z_kinds(const ZGroups& zg, int a, int nz) {
     return r;
 }
 
-// One task of the 3-D STEP 5 kernel: the local expansion in `slot`,
-// evaluated at up to four leaves of level `lev` that share the x table
-// variant vx (0 plain table; 1 / 2 table times the + / conjugate
-// parent->child split phase).  Leaf c: box[c] (-1 = unused), y variant
-// vy[code[c] & 1], z variant code[c] >> 1.  A leaf evaluating its own
-// expansion is a task with one leaf and all variants 0; the leaves of one
-// parent with the same x split sign form one task, so the x contraction of
-// the parent's expansion is done once for all of them.
-struct PotTask {
-    int slot, lev, vx, nvy;
-    int vy[2];
-    int box[4];
-    int code[4];
-};
-
-// One task of the symmetric 3-D STEP 1 / STEP 5 kernels: a leaf with an
+// One task of the 3-D STEP 1 (FP64) and STEP 5 kernels: a leaf with an
 // expansion of its own (box[0]), or a family, the leaf children of the box
 // whose expansion is in `slot`.  A family's child c has bit a (x, y, z) set
 // when it is the side whose table carries the conjugate parent-child phase
@@ -269,11 +254,9 @@ struct DevTables {
 bool launch_p2pw_3d(const Geom& g, const DevTables& t, int ntask, const int* box, const int* lev,
                     const int* slot, const double* fvals, double2* expn, hipStream_t s, size_t lds_limit,
                     const Multi& mu = Multi{});
-// STEP 5 in reduced precision over PotTask lists, tasks [0, nsib) sibling
-// tasks (up to four leaves), [nsib, ntask) one leaf: for the components of zo
-// (x and y kinds kd.x, kd.y) the one-leaf tasks share their x and y stages
-// across the z kinds
-bool launch_pw2pot_3d_z(const Geom& g, const DevTables& t, int ntask, int nsib, const PotTask* tasks,
+// STEP 5 with a reduced-precision x stage: tasks [0, nfam) families, then
+// nown single leaves; the components of zo (x and y kinds kd.x, kd.y)
+bool launch_pw2pot_3d_z(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks,
                         const double2* expn, Kinds kd, const ZOut& zo, hipStream_t s, size_t lds_limit,
                         const Multi& mu = Multi{});
 // STEP 5 in FP64 arithmetic (FP64 or FP32 expansions) through the tables'
@@ -384,12 +367,9 @@ void launch_pw2pot(const Geom& g, const DevTables& t, int ntask, const int* box,
 // 3-D STEP 5 for the components of zg, in the form pw2pot_lowp picks (throws
 // when the shape is not covered)
 struct Step5Lists {
-    int ntask, nsib;          // PotTask list (reduced precision)
-    const PotTask* tasks;
-    const int* tprob;         // its problem indices (batches)
     int nfam, nown;           // SymTask list
     const SymTask* sym;
-    const int* symprob;
+    const int* symprob;       // its problem indices (batches)
 };
 void launch_pw2pot_tasks(const Geom& g, const DevTables& t, const Step5Lists& l, const double2* expn,
                          const ZGroups& zg, hipStream_t s, const ProbPtrs* pp = nullptr);

@@ -406,6 +406,10 @@ __global__ void __launch_bounds__(kBrickBlock) k_m2l_brick(Geom g, DevTables t, 
         if (i < n) s_code[i] = scode[g0 + i];
     }
     __syncthreads();
+    // the opposite element's phase is the conjugate; the sign is opaque, so that
+    // both elements' products round alike (as the one-element form's did)
+    long long flip = 1LL << 63;
+    asm volatile("" : "+s"(flip));
     double2 acc[8], acc2[8];
 #pragma unroll
     for (int q = 0; q < 8; ++q) acc[q] = acc2[q] = make_double2(0.0, 0.0);
@@ -429,10 +433,12 @@ __global__ void __launch_bounds__(kBrickBlock) k_m2l_brick(Geom g, DevTables t, 
                 zf.y = __longlong_as_double(__double_as_longlong(zf.y) ^                 \
                                             ((long long)(oz == 0) << 63));               \
                 double2 fxy = s_fxy[(kM2lRow >> (3 * oxy)) & 7][tid];                    \
-                fxy.y = __longlong_as_double(__double_as_longlong(fxy.y) ^               \
-                                             ((long long)((kM2lConj >> oxy) & 1) << 63)); \
+                const long long cj = (long long)((kM2lConj >> oxy) & 1) << 63;           \
+                const long long fy = __double_as_longlong(fxy.y);                        \
+                fxy.y = __longlong_as_double(fy ^ cj);                                   \
                 acc[q] = cfma(cmul(ldE(v[2 * u]), fxy), zf, acc[q]);                     \
-                acc2[q] = cfma(cmul(ldE(v[2 * u + 1]), conjd(fxy)), zf, acc2[q]);        \
+                fxy.y = __longlong_as_double(fy ^ cj ^ flip);                            \
+                acc2[q] = cfma(cmul(ldE(v[2 * u + 1]), fxy), zf, acc2[q]);               \
             }                                                                            \
         }                                                                                \
     }
@@ -1017,15 +1023,15 @@ void launch_split(const Geom& g, const DevTables& t, int nentry, const int* pc_p
 void launch_pw2pot_tasks(const Geom& g, const DevTables& t, const Step5Lists& l, const double2* expn,
                          const ZGroups& zg, hipStream_t s, const ProbPtrs* pp) {
     const bool lowp = pw2pot_lowp(t);
-    if ((lowp ? l.ntask : l.nfam + l.nown) <= 0) return;
+    if (l.nfam + l.nown <= 0) return;
     Multi mu;
     mu.pp = pp;
-    mu.tprob = lowp ? l.tprob : l.symprob;
+    mu.tprob = l.symprob;
     bool ok = true;
     if (!lowp) ok = launch_pw2pot_sym(g, t, l.nfam, l.nown, l.sym, expn, zg, s, mu);
     else
         for (int q = 0; q < zg.n; ++q)
-            ok = ok && launch_pw2pot_3d_z(g, t, l.ntask, l.nsib, l.tasks, expn, zg.kd[q], zg.zo[q], s, t.lds_limit, mu);
+            ok = ok && launch_pw2pot_3d_z(g, t, l.nfam, l.nown, l.sym, expn, zg.kd[q], zg.zo[q], s, t.lds_limit, mu);
     if (!ok) throw std::runtime_error("3-D STEP 5 kernel not available for this shape");
     check(hipGetLastError(), "3-D STEP 5 launch");
 }

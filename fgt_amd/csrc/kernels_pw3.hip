@@ -26,19 +26,6 @@ __device__ __forceinline__ double2 zfma(double2 t, double2 f, double2 c) {
     return make_double2(c.x + t.x * f.x - t.y * f.y, c.y + t.x * f.y + t.y * f.x);
 }
 
-// Complex 16x16x4 tile product on the FP64 matrix cores: (re, im) += A B with
-// A, B complex, as four v_mfma_f64_16x16x4f64 (Ar Br - Ai Bi, Ar Bi + Ai Br).
-// Operand layout of that instruction: A lane l = A[l%16][l/16], B lane l =
-// B[l/16][l%16]; result lane l, element v = D[l/16 + 4v][l%16].
-typedef double dbl4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ void cmfma(double2 a, double2 b, dbl4& re, dbl4& im) {
-    re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.x, re, 0, 0, 0);
-    re = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, b.y, re, 0, 0, 0);
-    im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.y, im, 0, 0, 0);
-    im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.x, im, 0, 0, 0);
-}
-
 // Reduced-precision matrix-core contractions (mixed-precision forms).  A
 // complex product C[row][kk] = sum_k A[row][k] U[kk][k] becomes a real GEMM
 // with columns (kk, part) -- part 0 the real, 1 the imaginary part of C:
@@ -510,34 +497,43 @@ __global__ void __launch_bounds__(256) k_p2pwF3(Geom g, const double2* __restric
     }
 }
 
-// XS 4 (FP32, one column tile: norder 8): the x table operands of every K
-// step, converted once per task (the table depends only on the task's
-// level, x variant and kind) for all its rounds and row tiles (registers:
-// the largest plane-wave count's steps, uniform guards past npw; 147 VGPRs,
-// three waves per SIMD, against four for XS 2, which converts them per row
-// tile: STEP 5 of 21 norder-8, npw <= 32 problems 1.80 -> 1.47 ms)
-template <int N, int XS>
-struct XHoist {
-    static constexpr bool on = XS == 4 && (2 * N + 15) / 16 == 1;
-    static constexpr int KSH = on ? kLowpMaxPw / 4 : 1;
-    float b0[KSH], b1[KSH];
-    __device__ __forceinline__ void load(const CTab2 UX, int npw, int lane) {
-        if constexpr (on) {
-            const int li = lane & 15, lq = lane >> 4;
-            const bool cval = li < 2 * N;
-            const int cpart = li >= N ? 1 : 0;
-            const int ckk = cval ? li - N * cpart : 0;
-            const int ks = (npw + 3) >> 2;
+// The x table of a STEP 5 task as the operands of its matrix products, in LDS
+// once per task (read from memory and converted again for every row tile, the
+// wait for them had set the x stage's time): XS 2 (FP32) per K step, column
+// tile and lane the two parts' entries, XS 3 (BF16) the hi and lo halves of
+// the lane's eight K entries.  Zero past npw and past the last column.
+template <int XS> struct XEntry;
+template <> struct XEntry<2> { typedef float2 type; };
+struct BfPair { bf8 hi, lo; };
+template <> struct XEntry<3> { typedef BfPair type; };
+template <int N, int XS> struct XTable {
+    static constexpr int NT = (2 * N + 15) / 16;
+    typedef typename XEntry<XS>::type E;
+    static __host__ __device__ int steps(int npw) { return XS == 2 ? (npw + 3) >> 2 : (npw + 15) >> 4; }
+    static __host__ __device__ size_t bytes(int npw) { return sizeof(E) * steps(npw) * NT * 64; }
+    static __device__ __forceinline__ void fill(E* __restrict__ tab, const CTab2 UX, int npw, int tid) {
+        const int n = steps(npw) * NT * 64;
+        for (int o = tid; o < n; o += 256) {
+            const int lane = o & 63, t = (o >> 6) % NT, st = (o >> 6) / NT;
+            const int c = 16 * t + (lane & 15), lq = lane >> 4;
+            const bool cval = c < 2 * N;
+            const int part = c >= N ? 1 : 0, kk = cval ? c - N * part : 0;
+            if constexpr (XS == 2) {
+                const int k1 = 4 * st + lq;
+                const double2 u = UX[min(k1, npw - 1) * N + kk];
+                const bool ok = k1 < npw && cval;
+                tab[o] = make_float2(ok ? bcol(u, part, 0) : 0.f, ok ? bcol(u, part, 1) : 0.f);
+            } else {
+                float bx[8];
 #pragma unroll
-            for (int st = 0; st < KSH; ++st) {
-                if (st < ks) {
-                    const int k1 = 4 * st + lq;
-                    const bool kv = k1 < npw;
-                    const double2 u = UX[(kv ? k1 : npw - 1) * N + ckk];
-                    const bool ok = kv && cval;
-                    b0[st] = ok ? bcol(u, cpart, 0) : 0.f;
-                    b1[st] = ok ? bcol(u, cpart, 1) : 0.f;
+                for (int j = 0; j < 4; ++j) {
+                    const int k1 = 16 * st + 4 * lq + j;
+                    const double2 u = UX[min(k1, npw - 1) * N + kk];
+                    const bool ok = k1 < npw && cval;
+                    bx[2 * j] = ok ? bcol(u, part, 0) : 0.f;
+                    bx[2 * j + 1] = ok ? bcol(u, part, 1) : 0.f;
                 }
+                split_bf(bx, tab[o].hi, tab[o].lo);
             }
         }
     }
@@ -549,17 +545,16 @@ struct XHoist {
 // rows k2 (row tiles of 16, up to 80 frequencies), columns (kk1, part), K =
 // k1.  XS 2: FP32 operands; XS 3: BF16 hi/lo operands.  The result goes to
 // sff[(k2*SR + slab)*KW + (kk1 ^ (k2 & (KW-1)))], KW = 64 / SR (FP32
-// complex: the two accumulator chains' FP32 sum, stored exactly; for SR = 4
-// the layout of the FP64 x stages), where the y stage reads it.  Lanes past npw read a valid duplicate row (discarded); K
-// entries past npw get zero table values.
+// complex: the two accumulator chains' FP32 sum, stored exactly), where the y
+// stage reads it.  Lanes past npw read a valid duplicate row (discarded).
 template <int N, int XS, int SR>
-__device__ __forceinline__ void pw2pot_x_lowp(const float2* __restrict__ E, const CTab2 UX,
-                                              int npw, int nh, int r, int wave, int lane, float2* sff,
-                                              const XHoist<N, XS>& hx) {
+__device__ __forceinline__ void pw2pot_x_lowp(const float2* __restrict__ E,
+                                              const typename XTable<N, XS>::E* __restrict__ tab, int npw, int nh,
+                                              int r, int wave, int lane, float2* sff) {
     constexpr int KW = 64 / SR;
     static_assert(KW >= N, "a (k2, slab) row of sff holds the N values kk1");
     if (r + wave >= nh) return;
-    constexpr int NT = (2 * N + 15) / 16;
+    constexpr int NT = XTable<N, XS>::NT;
     const int MT = (npw + 15) >> 4;
     const int li = lane & 15, lq = lane >> 4;
     int ckk[NT], cpart[NT];
@@ -572,8 +567,7 @@ __device__ __forceinline__ void pw2pot_x_lowp(const float2* __restrict__ E, cons
         ckk[t] = cval[t] ? c - N * cpart[t] : 0;
     }
     float* __restrict__ sffd = reinterpret_cast<float*>(sff);
-    constexpr bool HOIST = XHoist<N, XS>::on;
-    constexpr int KSH = XHoist<N, XS>::KSH;
+    const int ks = XTable<N, XS>::steps(npw);
     for (int sl = wave; sl < SR; sl += 4) {
         const int k3 = r + sl;
         if (k3 >= nh) break;
@@ -585,110 +579,59 @@ __device__ __forceinline__ void pw2pot_x_lowp(const float2* __restrict__ E, cons
             flt4 acc[NT][2];
 #pragma unroll
             for (int t = 0; t < NT; ++t) acc[t][0] = acc[t][1] = flt4{0.f, 0.f, 0.f, 0.f};
-            if constexpr (HOIST) {
-                // E rows in chunks of four K steps, the next chunk loaded before
-                // the current one's products (chunks unrolled to the largest
-                // plane-wave count, uniform guards past npw)
-                const int ks = (npw + 3) >> 2;
-                constexpr int NCH = KSH / 4;
-                float2 e[2][4];
+            // K steps in chunks of KC, the next chunk's rows of E loaded (from
+            // valid clamped addresses, past npw against zero table entries)
+            // before this chunk's products
+            constexpr int KC = XS == 2 ? 8 : 2, KE = XS == 2 ? 1 : 4;
+            float2 ea[KC][KE], eb[KC][KE];
+            auto load = [&](float2 (&e)[KC][KE], int st0) {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) e[0][j] = Ek[(size_t)min(4 * j + lq, npw - 1) * npw + k2r];
+                for (int j = 0; j < KC; ++j)
 #pragma unroll
-                for (int c = 0; c < NCH; ++c) {
-                    if (4 * c < ks) {
-                        if (c + 1 < NCH && 4 * (c + 1) < ks) {
+                    for (int i = 0; i < KE; ++i)
+                        e[j][i] = gload(Ek, (unsigned)(min(4 * KE * (st0 + j) + KE * lq + i, npw - 1) * npw + k2r));
+            };
+            auto apply = [&](const float2 (&e)[KC][KE], int st0) {
 #pragma unroll
-                            for (int j = 0; j < 4; ++j)
-                                e[(c + 1) & 1][j] = Ek[(size_t)min(4 * (4 * (c + 1) + j) + lq, npw - 1) * npw + k2r];
-                        }
-                        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            if (4 * c + j < ks) {
-                                acc[0][0] = mfma32(e[c & 1][j].x, hx.b0[4 * c + j], acc[0][0]);
-                                acc[0][1] = mfma32(e[c & 1][j].y, hx.b1[4 * c + j], acc[0][1]);
-                            }
-                        }
-                    }
-                }
-            } else if constexpr (XS == 2) {
-                // FP32: K steps in chunks of KC, the next chunk's operand row and
-                // table entries loaded (from valid clamped addresses, zeroed past
-                // npw) before the current chunk's products, into two register sets
-                // (two steps per chunk where two column tiles hold the registers)
-                constexpr int KC = NT == 1 ? 4 : 2;
-                const int ks = (npw + 3) >> 2;
-                const int nchunk = (ks + KC - 1) / KC;
-                float2 ea[KC], eb[KC];
-                float ba[NT][KC][2], bb[NT][KC][2];
-                auto load = [&](float2 (&e)[KC], float (&bv)[NT][KC][2], int c) {
-#pragma unroll
-                    for (int j = 0; j < KC; ++j) {
-                        const int k1 = 4 * (KC * c + j) + lq;
-                        const bool kv = k1 < npw;
-                        const int k1c = kv ? k1 : npw - 1;
-                        e[j] = Ek[(size_t)k1c * npw + k2r];
+                for (int j = 0; j < KC; ++j) {
+                    if (st0 + j >= ks) break;
+                    const typename XTable<N, XS>::E* __restrict__ b = tab + (st0 + j) * NT * 64 + lane;
+                    if constexpr (XS == 2) {
 #pragma unroll
                         for (int t = 0; t < NT; ++t) {
-                            const double2 u = UX[k1c * N + ckk[t]];
-                            const bool ok = kv && cval[t];
-                            bv[t][j][0] = ok ? bcol(u, cpart[t], 0) : 0.f;
-                            bv[t][j][1] = ok ? bcol(u, cpart[t], 1) : 0.f;
+                            const float2 u = b[64 * t];
+                            acc[t][0] = mfma32(e[j][0].x, u.x, acc[t][0]);
+                            acc[t][1] = mfma32(e[j][0].y, u.y, acc[t][1]);
                         }
-                    }
-                };
-                auto apply = [&](const float2 (&e)[KC], const float (&bv)[NT][KC][2]) {
+                    } else {
+                        // K = (k1, part): 16 frequencies per step; lane K entries 8 lq .. 8 lq + 7
+                        float ax[8];
 #pragma unroll
-                    for (int j = 0; j < KC; ++j)
+                        for (int i = 0; i < 4; ++i) {
+                            ax[2 * i] = e[j][i].x;
+                            ax[2 * i + 1] = e[j][i].y;
+                        }
+                        bf8 ah, al;
+                        split_bf(ax, ah, al);
 #pragma unroll
                         for (int t = 0; t < NT; ++t) {
-                            acc[t][0] = mfma32(e[j].x, bv[t][j][0], acc[t][0]);
-                            acc[t][1] = mfma32(e[j].y, bv[t][j][1], acc[t][1]);
+                            const bf8 bh = b[64 * t].hi, bl = b[64 * t].lo;
+                            acc[t][0] = mfma_bf(ah, bh, acc[t][0]);
+                            acc[t][1] = mfma_bf(ah, bl, acc[t][1]);
+                            acc[t][1] = mfma_bf(al, bh, acc[t][1]);
                         }
-                };
-                load(ea, ba, 0);
-                for (int c = 0; c < nchunk; c += 2) {
-                    load(eb, bb, min(c + 1, nchunk - 1));
-                    __builtin_amdgcn_sched_barrier(0);
-                    apply(ea, ba);
-                    if (c + 1 >= nchunk) break;
-                    load(ea, ba, min(c + 2, nchunk - 1));
-                    __builtin_amdgcn_sched_barrier(0);
-                    apply(eb, bb);
-                }
-            } else {
-                // K = (k1, part): 16 frequencies per step; lane K entries 8 lq .. 8 lq + 7
-                const int ks = (npw + 15) >> 4;
-                for (int st = 0; st < ks; ++st) {
-                    float ax[8];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int k1c = min(16 * st + 4 * lq + j, npw - 1);
-                        const float2 e = Ek[(size_t)k1c * npw + k2r];
-                        ax[2 * j] = e.x;
-                        ax[2 * j + 1] = e.y;
-                    }
-                    bf8 ah, al;
-                    split_bf(ax, ah, al);
-#pragma unroll
-                    for (int t = 0; t < NT; ++t) {
-                        float bx[8];
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const int k1 = 16 * st + 4 * lq + j;
-                            const bool ok = k1 < npw && cval[t];
-                            const double2 u = UX[min(k1, npw - 1) * N + ckk[t]];
-                            bx[2 * j] = ok ? bcol(u, cpart[t], 0) : 0.f;
-                            bx[2 * j + 1] = ok ? bcol(u, cpart[t], 1) : 0.f;
-                        }
-                        bf8 bh, bl;
-                        split_bf(bx, bh, bl);
-                        acc[t][0] = mfma_bf(ah, bh, acc[t][0]);
-                        acc[t][1] = mfma_bf(ah, bl, acc[t][1]);
-                        acc[t][1] = mfma_bf(al, bh, acc[t][1]);
                     }
                 }
+            };
+            load(ea, 0);
+            for (int st = 0; st < ks; st += 2 * KC) {
+                if (st + KC < ks) load(eb, st + KC);
+                __builtin_amdgcn_sched_barrier(0);
+                apply(ea, st);
+                if (st + KC >= ks) break;
+                if (st + 2 * KC < ks) load(ea, st + 2 * KC);
+                __builtin_amdgcn_sched_barrier(0);
+                apply(eb, st + KC);
             }
 #pragma unroll
             for (int t = 0; t < NT; ++t)
@@ -706,214 +649,199 @@ __device__ __forceinline__ void pw2pot_x_lowp(const float2* __restrict__ E, cons
 
 // ---------------------------------------------------------------- STEP 5
 // The reduced-precision form (FP32 expansions, x stage on the matrix cores;
-// the FP64 form is k_pw2pot_sym).  Tables: tabS[kind][l][v][k][i] (frequency k, node i), v = 0 the plain
-// PW->value table, 1 / 2 the table times the + / conjugate parent->child
-// split phase.  A task (PotTask) evaluates one expansion at up to four
-// leaves: for a leaf evaluating its parent's expansion the phase is folded
-// into the tables (STEP 4 folded into STEP 5), and the x variant depends only
-// on the x split sign, so four siblings share one x contraction.
+// the FP64 form is k_pw2pot_sym).  Tables: tabS[kind][l][v][k][i] (frequency k,
+// node i), v = 0 the plain PW->value table, 1 / 2 the table times the + /
+// conjugate parent->child split phase (STEP 4 folded into STEP 5).
+// A block evaluates one expansion at the leaf children of its box that share
+// their x side (FAM; SymTask families, two blocks each, whose x contraction is
+// that of the side's table) or at the leaf that holds it.
 // Per round of SR k3 slabs (4; 8 for norder 8):
 //   x: ff[k2][s][kk1] = sum_k1 Ux[kk1][k1] E[k3][k1][k2]   (wave = slab,
-//      or slabs w and w + 4)
-//   y: yres[s][kk1][kk2] = sum_k2 Uy[kk2][k2] ff[k2][s][kk1], per y variant
-//   z: G_c[kk3] += Re(Uz_c[kk3][k3] yres[s][zk1][zk2]), per leaf c, with one
-//      thread per output column (zk1, zk2) holding all kk3 in registers.
+//      or slabs w and w + 4), FP32 products of FP32 or BF16 hi/lo operands;
+//   y, z: FP64, through the tables' symmetries as in k_pw2pot_sym (pairs of
+//      opposite frequencies and of mirror nodes, these of the two children
+//      along the axis where there are two): y lane = (kk1, slab), the pairs
+//      split over the waves; z thread = output column, all (or ZP) pairs of
+//      every z kind in registers.
+// Bound by the latencies of each round's three stages.  Order 12, npw 28, 3423
+// leaves: 253 us with the plain complex y and z stages, one leaf after another,
+// and the x table read per row tile; 188 with the symmetric stages, 119 with
+// the x table in LDS as well.  BF16 order 8, npw 20, 1332 leaves: 51, 39, 32.
 // LDS: sff [k2][s][KW] (npw*64 complex, KW = 64 / SR; the x stage's FP32
-// results, held exactly), yres [s][kk1][16]
-// (1024 complex, entry kk2 at kk2 ^ kk1), sUr [v][s][kk3] (3*SR*N complex:
-// the round's z table rows of the three variants, zero past nh).
-// C: most leaves per task (4 for sibling tasks, 1 for a leaf's own expansion).
-// NZ: output components sharing the x and y table kinds and differing in the
-// z kind zo.kz[q] (one-leaf tasks only: all their variants are 0, so sUr
-// holds the round's rows of NZ <= 3 z kinds in place of the three
-// variants).  The x and y stages run once for all of them, the z stage once
-// per kind, into zo.od[q].
-template <int N, int XS, int C, typename ET, int NZ = 1>
-__global__ void __launch_bounds__(256, 2) k_pw2pot3(Geom g, const double2* __restrict__ tabS_a, int npw,
-                                                const PotTask* __restrict__ tasks, const ET* __restrict__ expn_a,
-                                                size_t ks, Kinds kd, ZOut zo, Multi mu) {
-    static_assert(NZ >= 1 && NZ <= 3 && (NZ == 1 || C == 1), "z kinds are grouped for one-leaf tasks only");
+// results, held exactly), yres [s][kk1][y node] (rows padded by one), the x
+// table's operands (XTable).
+// NZ: output components that differ in their z kind zo.kz[q] only share the x
+// and y stages.
+template <int N> constexpr int mix_slabs() { return N == 8 ? 8 : 4; }
+template <int N, int XS, bool FAM, int NZ>
+__global__ void __launch_bounds__(256, 2) k_pw2pot3(Geom g, const double2* __restrict__ tabS, int npw,
+                                                    const SymTask* __restrict__ tasks,
+                                                    const float2* __restrict__ expn, size_t ks, Kinds kd, ZOut zo,
+                                                    Multi mu) {
+    constexpr int SR = mix_slabs<N>(), KW = 64 / SR;
+    constexpr int NP = FAM ? N : N / 2, NODY = 2 * NP, COLS = N * NODY;
+    constexpr int YP = (NP + 3) / 4;                                       // y pairs per wave
+    constexpr int ZS = COLS <= 64 ? 4 : (COLS <= 128 ? 2 : 1);             // thread groups sharing the z pairs
+    constexpr int ZP = (NP + ZS - 1) / ZS, CPT = (COLS + 255) / 256;       // pairs, columns per thread
+    constexpr int V = FAM ? 1 : 0;
     extern __shared__ double2 sm[];
-    static_assert(XS >= 2, "the FP64 form is k_pw2pot_sym");
     float2* sff = reinterpret_cast<float2*>(sm);
     double2* yres = reinterpret_cast<double2*>(sff + (size_t)npw * 64);
-    double2* sUr = yres + 4 * 16 * 16;
-    constexpr int NQ = N / 4;
-    // slabs per round: 8 for norder 8 (each wave
-    // computes two slabs, and the y stage's 64 lanes are (kk1, slab) with no
-    // idle half), else 4; KW: kk1 slots per (k2, slab) row of sff, per
-    // (slab, kk1) group of yres
-    constexpr int SR = N == 8 ? 8 : 4;
-    constexpr int KW = 64 / SR;
-    const int tix = xcd_task(blockIdx.x, gridDim.x);
-    const PotTask* __restrict__ T = tasks + tix;
-    const double2* __restrict__ tabS = tabS_a;
-    const ET* __restrict__ expn = expn_a;
+    auto* xtab = reinterpret_cast<typename XTable<N, XS>::E*>(yres + SR * N * (2 * N + 1));
+    const int lin = xcd_task(blockIdx.x, gridDim.x);
+    const int tix = FAM ? lin >> 1 : lin, sx = FAM ? lin & 1 : 0;
+    const SymTask* __restrict__ T = tasks + tix;
+    const ProbPtrs* prob = nullptr;
     if (mu.pp) {
-        const ProbPtrs& q = mu.pp[mu.tprob[tix]];
-        g = q.g;
-        npw = q.g.npw;
-        tabS = q.pw2potS;
-        expn = static_cast<const ET*>(q.expn);
-        zo.od[0].p = zo.od[1].p = zo.od[2].p = q.pot;
+        prob = mu.pp + mu.tprob[tix];
+        npw = prob->g.npw;
+        tabS = prob->pw2potS;
+        expn = static_cast<const float2*>(prob->expn);
     }
-    const int sl = T->slot, l = T->lev, nvy = T->nvy;
-    int cbox[C], ccode[C];
+    if (FAM && T->box[sx] < 0 && T->box[sx | 2] < 0 && T->box[sx | 4] < 0 && T->box[sx | 6] < 0) return;
+    const int nh = (npw + 1) >> 1, nd = g.nd;
+    const bool odd = (npw & 1) != 0;
+    const long long per = (long long)npw * N;
+    const long long row3 = 3LL * __builtin_amdgcn_readfirstlane(T->lev) * per;
+    const CTab2 UX = ctab(tabS) + ((long long)(kd.x * ks) + row3 + (FAM ? 1 + sx : 0) * per);
+    const CTab2 UY = ctab(tabS) + ((long long)(kd.y * ks) + row3 + V * per);
+    CTab2 UZ[NZ];
 #pragma unroll
-    for (int c = 0; c < C; ++c) {
-        cbox[c] = T->box[c];
-        ccode[c] = T->code[c];
-    }
-    // table kind per axis (value / first / second derivative) at stride ks;
-    // offsets are wave-uniform so the table reads stay on the scalar path
-    const int per = npw * N;
-    const int ox = __builtin_amdgcn_readfirstlane((int)(kd.x * ks) + (3 * l + T->vx) * per);
-    const int oz = __builtin_amdgcn_readfirstlane((int)(zo.kz[0] * ks) + 3 * l * per);
-    const CTab2 UX = ctab(tabS) + ox;
-    const CTab2 UZ = ctab(tabS) + oz;
+    for (int z = 0; z < NZ; ++z) UZ[z] = ctab(tabS) + ((long long)(zo.kz[z] * ks) + row3 + V * per);
+    const double sgy = kd.y == 1 ? -1.0 : 1.0;
+    const int slot = __builtin_amdgcn_readfirstlane(T->slot);
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
-    const int nh = g.pz, nd = g.nd;
     const int kk1 = lane & (KW - 1), s = lane / KW;
-    const bool halve = (npw & 1) != 0;
-    // z stage: one thread per output column (zk1, zk2), all kk3 in
-    // registers; where the block holds exactly one column per thread and leaf
-    // (N = 8, four leaves) each wave takes one leaf (ZW), where it holds one
-    // column per thread and z kind (N = 8, NZ kinds) wave q takes kind q
-    // (ZK), else every thread below N^2 takes all the leaves or kinds
-    constexpr bool ZW = C > 1 && N * N * C == 256;
-    constexpr bool ZK = NZ > 1 && N * N == 64;
-    constexpr int CG = (ZW || ZK) ? 1 : C * NZ;
-    const bool zact = ZW || (ZK ? wave < NZ : tid < N * N);
-    const int zt = (ZW || ZK) ? lane : tid;
-    const int zk1 = zt % N, zk2 = zt / N;
-    const int wbox = ZW ? T->box[wave] : -1, wcode = ZW ? T->code[wave] : 0;
-    // x-stage table operands of the task (XS 4 only)
-    XHoist<N, XS> hx;
-    hx.load(UX, npw, lane);
+    const bool yact = kk1 < N;
+    const int kk1c = yact ? kk1 : N - 1;
+    const int zset = ZS == 1 ? 0 : (ZS == 2 ? wave >> 1 : wave);
+    const int col0 = ZS == 1 ? tid : (ZS == 2 ? (tid & 127) : lane);
+    XTable<N, XS>::fill(xtab, UX, npw, tid);
+    __syncthreads();
     for (int ind = 0; ind < nd; ++ind) {
-        double G[CG][N];
+        double GP[CPT][NZ][ZP], GQ[CPT][NZ][ZP];
 #pragma unroll
-        for (int c = 0; c < CG; ++c)
+        for (int c = 0; c < CPT; ++c)
 #pragma unroll
-            for (int k = 0; k < N; ++k) G[c][k] = 0.0;
-        const ET* __restrict__ E = expn + ((size_t)sl * 2 * nd + nd + ind) * g.nexp;
+            for (int z = 0; z < NZ; ++z)
+#pragma unroll
+                for (int q = 0; q < ZP; ++q) GP[c][z][q] = GQ[c][z][q] = 0.0;
+        const float2* __restrict__ E = expn + (size_t)(slot * 2 * nd + nd + ind) * (size_t)(nh * npw * npw);
         for (int r = 0; r < nh; r += SR) {
-            __syncthreads();
-            // the round's z table rows, all three variants or (NZ > 1) the
-            // plain rows of each z kind (zero past nh)
-            if constexpr (NZ == 1) {
-                if (tid < 3 * SR * N) {
-                    const int v = tid / (SR * N), s2 = (tid / N) % SR, k = tid % N;
-                    sUr[tid] = (r + s2 < nh) ? UZ[v * per + (r + s2) * N + k] : make_double2(0.0, 0.0);
-                }
-            } else {
-                if (tid < SR * N * NZ) {
-                    const int z = tid / (SR * N), s2 = (tid / N) % SR, k = tid % N;
-                    const int kz = z == 0 ? zo.kz[0] : (z == 1 ? zo.kz[1] : zo.kz[2]);
-                    const CTab2 U = ctab(tabS) + ((long long)kz * ks + 3 * l * per);
-                    sUr[tid] = (r + s2 < nh) ? U[(r + s2) * N + k] : make_double2(0.0, 0.0);
-                }
-            }
-            pw2pot_x_lowp<N, XS, SR>(E, UX, npw, nh, r, wave, lane, sff, hx);
-            __syncthreads();
-            for (int j = 0; j < nvy; ++j) {
-                if (j) __syncthreads();   // the z stage of the previous y variant is done with yres
-                // y: lane = (kk1, s), wave owns kk2 in [wave*NQ, wave*NQ+NQ)
-                const int oy = __builtin_amdgcn_readfirstlane((int)(kd.y * ks) + (3 * l + T->vy[j]) * per);
-                const CTab2 UY = ctab(tabS) + oy;
-                const int k3 = r + s;
-                if (kk1 < N && k3 < nh) {
-                    double2 y[NQ];
+            pw2pot_x_lowp<N, XS, SR>(E, xtab, npw, nh, r, wave, lane, sff);
+            __syncthreads();   // (and the last round's z stage is done with yres)
+            {
+                double2 P[YP], Q[YP];
 #pragma unroll
-                    for (int q = 0; q < NQ; ++q) y[q] = make_double2(0.0, 0.0);
-                    for (int k2 = 0; k2 < npw; ++k2) {
-                        const float2 fs = sff[(k2 * SR + s) * KW + (kk1 ^ (k2 & (KW - 1)))];
-                        const double2 f = make_double2(fs.x, fs.y);
+                for (int p = 0; p < YP; ++p) P[p] = Q[p] = make_double2(0.0, 0.0);
+                // several steps' table and LDS reads together (a slab past nh
+                // holds stale values, never read back)
+                constexpr int YU = YP <= 2 ? 4 : 2;
+                for (int k0 = 0; k0 < nh; k0 += YU) {
+                    float2 a[YU], b[YU];
+                    double2 t[YU][YP];
 #pragma unroll
-                        for (int q = 0; q < NQ; ++q) y[q] = zfma(UY[k2 * N + wave * NQ + q], f, y[q]);
+                    for (int j = 0; j < YU; ++j) {
+                        const int k = min(k0 + j, nh - 1), m = npw - 1 - k;
+                        a[j] = sff[(k * SR + s) * KW + (kk1c ^ (k & (KW - 1)))];
+                        b[j] = sff[(m * SR + s) * KW + (kk1c ^ (m & (KW - 1)))];
+#pragma unroll
+                        for (int p = 0; p < YP; ++p) t[j][p] = UY[(long long)k * N + min(wave * YP + p, NP - 1)];
                     }
 #pragma unroll
-                    for (int q = 0; q < NQ; ++q) yres[(s * KW + kk1) * 16 + ((wave * NQ + q) ^ kk1)] = y[q];
+                    for (int j = 0; j < YU; ++j) {
+                        if (k0 + j >= nh) break;
+                        const double ax = a[j].x, ay = a[j].y, bx = b[j].x, by = b[j].y;
+                        const bool self = odd && k0 + j == nh - 1;   // the zero frequency pairs with itself
+                        const double Sx = self ? ax : ax + bx, Sy = self ? ay : ay + by, Dx = ax - bx, Dy = ay - by;
+#pragma unroll
+                        for (int p = 0; p < YP; ++p) {
+                            P[p].x += t[j][p].x * Sx;
+                            P[p].y += t[j][p].x * Sy;
+                            Q[p].x += t[j][p].y * Dx;
+                            Q[p].y += t[j][p].y * Dy;
+                        }
+                    }
                 }
-                __syncthreads();
-                // z, for the leaves that use this y variant
-                if (zact) {
-#pragma unroll 1
-                    for (int s2 = 0; s2 < SR; ++s2) {
-                        const int k3z = r + s2;
-                        if (k3z >= nh) break;
-                        const double2 yv = yres[(s2 * KW + zk1) * 16 + (zk2 ^ zk1)];
-                        const double w = (halve && k3z == nh - 1) ? 0.5 : 1.0;
-                        const double yr = yv.x * w, yi = yv.y * w;
-                        if constexpr (ZW) {
-                            if (wbox >= 0 && (wcode & 1) == j) {
-                                const double2* __restrict__ uz = sUr + ((wcode >> 1) * SR + s2) * N;
+                if (yact && r + s < nh) {
+                    double2* __restrict__ o = yres + (s * N + kk1) * (NODY + 1);
 #pragma unroll
-                                for (int kk3 = 0; kk3 < N; ++kk3) {
-                                    const double2 u = uz[kk3];
-                                    G[0][kk3] += u.x * yr - u.y * yi;
+                    for (int p = 0; p < YP; ++p) {
+                        const int q = wave * YP + p;
+                        if (q < NP) {
+                            o[q] = make_double2(P[p].x - Q[p].y, P[p].y + Q[p].x);
+                            o[NP + q] = make_double2(sgy * (P[p].x + Q[p].y), sgy * (P[p].y - Q[p].x));
+                        }
+                    }
+                }
+            }
+            __syncthreads();
+            const int ns = min(SR, nh - r);
+#pragma unroll
+            for (int c = 0; c < CPT; ++c) {
+                const int col = col0 + 256 * c;
+                if (col < COLS) {
+                    const double2* __restrict__ yc = yres + (col % N) * (NODY + 1) + col / N;
+                    constexpr int ZU = NZ * ZP <= 4 ? 4 : (NZ * ZP <= 8 ? 2 : 1);
+                    for (int s0 = 0; s0 < ns; s0 += ZU) {
+                        double2 yv[ZU], t[ZU][NZ][ZP];
+#pragma unroll
+                        for (int j = 0; j < ZU; ++j) {
+                            const int s2 = min(s0 + j, ns - 1);
+                            yv[j] = yc[s2 * N * (NODY + 1)];
+#pragma unroll
+                            for (int z = 0; z < NZ; ++z)
+#pragma unroll
+                                for (int q = 0; q < ZP; ++q)
+                                    t[j][z][q] = UZ[z][(long long)(r + s2) * N + min(zset * ZP + q, NP - 1)];
+                        }
+#pragma unroll
+                        for (int j = 0; j < ZU; ++j) {
+                            if (s0 + j >= ns) break;
+                            const double w = (odd && r + s0 + j == nh - 1) ? 0.5 : 1.0;
+                            const double yr = yv[j].x * w, yi = yv[j].y * w;
+#pragma unroll
+                            for (int z = 0; z < NZ; ++z)
+#pragma unroll
+                                for (int q = 0; q < ZP; ++q) {
+                                    GP[c][z][q] += t[j][z][q].x * yr;
+                                    GQ[c][z][q] += t[j][z][q].y * yi;
                                 }
-                            }
-                        } else if constexpr (ZK) {
-                            if (cbox[0] >= 0) {
-                                const double2* __restrict__ uz = sUr + (wave * SR + s2) * N;
-#pragma unroll
-                                for (int kk3 = 0; kk3 < N; ++kk3) {
-                                    const double2 u = uz[kk3];
-                                    G[0][kk3] += u.x * yr - u.y * yi;
-                                }
-                            }
-                        } else if constexpr (NZ > 1) {
-                            if (cbox[0] >= 0) {
-#pragma unroll
-                                for (int z = 0; z < NZ; ++z) {
-                                    const double2* __restrict__ uz = sUr + (z * SR + s2) * N;
-#pragma unroll
-                                    for (int kk3 = 0; kk3 < N; ++kk3) {
-                                        const double2 u = uz[kk3];
-                                        G[z][kk3] += u.x * yr - u.y * yi;
-                                    }
-                                }
-                            }
-                        } else {
-#pragma unroll
-                            for (int c = 0; c < C; ++c) {
-                                if (cbox[c] >= 0 && (ccode[c] & 1) == j) {
-                                    const double2* __restrict__ uz = sUr + ((ccode[c] >> 1) * SR + s2) * N;
-#pragma unroll
-                                    for (int kk3 = 0; kk3 < N; ++kk3) {
-                                        const double2 u = uz[kk3];
-                                        G[c][kk3] += u.x * yr - u.y * yi;
-                                    }
-                                }
-                            }
                         }
                     }
                 }
             }
         }
-        if (zact) {
-            // the empty asm makes col opaque here, so the 64 output addresses
-            // are formed now and not hoisted out of the loops (where they
-            // would be held, or spilled, through the whole task)
-            int col = zk1 + N * zk2;
-            asm volatile("" : "+v"(col));
+        // node pair -> (child bit, node): side b is the mirrored node, of the
+        // other child (FAM) or of the same leaf
 #pragma unroll
-            for (int c = 0; c < CG; ++c) {
-                const int b = ZW ? wbox : cbox[C > 1 ? c : 0];
-                // output of kind c (NZ > 1), of this wave's kind (ZK), else
-                // the one output (selected field by field: a whole-struct
-                // select by a run-time index would put zo in scratch memory)
-                const int q = ZK ? wave : (NZ > 1 ? c : 0);
-                double* const op = q == 0 ? zo.od[0].p : (q == 1 ? zo.od[1].p : zo.od[2].p);
-                const int ons = q == 0 ? zo.od[0].ns : (q == 1 ? zo.od[1].ns : zo.od[2].ns);
-                const int ocoff = q == 0 ? zo.od[0].coff : (q == 1 ? zo.od[1].coff : zo.od[2].coff);
-                if (b >= 0) {
-                    double* __restrict__ o = op + (size_t)b * g.npbox * ons + ocoff + ind;
+        for (int c = 0; c < CPT; ++c) {
+            const int col = col0 + 256 * c;
+            if (col >= COLS) continue;
+            const int ix = col % N, zy = col / N, by = zy >= NP, py = zy - by * NP, iy = by ? N - 1 - py : py;
+            const int cxy = FAM ? sx | by << 1 : 0;
+            const int ba = T->box[cxy], bb = T->box[FAM ? cxy | 4 : 0];
+            int node = ix + N * iy;
+            // opaque: the output addresses are formed here, not held through
+            // the whole task
+            asm volatile("" : "+v"(node));
 #pragma unroll
-                    for (int kk3 = 0; kk3 < N; ++kk3) o[(size_t)(col + N * N * kk3) * ons] += 2.0 * G[c][kk3];
+            for (int z = 0; z < NZ; ++z) {
+                double* const op = (prob ? prob->pot : zo.od[z].p) + zo.od[z].coff + ind;
+                const int ns = zo.od[z].ns;
+                const double sgz = zo.kz[z] == 1 ? -2.0 : 2.0;
+#pragma unroll
+                for (int q = 0; q < ZP; ++q) {
+                    const int pz = zset * ZP + q;
+                    if (pz >= NP) break;
+                    if (ba >= 0)
+                        gadd(op + (size_t)ba * (N * N * N) * ns, (node + N * N * pz) * ns,
+                             2.0 * (GP[c][z][q] - GQ[c][z][q]));
+                    if (bb >= 0)
+                        gadd(op + (size_t)bb * (N * N * N) * ns, (node + N * N * (N - 1 - pz)) * ns,
+                             sgz * (GP[c][z][q] + GQ[c][z][q]));
                 }
             }
         }
@@ -935,16 +863,18 @@ bool try_p2pw3(const Geom& g, const DevTables& t, int ntask, const int* box, con
     return true;
 }
 
-size_t pw2pot3_lds(int n, int npw) {
-    // sff, yres, sUr (three variants of up to eight slabs at norder 8, four above)
-    return sizeof(float2) * (size_t)npw * 64 + sizeof(double2) * (4 * 16 * 16 + (n == 8 ? 24 : 12) * (size_t)n);
+size_t pw2pot3_lds(int n, int npw, int xs) {
+    // sff, yres (a family's, the larger), x table
+    const size_t sr = n == 8 ? 8 : 4;
+    const size_t tab = n == 8 ? (xs == 2 ? XTable<8, 2>::bytes(npw) : XTable<8, 3>::bytes(npw))
+                              : (xs == 2 ? XTable<16, 2>::bytes(npw) : XTable<16, 3>::bytes(npw));
+    return sizeof(float2) * (size_t)npw * 64 + sizeof(double2) * sr * n * (2 * (size_t)n + 1) + tab;
 }
 
-template <int N, int XS, int C, int NZ = 1>
-void launch_pw2pot3_c(const Geom& g, const DevTables& t, int ntask, const PotTask* tasks, const double2* expn,
+template <int N, int XS, bool FAM, int NZ>
+void launch_pw2pot3_z(const Geom& g, const DevTables& t, int nblk, const SymTask* tasks, const double2* expn,
                       Kinds kd, const ZOut& zo, hipStream_t s, size_t lds, const Multi& mu) {
-    if (ntask <= 0) return;
-    hipLaunchKernelGGL((k_pw2pot3<N, XS, C, float2, NZ>), dim3(ntask), dim3(256), lds, s, g, t.pw2potS, t.npw, tasks,
+    hipLaunchKernelGGL((k_pw2pot3<N, XS, FAM, NZ>), dim3(nblk), dim3(256), lds, s, g, t.pw2potS, t.npw, tasks,
                        reinterpret_cast<const float2*>(expn), t.pw2potS_ks, kd, zo, mu);
 }
 
@@ -959,34 +889,42 @@ ZOut zsub(const ZOut& zo, int a, int nz) {
     return r;
 }
 
-// tasks [0, nsib) hold up to four leaves and run once per z kind; [nsib,
-// ntask) hold one leaf each and run once for all the kinds
-template <int N, int XS>
-void launch_pw2pot3_typed(const Geom& g, const DevTables& t, int ntask, int nsib, const PotTask* tasks,
-                          const double2* expn, Kinds kd, const ZOut& zo, hipStream_t s, size_t lds,
-                          const Multi& mu) {
-    for (int q = 0; q < zo.nz; ++q) launch_pw2pot3_c<N, XS, 4>(g, t, nsib, tasks, expn, kd, zsub(zo, q, 1), s, lds, mu);
-    Multi m1 = mu;
-    if (m1.tprob) m1.tprob += nsib;
-    const int n1 = ntask - nsib;
-    const PotTask* t1 = tasks + nsib;
-    if (zo.nz == 3) {
-        launch_pw2pot3_c<N, XS, 1, 3>(g, t, n1, t1, expn, kd, zo, s, lds, m1);
-    } else if (zo.nz == 2) {
-        launch_pw2pot3_c<N, XS, 1, 2>(g, t, n1, t1, expn, kd, zo, s, lds, m1);
+// nblk blocks of one kind of task: the z kinds together, or (a family's z
+// sums of several kinds exceed the registers above norder 8) one after another
+template <int N, int XS, bool FAM>
+void launch_pw2pot3_kind(const Geom& g, const DevTables& t, int nblk, const SymTask* tasks, const double2* expn,
+                         Kinds kd, const ZOut& zo, hipStream_t s, size_t lds, const Multi& mu) {
+    if (nblk <= 0) return;
+    if constexpr (!FAM || N == 8) {
+        switch (zo.nz) {
+            case 3: launch_pw2pot3_z<N, XS, FAM, 3>(g, t, nblk, tasks, expn, kd, zo, s, lds, mu); return;
+            case 2: launch_pw2pot3_z<N, XS, FAM, 2>(g, t, nblk, tasks, expn, kd, zo, s, lds, mu); return;
+            default: launch_pw2pot3_z<N, XS, FAM, 1>(g, t, nblk, tasks, expn, kd, zo, s, lds, mu); return;
+        }
     } else {
-        launch_pw2pot3_c<N, XS, 1, 1>(g, t, n1, t1, expn, kd, zo, s, lds, m1);
+        for (int q = 0; q < zo.nz; ++q)
+            launch_pw2pot3_z<N, XS, FAM, 1>(g, t, nblk, tasks, expn, kd, zsub(zo, q, 1), s, lds, mu);
     }
 }
 
+template <int N, int XS>
+void launch_pw2pot3_typed(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks,
+                          const double2* expn, Kinds kd, const ZOut& zo, hipStream_t s, size_t lds,
+                          const Multi& mu) {
+    launch_pw2pot3_kind<N, XS, true>(g, t, 2 * nfam, tasks, expn, kd, zo, s, lds, mu);
+    Multi m1 = mu;
+    if (m1.tprob) m1.tprob += nfam;
+    launch_pw2pot3_kind<N, XS, false>(g, t, nown, tasks + nfam, expn, kd, zo, s, lds, m1);
+}
+
 template <int N>
-bool try_pw2pot3(const Geom& g, const DevTables& t, int ntask, int nsib, const PotTask* tasks,
+bool try_pw2pot3(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks,
                  const double2* expn, Kinds kd, const ZOut& zo, hipStream_t s, size_t lds_limit, const Multi& mu) {
-    const size_t lds = pw2pot3_lds(N, t.npw);
-    if (lds > lds_limit || 3 * t.pw2potS_ks > 0x7fffffffULL) return false;
-    // BF16 hi/lo, or FP32 (its table operands hoisted at norder 8)
-    if (t.prec == 2) launch_pw2pot3_typed<N, 3>(g, t, ntask, nsib, tasks, expn, kd, zo, s, lds, mu);
-    else launch_pw2pot3_typed<N, (N == 8 ? 4 : 2)>(g, t, ntask, nsib, tasks, expn, kd, zo, s, lds, mu);
+    const size_t lds = pw2pot3_lds(N, t.npw, t.prec == 2 ? 3 : 2);
+    if (lds > lds_limit || nfam > 0x3fffffff) return false;
+    // BF16 hi/lo, or FP32
+    if (t.prec == 2) launch_pw2pot3_typed<N, 3>(g, t, nfam, nown, tasks, expn, kd, zo, s, lds, mu);
+    else launch_pw2pot3_typed<N, 2>(g, t, nfam, nown, tasks, expn, kd, zo, s, lds, mu);
     return true;
 }
 
@@ -1079,20 +1017,20 @@ bool p2pw_fused_3d(const Geom& g, const DevTables& t, int ntask, const int* plev
 
 bool pw2pot_3d_supported(const Geom& g, const DevTables& t) {
     if (g.ndim != 3 || (t.n != 8 && t.n != 12 && t.n != 16)) return false;
-    const size_t lds = sizeof(double2) * ((size_t)t.npw * 64 + 4 * 16 * 16 + (t.n == 8 ? 24 : 12) * (size_t)t.n);
+    const size_t lds = std::max(pw2pot3_lds(t.n, t.npw, 2), pw2pot3_lds(t.n, t.npw, 3));
     const size_t lds1 = sizeof(double2) * std::max(4 * (size_t)t.n * t.n, 4 * (size_t)t.n * t.npw);
     const size_t lds2 = sizeof(double2) * std::max(8 * (size_t)t.n * t.n, 4 * (size_t)t.n * t.npw);
     return lds <= t.lds_limit && lds1 <= t.lds_limit && lds2 <= t.lds_limit;
 }
 
-bool launch_pw2pot_3d_z(const Geom& g, const DevTables& t, int ntask, int nsib, const PotTask* tasks,
+bool launch_pw2pot_3d_z(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks,
                         const double2* expn, Kinds kd, const ZOut& zo, hipStream_t s, size_t lds_limit,
                         const Multi& mu) {
-    if (g.ndim != 3 || ntask <= 0 || zo.nz < 1 || zo.nz > 3) return false;
+    if (g.ndim != 3 || nfam + nown <= 0 || zo.nz < 1 || zo.nz > 3) return false;
     switch (t.n) {
-        case 8: return try_pw2pot3<8>(g, t, ntask, nsib, tasks, expn, kd, zo, s, lds_limit, mu);
-        case 12: return try_pw2pot3<12>(g, t, ntask, nsib, tasks, expn, kd, zo, s, lds_limit, mu);
-        case 16: return try_pw2pot3<16>(g, t, ntask, nsib, tasks, expn, kd, zo, s, lds_limit, mu);
+        case 8: return try_pw2pot3<8>(g, t, nfam, nown, tasks, expn, kd, zo, s, lds_limit, mu);
+        case 12: return try_pw2pot3<12>(g, t, nfam, nown, tasks, expn, kd, zo, s, lds_limit, mu);
+        case 16: return try_pw2pot3<16>(g, t, nfam, nown, tasks, expn, kd, zo, s, lds_limit, mu);
         default: return false;
     }
 }
