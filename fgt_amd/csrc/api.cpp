@@ -493,6 +493,90 @@ int mode_precision(int mode, double eps, bool ok) {
     return eps >= kEpsBf16 ? 2 : (eps >= kEpsFp32 ? 1 : 0);
 }
 
+// STEP 4 and STEP 5 lists of the 3-D fast path.  The leaf children of a box, at
+// levels below the first PW level, evaluate its expansion through the
+// split-phased tables, a family in one task.  Those come first (more work per
+// task), then one task per leaf evaluating its own expansion.  Splits go into
+// non-leaf children only, and with FP64 expansions only into those that have
+// non-leaf children themselves: the families of the others take the expansion
+// from one level up and split it as they read it, so most of the split
+// expansions (7 of 8 on a uniform tree) are never written or read: order 12,
+// npw 60, 4250 leaves STEP 4 217 -> 43 us and STEP 5, which reads an eighth of
+// the bytes for a few per cent more products, 393 -> 360; order 8, 8382 leaves
+// 44 -> 13 and 88 -> 77.  FP32 expansions round at every level and keep every
+// split.
+void step45_lists(fgt_solver& S) {
+    const fgt::Plan& P = S.plan;
+    const fgt::TreeView& T = P.tree;
+    const int nl = P.nlevels;
+    const bool fold = S.tabs.expn_f32 == 0;
+    auto sides = [&](int c, int b) {   // bit a: c lies below b's centre along axis a
+        int k = 0;
+        for (int a = 0; a < 3; ++a)
+            if (T.centers[3 * c + a] - T.centers[3 * b + a] < 0) k |= 1 << a;
+        return k;
+    };
+    // boxes whose own local expansion is formed: the first PW level's, and
+    // below it those that are split into
+    std::vector<char> formed(P.nboxes, 0);
+    std::vector<int> pp, pcc, psg;
+    S.pcs_level_off.assign(nl + 2, 0);
+    for (int l = 0; l <= nl; ++l) {
+        S.pcs_level_off[l] = (int)pp.size();
+        if (l < P.nlevstart || l >= nl) continue;
+        for (int b = T.lfirst[l]; b <= T.llast[l]; ++b) {
+            if (T.nchild[b] == 0) continue;
+            if (l == P.nlevstart) formed[b] = 1;
+            for (int i = 0; i < T.nchild[b]; ++i) {
+                const int c = T.child[static_cast<size_t>(T.mc) * b + i];
+                if (T.nchild[c] == 0) continue;
+                bool deep = !fold;
+                for (int m = 0; m < T.nchild[c] && !deep; ++m)
+                    deep = T.nchild[T.child[static_cast<size_t>(T.mc) * c + m]] > 0;
+                if (!deep) continue;
+                formed[c] = 1;
+                pp.push_back(P.slot_of_box[b]);
+                pcc.push_back(P.slot_of_box[c]);
+                psg.push_back(sides(c, b));
+            }
+        }
+    }
+    S.pcs_level_off[nl + 1] = (int)pp.size();
+    std::vector<fgt::SymTask> sfam, sown;
+    std::unordered_map<int, int> sfam_of;
+    for (size_t i = 0; i < P.leaf_box.size(); ++i) {
+        const int b = P.leaf_box[i], l = P.leaf_lev[i];
+        if (l > P.nlevstart) {
+            const int par = T.parent[b];
+            auto is = sfam_of.find(par);
+            if (is == sfam_of.end()) {
+                is = sfam_of.emplace(par, (int)sfam.size()).first;
+                fgt::SymTask f{P.slot_of_box[par], l, {-1, -1, -1, -1, -1, -1, -1, -1}};
+                if (!formed[par]) {
+                    f.slot = P.slot_of_box[T.parent[par]];
+                    f.klev = nl - (l - 2);   // the phase row of the splits out of level l - 2
+                    f.sign = sides(par, T.parent[par]);
+                }
+                sfam.push_back(f);
+            }
+            sfam[is->second].box[sides(b, par)] = b;
+        } else {
+            sown.push_back({P.leaf_slot[i], l, {b, -1, -1, -1, -1, -1, -1, -1}});
+        }
+    }
+    S.n_s5_fam = (int)sfam.size();
+    S.n_s5_own = (int)sown.size();
+    sfam.insert(sfam.end(), sown.begin(), sown.end());
+    S.d_s5_sym.upload(sfam);
+    S.h.s5_sym = sfam;
+    S.d_pcs_parent.upload(pp);
+    S.h.pcs_parent = pp;
+    S.d_pcs_child.upload(pcc);
+    S.h.pcs_child = pcc;
+    S.d_pcs_sign.upload(psg);
+    S.h.pcs_sign = psg;
+}
+
 void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, fgt::Plan* planned = nullptr,
                   int prec_mode = 0) {
     if (planned) {
@@ -581,60 +665,7 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
         S.d_pw2potS.upload(to_d2(ts));
         t.pw2potS_ks = sks;
         const fgt::TreeView& T = P.tree;
-        // STEP 5 tasks: the leaf children of a box, at levels below the first
-        // PW level, evaluate its expansion through the split-phased tables, a
-        // family in one task.  Those come first (more work per task), then one
-        // task per leaf evaluating its own expansion.
-        std::vector<fgt::SymTask> sfam, sown;
-        std::unordered_map<int, int> sfam_of;
-        for (size_t i = 0; i < P.leaf_box.size(); ++i) {
-            const int b = P.leaf_box[i], l = P.leaf_lev[i];
-            if (l > P.nlevstart) {
-                const int par = T.parent[b];
-                int sg[3];
-                for (int a = 0; a < 3; ++a) sg[a] = T.centers[3 * b + a] - T.centers[3 * par + a] < 0 ? 1 : 0;
-                auto is = sfam_of.find(par);
-                if (is == sfam_of.end()) {
-                    is = sfam_of.emplace(par, (int)sfam.size()).first;
-                    sfam.push_back({P.slot_of_box[par], l, {-1, -1, -1, -1, -1, -1, -1, -1}});
-                }
-                sfam[is->second].box[sg[0] | sg[1] << 1 | sg[2] << 2] = b;
-            } else {
-                sown.push_back({P.leaf_slot[i], l, {b, -1, -1, -1, -1, -1, -1, -1}});
-            }
-        }
-        S.n_s5_fam = (int)sfam.size();
-        S.n_s5_own = (int)sown.size();
-        sfam.insert(sfam.end(), sown.begin(), sown.end());
-        S.d_s5_sym.upload(sfam);
-        S.h.s5_sym = sfam;
-        // split entries, keeping non-leaf children only
-        std::vector<int> pp, pcc, psg;
-        S.pcs_level_off.assign(nl + 2, 0);
-        for (int l = 0; l <= nl; ++l) {
-            S.pcs_level_off[l] = (int)pp.size();
-            if (l < P.nlevstart || l >= nl) continue;
-            for (int b = T.lfirst[l]; b <= T.llast[l]; ++b) {
-                if (T.nchild[b] == 0) continue;
-                for (int i = 0; i < T.nchild[b]; ++i) {
-                    const int c = T.child[(size_t)T.mc * b + i];
-                    if (T.nchild[c] == 0) continue;
-                    int k = 0;
-                    for (int a = 0; a < 3; ++a)
-                        if (T.centers[3 * c + a] - T.centers[3 * b + a] < 0) k |= 1 << a;
-                    pp.push_back(P.slot_of_box[b]);
-                    pcc.push_back(P.slot_of_box[c]);
-                    psg.push_back(k);
-                }
-            }
-        }
-        S.pcs_level_off[nl + 1] = (int)pp.size();
-        S.d_pcs_parent.upload(pp);
-        S.h.pcs_parent = pp;
-        S.d_pcs_child.upload(pcc);
-        S.h.pcs_child = pcc;
-        S.d_pcs_sign.upload(psg);
-        S.h.pcs_sign = psg;
+        step45_lists(S);
 
         // fused STEP 1+2: value->PW tables times the child->parent merge phase
         std::vector<fgt::cplx> t1(3 * per * (nl + 1), fgt::cplx(0.0));
@@ -2175,12 +2206,14 @@ struct Refiner {
             }
         std::unordered_map<int, int> tmp;     // solve slot of a grandparent -> workspace slot
         int ns = 0;
-        // (2-D: only the cutoff boxes have theirs, so the boxes from there down)
+        // (on the fast paths only some boxes below the cutoff have theirs: the
+        // boxes from there down)
+        const bool from_cutoff = S.plane || S.fast3d;
         for (int p : parents)
             for (int q = p; q < nb0 && T.level[q] > P.nlevstart;) {
                 q = T.parent[q];
                 if (!tmp.count(q)) tmp[q] = ns++;
-                if (!S.plane) break;
+                if (!from_cutoff) break;
             }
         for (int p : parents) aslot[p] = ns++;
         std::vector<int> bslot(nk, -1);
@@ -2194,7 +2227,7 @@ struct Refiner {
         // entries per split level code: (source slot, target slot, sign)
         std::map<int, std::array<std::vector<int>, 3>> splits;
         for (const auto& kv : tmp) {
-            if (S.plane && T.level[kv.first] > P.nlevstart) {
+            if (from_cutoff && T.level[kv.first] > P.nlevstart) {
                 const int q = T.parent[kv.first];
                 auto& e = splits[P.nlevels - T.level[q]];
                 e[0].push_back(tmp.at(q));
@@ -2822,6 +2855,7 @@ int fgt_solver_set_precision(fgt_solver* s, int mode) {
             hcheck(hipDeviceSynchronize(), "hipDeviceSynchronize");
             alloc_expansions(*s, f32 ? sizeof(float2) : sizeof(double2));
             s->tabs.expn_f32 = f32;
+            step45_lists(*s);
         }
         s->tabs.prec = mode;
     });

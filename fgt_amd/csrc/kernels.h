@@ -157,10 +157,13 @@ inline ZGroups z_kinds(const ZGroups& zg, int a, int nz) {
 // expansion of its own (box[0]), or a family, the leaf children of the box
 // whose expansion is in `slot`.  A family's child c has bit a (x, y, z) set
 // when it is the side whose table carries the conjugate parent-child phase
-// along axis a (-1: no leaf there); lev is the leaves' level.
+// along axis a (-1: no leaf there); lev is the leaves' level.  STEP 5 of FP64
+// expansions (klev > 0): slot holds the expansion of that box's parent, still
+// to be split to it with phase row klev and the signs of k_split.
 struct SymTask {
     int slot, lev;
     int box[8];
+    int klev = 0, sign = 0;
 };
 
 // 2-D: a leaf with an expansion (at `depth` levels below its cutoff box, whose

@@ -38,6 +38,9 @@ constexpr int kThreads = 256;
 
 __device__ __forceinline__ double2 cplus(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ double2 cminus(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
+__device__ __forceinline__ double2 cprod(double2 a, double2 b) {
+    return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+}
 
 // Touches every 64-byte line of n table entries once, eight scalar loads at a
 // time, the lines dealt to the block's waves: the scalar cache starts a
@@ -90,16 +93,22 @@ inline size_t sym5_lds_entries(int npw, int nodx, int nody) {
 // Bound by the expansion reads and by the latency of each round's three
 // stages (norder 8, npw 28, 8382 leaves: 84 us for 210 MB, 2.5 TB/s; the
 // sixteen-multiply-add form over half the siblings 244 us; norder 12, npw 60,
-// 4250 leaves: 402 us, 1182 before).  x pairs over more blocks at eight pairs
+// 4250 leaves: 402 us, 1182 before).  A family whose box's expansion is not
+// formed reads the one above it and splits it on the way: the x phase on each
+// row pair's sum and difference, the y and z phases on the column's results
+// (77 and 360 us, with the siblings' rows shared through the caches).  x pairs over more blocks at eight pairs
 // (two of four rather than one of eight: smaller LDS tiles, four blocks per
 // CU instead of three) measured 106 -> 102 us, the scalar cache's warm-up,
 // the unrolled y and z stages and one launch for both kinds of task 102 -> 84.
 template <int N, bool FAM, int NZ, typename ET>
 __device__ __forceinline__ void pw2pot_sym_block(int npw, int nd, const double2* __restrict__ tabS,
                                                  const SymTask* __restrict__ T, int part,
-                                                 const ET* __restrict__ expn, size_t ks, Kinds kd, const ZOut& zo,
+                                                 const ET* __restrict__ expn, const double2* __restrict__ wms,
+                                                 size_t ks, Kinds kd, const ZOut& zo,
                                                  const ProbPtrs* __restrict__ prob, double2* __restrict__ sm) {
     constexpr int NP = sym_pairs<N, FAM>(), NX = sym5_nx<N, FAM>();
+    // (FP32 expansions round after every split: none is folded in)
+    constexpr bool FOLD = FAM && std::is_same<ET, double2>::value;
     constexpr int NODX = 2 * NX, NODY = 2 * NP, COLS = NODX * NODY;
     static_assert(COLS <= kThreads, "one output column per thread");
     constexpr int YS = NODX <= 8 ? 4 : 2;                  // waves sharing one y row batch
@@ -122,6 +131,13 @@ __device__ __forceinline__ void pw2pot_sym_block(int npw, int nd, const double2*
     const int lane = tid & 63;
     const int slot = __builtin_amdgcn_readfirstlane(T->slot);
     const double sgx = kd.x == 1 ? -1.0 : 1.0, sgy = kd.y == 1 ? -1.0 : 1.0;
+    // the split of the expansion to the family's box: per axis the phase row,
+    // conjugated as the box lies (only the imaginary parts' signs)
+    const int klev = FOLD ? __builtin_amdgcn_readfirstlane(T->klev) : 0;
+    const int fsg = FOLD ? __builtin_amdgcn_readfirstlane(T->sign) : 0;
+    const double2* __restrict__ W = wms + (long long)(klev > 0 ? klev - 1 : 0) * npw;
+    const CTab2 WX = ctab(W);
+    const double wsx = fsg & 1 ? -1.0 : 1.0, wsy = fsg & 2 ? -1.0 : 1.0, wsz = fsg & 4 ? -1.0 : 1.0;
     CTab2 UZ[NZ];
 #pragma unroll
     for (int z = 0; z < NZ; ++z) UZ[z] = ctab(tabS) + ((long long)(zo.kz[z] * ks) + row3);
@@ -169,8 +185,16 @@ __device__ __forceinline__ void pw2pot_sym_block(int npw, int nd, const double2*
                         if (k + j >= nh) break;
                         const double2 a = ldE(e[j][0]), b = ldE(e[j][1]);
                         // the zero frequency of an odd count pairs with itself
-                        const double2 S = (odd && k + j == nh - 1) ? a : cplus(a, b);
-                        const double2 D = cminus(a, b);
+                        double2 S = (odd && k + j == nh - 1) ? a : cplus(a, b);
+                        double2 D = cminus(a, b);
+                        if (FOLD && klev > 0) {
+                            // sum and difference of a w and b conj(w)
+                            const double2 w = WX[k + j];
+                            const double wi = wsx * w.y;
+                            const double2 S0 = S;
+                            S = make_double2(S0.x * w.x - D.y * wi, S0.y * w.x + D.x * wi);
+                            D = make_double2(D.x * w.x - S0.y * wi, D.y * w.x + S0.x * wi);
+                        }
 #pragma unroll
                         for (int p = 0; p < NX; ++p) {
                             const double2 t = UX[(long long)(k + j) * N + p];
@@ -192,10 +216,18 @@ __device__ __forceinline__ void pw2pot_sym_block(int npw, int nd, const double2*
                     apply(v, k + KU);
                 }
                 double2* __restrict__ o = sm + k2 * ST + s * NODX;
+                double2 yz = make_double2(1.0, 0.0);   // the column's y and z phases
+                if (FOLD && klev > 0) {
+                    const double2 wy = gload(W, (unsigned)k2), wz = gload(W, (unsigned)min(r + s, nh - 1));
+                    yz = cprod(make_double2(wy.x, wsy * wy.y), make_double2(wz.x, wsz * wz.y));
+                }
 #pragma unroll
                 for (int p = 0; p < NX; ++p) {
-                    o[p] = make_double2(P[p].x - Q[p].y, P[p].y + Q[p].x);
-                    o[NX + p] = make_double2(sgx * (P[p].x + Q[p].y), sgx * (P[p].y - Q[p].x));
+                    double2 a = make_double2(P[p].x - Q[p].y, P[p].y + Q[p].x);
+                    double2 b = make_double2(sgx * (P[p].x + Q[p].y), sgx * (P[p].y - Q[p].x));
+                    if (FOLD && klev > 0) a = cprod(a, yz), b = cprod(b, yz);
+                    o[p] = a;
+                    o[NX + p] = b;
                 }
             }
             __syncthreads();
@@ -325,7 +357,7 @@ __device__ __forceinline__ void pw2pot_sym_block(int npw, int nd, const double2*
 template <int N, int NZ, typename ET>
 __global__ void __launch_bounds__(kThreads, (NZ > 1 && NZ * N >= 16) ? 2 : 3)
     k_pw2pot_sym(int nd, const double2* __restrict__ tabS, int npw, const SymTask* __restrict__ tasks, int nfam,
-                 int nown, const ET* __restrict__ expn, size_t ks, ZGroups zg, Multi mu) {
+                 int nown, const ET* __restrict__ expn, const double2* __restrict__ wms, size_t ks, ZGroups zg, Multi mu) {
     constexpr int PF = sym5_parts<N, true>(), PO = sym5_parts<N, false>();
     extern __shared__ double2 sm[];
     const int nfb = nfam * PF, per = nfb + nown * PO;
@@ -340,10 +372,11 @@ __global__ void __launch_bounds__(kThreads, (NZ > 1 && NZ * N >= 16) ? 2 : 3)
         prob = mu.pp + mu.tprob[tix];
         npw = prob->g.npw;
         tabS = prob->pw2potS;
+        wms = prob->wms;
         expn = static_cast<const ET*>(prob->expn);
     }
-    if (fam) pw2pot_sym_block<N, true, NZ, ET>(npw, nd, tabS, tasks + tix, part, expn, ks, kd, zo, prob, sm);
-    else pw2pot_sym_block<N, false, NZ, ET>(npw, nd, tabS, tasks + tix, part, expn, ks, kd, zo, prob, sm);
+    if (fam) pw2pot_sym_block<N, true, NZ, ET>(npw, nd, tabS, tasks + tix, part, expn, wms, ks, kd, zo, prob, sm);
+    else pw2pot_sym_block<N, false, NZ, ET>(npw, nd, tabS, tasks + tix, part, expn, wms, ks, kd, zo, prob, sm);
 }
 
 // f(std::integral_constant<int, n>) for the orders covered here
@@ -384,12 +417,12 @@ void launch_sym5_z(const Geom& g, const DevTables& t, int nfam, int nown, const 
     if constexpr (has_fp32(N)) {
         if (t.expn_f32) {
             hipLaunchKernelGGL((k_pw2pot_sym<N, NZ, float2>), grid, block, lds, s, g.nd, t.pw2potS, t.npw, tasks, nfam,
-                               nown, reinterpret_cast<const float2*>(expn), t.pw2potS_ks, zg, mu);
+                               nown, reinterpret_cast<const float2*>(expn), t.wms, t.pw2potS_ks, zg, mu);
             return;
         }
     }
     hipLaunchKernelGGL((k_pw2pot_sym<N, NZ, double2>), grid, block, lds, s, g.nd, t.pw2potS, t.npw, tasks, nfam, nown,
-                       expn, t.pw2potS_ks, zg, mu);
+                       expn, t.wms, t.pw2potS_ks, zg, mu);
 }
 
 template <int N>
