@@ -76,9 +76,39 @@ __device__ __forceinline__ float bcol(double2 u, int part, int kpart) {
 // of their four, part-1 lanes 2, 3.
 constexpr int kLowpColGroup = 2;
 
+// BF16: the table operands of every column tile and K step, split, in LDS once
+// per task: tab[(ct * KB + st) * 64 + lane], KB = K steps of 16 (prepared per
+// row tile and round, with the result's part picked by an index through
+// scratch, k_p2pw3 over the 779 leaves of an order-8 problem took 39 us, per
+// column group and round 30; in LDS STEP 1 beside the near field 66 -> 41 us)
+struct BfPair { bf8 hi, lo; };
+__host__ __device__ constexpr size_t x1_tab_entries(int KN, int npw) {
+    return (size_t)((2 * npw + 15) >> 4) * ((KN + 15) / 16) * 64;
+}
+template <int KN, class FB>
+__device__ __forceinline__ void x1_fill(BfPair* __restrict__ tab, int npw, int tid, FB fb) {
+    constexpr int KB = (KN + 15) / 16;
+    const int n = (int)x1_tab_entries(KN, npw);
+    for (int o = tid; o < n; o += 256) {
+        const int lane = o & 63, st = (o >> 6) % KB, c = 16 * ((o >> 6) / KB) + (lane & 15), lq = lane >> 4;
+        const bool cval = (c >> 1) < npw;
+        float bx[8];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int kk = 16 * st + 4 * lq + j;
+            const bool ok = kk < KN && cval;
+            const double2 u = fb(kk < KN ? kk : KN - 1, cval ? (c >> 1) : 0);
+            bx[2 * j] = ok ? bcol(u, c & 1, 0) : 0.f;
+            bx[2 * j + 1] = ok ? bcol(u, c & 1, 1) : 0.f;
+        }
+        split_bf(bx, tab[o].hi, tab[o].lo);
+    }
+}
+
 // column tiles c0, c0 + ctstep, ... (CG of them, all below CT)
 template <int KN, int XS, int CG, class FA, class FB, class FW>
-__device__ __forceinline__ void x1_lowp_group(int npw, int lane, int c0, int ctstep, FA fa, FB fb, FW fw) {
+__device__ __forceinline__ void x1_lowp_group(int npw, int lane, int c0, int ctstep, FA fa, FB fb, FW fw,
+                                              const BfPair* __restrict__ tab) {
     const int MT = (npw + 15) >> 4;
     const int CT = (2 * npw + 15) >> 4;
     const int li = lane & 15, lq = lane >> 4;
@@ -92,10 +122,8 @@ __device__ __forceinline__ void x1_lowp_group(int npw, int lane, int c0, int cts
             cval[gi] = (c >> 1) < npw && c0 + gi * ctstep < CT;
             k1c[gi] = cval[gi] ? (c >> 1) : 0;
         }
-        // the column tiles' table operands of every K step, read (BF16: and
-        // split) once for all row tiles (BF16 per row tile, with the result's
-        // part picked by an index through scratch: k_p2pw3 over the 779 leaves
-        // of an order-8 problem 39 us, now 30)
+        // FP32: the column tiles' table operands of every K step, read once for
+        // all row tiles
         constexpr int KS = (KN + 3) / 4, KB = (KN + 15) / 16;
         float tb1[CG][XS == 2 ? KS : 1], tb2[CG][XS == 2 ? KS : 1];
         if constexpr (XS == 2) {
@@ -112,24 +140,6 @@ __device__ __forceinline__ void x1_lowp_group(int npw, int lane, int c0, int cts
                     tb2[gi][st] = ok ? bcol(u, part[gi], 1) : 0.f;
                 }
             }
-        }
-        bf8 bh[CG][XS == 2 ? 1 : KB], bl[CG][XS == 2 ? 1 : KB];
-        if constexpr (XS != 2) {
-#pragma unroll
-            for (int st = 0; st < KB; ++st)
-#pragma unroll
-                for (int gi = 0; gi < CG; ++gi) {
-                    float bx[8];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int kk = 16 * st + 4 * lq + j;
-                        const bool ok = kk < KN && cval[gi];
-                        const double2 u = fb(kk < KN ? kk : KN - 1, k1c[gi]);
-                        bx[2 * j] = ok ? bcol(u, part[gi], 0) : 0.f;
-                        bx[2 * j + 1] = ok ? bcol(u, part[gi], 1) : 0.f;
-                    }
-                    split_bf(bx, bh[gi][st], bl[gi][st]);
-                }
         }
         // one row tile at a time (few live accumulators, high occupancy)
         for (int mt = 0; mt < MT; ++mt) {
@@ -165,9 +175,12 @@ __device__ __forceinline__ void x1_lowp_group(int npw, int lane, int c0, int cts
                     split_bf(ax, ah, al);
 #pragma unroll
                     for (int gi = 0; gi < CG; ++gi) {
-                        acc[gi][0] = mfma_bf(ah, bh[gi][st], acc[gi][0]);
-                        acc[gi][1] = mfma_bf(ah, bl[gi][st], acc[gi][1]);
-                        acc[gi][1] = mfma_bf(al, bh[gi][st], acc[gi][1]);
+                        // (a group's tile past the last is discarded)
+                        const BfPair* __restrict__ b = tab + (min(c0 + gi * ctstep, CT - 1) * KB + st) * 64 + lane;
+                        const bf8 bh = b->hi, bl = b->lo;
+                        acc[gi][0] = mfma_bf(ah, bh, acc[gi][0]);
+                        acc[gi][1] = mfma_bf(ah, bl, acc[gi][1]);
+                        acc[gi][1] = mfma_bf(al, bh, acc[gi][1]);
                     }
                 }
             }
@@ -194,15 +207,16 @@ __device__ __forceinline__ void x1_lowp_group(int npw, int lane, int c0, int cts
 }
 
 template <int KN, int XS, class FA, class FB, class FW>
-__device__ __forceinline__ void x1_lowp(int npw, int lane, int ct0, int ctstep, FA fa, FB fb, FW fw) {
+__device__ __forceinline__ void x1_lowp(int npw, int lane, int ct0, int ctstep, FA fa, FB fb, FW fw,
+                                        const BfPair* __restrict__ tab) {
     constexpr int CG = kLowpColGroup;
     const int CT = (2 * npw + 15) >> 4;
     for (int c0 = ct0; c0 < CT; c0 += CG * ctstep) {
         // (BF16: the one-tile form's registers would cost a block per CU)
         if (XS != 2 || c0 + (CG - 1) * ctstep < CT)
-            x1_lowp_group<KN, XS, CG>(npw, lane, c0, ctstep, fa, fb, fw);
+            x1_lowp_group<KN, XS, CG>(npw, lane, c0, ctstep, fa, fb, fw, tab);
         else
-            x1_lowp_group<KN, XS, 1>(npw, lane, c0, ctstep, fa, fb, fw);
+            x1_lowp_group<KN, XS, 1>(npw, lane, c0, ctstep, fa, fb, fw, tab);
     }
 }
 
@@ -210,6 +224,9 @@ __device__ __forceinline__ void x1_lowp(int npw, int lane, int ct0, int ctstep, 
 // LDS: sff [m2][s][m1] (N*4*N complex) and sff2 [s][m1][k2] (4*N*npw
 // complex) share one buffer: the y stage reads its sff column into registers
 // and passes a barrier before writing sff2 (more blocks fit on a CU).
+__host__ __device__ constexpr size_t p2pw3_entries(int n, int npw) {
+    return 4 * (size_t)n * (npw > n ? npw : n);
+}
 template <int N, int XS, typename ET>
 __global__ void __launch_bounds__(256) k_p2pw3(Geom g, const double2* __restrict__ tab_a, int npw,
                                               const int* __restrict__ box, const int* __restrict__ lev,
@@ -237,6 +254,8 @@ __global__ void __launch_bounds__(256) k_p2pw3(Geom g, const double2* __restrict
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
     const int nh = g.pz, nd = g.nd;
+    BfPair* xtab = reinterpret_cast<BfPair*>(sm + p2pw3_entries(N, npw));
+    if (XS == 3) x1_fill<N>(xtab, npw, tid, [&](int m1, int k1) { return T[k1 * N + m1]; });   // (a barrier follows)
     for (int ind = 0; ind < nd; ++ind) {
         double fr[N];
         if (tid < N * N) {
@@ -295,7 +314,7 @@ __global__ void __launch_bounds__(256) k_p2pw3(Geom g, const double2* __restrict
                         npw, lane, 0, 1,
                         [&](int k2, int m1) { return sff2[(wave * N + m1) * npw + k2]; },
                         [&](int m1, int k1) { return T[k1 * N + m1]; },
-                        [&](int k2, int k1, float2 v) { Ek[(size_t)k1 * npw + k2] = v; });
+                        [&](int k2, int k1, float2 v) { Ek[(size_t)k1 * npw + k2] = v; }, xtab);
                 }
             }
             __syncthreads();
@@ -325,6 +344,9 @@ __global__ void __launch_bounds__(256) k_p2pw3(Geom g, const double2* __restrict
 // share one buffer: sH is fully read into registers before sF is written.
 constexpr int kFusedParts = 4;
 
+__host__ __device__ constexpr size_t p2pwF3_entries(int n, int sr, int npw) {
+    return 2 * (size_t)sr * n * (npw > 2 * n ? npw : 2 * n);
+}
 template <int N, int XS, typename ET, int SR = 2>
 __global__ void __launch_bounds__(256) k_p2pwF3(Geom g, const double2* __restrict__ tabS_a, int npw,
                                                const int* __restrict__ plev, const int* __restrict__ pslot,
@@ -360,6 +382,13 @@ __global__ void __launch_bounds__(256) k_p2pwF3(Geom g, const double2* __restric
     while (nk < 8 && kids[8 * task + nk] >= 0) ++nk;   // leaf children are packed first
     const int nround = (nh + SR - 1) / SR;
     const int rb = SR * (part * nround / kFusedParts), re = SR * ((part + 1) * nround / kFusedParts);
+    BfPair* xtab = reinterpret_cast<BfPair*>(sm + p2pwF3_entries(N, SR, npw));
+    if (XS == 3) {   // (barriers follow)
+        const CTab2 Txp = T + base0 + 1 * per;
+        const CTab2 Txm = T + base0 + 2 * per;
+        x1_fill<2 * N>(xtab, npw, tid,
+                       [&](int kk, int k1) { return kk >= N ? Txm[k1 * N + kk - N] : Txp[k1 * N + kk]; });
+    }
     for (int ind = 0; ind < nd; ++ind) {
         ET* __restrict__ E = expn + ((size_t)sl * 2 * nd + ind) * g.nexp;
         // norder 8: one wave per group g = (sx, sy) of children; the values
@@ -489,7 +518,7 @@ __global__ void __launch_bounds__(256) k_p2pwF3(Geom g, const double2* __restric
                             return sF[((sx * SR + s) * N + (kk - N * sx)) * npw + k2];
                         },
                         [&](int kk, int k1) { return kk >= N ? Txm[k1 * N + kk - N] : Txp[k1 * N + kk]; },
-                        [&](int k2, int k1, float2 v) { Ek[(size_t)k1 * npw + k2] = v; });
+                        [&](int k2, int k1, float2 v) { Ek[(size_t)k1 * npw + k2] = v; }, xtab);
                 }
             }
             __syncthreads();
@@ -504,7 +533,6 @@ __global__ void __launch_bounds__(256) k_p2pwF3(Geom g, const double2* __restric
 // the lane's eight K entries.  Zero past npw and past the last column.
 template <int XS> struct XEntry;
 template <> struct XEntry<2> { typedef float2 type; };
-struct BfPair { bf8 hi, lo; };
 template <> struct XEntry<3> { typedef BfPair type; };
 template <int N, int XS> struct XTable {
     static constexpr int NT = (2 * N + 15) / 16;
@@ -851,7 +879,8 @@ __global__ void __launch_bounds__(256, 2) k_pw2pot3(Geom g, const double2* __res
 template <int N>
 bool try_p2pw3(const Geom& g, const DevTables& t, int ntask, const int* box, const int* lev, const int* slot,
                const double* fvals, double2* expn, hipStream_t s, size_t lds_limit, const Multi& mu) {
-    const size_t lds = sizeof(double2) * std::max(4 * (size_t)N * N, 4 * (size_t)N * t.npw);
+    const size_t lds = sizeof(double2) * p2pw3_entries(N, t.npw) +
+                       (t.prec == 2 ? sizeof(BfPair) * x1_tab_entries(N, t.npw) : 0);
     if (lds > lds_limit) return false;
     float2* e32 = reinterpret_cast<float2*>(expn);
     if (t.prec == 2)
@@ -1003,7 +1032,8 @@ bool p2pw_fused_3d(const Geom& g, const DevTables& t, int ntask, const int* plev
     if (g.ndim != 3 || ntask <= 0) return ntask <= 0;
     const int N = t.n;
     const size_t sr = (size_t)p2pwF3_slabs(N, t);
-    const size_t lds = sizeof(double2) * std::max(4 * sr * N * N, 2 * sr * N * t.npw);
+    const size_t lds = sizeof(double2) * p2pwF3_entries(N, (int)sr, t.npw) +
+                       (t.prec == 2 ? sizeof(BfPair) * x1_tab_entries(2 * N, t.npw) : 0);
     if (lds > t.lds_limit) return false;
     if ((long long)ntask * kFusedParts > 0x7fffffffLL) return false;
     const unsigned nblk = (unsigned)(ntask * kFusedParts);
