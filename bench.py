@@ -62,8 +62,9 @@ M2L_KERNEL = {0: "k_m2l27", 1: "k_m2l_brick", 2: "k_m2l_sep"}
 def stage_model(st, n, nd=1):
     """Algorithmic FLOPs and HBM bytes of one launch of the single-kernel stages.
 
-    STEP 5 (k_pw2pot3, per PW leaf, 3-D): 4 n^3 nh + 8 n^2 npw nh + 8 n npw^2 nh
-    flops (the x/y stages complex x complex, the last stage real output);
+    STEP 5 (k_pw2pot_sym, per PW leaf, 3-D): a quarter (the tables' symmetries) of
+    4 n^3 nh + 8 n^2 npw nh + 8 n npw^2 nh flops (the x/y stages complex x
+    complex, the last stage real output);
     bytes: read one local expansion (16 nexp) + read/write pot (16 n^3).
     STEP 3 (k_m2l_sep / k_m2l_brick / k_m2l27, per cutoff-level box): 8 nexp flops per list entry; compulsory
     bytes: every cutoff-level mp read once and every loc written once,
@@ -74,7 +75,7 @@ def stage_model(st, n, nd=1):
     L = st["npw_leaves"]
     f15 = 4 * n ** 3 * nh + 8 * n * n * npw * nh + 8 * n * npw * npw * nh
     return {
-        "pw2pot": {"kernel": "k_pw2pot3", "bound": "mfma", "flops": L * nd * f15,
+        "pw2pot": {"kernel": "k_pw2pot_sym", "bound": "mfma", "flops": L * nd * f15 // 4,
                    "bytes": L * nd * (16 * nexp + 16 * n ** 3)},
         "m2l": {"kernel": M2L_KERNEL[st.get("m2l_form", 0)], "bound": "hbm",
                 "flops": 8 * nd * nexp * st["n_m2l_pairs"],
@@ -174,13 +175,22 @@ def pot_error(pot, ref):
     return l2, mx
 
 
+def lowp(prec, xs, step):
+    """STEP 1 / 5 of a class has its x stage on the reduced-precision matrix
+    cores: the autotuner's choice, else both in BF16 and STEP 5 in FP32."""
+    if prec == 0:
+        return 0
+    return int(xs == 2) if xs >= 0 else int(step == 5 or prec == 2)
+
+
 def batch_roofline(probs, prof):
     """Per class and stage: device ms of the profiled execute and the
     algorithmic work of that launch group; roofline of the longest one among
-    STEP 1 (k_p2pwF3 / k_p2pw3), STEP 3 (k_m2l27) and STEP 5 (k_pw2pot3).
-    STEP 1 and 5 flops: the reference's per-leaf count 4 n^3 nh + 8 n^2 npw nh
-    + 8 n npw^2 nh (nh = (npw+1)/2) per plane-wave leaf of every member;
-    STEP 3 bytes: every cutoff-level expansion read once and every local
+    STEP 1 (k_p2pw_sym, or k_p2pwF3 / k_p2pw3 in reduced precision), STEP 3
+    (k_m2l27) and STEP 5 (k_pw2pot_sym or k_pw2pot3).  STEP 1 and 5 flops: the
+    reference's per-leaf count 4 n^3 nh + 8 n^2 npw nh + 8 n npw^2 nh (nh =
+    (npw+1)/2) per plane-wave leaf of every member, a quarter of it where a
+    stage goes through the tables' symmetries; STEP 3 bytes: every cutoff-level expansion read once and every local
     expansion written once (2 x nexp complex of the storage precision per
     target)."""
     import fgt_amd
@@ -188,22 +198,28 @@ def batch_roofline(probs, prof):
     for c in prof:
         n, prec = c["norder"], c["prec"]
         elem = 16 if prec == 0 else 8
-        flops = byts = 0
+        flops5 = flops1 = byts = 0
         for i in c["member_ids"]:
             tr, delta, eps = probs[i]
             ps = fgt_amd.plan_summary(tr, delta, eps)
             npw = ps["npw"]
             nh = (npw + 1) // 2
-            flops += ps["npw_leaves"] * (4 * n ** 3 * nh + 8 * n * n * npw * nh + 8 * n * npw * npw * nh)
+            # z, y and x stages through the tables' symmetries (a quarter of the
+            # complex products); a reduced-precision x stage is plain, and so is
+            # all of STEP 1 beside it
+            zy, x = 4 * n ** 3 * nh + 8 * n * n * npw * nh, 8 * n * npw * npw * nh
+            flops5 += ps["npw_leaves"] * (zy // 4 + (x if lowp(prec, c["xs5"], 5) else x // 4))
+            flops1 += ps["npw_leaves"] * (zy + x if lowp(prec, c["xs1"], 1) else (zy + x) // 4)
             byts += 2 * elem * ps["nexp"] * ps["n_m2l_targets"]
         ms = c["stage_ms"]
         rows.append({"norder": n, "prec": prec, "npw_cap": c["npw_cap"], "members": c["members"],
                      "group": c["group"], "xs1": c["xs1"], "xs5": c["xs5"], "m2l_brick": c["m2l_brick"],
                      "m2l_ept": c["m2l_ept"],
-                     "stage_ms": [round(v, 4) for v in ms], "step15_gflop": round(flops / 1e9, 3),
+                     "stage_ms": [round(v, 4) for v in ms], "step5_gflop": round(flops5 / 1e9, 3), "step1_gflop": round(flops1 / 1e9, 3),
                      "step3_gb": round(byts / 1e9, 3)})
-        for stg, kern, kind, work, xs in ((4, "k_pw2pot3", "flops", flops, c["xs5"]),
-                                          (0, "k_p2pwF3+k_p2pw3", "flops", flops, c["xs1"]),
+        xs5, xs1 = 2 * lowp(prec, c["xs5"], 5), 2 * lowp(prec, c["xs1"], 1)
+        for stg, kern, kind, work, xs in ((4, "k_pw2pot3" if xs5 else "k_pw2pot_sym", "flops", flops5, xs5),
+                                          (0, "k_p2pwF3+k_p2pw3" if xs1 else "k_p2pw_sym", "flops", flops1, xs1),
                                           (2, M2L_KERNEL[c["m2l_brick"]], "bytes", byts, -1)):
             if ms[stg] > 0 and work > 0 and (best is None or ms[stg] > best[0]):
                 best = (ms[stg], kern, kind, work, n, prec, c["npw_cap"], xs)
@@ -213,11 +229,10 @@ def batch_roofline(probs, prof):
     arith = None
     if kind == "flops":
         # the peak of the arithmetic the launch group runs: its x stage (the
-        # bulk of the flops) on the VALU in FP64 (xs 0), on the FP64 matrix
-        # cores (xs 1) or on the reduced-precision matrix cores of the mode
-        # (xs 2); FP64 vector and matrix peaks are equal on MI355X
-        if xs in (0, 1):
-            peak, arith = PEAK_FP64_TFLOPS, "FP64 x stage (" + ("VALU" if xs == 0 else "matrix cores") + ")"
+        # bulk of the flops) on the VALU in FP64 (xs 0) or on the
+        # reduced-precision matrix cores of the mode (xs 2)
+        if xs == 0:
+            peak, arith = PEAK_FP64_TFLOPS, "FP64 x stage (VALU)"
         else:
             peak, arith = PEAK_MODE_TFLOPS[prec], f"x stage on the precision-mode-{prec} matrix cores"
         ach, unit, bound = work / (ms * 1e-3) / 1e12, "TFLOP/s", "mfma"
