@@ -250,7 +250,7 @@ def batch_roofline(probs, prof):
 
 
 def headline(probs, steps, warmup, mode, drop_in=True):
-    """North-star comparison on one problem set.
+    """Headline comparison on one problem set.
 
     value: the batched mixed-precision form (precision `mode` for every
     problem whose eps allows it; fvals resident in HBM, potential written to
