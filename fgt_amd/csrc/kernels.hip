@@ -330,6 +330,14 @@ __global__ void __launch_bounds__(kBlock) k_m2l27(Geom g, DevTables t, int ngrou
 #undef M2L_LOAD
 }
 
+// store past the caches
+__device__ __forceinline__ void stNT(double2* p, double2 v) {
+    __builtin_nontemporal_store(dvec2_t{v.x, v.y}, (FGT_GLOBAL dvec2_t*)p);
+}
+__device__ __forceinline__ void stNT(float2* p, double2 v) {
+    __builtin_nontemporal_store(fvec2_t{(float)v.x, (float)v.y}, (FGT_GLOBAL fvec2_t*)p);
+}
+
 // STEP 3 over sibling bricks (3-D): a block owns one element range and the
 // (up to) eight cutoff-level children of one parent, whose M2L sources lie
 // in the 4x4x4 boxes around them.  Each source is loaded once per brick and
@@ -347,14 +355,20 @@ __global__ void __launch_bounds__(kBlock) k_m2l27(Geom g, DevTables t, int ngrou
 // one element range then share fewer source bytes than an XCD's L2 holds), and
 // entries padded to two, not four.  Whole solves: periodic order 16 with 1245
 // targets 1864 -> 1743 us, order-8 gradient with 752 targets 452 -> 418.
+// past: the results go past the caches.  Where the expansions exceed the
+// memory-side cache, STEP 5 would not find them there anyway, and the sources
+// keep the L2 (periodic order 16 1715 -> 1668 us, order-8 gradient 405 -> 387,
+// 1.2 GB and 0.16 GB of results); below that STEP 5 reads them from the cache
+// (order 8, 64 MB: 264 -> 267 us with the stores past it).
 constexpr int kBrickBlock = 128;
+constexpr long long kBrickPastBytes = 128LL << 20;
 template <typename ET>
 __global__ void __launch_bounds__(kBrickBlock) k_m2l_brick(Geom g, DevTables t, int nbrick, long long zero_off,
                                                       const long long* __restrict__ toff,
                                                       const int* __restrict__ gent,
                                                       const long long* __restrict__ soff,
                                                       const int* __restrict__ scode,
-                                                      ET* __restrict__ expn_a, Multi mu) {
+                                                      ET* __restrict__ expn_a, Multi mu, int past) {
     const int lin = xcd_task(blockIdx.x, gridDim.x);
     const int brk = lin % nbrick, chunk = lin / nbrick;
     ET* __restrict__ expn = expn_a;
@@ -459,8 +473,13 @@ __global__ void __launch_bounds__(kBrickBlock) k_m2l_brick(Geom g, DevTables t, 
         for (int q = 0; q < 8; ++q) {
             const long long o = to[q];
             if (o >= 0) {
-                stE(expn + o + tot + e, acc[q]);
-                stE(expn + o + tot + e2, acc2[q]);
+                if (past) {
+                    stNT(expn + o + tot + e, acc[q]);
+                    stNT(expn + o + tot + e2, acc2[q]);
+                } else {
+                    stE(expn + o + tot + e, acc[q]);
+                    stE(expn + o + tot + e2, acc2[q]);
+                }
             }
         }
     }
@@ -931,12 +950,14 @@ void launch_m2l_brick(const Geom& g, const DevTables& t, int nbrick, long long z
     const long long pairs = (long long)g.nd * g.pz * ((g.px * g.py + 1) / 2);
     const long long nblk = ((pairs + kBrickBlock - 1) / kBrickBlock) * nbrick;
     if (pairs > 0x7fffff00LL || nblk > 0x7fffffffLL) throw std::runtime_error("k_m2l_brick: grid too large");
+    // (eight targets per brick at most)
+    const int past = 8LL * nbrick * g.nd * g.nexp * (t.expn_f32 ? 8 : 16) > kBrickPastBytes;
     if (t.expn_f32)
         hipLaunchKernelGGL(k_m2l_brick<float2>, dim3((unsigned)nblk), dim3(kBrickBlock), 0, s, g, t, nbrick, zero_off,
-                           toff, gent, soff, scode, reinterpret_cast<float2*>(expn), mu);
+                           toff, gent, soff, scode, reinterpret_cast<float2*>(expn), mu, past);
     else
         hipLaunchKernelGGL(k_m2l_brick<double2>, dim3((unsigned)nblk), dim3(kBrickBlock), 0, s, g, t, nbrick, zero_off,
-                           toff, gent, soff, scode, expn, mu);
+                           toff, gent, soff, scode, expn, mu, past);
     check(hipGetLastError(), "k_m2l_brick launch");
 }
 
