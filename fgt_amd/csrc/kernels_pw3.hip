@@ -4,7 +4,7 @@
 // STEP 1 (values -> PW, g3d_tens_prod_to_pw, bfgt_pwrouts.f:153-222) and
 // STEP 5 (PW -> values, g3d_pw2pot, bfgt_pwrouts.f:719-790) for norder
 // N in {8, 12, 16}, one 256-thread block (4 waves) per task (a leaf, a
-// parent with leaf children, or up to four sibling leaves).
+// quarter of a parent with leaf children, or one side of such a family).
 //
 // The y and z stages run on the FP64 VALU with a wave-uniform 1-D table
 // operand (its address depends only on loop counters and the wave index, so
