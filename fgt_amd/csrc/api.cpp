@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "../../include/fgt.h"
+#include "device_buffer.h"
 #include "kernels.h"
 #include "plan.h"
 #include "retree.h"
@@ -39,76 +40,11 @@ void set_status(int st, const std::string& m) {
     g_msg = m;
 }
 
-void hcheck(hipError_t e, const char* what) {
-    if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
-}
-
-// Bump allocator over a caller-provided device range (the no-allocation
-// entry point's scratch): while one is installed on this thread, device
-// buffers are carved from it instead of hipMalloc'd.
-struct Arena {
-    char* base = nullptr;
-    size_t cap = 0, used = 0;
-    void* take(size_t b) {
-        const size_t off = (used + 255) & ~size_t(255);
-        if (off + b > cap)
-            throw std::invalid_argument("problem needs more device workspace than the " +
-                                        std::to_string(cap >> 20) + " MiB no-allocation scratch");
-        used = off + b;
-        return base + off;
-    }
-};
-thread_local Arena* g_arena = nullptr;
-// device bytes allocated on this thread by DBuf::alloc (the server's
-// admission accounting reads it around a solver build)
-thread_local size_t g_tally = 0;
-
-// A device buffer owned by the solver (or carved from the installed arena).
-struct DBuf {
-    void* p = nullptr;
-    size_t bytes = 0;
-    bool from_arena = false;
-    DBuf() = default;
-    DBuf(const DBuf&) = delete;
-    DBuf& operator=(const DBuf&) = delete;
-    DBuf& operator=(DBuf&& o) noexcept {
-        if (this != &o) {
-            release();
-            p = o.p;
-            bytes = o.bytes;
-            from_arena = o.from_arena;
-            o.p = nullptr;
-            o.bytes = 0;
-            o.from_arena = false;
-        }
-        return *this;
-    }
-    ~DBuf() { release(); }
-    void release() {
-        if (p && !from_arena) (void)hipFree(p);
-        p = nullptr;
-        from_arena = false;
-    }
-    void alloc(size_t b) {
-        release();
-        bytes = b;
-        if (!b) return;
-        if (g_arena) {
-            p = g_arena->take(b);
-            from_arena = true;
-        } else {
-            hcheck(hipMalloc(&p, b), "hipMalloc");
-            g_tally += b;
-        }
-    }
-    template <class T>
-    void upload(const std::vector<T>& v) {
-        alloc(sizeof(T) * v.size());
-        if (!v.empty()) hcheck(hipMemcpy(p, v.data(), bytes, hipMemcpyHostToDevice), "hipMemcpy H2D");
-    }
-    template <class T>
-    T* as() const { return static_cast<T*>(p); }
-};
+using fgt::Arena;
+using fgt::DBuf;
+using fgt::g_arena;
+using fgt::g_tally;
+using fgt::hcheck;
 
 }  // namespace
 
@@ -1260,10 +1196,7 @@ void eval_targets(fgt_solver& S, int nt, const double* targs, int ifpghtarg, dou
         hcheck(hipMemcpy(outs[L].host, out, sizeof(double) * (size_t)ncd * nt, hipMemcpyDeviceToHost),
                "download target values");
     }
-    if (S.d_t_work.bytes > kTargetWorkKept) {
-        S.d_t_work.release();
-        S.d_t_work.bytes = 0;
-    }
+    if (S.d_t_work.bytes > kTargetWorkKept) S.d_t_work.release();
 }
 
 template <class F>
