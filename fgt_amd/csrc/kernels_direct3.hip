@@ -68,6 +68,15 @@ struct Entry {
 __device__ __forceinline__ Entry uniform(int2 v) {
     return Entry{__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y)};
 }
+// What one lane of a wave wrote to LDS and another reads after: the wave's LDS
+// accesses complete in program order, so only the compiler has to keep it.  The
+// barrier alone stops the scheduler, not the passes that move memory accesses.
+__device__ __forceinline__ void wave_lds_exchange() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // entries [j0, j0 + n), n <= kChunk, by the block's first wave; the caller's
 // barrier follows
 template <int TEAMS>
@@ -291,7 +300,7 @@ __global__ void __launch_bounds__(64 * direct3_waves<N>() * direct3_teams<N>())
                         X[s][m][r] = 0.0;
                     }
             if (W > 1) __syncthreads();
-            else __builtin_amdgcn_wave_barrier();
+            else wave_lds_exchange();
             // z: Z[k3][k1] += sum_j3 Az[k3][j3] X[j3][k1], rows k2
             double V[S][NB][NB];
 #pragma unroll
@@ -317,7 +326,7 @@ __global__ void __launch_bounds__(64 * direct3_waves<N>() * direct3_teams<N>())
                                     __builtin_amdgcn_mfma_f64_4x4x4f64(A[m][h], V[s][h][r], Z[c][s][m][r], 0, 0, 0);
             }
             if (W > 1) __syncthreads();   // the x sums are read
-            else __builtin_amdgcn_wave_barrier();
+            else wave_lds_exchange();
         };
         for (int c0 = j0; c0 < j1; c0 += kChunk) {
             if (ind == 0 || j1 - j0 > kChunk) {
