@@ -61,7 +61,7 @@ struct fgt_solver {
     // extra targets (STEP 11): set up on first use
     bool t_ready = false;
     DBuf d_t_u, d_t_child, d_t_centers, d_t_bsz, d_t_work;
-    int t_nleaf = 0;
+    int t_nend = 0;         // boxes where a target's path can end: leaves, parents that lack a child
     bool t_whole = true;    // no parent lacks a child
     // lists
     DBuf d_leaf_box, d_leaf_lev, d_leaf_slot;
@@ -1130,18 +1130,23 @@ void eval_targets(fgt_solver& S, int nt, const double* targs, int ifpghtarg, dou
         S.d_t_u.upload(u);
         std::vector<int> child((size_t)mc * P.nboxes, -1);
         std::vector<double> bsz(P.nboxes);
-        S.t_nleaf = 0;
+        S.t_nend = 0;
         S.t_whole = true;
         for (int b = 0; b < P.nboxes; ++b) {
             bsz[b] = T.boxsize[T.level[b]];
             if (T.nchild[b] == 0) {
-                ++S.t_nleaf;
+                ++S.t_nend;
                 continue;
             }
+            bool whole = true;
             for (int k = 0; k < mc; ++k) {
                 const int c = T.child[(size_t)mc * b + k];
                 child[(size_t)mc * b + k] = c >= 0 ? c : -2;
-                if (c < 0) S.t_whole = false;
+                if (c < 0) whole = false;
+            }
+            if (!whole) {
+                ++S.t_nend;
+                S.t_whole = false;
             }
         }
         S.d_t_child.upload(child);
@@ -1155,7 +1160,7 @@ void eval_targets(fgt_solver& S, int nt, const double* targs, int ifpghtarg, dou
     int ncdmax = 0;
     for (int L = 0; L < ifpghtarg; ++L) ncdmax = std::max(ncdmax, nd * outs[L].ncomp);
     // one workspace; each part starts on 16 bytes
-    const int maxtask = fgt::target_tasks_max(nt, S.t_nleaf);
+    const int maxtask = fgt::target_tasks_max(nt, S.t_nend);
     size_t bytes = 0;
     auto part = [&](size_t b) {
         const size_t at = bytes;

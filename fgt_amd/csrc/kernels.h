@@ -421,7 +421,8 @@ void launch_zero(void* p, size_t bytes, hipStream_t s);
 // ends at a missing child.  launch_targets evaluates values (ncd, npbox,
 // nboxes) at the targets, out[t*ncd + q] (u = values->coefficients, u(k,j) at
 // u[k + j*n]).
-int target_tasks_max(int nt, int nleaf);
+// (nend: boxes where a target's path can end, leaves and boxes that lack a child)
+int target_tasks_max(int nt, int nend);
 bool launch_target_groups(int nt, int ndim, int nlevels, int nboxes, const double* targs, const double* centers,
                           const int* child, int* count, int* first, int2* place, int* perm, int4* tasks, int* ntask,
                           int* missing, hipStream_t s);

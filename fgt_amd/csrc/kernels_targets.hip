@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(256) k_targets(int ndim, int ipoly, int ncd, c
 
 }  // namespace
 
-int target_tasks_max(int nt, int nleaf) { return (int)std::min<long long>(nt, (long long)nleaf + nt / kTaskTargets); }
+int target_tasks_max(int nt, int nend) { return (int)std::min<long long>(nt, (long long)nend + nt / kTaskTargets); }
 
 bool launch_target_groups(int nt, int ndim, int nlevels, int nboxes, const double* targs, const double* centers,
                           const int* child, int* count, int* first, int2* place, int* perm, int4* tasks, int* ntask,
