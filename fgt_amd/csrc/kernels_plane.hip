@@ -389,8 +389,10 @@ void for_y(int n, F&& launch) {
 
 bool ok_launch() { return hipGetLastError() == hipSuccess; }
 
-// rows k3 of a STEP 1 block
-int plane_rows(int nh) { return kBlock / nh * kRows; }
+// rows k3 of a STEP 1 block: as its threads take them, of those there are (LDS
+// holds the rows: three plane waves at order 16, 256 / nh threads a row, would
+// ask for 209 KB and go the general way, 166 leaves 63 us and not 22)
+int plane_rows(int nh) { return std::min(kBlock / nh * kRows, nh); }
 size_t p2pw2_lds(int n, int nh) {
     const size_t R = plane_rows(nh), h = (n + 1) / 2;
     return sizeof(double2) * (nh * h + 2 * (nh + R) + 4 * R * h) + sizeof(double) * 2 * n * n;
