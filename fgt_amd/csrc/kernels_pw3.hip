@@ -876,11 +876,24 @@ __global__ void __launch_bounds__(256, 2) k_pw2pot3(Geom g, const double2* __res
     }
 }
 
+// slabs per round of the fused STEP 1 kernel: four for norder 8 while sF (8 n npw complex) leaves room for three blocks
+// per CU, else two
+int p2pwF3_slabs(int n, int npw) { return n == 8 && npw <= 48 ? 4 : 2; }
+
+// LDS of the STEP 1 kernels, the BF16 table included: the launchers and
+// pw2pot_3d_supported, which answers before anything is launched, ask the same
+size_t p2pw3_lds(int n, int npw, int prec) {
+    return sizeof(double2) * p2pw3_entries(n, npw) + (prec == 2 ? sizeof(BfPair) * x1_tab_entries(n, npw) : 0);
+}
+size_t p2pwF3_lds(int n, int npw, int prec) {
+    return sizeof(double2) * p2pwF3_entries(n, p2pwF3_slabs(n, npw), npw) +
+           (prec == 2 ? sizeof(BfPair) * x1_tab_entries(2 * n, npw) : 0);
+}
+
 template <int N>
 bool try_p2pw3(const Geom& g, const DevTables& t, int ntask, const int* box, const int* lev, const int* slot,
                const double* fvals, double2* expn, hipStream_t s, size_t lds_limit, const Multi& mu) {
-    const size_t lds = sizeof(double2) * p2pw3_entries(N, t.npw) +
-                       (t.prec == 2 ? sizeof(BfPair) * x1_tab_entries(N, t.npw) : 0);
+    const size_t lds = p2pw3_lds(N, t.npw, t.prec);
     if (lds > lds_limit) return false;
     float2* e32 = reinterpret_cast<float2*>(expn);
     if (t.prec == 2)
@@ -957,19 +970,13 @@ bool try_pw2pot3(const Geom& g, const DevTables& t, int nfam, int nown, const Sy
     return true;
 }
 
-// slabs per round of the fused STEP 1 kernel: four for norder 8 while sF (8 n npw complex) leaves room for three blocks
-// per CU, else two
-int p2pwF3_slabs(int n, const DevTables& t) {
-    return n == 8 && t.npw <= 48 ? 4 : 2;
-}
-
 template <int N>
 void launch_p2pwF3_typed(const Geom& g, const DevTables& t, unsigned nblk, size_t lds, const int* plev,
                          const int* pslot, const int* kids, const int* ksg, const double* fvals, double2* expn,
                          hipStream_t s, const Multi& mu) {
     float2* e32 = reinterpret_cast<float2*>(expn);
     if constexpr (N == 8) {
-        if (p2pwF3_slabs(N, t) == 4) {
+        if (p2pwF3_slabs(N, t.npw) == 4) {
             if (t.prec == 2)
                 hipLaunchKernelGGL((k_p2pwF3<N, 3, float2, 4>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS, t.npw, plev,
                                    pslot, kids, ksg, fvals, e32, mu);
@@ -1031,9 +1038,7 @@ bool p2pw_fused_3d(const Geom& g, const DevTables& t, int ntask, const int* plev
                    const Multi& mu) {
     if (g.ndim != 3 || ntask <= 0) return ntask <= 0;
     const int N = t.n;
-    const size_t sr = (size_t)p2pwF3_slabs(N, t);
-    const size_t lds = sizeof(double2) * p2pwF3_entries(N, (int)sr, t.npw) +
-                       (t.prec == 2 ? sizeof(BfPair) * x1_tab_entries(2 * N, t.npw) : 0);
+    const size_t lds = p2pwF3_lds(N, t.npw, t.prec);
     if (lds > t.lds_limit) return false;
     if ((long long)ntask * kFusedParts > 0x7fffffffLL) return false;
     const unsigned nblk = (unsigned)(ntask * kFusedParts);
@@ -1047,10 +1052,12 @@ bool p2pw_fused_3d(const Geom& g, const DevTables& t, int ntask, const int* plev
 
 bool pw2pot_3d_supported(const Geom& g, const DevTables& t) {
     if (g.ndim != 3 || (t.n != 8 && t.n != 12 && t.n != 16)) return false;
-    const size_t lds = std::max(pw2pot3_lds(t.n, t.npw, 2), pw2pot3_lds(t.n, t.npw, 3));
-    const size_t lds1 = sizeof(double2) * std::max(4 * (size_t)t.n * t.n, 4 * (size_t)t.n * t.npw);
-    const size_t lds2 = sizeof(double2) * std::max(8 * (size_t)t.n * t.n, 4 * (size_t)t.n * t.npw);
-    return lds <= t.lds_limit && lds1 <= t.lds_limit && lds2 <= t.lds_limit;
+    size_t need = std::max(pw2pot3_lds(t.n, t.npw, 2), pw2pot3_lds(t.n, t.npw, 3));
+    // (beyond kLowpMaxPw both steps stay in FP64 arithmetic)
+    if (t.npw <= kLowpMaxPw)
+        for (int prec = 1; prec <= 2; ++prec)
+            need = std::max({need, p2pw3_lds(t.n, t.npw, prec), p2pwF3_lds(t.n, t.npw, prec)});
+    return need <= t.lds_limit;
 }
 
 bool launch_pw2pot_3d_z(const Geom& g, const DevTables& t, int nfam, int nown, const SymTask* tasks,

@@ -39,6 +39,33 @@ def test_plane_kernels_take_few_plane_waves(shapes, n):
     assert all(shapes("plane", n, npw, LDS // 4) for npw in (1, 2, 3, 4, 5, 13))
 
 
+@pytest.mark.parametrize("n", [8, 12, 16])
+@pytest.mark.parametrize("npw", [13, 20, 47, 48, 49, 64, 80])
+def test_reduced_precision_asks_for_all_its_steps_need(shapes, n, npw):
+    """What a device must offer a block for reduced precision, step by step
+    from the kernels' layouts, and one byte less: accepted and refused (a
+    problem accepted with less fails at its first STEP 1)."""
+    slabs = 4 if n == 8 and npw <= 48 else 2
+    tiles = (2 * npw + 15) // 16   # column tiles of the BF16 STEP 1 tables, 64 pairs of 16 bytes per K step
+
+    def table(kn):
+        return 32 * 64 * tiles * ((kn + 15) // 16)
+    leaf = 16 * 4 * n * max(n, npw) + table(n)
+    family = 16 * 2 * slabs * n * max(2 * n, npw) + table(2 * n)
+    cols, ns = (1, 8) if n == 8 else (2, 4)
+    step5 = 8 * 64 * npw + 16 * ns * n * (2 * n + 1) + 64 * cols * max(8 * ((npw + 3) // 4), 32 * ((npw + 15) // 16))
+    need = max(leaf, family, step5)
+    assert shapes("lowp", n, npw, need) and not shapes("lowp", n, npw, need - 1)
+    assert need <= LDS
+
+
+@pytest.mark.parametrize("n,most", [(8, 141), (12, 141), (16, 141)])
+def test_reduced_precision_keeps_its_range(shapes, n, most):
+    """Accepted up to this many plane waves when a block's LDS was first
+    counted (FP64 x stage, two slabs); never fewer."""
+    assert all(shapes("lowp", n, npw, LDS) for npw in range(1, most + 1))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,eps,delta,nd,npw", [(16, 1e-3, 5.0, 1, 3), (13, 1e-6, 20.0, 2, 3), (16, 1e-9, 2.0, 2, 7),
                                                 (14, 1e-1, 1e3, 1, 3)])
