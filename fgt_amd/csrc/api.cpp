@@ -513,6 +513,34 @@ void step45_lists(fgt_solver& S) {
     S.h.pcs_sign = psg;
 }
 
+// Geometry of a plan on the current device, and whether the 3-D fast path and
+// its reduced-precision kernels cover it (t: n, npw and the LDS limit are set).
+void plan_shape(const fgt::Plan& P, fgt::Geom& g, fgt::DevTables& t, bool& fast3d, bool& lowp3d) {
+    const int ndim = P.ndim, n = P.n;
+    g.nd = P.nd;
+    g.ndim = ndim;
+    g.nx = ndim == 1 ? 1 : n;
+    g.ny = ndim == 3 ? n : 1;
+    g.nz = n;
+    g.px = ndim == 1 ? 1 : P.npw;
+    g.py = ndim == 3 ? P.npw : 1;
+    g.pz = P.nh;
+    g.npw = P.npw;
+    g.npbox = P.npbox;
+    g.nexp = P.nexp;
+    t.n = n;
+    t.npw = P.npw;
+    // device limit for the LDS-staged kernels
+    int dev = 0;
+    hcheck(hipGetDevice(&dev), "hipGetDevice");
+    int lds_max = 0;   // one attribute query (the full property struct is slow to fill)
+    hcheck(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev),
+           "hipDeviceGetAttribute");
+    t.lds_limit = static_cast<size_t>(lds_max);
+    fast3d = P.do_pw && fgt::sym3_supported(g, t);
+    lowp3d = fast3d && fgt::pw2pot_3d_supported(g, t);
+}
+
 void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, fgt::Plan* planned = nullptr,
                   int prec_mode = 0) {
     if (planned) {
@@ -525,25 +553,9 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
     const fgt::Plan& P = S.plan;
     const int ndim = P.ndim, n = P.n;
     fgt::Geom& g = S.geom;
-    g.nd = P.nd;
-    g.ndim = ndim;
-    g.nx = ndim == 1 ? 1 : n;
-    g.ny = ndim == 3 ? n : 1;
-    g.nz = n;
-    g.px = ndim == 1 ? 1 : P.npw;
-    g.py = ndim == 3 ? P.npw : 1;
-    g.pz = P.nh;
-    g.npw = P.npw;
-    g.npbox = P.npbox;
-    g.nexp = P.nexp;
-
-    // device limits for the LDS-staged kernels
-    int dev = 0;
-    hcheck(hipGetDevice(&dev), "hipGetDevice");
-    int lds_max = 0;   // one attribute query (the full property struct is slow to fill)
-    hcheck(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev),
-           "hipDeviceGetAttribute");
-    const size_t lds_limit = static_cast<size_t>(lds_max);
+    fgt::DevTables& t = S.tabs;
+    plan_shape(P, g, t, S.fast3d, S.lowp3d);
+    const size_t lds_limit = t.lds_limit;
     const size_t lds_p2pw = sizeof(double2) * ((size_t)P.npw * n + (size_t)g.nx * g.ny + (size_t)g.py * g.nx);
     const size_t lds_pw2pot = sizeof(double2) * ((size_t)n * P.npw + (size_t)g.nx * g.py);
     if (P.do_pw && (lds_p2pw > lds_limit || lds_pw2pot > lds_limit))
@@ -562,16 +574,10 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
         S.d_wms.upload(to_d2(P.wms));
         S.d_wm2l.upload(to_d2(P.wm2l));
     }
-    fgt::DevTables& t = S.tabs;
     t.p2pw = S.d_p2pw.as<double2>();
     t.pw2pot = S.d_pw2pot.as<double2>();
     t.pw2pot_ks = P.pw2pot_ks;
     t.loctab_ks = P.loctab_ks;
-    t.lds_limit = lds_limit;
-    t.n = n;
-    t.npw = P.npw;
-    S.fast3d = P.do_pw && fgt::sym3_supported(g, t);
-    S.lowp3d = S.fast3d && fgt::pw2pot_3d_supported(g, t);
     if (S.fast3d) compact_slots(S.plan);
     t.prec = mode_precision(prec_mode, P.eps, S.lowp3d);
     t.expn_f32 = t.prec > 0 ? 1 : 0;
@@ -2579,14 +2585,17 @@ size_t estimate_bytes(const fgt::Plan& P, int mode) {
     const fgt::TreeView& T = P.tree;
     const size_t io = 2 * sizeof(double) * (size_t)P.nd * P.npbox * P.nboxes;
     size_t slots = (size_t)P.nslots;
-    const bool fast = P.do_pw && P.ndim == 3 && (P.n == 8 || P.n == 12 || P.n == 16);
+    fgt::Geom g{};
+    fgt::DevTables t{};
+    bool fast = false, lowp = false;
+    plan_shape(P, g, t, fast, lowp);
     if (fast) {
         slots = 0;
         for (int l = P.nlevstart; l <= P.nlevels; ++l)
             for (int b = T.lfirst[l]; b <= T.llast[l]; ++b)
                 if (P.slot_of_box[b] >= 0 && (T.nchild[b] > 0 || l == P.nlevstart)) ++slots;
     }
-    const size_t elem = mode_precision(mode, P.eps, fast) > 0 ? sizeof(float2) : sizeof(double2);
+    const size_t elem = mode_precision(mode, P.eps, lowp) > 0 ? sizeof(float2) : sizeof(double2);
     const size_t expn = P.do_pw ? elem * 2 * (size_t)P.nd * P.nexp * (slots + 1) : 0;
     const size_t tabs = sizeof(double) * P.loctab.size() + 10 * sizeof(double2) * (P.p2pw.size() + P.pw2pot.size()) +
                         sizeof(int) * (P.dir_src.size() * 3 + P.locband.size() + 16 * (size_t)P.nboxes);
