@@ -75,6 +75,9 @@ struct fgt_solver {
     // 3-D fast path: STEP 4 folded into STEP 5 for leaves below the cutoff level
     bool fast3d = false;
     bool lowp3d = false;   // the reduced-precision kernels cover the problem as well
+    // the expansions and the STEP 4 / 5 lists are those of tabs.expn_f32 (not
+    // while they change, and not after a change that failed)
+    bool expn_ready = true;
     DBuf d_s5_sym;     // fgt::SymTask list of STEP 5
     int n_s5_fam = 0, n_s5_own = 0;   // families first, then single leaves
     DBuf d_p2pwS, d_fz_lev, d_fz_slot, d_fz_kids, d_fz_ksg;          // fused STEP 1+2 parents
@@ -957,6 +960,7 @@ void execute(fgt_solver& S, hipStream_t st, bool timed, bool fork_near = false,
     const fgt::DevTables& t = S.tabs;
     const double* fv = ov ? ov->fvals : S.d_fvals.as<double>();
     double2* ex = ov ? ov->expn : S.d_expn.as<double2>();
+    if (!S.expn_ready) throw std::runtime_error("the last change of precision failed: set the precision again");
     if (ov) timed = fork_near = false;
     hipEvent_t ev[8], evn[2];
     if (timed) {
@@ -1302,7 +1306,11 @@ struct fgt_batch {
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     bool use_graph = true;
+    bool ready = true;   // the classes match the solvers (not after a change of precision that failed)
     double last_ms = 0.0;
+    void check_ready() const {
+        if (!ready) throw std::runtime_error("the last change of precision failed: set the precision again");
+    }
     void drop_graph() {
         if (gexec) (void)hipGraphExecDestroy(gexec);
         if (graph) (void)hipGraphDestroy(graph);
@@ -2798,11 +2806,13 @@ int fgt_solver_set_precision(fgt_solver* s, int mode) {
         if (mode >= 1 && !s->lowp3d)
             throw std::invalid_argument("mixed precision needs the 3-D register-blocked path (ndim 3, norder 8/12/16)");
         const int f32 = mode >= 1 ? 1 : 0;
-        if (f32 != s->tabs.expn_f32) {
+        if (f32 != s->tabs.expn_f32 || !s->expn_ready) {
             hcheck(hipDeviceSynchronize(), "hipDeviceSynchronize");
+            s->expn_ready = false;
             alloc_expansions(*s, f32 ? sizeof(float2) : sizeof(double2));
             s->tabs.expn_f32 = f32;
             step45_lists(*s);
+            s->expn_ready = true;
         }
         s->tabs.prec = mode;
     });
@@ -2886,6 +2896,7 @@ int fgt_batch_set_precision(fgt_batch* b, int mode, double eps_min, int* nmixed)
         if (!b) throw std::invalid_argument("null batch");
         if (mode < 0 || mode > 3) throw std::invalid_argument("batch precision mode must be 0..3");
         int cnt = 0;
+        b->ready = false;
         for (auto& S : b->solvers) {
             const double eps = S->plan.eps;
             const bool ok = mode >= 1 && S->plan.do_pw && S->lowp3d && eps >= eps_min;
@@ -2904,6 +2915,7 @@ int fgt_batch_set_precision(fgt_batch* b, int mode, double eps_min, int* nmixed)
         std::stable_sort(b->loose.begin(), b->loose.end(), [&](int x, int y) {
             return b->solvers[x]->plan.nleaves > b->solvers[y]->plan.nleaves;
         });
+        b->ready = true;
         if (nmixed) *nmixed = cnt;
     });
 }
@@ -2929,6 +2941,7 @@ int fgt_batch_set_graph(fgt_batch* b, int on) {
 int fgt_batch_autotune(fgt_batch* b, int reps) {
     return guarded([&] {
         if (!b) throw std::invalid_argument("null batch");
+        b->check_ready();
         if (reps < 1 || reps > 100) throw std::invalid_argument("reps must be 1..100");
         batch_autotune(*b, reps);
     });
@@ -2948,6 +2961,7 @@ int fgt_batch_class_info(const fgt_batch* b, int k, int* info) {
 int fgt_batch_profile(fgt_batch* b) {
     return guarded([&] {
         if (!b) throw std::invalid_argument("null batch");
+        b->check_ready();
         hcheck(hipDeviceSynchronize(), "hipDeviceSynchronize");
         batch_chain_objects(*b);
         StageEvents prof;
@@ -2983,6 +2997,7 @@ int fgt_batch_class_members(const fgt_batch* b, int k, int* members) {
 int fgt_batch_execute(fgt_batch* b) {
     return guarded([&] {
         if (!b) throw std::invalid_argument("null batch");
+        b->check_ready();
         hipStream_t st = b->streams[0];
         // earlier work on any stream (uploads, other executes) comes first
         hcheck(hipDeviceSynchronize(), "hipDeviceSynchronize");

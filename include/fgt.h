@@ -156,7 +156,8 @@ int fgt_solver_set_ifpgh(fgt_solver *s, int ifpgh);
  * Modes 1 and 2 need the 3-D register-blocked path (ndim 3, norder
  * 8/12/16) and a plan that forms plane-wave expansions.  A mode the
  * solver's eps or shape does not allow returns status 2 and changes
- * nothing. */
+ * nothing.  A change that runs out of device memory leaves the solver without
+ * its expansions: executes fail until a mode has been set again. */
 int fgt_solver_set_precision(fgt_solver *s, int mode);
 /* device gradient / Hessian -> host (accumulate != 0 adds, reference +=);
  * status 2 when not requested by fgt_solver_set_ifpgh. */

@@ -32,7 +32,7 @@ def test_targets_after_a_request_beyond_the_memory():
     the next, smaller one gives the values it gave before."""
     import torch
     nd = 1024
-    tr = fgt_amd.vol_tree_build(3, 4, 0, 0, 1e-1, gauss_source(np.zeros((1, 3)), np.array([1e-2]), np.ones(1)))
+    tr = fgt_amd.vol_tree_build(3, 4, 0, 0, 1e-1, gauss_source(np.zeros((1, 3)), np.full((1, 3), 1e-2), np.ones(1)))
     s = fgt_amd.Solver.from_tree(tr, 1e-3, 1e-3, nd=nd)
     rng = np.random.default_rng(3)
     s.set_fvals(rng.uniform(-1, 1, tr.nboxes * tr.npbox * nd))
@@ -53,3 +53,19 @@ def test_targets_after_a_request_beyond_the_memory():
     after = s.eval_targets(targs)[0]
     assert np.array_equal(before, after)
     s.close()
+
+
+def test_nothing_runs_after_a_failed_change_of_precision(tmp_path):
+    g = gauss_source(np.array([[0.1, -0.2, 0.05]]), np.array([[4e-3, 7e-3, 5e-3]]), np.ones(1))
+    tr = fgt_amd.vol_tree_build(3, 8, 0, 0, 1e-3, g)
+    assert fgt_amd.plan_summary(tr, 1e-2, 1e-3)["npw_leaves"] > 0
+    with open(tmp_path / "problem", "wb") as f:
+        for a, dt in (([tr.nboxes, tr.nlevels, tr.ltree, tr.norder], np.int32), (tr.itree, np.int32),
+                      (tr.iptr, np.int32), (tr.centers, np.float64), (tr.boxsize, np.float64)):
+            f.write(np.ascontiguousarray(a, dt).tobytes())
+    exe, lib = str(tmp_path / "alloc_failures"), os.path.join(ROOT, "fgt_amd")
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-rdynamic", "-I/opt/rocm/include",
+                    "-I" + os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "csrc", "alloc_failures.cpp"),
+                    "-o", exe, "-L" + lib, "-lfgt_amd", "-Wl,-rpath," + lib, "-Wl,--allow-shlib-undefined"], check=True)
+    r = subprocess.run([exe, str(tmp_path / "problem")], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
