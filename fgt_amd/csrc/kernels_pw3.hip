@@ -227,26 +227,26 @@ __device__ __forceinline__ void x1_lowp(int npw, int lane, int ct0, int ctstep, 
 __host__ __device__ constexpr size_t p2pw3_entries(int n, int npw) {
     return 4 * (size_t)n * (npw > n ? npw : n);
 }
-template <int N, int XS, typename ET>
+template <int N, int XS>
 __global__ void __launch_bounds__(256) k_p2pw3(Geom g, const double2* __restrict__ tab_a, int npw,
                                               const int* __restrict__ box, const int* __restrict__ lev,
                                               const int* __restrict__ slot,
                                               const double* __restrict__ fvals_a,
-                                              ET* __restrict__ expn_a, Multi mu) {
+                                              float2* __restrict__ expn_a, Multi mu) {
     extern __shared__ double2 sm[];
     double2* sff = sm;
     double2* sff2 = sm;
     const int task = blockIdx.x;
     const double2* __restrict__ tab = tab_a;
     const double* __restrict__ fvals = fvals_a;
-    ET* __restrict__ expn = expn_a;
+    float2* __restrict__ expn = expn_a;
     if (mu.pp) {
         const ProbPtrs& q = mu.pp[mu.tprob[task]];
         g = q.g;
         npw = q.g.npw;
         tab = q.p2pw;
         fvals = q.fvals;
-        expn = static_cast<ET*>(q.expn);
+        expn = static_cast<float2*>(q.expn);
     }
     const int b = box[task], l = lev[task], sl = slot[task];
     const CTab2 T = ctab(tab) + (long long)l * npw * N;   // T[k][m]
@@ -263,7 +263,7 @@ __global__ void __launch_bounds__(256) k_p2pw3(Geom g, const double2* __restrict
             for (int m3 = 0; m3 < N; ++m3)
                 fr[m3] = fvals[((size_t)b * g.npbox + tid + N * N * m3) * nd + ind];
         }
-        ET* __restrict__ E = expn + ((size_t)sl * 2 * nd + ind) * g.nexp;
+        float2* __restrict__ E = expn + ((size_t)sl * 2 * nd + ind) * g.nexp;
         for (int r = 0; r < nh; r += 4) {
             // z: ff[s][m1][m2] = sum_m3 T[k3_s][m3] f[m1,m2,m3], thread = (m1,m2)
             if (tid < N * N) {
@@ -309,7 +309,7 @@ __global__ void __launch_bounds__(256) k_p2pw3(Geom g, const double2* __restrict
             {
                 const int k3 = r + wave;
                 if (k3 < nh) {
-                    ET* __restrict__ Ek = E + (size_t)k3 * npw * npw;
+                    float2* __restrict__ Ek = E + (size_t)k3 * npw * npw;
                     x1_lowp<N, XS>(
                         npw, lane, 0, 1,
                         [&](int k2, int m1) { return sff2[(wave * N + m1) * npw + k2]; },
@@ -347,12 +347,12 @@ constexpr int kFusedParts = 4;
 __host__ __device__ constexpr size_t p2pwF3_entries(int n, int sr, int npw) {
     return 2 * (size_t)sr * n * (npw > 2 * n ? npw : 2 * n);
 }
-template <int N, int XS, typename ET, int SR = 2>
+template <int N, int XS, int SR = 2>
 __global__ void __launch_bounds__(256) k_p2pwF3(Geom g, const double2* __restrict__ tabS_a, int npw,
                                                const int* __restrict__ plev, const int* __restrict__ pslot,
                                                const int* __restrict__ kids, const int* __restrict__ ksg,
                                                const double* __restrict__ fvals_a,
-                                               ET* __restrict__ expn_a, Multi mu) {
+                                               float2* __restrict__ expn_a, Multi mu) {
     static_assert(SR == 2 || (SR == 4 && N == 8 && XS >= 2), "four-slab rounds: norder 8, matrix-core x stage");
     extern __shared__ double2 sm[];
     double2* sH = sm;                     // 4*SR*N*N
@@ -361,14 +361,14 @@ __global__ void __launch_bounds__(256) k_p2pwF3(Geom g, const double2* __restric
     const int task = lin / kFusedParts, part = lin % kFusedParts;
     const double2* __restrict__ tabS = tabS_a;
     const double* __restrict__ fvals = fvals_a;
-    ET* __restrict__ expn = expn_a;
+    float2* __restrict__ expn = expn_a;
     if (mu.pp) {
         const ProbPtrs& q = mu.pp[mu.tprob[task]];
         g = q.g;
         npw = q.g.npw;
         tabS = q.p2pwS;
         fvals = q.fvals;
-        expn = static_cast<ET*>(q.expn);
+        expn = static_cast<float2*>(q.expn);
     }
     const int l = plev[task] + 1, sl = pslot[task];
     const int per = npw * N;
@@ -390,7 +390,7 @@ __global__ void __launch_bounds__(256) k_p2pwF3(Geom g, const double2* __restric
                        [&](int kk, int k1) { return kk >= N ? Txm[k1 * N + kk - N] : Txp[k1 * N + kk]; });
     }
     for (int ind = 0; ind < nd; ++ind) {
-        ET* __restrict__ E = expn + ((size_t)sl * 2 * nd + ind) * g.nexp;
+        float2* __restrict__ E = expn + ((size_t)sl * 2 * nd + ind) * g.nexp;
         // norder 8: one wave per group g = (sx, sy) of children; the values
         // of its (up to two) children -- the z sign tells them apart -- stay
         // in registers for every round
@@ -508,7 +508,7 @@ __global__ void __launch_bounds__(256) k_p2pwF3(Geom g, const double2* __restric
                 const int s = SR == 4 ? wave : (wave & 1), hlf = SR == 4 ? 0 : wave >> 1;
                 const int k3 = r + s;
                 if (k3 < nh) {
-                    ET* __restrict__ Ek = E + (size_t)k3 * npw * npw;
+                    float2* __restrict__ Ek = E + (size_t)k3 * npw * npw;
                     const CTab2 Txp = T + base0 + 1 * per;
                     const CTab2 Txm = T + base0 + 2 * per;
                     x1_lowp<2 * N, XS>(
@@ -897,10 +897,10 @@ bool try_p2pw3(const Geom& g, const DevTables& t, int ntask, const int* box, con
     if (lds > lds_limit) return false;
     float2* e32 = reinterpret_cast<float2*>(expn);
     if (t.prec == 2)
-        hipLaunchKernelGGL((k_p2pw3<N, 3, float2>), dim3(ntask), dim3(256), lds, s, g, t.p2pw, t.npw, box, lev, slot,
+        hipLaunchKernelGGL((k_p2pw3<N, 3>), dim3(ntask), dim3(256), lds, s, g, t.p2pw, t.npw, box, lev, slot,
                            fvals, e32, mu);
     else
-        hipLaunchKernelGGL((k_p2pw3<N, 2, float2>), dim3(ntask), dim3(256), lds, s, g, t.p2pw, t.npw, box, lev, slot,
+        hipLaunchKernelGGL((k_p2pw3<N, 2>), dim3(ntask), dim3(256), lds, s, g, t.p2pw, t.npw, box, lev, slot,
                            fvals, e32, mu);
     return true;
 }
@@ -978,19 +978,19 @@ void launch_p2pwF3_typed(const Geom& g, const DevTables& t, unsigned nblk, size_
     if constexpr (N == 8) {
         if (p2pwF3_slabs(N, t.npw) == 4) {
             if (t.prec == 2)
-                hipLaunchKernelGGL((k_p2pwF3<N, 3, float2, 4>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS, t.npw, plev,
+                hipLaunchKernelGGL((k_p2pwF3<N, 3, 4>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS, t.npw, plev,
                                    pslot, kids, ksg, fvals, e32, mu);
             else
-                hipLaunchKernelGGL((k_p2pwF3<N, 2, float2, 4>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS, t.npw, plev,
+                hipLaunchKernelGGL((k_p2pwF3<N, 2, 4>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS, t.npw, plev,
                                    pslot, kids, ksg, fvals, e32, mu);
             return;
         }
     }
     if (t.prec == 2)
-        hipLaunchKernelGGL((k_p2pwF3<N, 3, float2>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS, t.npw, plev, pslot,
+        hipLaunchKernelGGL((k_p2pwF3<N, 3>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS, t.npw, plev, pslot,
                            kids, ksg, fvals, e32, mu);
     else
-        hipLaunchKernelGGL((k_p2pwF3<N, 2, float2>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS, t.npw, plev, pslot,
+        hipLaunchKernelGGL((k_p2pwF3<N, 2>), dim3(nblk), dim3(256), lds, s, g, t.p2pwS, t.npw, plev, pslot,
                            kids, ksg, fvals, e32, mu);
 }
 
