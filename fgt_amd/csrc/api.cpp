@@ -570,7 +570,7 @@ void build_solver(fgt_solver& S, const fgt::PlanInput& in, bool own_io = true, f
     }
 
     S.d_loctab.upload(loctab_for(ndim, n, P.loctab));
-    S.d_locband.upload(P.locband);
+    if (!fgt::loctab_by_source(ndim, n)) S.d_locband.upload(P.locband);   // k_direct's
     if (P.do_pw) {
         S.d_p2pw.upload(to_d2(P.p2pw));
         S.d_pw2pot.upload(to_d2(P.pw2pot));
@@ -1119,14 +1119,15 @@ void execute(fgt_solver& S, hipStream_t st, bool timed, bool fork_near = false,
     }
 }
 
-// STEP 11 (extra targets, src/bfgt/boxfgt.f:1343-1378): values of the last
-// execute (device pot / grad / hess) -> coefficients on every leaf -> values
-// at the targets.  Targets are assigned to leaves on the host by the
-// reference's root-to-leaf descent (child bit a set when t_a - c_a >= 0,
-// find_childbox_ind, src/common/pts_tree_nd.f:713-740) and grouped by leaf.
 // per-solver target workspaces up to this size are kept between calls
 constexpr size_t kTargetWorkKept = size_t(32) << 20;
 
+// STEP 11 (extra targets, src/bfgt/boxfgt.f:1343-1378): values of the last
+// execute (device pot / grad / hess) at the targets.  The targets are grouped
+// by leaf on the device (kernels_targets.hip): each takes the reference's
+// root-to-leaf descent (child bit a set when t_a - c_a >= 0, find_childbox_ind,
+// src/common/pts_tree_nd.f:713-740), and a block per group of one leaf turns
+// the leaf's values into coefficients and evaluates them.
 void eval_targets(fgt_solver& S, int nt, const double* targs, int ifpghtarg, double* pote, double* grade,
                   double* hesse, hipStream_t st) {
     const fgt::Plan& P = S.plan;
@@ -2113,7 +2114,7 @@ struct Refiner {
                                    &band[(size_t)2 * n * nslot * l], &loccols[(size_t)2 * nslot * l],
                                    &tab[ks + per * l], &tab[2 * ks + per * l], 3);
         d_loctab.upload(loctab_for(P.ndim, n, tab));
-        d_locband.upload(band);
+        if (!fgt::loctab_by_source(P.ndim, n)) d_locband.upload(band);
         tr = S.tabs;
         tr.loctab = d_loctab.as<double>();
         tr.locband = d_locband.as<int>();
