@@ -227,7 +227,7 @@ struct DevTables {
     const double2* wms;
     const double2* wm2l;
     // near-field masked tables loc[kind][l][slot][k][j] ([j][k] where
-    // loctab_by_source), bands [l][slot][k][2];
+    // loctab_by_source), else with bands [l][slot][k][2];
     // loc_slots table slots per level (13 for the solve, 193 for the
     // refinement of a new tree); a pair's table slots are packed 8 bits per
     // kernel axis: x | y << 8 | z << 16
@@ -319,13 +319,20 @@ void launch_merge(const Geom& g, const DevTables& t, int ntask, const int* par_s
 // points at an all-zero slot, whose element offset is zero_off); scode[j] =
 // o | last << 5 with o = ox + 3 oy + 9 oz in 0..26 and last set on each
 // target's final entry.
-constexpr int kM2lGroup = 4;   // best at 4-5 with six blocks per CU (8 was best at four)
+// (2-D with entries in batches of two: 1062 targets x 16 densities 204 / 175 /
+// 176 / 180 / 187 us in groups of 1 / 2 / 4 / 5 / 8, 3184 targets 43 / 36 / 36 /
+// 41 / 49, periodic 2933 x 4 107 / 93 / 92 / 97 / 105)
+constexpr int kM2lGroup = 4;
 constexpr int kM2lGroupMax = 12;
 // targets per STEP 3 block of a problem with `blocks` targets x element
 // ranges: kM2lGroup, or one where even that leaves each CU fewer than sixteen
 // blocks (178 targets of 800 elements: 13 us in groups of four, now 9), or
 // FGT_M2L_GROUP (1..kM2lGroupMax, tuning runs)
 int m2l_group(long long blocks);
+// source loads per register batch (STEP 3 in groups and over bricks): the
+// grouped kernel keeps two batches in flight, and with four loads in each
+// measured the same or slower (2-D, 1062 / 3184 targets 19.8 -> 20.4 / 36.4 ->
+// 38.4 us; 3-D without bricks, 752 targets 158 -> 164)
 constexpr int kM2lBatch = 2;
 // longest entry stream of a group: kM2lGroupMax targets x (own + 26 list
 // entries), padded

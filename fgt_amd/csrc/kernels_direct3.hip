@@ -49,7 +49,9 @@ int direct_runs(const Multi& mu) {
 // wave-uniform address they keep the vector-memory counter for the values
 // and tables alone (read from global memory between the products, every step
 // waited for all loads in flight).  z group g of the chunk goes to team
-// g % TEAMS; a chunk's last entry closes its groups.
+// g % TEAMS; a chunk's last entry closes its groups.  (The lists of list 1 are
+// one chunk: a leaf has at most 26 colleagues, each a leaf or its 8 children,
+// itself, and 27 colleagues of its parent, 236 entries.)
 // flags per entry: bit0 = last of its (x,z) group, bit1 = last of its z group.
 constexpr int kChunk = 256;
 template <int TEAMS>
