@@ -59,13 +59,14 @@ def make_workload(seed=1, ng=20, n=16, eps=1e-9, delta=1e-4, iperiod=1):
 M2L_KERNEL = {0: "k_m2l27", 1: "k_m2l_brick", 2: "k_m2l_sep"}
 
 
-def stage_model(st, n, nd=1):
+def stage_model(st, tree, n, nd=1):
     """Algorithmic FLOPs and HBM bytes of one launch of the single-kernel stages.
 
     STEP 5 (k_pw2pot_sym, per PW leaf, 3-D): a quarter (the tables' symmetries) of
     4 n^3 nh + 8 n^2 npw nh + 8 n npw^2 nh flops (the x/y stages complex x
     complex, the last stage real output);
-    bytes: read one local expansion (16 nexp) + read/write pot (16 n^3).
+    bytes: one local expansion (16 nexp) per family of leaves below the cutoff
+    level and per leaf of that level, + read/write pot (16 n^3) per leaf.
     STEP 3 (k_m2l_sep / k_m2l_brick / k_m2l27, per cutoff-level box): 8 nexp flops per list entry; compulsory
     bytes: every cutoff-level mp read once and every loc written once,
     2 x 16 nexp per box (re-reads of a shared source are not algorithmic).
@@ -73,10 +74,12 @@ def stage_model(st, n, nd=1):
     npw, nexp = st["npw"], st["nexp"]
     nh = (npw + 1) // 2
     L = st["npw_leaves"]
+    below = tree.leaves[tree.level[tree.leaves] > st["npwlevel"]]
+    nread = len(set(tree.section(3)[below, 0])) + L - len(below)
     f15 = 4 * n ** 3 * nh + 8 * n * n * npw * nh + 8 * n * npw * npw * nh
     return {
         "pw2pot": {"kernel": "k_pw2pot_sym", "bound": "mfma", "flops": L * nd * f15 // 4,
-                   "bytes": L * nd * (16 * nexp + 16 * n ** 3)},
+                   "bytes": nd * (16 * nexp * nread + 16 * n ** 3 * L)},
         "m2l": {"kernel": M2L_KERNEL[st.get("m2l_form", 0)], "bound": "hbm",
                 "flops": 8 * nd * nexp * st["n_m2l_pairs"],
                 "bytes": 2 * 16 * nd * nexp * st["n_m2l_targets"]},
@@ -187,7 +190,8 @@ def batch_roofline(probs, prof):
     """Per class and stage: device ms of the profiled execute and the
     algorithmic work of that launch group; roofline of the longest one among
     STEP 1 (k_p2pw_sym, or k_p2pwF3 / k_p2pw3 in reduced precision), STEP 3
-    (k_m2l27) and STEP 5 (k_pw2pot_sym or k_pw2pot3).  STEP 1 and 5 flops: the
+    (k_m2l_brick, or k_m2l27 without bricks) and STEP 5 (k_pw2pot_sym or
+    k_pw2pot3).  STEP 1 and 5 flops: the
     reference's per-leaf count 4 n^3 nh + 8 n^2 npw nh + 8 n npw^2 nh (nh =
     (npw+1)/2) per plane-wave leaf of every member, a quarter of it where a
     stage goes through the tables' symmetries; STEP 3 bytes: every cutoff-level expansion read once and every local
@@ -580,7 +584,7 @@ def c2_leg(args):
     names = ["p2pw", "merge", "m2l", "split", "pw2pot", "direct"]
     stage = dict(zip(names, st2["stage_ms"][:6]))
     log("c2 stage ms: " + ", ".join(f"{k}={v:.3f}" for k, v in stage.items()))
-    model = stage_model(st2, n)
+    model = stage_model(st2, tree, n)
     dom = max(model, key=lambda k: stage[k])
     m = model[dom]
     secs = stage[dom] * 1e-3

@@ -177,7 +177,7 @@ __global__ void __launch_bounds__(kBlock) k_merge(Geom g, DevTables t, const int
 // group.  The 1-D phases are conj(z), 1, z for offsets 0, 1, 2, so the nine
 // products w_x w_y are a b, a conj(b), a, b, 1 (a = z[k1], b = z[k2]) or
 // their conjugates: five LDS rows, and a conjugate is an (exact) sign flip
-// of the imaginary part -- 20 KB of LDS per block instead of 36 KB, six
+// of the imaginary part -- 20 KB of LDS per block instead of 36 KB, seven
 // blocks per CU instead of four.  The group's entries (each target's own expansion first, then its
 // list) form one stream; source loads go kM2lBatch at a time into three
 // register batches, the batch two ahead issued before the current one is
@@ -396,8 +396,8 @@ __global__ void __launch_bounds__(kBrickBlock) k_m2l_brick(Geom g, DevTables t, 
     // for oz = 0, 1, 2 is conj(c), 1, c (the table's rows are exactly that),
     // read at a uniform row (5 with a sign flip, 4, 5) instead of selected
     // from registers per pair (STEP 3 at a norder-16 periodic problem 0.745
-    // -> 0.696 ms); six rows rather than eight leave room for six blocks per
-    // CU in LDS instead of four
+    // -> 0.696 ms, with one element per thread); 13 KB of LDS per block leave
+    // the blocks per CU to the registers (106 and 118: eight)
     __shared__ double2 s_fxy[6][kBrickBlock];
     const int tid = threadIdx.x;
     {
