@@ -1005,9 +1005,12 @@ int lowp_stages(int prec) {
         const char* e = std::getenv("FGT_LOWP_STAGES");
         return e ? (std::atoi(e) & 3) : -1;
     }();
-    // defaults: FP32 keeps STEP 1 on the VALU (its matrix-core form measured
-    // slower: 50 x 50-class outputs pad to 64-row / 16-column tiles with K = 8
-    // or 16); BF16 hi/lo runs both stages on the matrix cores
+    // defaults by mode: FP32 runs STEP 5's x stage on the matrix cores, BF16
+    // hi/lo both steps'.  The FP64 arithmetic of the symmetric kernels on FP32
+    // expansions is a quarter of the plain products, and at order 8 with up to
+    // 48 plane waves (35 problems in one launch) the faster one: STEP 1 2.0 ms
+    // against 4.4, STEP 5 2.7 against 3.7.  A batch's autotuner times both; a
+    // single solver keeps the arithmetic that its mode names.
     return v >= 0 ? v : (prec == 2 ? 3 : 2);
 }
 
